@@ -208,7 +208,8 @@ class _State:
     """A simulator and what its user reads after a call; closed with its last reference."""
 
     def __init__(self, case, seed):
-        net, self.probes, learned = _network(case, seed % (2 ** 31 - 1))
+        # `configs` multiplies the seed by up to 7919, and NumPy takes 32 bits of it
+        net, self.probes, learned = _network(case, seed % 500009)
         self.sim = Simulator(net, progress_bar=False)
         self.learned = [self.sim.model.sig[c]["weights"] for c in learned]
         self.steps = case["steps"]
