@@ -172,6 +172,140 @@ __global__ __launch_bounds__(NHIP_WG) void conv2d_kernel(const ConvGeom g, const
         Y[g.y_start + (size_t)k * g.ys_f + (size_t)i * g.ys_i + (size_t)j * g.ys_j] = out;
 }
 
+// The same convolution (channels last) for images with too few outputs to fill the device with
+// the tiles above.  A group is one wave: 16 filters x 4 consecutive pixels, an output per lane,
+// so a few thousand outputs spread over all compute units instead of sharing a few.  All taps
+// of the 16 filters and the windows of the 4 pixels are staged at once, every load of a lane in
+// flight before the first is stored (memory is about a microsecond away and little else is
+// running), in the order the sum walks them: LDS reads of the chain have constant offsets
+// and no address arithmetic.  Same order, channel, kernel row, kernel column, one fused
+// multiply-add each; taps outside the image multiply a zero, as the padded patch above does.
+// 26 x 26 x 32 -> 12 x 12 x 64 (9,216 outputs of 288 links) 28.4 -> 7.7 us, 46 x 46 x 40 -> 22 x 22 x 80
+// 41.8 -> 13.0, 128 x 128 x 32 -> 126 x 126 x 32 70.1 -> 45.1, 128 x 128 x 8 -> 126 x 126 x 64 (a
+// million outputs) 42.2 -> 41.0; below 64 links the tiles above are as fast or faster (46 x 46 x 3 ->
+// 44 x 44 x 40 6.2 against 8.2).  Bound by the one trip to memory and the chain.
+constexpr int CONV_WF = 16, CONV_WP = 4;
+constexpr int CONV_WAVE_PF = 24;          // loads in flight per lane
+constexpr int CONV_WAVE_LINKS = 16;       // chain links whose operands are read together
+constexpr int CONV_WAVE_MAX_LINKS = 800;  // 64,000 bytes of LDS
+constexpr int CONV_WAVE_MIN_LINKS = 64;
+constexpr long long CONV_WAVE_MAX_OUT = 1 << 20;
+
+// VEC: filters in whole aligned quads
+template <bool VEC>
+__global__ __launch_bounds__(NHIP_WAVE) void conv2d_wave_kernel(
+    const ConvGeom g, const float* __restrict__ X, const float* __restrict__ F, float* Y) {
+    extern __shared__ float4 lds4[];
+    const int lane = threadIdx.x;
+    const int taps = g.si * g.sj, n_links = taps * g.nc, n_pix = g.nyi * g.nyj;
+    const int k0 = blockIdx.y * CONV_WF, pix0 = blockIdx.x * CONV_WP;
+    float* wl = reinterpret_cast<float*>(lds4);  // [link][filter]
+    float* xl = wl + n_links * CONV_WF;          // [link][pixel]
+    constexpr int PF = CONV_WAVE_PF;
+    {   // taps: memory order is (tap, channel, filter)
+        const float inv_nc = __frcp_rn((float)g.nc);
+        constexpr int PER = VEC ? 4 : 1, LANES = CONV_WF / PER, ROWS = NHIP_WAVE / LANES;
+        const int q = PER * (lane % LANES), row = lane / LANES;
+        const float* f = F + g.f_start + k0;
+        const int qc = min(q, max(g.nf - k0 - PER, 0));  // (filters past the last are not stored)
+#pragma unroll 1
+        for (int m0 = row; m0 < n_links; m0 += ROWS * PF) {
+            float v[PF][PER];
+#pragma unroll
+            for (int u = 0; u < PF; ++u) {
+                const float* src = f + (size_t)min(m0 + u * ROWS, n_links - 1) * g.nf + qc;
+                if (VEC) {
+                    const float4 t = *reinterpret_cast<const float4*>(src);
+                    v[u][0] = t.x; v[u][PER > 1 ? 1 : 0] = t.y;
+                    v[u][PER > 1 ? 2 : 0] = t.z; v[u][PER > 1 ? 3 : 0] = t.w;
+                } else {
+                    v[u][0] = *src;
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < PF; ++u) {
+                const int m = m0 + u * ROWS;
+                int tap = (int)((float)m * inv_nc);  // m < 800: exact after one correction
+                if ((tap + 1) * g.nc <= m) ++tap;
+                if (tap * g.nc > m) --tap;
+                const int e = (m - tap * g.nc) * taps + tap;
+                if (m < n_links) {
+#pragma unroll
+                    for (int p = 0; p < PER; ++p) wl[e * CONV_WF + q + p] = v[u][p];
+                }
+            }
+        }
+    }
+    {   // windows: 16 lanes per pixel, each a channel of 16; (tap, run of 16 channels) in turn
+        const int p = lane >> 4, cl = lane & 15;
+        const int pix = min(pix0 + p, n_pix - 1);
+        const int i = pix / g.nyj, j = pix - i * g.nyj;
+        const int i0 = i * g.sti - g.pi, j0 = j * g.stj - g.pj;
+        const float* x = X + g.x_start;
+        const int runs = (g.nc + 15) >> 4, n_loads = taps * runs;
+        int t_i = 0, t_j = 0, run = 0;  // of the next load, the same for all lanes
+#pragma unroll 1
+        for (int l0 = 0; l0 < n_loads; l0 += PF) {
+            float v[PF];
+            int where[PF];
+#pragma unroll
+            for (int u = 0; u < PF; ++u) {
+                const int c = 16 * run + cl, ii = i0 + t_i, jj = j0 + t_j;
+                const bool in = (unsigned)ii < (unsigned)g.nxi && (unsigned)jj < (unsigned)g.nxj;
+                where[u] = (l0 + u < n_loads && c < g.nc)
+                               ? (c * taps + t_i * g.sj + t_j) * CONV_WP + p : -1;
+                const float t = x[in ? (ii * g.nxj + jj) * g.nc + min(c, g.nc - 1) : 0];
+                v[u] = in ? t : 0.0f;
+                ++run;
+                const bool next_tap = run == runs;
+                run = next_tap ? 0 : run;
+                t_j += next_tap ? 1 : 0;
+                const bool next_row = t_j == g.sj;
+                t_j = next_row ? 0 : t_j;
+                t_i += next_row ? 1 : 0;
+            }
+#pragma unroll
+            for (int u = 0; u < PF; ++u)
+                if (where[u] >= 0) xl[where[u]] = v[u];
+        }
+    }
+    __syncthreads();
+    const int kf = lane & (CONV_WF - 1), p = lane / CONV_WF;
+    const float* wp = wl + kf;
+    const float* xp = xl + p;
+    constexpr int U = CONV_WAVE_LINKS;
+    float out = 0.0f;
+    float wa[U], xa[U], wb[U], xb[U];
+    auto read = [&](float (&w)[U], float (&x)[U], int e) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            w[u] = wp[(e + u) * CONV_WF];
+            x[u] = xp[(e + u) * CONV_WP];
+        }
+    };
+    auto sum = [&](const float (&w)[U], const float (&x)[U]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) out = fmaf(w[u], x[u], out);
+    };
+    int e = 0;
+    if (n_links >= U) {
+        read(wa, xa, 0);
+#pragma unroll 1
+        for (; e + 3 * U <= n_links; e += 2 * U) {
+            read(wb, xb, e + U);
+            sum(wa, xa);
+            read(wa, xa, e + 2 * U);
+            sum(wb, xb);
+        }
+        sum(wa, xa);
+        e += U;
+    }
+#pragma unroll 4
+    for (; e < n_links; ++e) out = fmaf(wp[e * CONV_WF], xp[e * CONV_WP], out);
+    const int k = k0 + kf, pix = pix0 + p;
+    if (k < g.nf && pix < n_pix) Y[g.y_start + (size_t)pix * g.nf + k] = out;
+}
+
 struct PoolGeom {
     int nc, nyi, nyj, nxi, nxj, si, sj, sti, stj, x_start, y_start;
 };
@@ -239,6 +373,22 @@ extern "C" int nhip_conv2d(void* stream, const int* geom, const float* X, const 
     const size_t lds = ((size_t)g.c_chunk * (g.nipatch * g.njpatch + (g.local ? 0 : taps * g.tile_f)) +
                         taps) * sizeof(float);
     if (lds > 64 * 1024) return NHIP_E_BADARG;
+    const long long n_out = (long long)g.nyi * g.nyj * g.nf;
+    const size_t n_links = taps * g.nc;
+    if (g.f_fast && !g.local && n_out <= CONV_WAVE_MAX_OUT && n_links >= CONV_WAVE_MIN_LINKS &&
+        n_links <= CONV_WAVE_MAX_LINKS) {
+        const dim3 waves((g.nyi * g.nyj + CONV_WP - 1) / CONV_WP, (g.nf + CONV_WF - 1) / CONV_WF);
+        const size_t words = n_links * (CONV_WF + CONV_WP);
+        const bool vec = !((g.nf | g.f_start) & 3) && !(reinterpret_cast<uintptr_t>(F) & 15);
+        if (vec)
+            NHIP_LAUNCH(conv2d_wave_kernel<true>, waves, dim3(NHIP_WAVE), words * sizeof(float),
+                        NHIP_STREAM(stream), g, X, F, Y);
+        else
+            NHIP_LAUNCH(conv2d_wave_kernel<false>, waves, dim3(NHIP_WAVE), words * sizeof(float),
+                        NHIP_STREAM(stream), g, X, F, Y);
+        NHIP_LAUNCH_CHECK();
+        return 0;
+    }
     const dim3 grid(g.tiles_j * tiles_i, (g.nf + g.tile_f - 1) / g.tile_f);
     NHIP_LAUNCH(conv2d_kernel, grid, dim3(NHIP_WG), lds, NHIP_STREAM(stream), g, X, F, Y);
     NHIP_LAUNCH_CHECK();
