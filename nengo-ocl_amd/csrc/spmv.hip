@@ -143,99 +143,214 @@ __global__ __launch_bounds__(NHIP_WG) void spmv_sell_kernel(
 }
 
 // ---- products whose X is mostly zero (spikes) -------------------------------------------
-// One bit per element of X ("is not +0.0"), made by a launch of its own, is kept in LDS by
-// every work-group; for a stored element whose bit is clear the operand is the constant +0.0
+// One bit per element of X ("is not +0.0"), made by a launch of its own (or, for an X of at most
+// SPMV_MASK_INLINE_COLS elements, by every work-group for itself), is kept in LDS by every
+// work-group; for a stored element whose bit is clear the operand is the constant +0.0
 // instead of a look-up in the cache.  The sum is formed as above, term by term, so the
 // result has the bits of the kernel above whatever X and the matrix hold.  Groups are
-// persistent: 16 waves per group take slices s, s + (waves of the grid), ... until none is
-// left; SPMV_SKIP_U quads of a row are in flight per lane while the previous ones are summed.
+// persistent: the waves of a group take quarters of slices t, t + (waves of the grid), ... until none
+// is left.  A lane per row, each element's bit and look-up waited for on its own, was bound by
+// that chain: 2,000 rows of 100 took 20.9 us and now take 6.0, 100,000 rows of 100 39.6 us and
+// now 23.8 (4.1 of them the launch for the bits; the rest is 80 MB through the caches at
+// 4 TB/s).  Every group's own copy of the bits made from X costs 400 KB of reads per compute
+// unit at that size (29.3 us in all): hence the limit below.
 constexpr int SPMV_SKIP_WG = 1024;
 constexpr int SPMV_MASK_WORDS = 36864;  // 144 KiB of LDS: X of up to 1,179,648 elements
-constexpr int SPMV_SKIP_U = 4;
+constexpr int SPMV_MASK_U = 16;
+// X of at most so many elements: every group forms the bits itself, without a launch for them
+constexpr int SPMV_MASK_INLINE_COLS = 32768;
 
+// Sixteen rows of a slice by one wave, four lanes per row: lane j of a row holds its quads j,
+// j + 4, ..., U of them at a time, so a row of 100 elements is two requests deep instead of
+// the seven it takes a lane alone, and four times as many waves have requests in flight.  The sum
+// still runs through the row element by element: each quad's lane adds its four products to the
+// sum the quad before left, which reaches it by an exchange inside the four lanes.  All the
+// bits of a batch are read first, then all the elements of X that are needed, then it is
+// summed: a batch waits for memory twice and not once per element.  Stored elements past a row's
+// end are +0 times -0, which changes no sum.  (Past the last quad that one again, unused.)
+// ONE: every element of X that is not +0.0 is `one` (spikes of one amplitude): the bits are all
+// there is to know, and X is not looked up at all.
+template <int U, bool ONE>
+__device__ __forceinline__ float spmv_skip_rows(const spmv_i4* c, const spmv_f4* v, int n_quads,
+                                                int len, int j, const float* x,
+                                                const unsigned* s_mask, float one, float acc) {
+    auto request = [&](int q, spmv_i4 (&cq)[U], spmv_f4 (&vq)[U]) {
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const size_t at = (size_t)min(q + 4 * i + j, n_quads - 1) * NHIP_WAVE;
+            cq[i] = __builtin_nontemporal_load(c + at);
+            vq[i] = __builtin_nontemporal_load(v + at);
+        }
+    };
+    auto add = [&](int q, const spmv_i4 (&cq)[U], const spmv_f4 (&vq)[U]) {
+        unsigned word[U][4];
+        float xi[U][4];
+#pragma unroll
+        for (int i = 0; i < U; ++i)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) word[i][u] = s_mask[(unsigned)cq[i][u] >> 5];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < U; ++i)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const unsigned col = (unsigned)cq[i][u];
+                const bool stored = 4 * (q + 4 * i + j) + u < len;
+                const bool set = stored & ((word[i][u] >> (col & 31u)) & 1u);
+                xi[i][u] = stored ? 0.0f : -0.0f;
+                if (ONE) xi[i][u] = set ? one : xi[i][u];
+                else if (set) xi[i][u] = x[col];
+            }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            if (q + 4 * i >= n_quads) break;  // uniform
+            const bool mine = q + 4 * i + j < n_quads;  // (else: the last quad's values again)
+            float w[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) w[u] = mine ? vq[i][u] : 0.0f;
+#define SPMV_LINK(J, CTRL)                                                               \
+            {                                                                            \
+                _Pragma("unroll") for (int u = 0; u < 4; ++u) acc = fmaf(w[u], xi[i][u], acc); \
+                acc = __int_as_float(__builtin_amdgcn_update_dpp(                        \
+                    0, __float_as_int(acc), CTRL, 0xF, 0xF, true));                      \
+            }
+            SPMV_LINK(0, 0x00)  // the sum of lane 0 of the four to all of them, then lane 1's, ...
+            SPMV_LINK(1, 0x55)
+            SPMV_LINK(2, 0xAA)
+            SPMV_LINK(3, 0xFF)
+#undef SPMV_LINK
+        }
+    };
+    spmv_i4 ca[U], cb[U];
+    spmv_f4 va[U], vb[U];
+    request(0, ca, va);
+#pragma unroll 1
+    for (int q = 0; q < n_quads; q += 8 * U) {
+        if (n_quads > 4 * U) request(q + 4 * U, cb, vb);
+        __builtin_amdgcn_sched_barrier(0);
+        add(q, ca, va);
+        if (q + 4 * U >= n_quads) break;
+        request(q + 8 * U, ca, va);
+        __builtin_amdgcn_sched_barrier(0);
+        add(q + 4 * U, cb, vb);
+    }
+    return acc;
+}
+
+// smallest and largest bits of the elements of X that are not +0.0
+__device__ __forceinline__ void spmv_wave_range(unsigned& lo, unsigned& hi) {
+#pragma unroll
+    for (int off = NHIP_WAVE / 2; off > 0; off >>= 1) {
+        lo = min(lo, (unsigned)__shfl_xor((int)lo, off, NHIP_WAVE));
+        hi = max(hi, (unsigned)__shfl_xor((int)hi, off, NHIP_WAVE));
+    }
+}
+
+// n_words words of bits, then {smallest, largest} of every 64 elements
 __global__ __launch_bounds__(NHIP_WG) void spmv_mask_kernel(const float* __restrict__ X, int n,
                                                             unsigned* __restrict__ mask,
                                                             int n_words) {
     const int i = blockIdx.x * NHIP_WG + threadIdx.x;
     const unsigned bits = i < n ? __float_as_uint(X[i]) : 0u;
     const unsigned long long b = __ballot(bits != 0u);
+    unsigned lo = bits != 0u ? bits : 0xffffffffu, hi = bits;
+    spmv_wave_range(lo, hi);
     if ((threadIdx.x & (NHIP_WAVE - 1)) == 0 && 2 * (i >> 6) < n_words) {
         // (words past the last element of X, up to a multiple of 4, are written as zero)
         mask[2 * (i >> 6)] = (unsigned)b;
         mask[2 * (i >> 6) + 1] = (unsigned)(b >> 32);
+        mask[n_words + 2 * (i >> 6)] = lo;
+        mask[n_words + 2 * (i >> 6) + 1] = hi;
     }
 }
 
 __global__ __launch_bounds__(SPMV_SKIP_WG) void spmv_sell_skip_kernel(
     const SpmvSlice* __restrict__ slices, int n_slices, const int* __restrict__ row_len,
     const int* __restrict__ cols, const float* __restrict__ vals, const float* X, float* Y,
-    const unsigned* __restrict__ mask, int n_mask_quads, SpmvEpi epi, SpmvSide side)
+    const unsigned* __restrict__ mask, int x_start, int n_cols, SpmvEpi epi, SpmvSide side)
 {
-    constexpr int U = SPMV_SKIP_U;
     __shared__ __attribute__((aligned(16))) unsigned s_mask[SPMV_MASK_WORDS];
+    __shared__ unsigned s_range[2];
     if (side.n_chains > 0 && (int)blockIdx.x >= side.n_groups) return spmv_side_chain(side, s_mask);
-    for (int i = threadIdx.x; i < n_mask_quads; i += SPMV_SKIP_WG)
-        reinterpret_cast<spmv_i4*>(s_mask)[i] = reinterpret_cast<const spmv_i4*>(mask)[i];
-    __syncthreads();  // the only barrier; every thread reaches it
     const int lane = threadIdx.x & (NHIP_WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int stride = side.n_groups * (SPMV_SKIP_WG / NHIP_WAVE);
-    for (int s = blockIdx.x * (SPMV_SKIP_WG / NHIP_WAVE) + wave; s < n_slices; s += stride) {
+    constexpr int WAVES = SPMV_SKIP_WG / NHIP_WAVE;
+    // Quarters of slices are dealt out over the groups first and the waves of a group second: a
+    // product that does not fill the grid then keeps every compute unit busy.
+    const int stride = side.n_groups * WAVES;
+    unsigned lo = 0xffffffffu, hi = 0u;  // smallest and largest bits of a set element
+    if (threadIdx.x == 0) {
+        s_range[0] = lo;
+        s_range[1] = hi;
+    }
+    __syncthreads();
+    if (mask) {
+        const int n_mask_quads = (n_cols + 127) / 128;
+        const spmv_i4* ranges = reinterpret_cast<const spmv_i4*>(mask) + n_mask_quads;
+        for (int i = threadIdx.x; i < n_mask_quads; i += SPMV_SKIP_WG) {
+            reinterpret_cast<spmv_i4*>(s_mask)[i] = reinterpret_cast<const spmv_i4*>(mask)[i];
+            const spmv_i4 r = ranges[i];
+            lo = min(lo, min((unsigned)r[0], (unsigned)r[2]));
+            hi = max(hi, max((unsigned)r[1], (unsigned)r[3]));
+        }
+    } else {
+        // the bits straight from X: a wave forms one 64-bit word per 64 elements, the
+        // elements of SPMV_MASK_U words requested together
+        const unsigned* bits = reinterpret_cast<const unsigned*>(X + x_start);
+        const int n_words = (n_cols + NHIP_WAVE - 1) / NHIP_WAVE;
+#pragma unroll 1
+        for (int w0 = wave; w0 < n_words; w0 += WAVES * SPMV_MASK_U) {
+            unsigned e[SPMV_MASK_U];
+#pragma unroll
+            for (int j = 0; j < SPMV_MASK_U; ++j) {
+                const int i = (w0 + j * WAVES) * NHIP_WAVE + lane;
+                const unsigned b = bits[min(i, n_cols - 1)];
+                e[j] = i < n_cols ? b : 0u;
+            }
+#pragma unroll
+            for (int j = 0; j < SPMV_MASK_U; ++j) {
+                const unsigned long long b = __ballot(e[j] != 0u);
+                const int w = w0 + j * WAVES;
+                if (lane == 0 && w < n_words)
+                    reinterpret_cast<unsigned long long*>(s_mask)[w] = b;
+                lo = min(lo, e[j] != 0u ? e[j] : 0xffffffffu);
+                hi = max(hi, e[j]);
+            }
+        }
+    }
+    spmv_wave_range(lo, hi);
+    if (lane == 0) {
+        atomicMin(&s_range[0], lo);
+        atomicMax(&s_range[1], hi);
+    }
+    __syncthreads();  // every thread reaches it
+    // all set elements have the same bits (or there are none)
+    const bool one_value = s_range[0] >= s_range[1];
+    const float one = __uint_as_float(s_range[1]);
+    for (int t = wave * side.n_groups + blockIdx.x; t < 4 * n_slices; t += stride) {
+        const int s = t >> 2, row = 16 * (t & 3) + (lane >> 2), j = lane & 3;
         const SpmvSlice sl = slices[s];
-        const bool live = lane < sl.n_rows;
-        const int len = live ? row_len[sl.len_start + lane] : 0;
-        const float* x = X + sl.x_start;
-        float acc = (live && sl.inc) ? Y[(size_t)sl.y_start + lane] : 0.0f;
+        if (16 * (t & 3) >= sl.n_rows) continue;  // uniform: a short last slice
+        const bool live = row < sl.n_rows;
+        const int len = live ? row_len[sl.len_start + row] : 0;
+        float acc = (live && sl.inc) ? Y[(size_t)sl.y_start + row] : 0.0f;
         const int n_quads = sl.width >> 2;
-        const spmv_i4* c = reinterpret_cast<const spmv_i4*>(cols + (size_t)sl.data_start) + lane;
-        const spmv_f4* v = reinterpret_cast<const spmv_f4*>(vals + (size_t)sl.data_start) + lane;
-        spmv_i4 ci[U];
-        spmv_f4 vi[U];
-#pragma unroll
-        for (int j = 0; j < U; ++j) {
-            ci[j] = spmv_i4{0, 0, 0, 0};
-            vi[j] = spmv_f4{0.0f, 0.0f, 0.0f, 0.0f};
-            if (j < n_quads) {  // the same for all lanes
-                ci[j] = __builtin_nontemporal_load(c + (size_t)j * NHIP_WAVE);
-                vi[j] = __builtin_nontemporal_load(v + (size_t)j * NHIP_WAVE);
-            }
-        }
-        for (int q = 0; q < n_quads; q += U) {
-            // the next U quads are requested before the look-ups of the current ones
-            spmv_i4 cn[U];
-            spmv_f4 vn[U];
-#pragma unroll
-            for (int j = 0; j < U; ++j) {
-                cn[j] = ci[j];
-                vn[j] = vi[j];
-                if (q + U + j < n_quads) {
-                    cn[j] = __builtin_nontemporal_load(c + (size_t)(q + U + j) * NHIP_WAVE);
-                    vn[j] = __builtin_nontemporal_load(v + (size_t)(q + U + j) * NHIP_WAVE);
-                }
-            }
-            float xi[U][4];
-#pragma unroll
-            for (int j = 0; j < U; ++j)
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const unsigned col = (unsigned)ci[j][u];
-                    const bool set = (4 * (q + j) + u < len) && ((s_mask[col >> 5] >> (col & 31u)) & 1u);
-                    xi[j][u] = set ? x[col] : 0.0f;
-                }
-#pragma unroll
-            for (int j = 0; j < U; ++j)
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (4 * (q + j) + u < len) acc = fmaf(vi[j][u], xi[j][u], acc);
-#pragma unroll
-            for (int j = 0; j < U; ++j) {
-                ci[j] = cn[j];
-                vi[j] = vn[j];
-            }
-        }
-        if (live) {
-            Y[(size_t)sl.y_start + lane] = acc;
-            if (epi.slice_epi) spmv_filter_rows(epi, s, lane, acc);
+        const spmv_i4* c = reinterpret_cast<const spmv_i4*>(cols + (size_t)sl.data_start) + row;
+        const spmv_f4* v = reinterpret_cast<const spmv_f4*>(vals + (size_t)sl.data_start) + row;
+        const float* x = X + sl.x_start;
+        // (all of these conditions are the same for all lanes)
+        if (n_quads > 4 && one_value)
+            acc = spmv_skip_rows<4, true>(c, v, n_quads, len, j, x, s_mask, one, acc);
+        else if (n_quads > 4)
+            acc = spmv_skip_rows<4, false>(c, v, n_quads, len, j, x, s_mask, one, acc);
+        else if (n_quads > 0 && one_value)
+            acc = spmv_skip_rows<1, true>(c, v, n_quads, len, j, x, s_mask, one, acc);
+        else if (n_quads > 0)
+            acc = spmv_skip_rows<1, false>(c, v, n_quads, len, j, x, s_mask, one, acc);
+        if (live && j == 0) {
+            Y[(size_t)sl.y_start + row] = acc;
+            if (epi.slice_epi) spmv_filter_rows(epi, s, row, acc);
         }
     }
 }
@@ -273,7 +388,7 @@ int launch_plain(void* stream, const int* slices, int n_slices, const int* row_l
     return 0;
 }
 
-// Two launches: the bits of X, then the product.
+// The product, behind a launch for the bits of X where X is long.
 int launch_skip(void* stream, const int* slices, int n_slices, const int* row_len,
                 const int* cols, const float* vals, const float* X, float* Y, int x_start,
                 int n_cols, unsigned* mask, SpmvEpi epi) {
@@ -287,11 +402,15 @@ int launch_skip(void* stream, const int* slices, int n_slices, const int* row_le
          reinterpret_cast<uintptr_t>(mask)) & 15)
         return NHIP_E_BADARG;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int n_mask_quads = (n_cols + 127) / 128;        // 128 bits per 16 bytes
-    const int n_mask_threads = n_mask_quads * 128;        // one thread per bit, whole quads
-    NHIP_LAUNCH_FIRST(spmv_mask_kernel, dim3(n_mask_threads / NHIP_WG + (n_mask_threads % NHIP_WG != 0)),
-                dim3(NHIP_WG), 0, s, X + x_start, n_cols, mask, 4 * n_mask_quads);
-    NHIP_LAUNCH_CHECK();
+    const bool bits_in_kernel = n_cols <= SPMV_MASK_INLINE_COLS;
+    if (!bits_in_kernel) {
+        const int n_mask_quads = (n_cols + 127) / 128;        // 128 bits per 16 bytes
+        const int n_mask_threads = n_mask_quads * 128;        // one thread per bit, whole quads
+        NHIP_LAUNCH_FIRST(spmv_mask_kernel,
+                          dim3(n_mask_threads / NHIP_WG + (n_mask_threads % NHIP_WG != 0)),
+                          dim3(NHIP_WG), 0, s, X + x_start, n_cols, mask, 4 * n_mask_quads);
+        NHIP_LAUNCH_CHECK();
+    }
     static int n_cu = 0;
     if (n_cu == 0) {
         int dev = 0;
@@ -300,14 +419,19 @@ int launch_skip(void* stream, const int* slices, int n_slices, const int* row_le
             return NHIP_E_BADARG;
         n_cu = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
     }
-    const int wpg = SPMV_SKIP_WG / NHIP_WAVE;
     // a group takes a whole compute unit (its LDS holds the bits of X), so the groups of a
     // carried sequence need compute units of their own: with one product group per compute
     // unit they would only start when the product is over
-    side.n_groups = min(n_cu > side.n_chains ? n_cu - side.n_chains : n_cu, (n_slices + wpg - 1) / wpg);
-    NHIP_LAUNCH_LAST(spmv_sell_skip_kernel, dim3(side.n_groups + side.n_chains), dim3(SPMV_SKIP_WG), 0, s,
-                reinterpret_cast<const SpmvSlice*>(slices), n_slices, row_len, cols, vals, X, Y,
-                mask, n_mask_quads, epi, side);
+    side.n_groups = min(n_cu > side.n_chains ? n_cu - side.n_chains : n_cu, 4 * n_slices);
+    const dim3 grid(side.n_groups + side.n_chains);
+    if (bits_in_kernel)
+        NHIP_LAUNCH(spmv_sell_skip_kernel, grid, dim3(SPMV_SKIP_WG), 0, s,
+                    reinterpret_cast<const SpmvSlice*>(slices), n_slices, row_len, cols, vals, X, Y,
+                    nullptr, x_start, n_cols, epi, side);
+    else
+        NHIP_LAUNCH_LAST(spmv_sell_skip_kernel, grid, dim3(SPMV_SKIP_WG), 0, s,
+                         reinterpret_cast<const SpmvSlice*>(slices), n_slices, row_len, cols, vals,
+                         X, Y, mask, x_start, n_cols, epi, side);
     NHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -321,8 +445,8 @@ extern "C" int nhip_spmv_sell(void* stream, const int* slices, int n_slices, con
 
 // The product for an X that is mostly zero.  All slices must read the same X:
 // `n_cols` elements at X + x_start, n_cols <= 32 * SPMV_MASK_WORDS.  `mask` is a workspace
-// of (n_cols + 127) / 128 * 4 words that the call fills (one bit per element of X) and
-// then reads.  Two launches; events armed for the next launch time the first, short one.
+// of (n_cols + 127) / 128 * 8 words that the call may fill (one bit per element of X, and which
+// values the set ones span) and then read.  One launch, or two where X has more than SPMV_MASK_INLINE_COLS elements.
 extern "C" int nhip_spmv_sell_skip(void* stream, const int* slices, int n_slices,
                                    const int* row_len, const int* cols, const float* vals,
                                    const float* X, float* Y, int x_start, int n_cols,

@@ -20,6 +20,10 @@ WG, WAVE = 256, 64
 QUAD = 4  # elements of a row stored side by side (one 16-byte access)
 WINDOW = 1024  # consecutive elements of X a wave can keep in LDS (SPMV_WINDOW in csrc/spmv.hip)
 SKIP_MAX_COLS = 32 * 36864  # longest X whose "is not zero" bits fit the LDS (SPMV_MASK_WORDS)
+# ... and slices whose rows hold at least so many elements on average.  Measured (with the launch
+# for the bits / the ordinary one): 100,000 rows of 10 11.9 / 8.7 us, 10,000 of 20 5.2 / 4.0,
+# 30,000 of 50 8.4 / 11.0, 2,000 of 100 6.0 / 13.5, 100,000 of 100 23.8 / 58.4
+SKIP_MIN_WIDTH = 32
 
 
 def slice_window(columns, n_cols, x_start):
@@ -151,14 +155,15 @@ class plan_sparse_dot_inc:
         n_groups = max(1, -(-n // (WG // WAVE)))
         flags = np.broadcast_to(np.asarray(x_mostly_zero, dtype=bool), (len(matrices),))
         same_x = len({(int(X.starts[b]), int(X.shape0s[b])) for b in range(len(matrices))}) == 1
-        skip = n > 0 and bool(flags.all()) and same_x and int(X.shape0s[0]) <= SKIP_MAX_COLS
+        skip = (n > 0 and bool(flags.all()) and same_x and int(X.shape0s[0]) <= SKIP_MAX_COLS
+                and vals.size > SKIP_MIN_WIDTH * WAVE * n)
         if skip:
             n_cols = int(X.shape0s[0])
-            mask = to_device(queue, np.zeros(-(-n_cols // 128) * 4, dtype=np.int32))
+            mask = to_device(queue, np.zeros(-(-n_cols // 128) * 8, dtype=np.int32))
             dev.append(mask)
             entry = queue.lib.nhip_spmv_sell_skip
             args = args + (int(X.starts[0]), n_cols, mask.ptr)
-            gsize, lsize = (1024 * min(queue.n_compute_units, -(-n // 16)),), (1024,)
+            gsize, lsize = (1024 * min(queue.n_compute_units, 4 * n),), (1024,)
         else:
             entry, gsize, lsize = queue.lib.nhip_spmv_sell, (WG * n_groups,), (WG,)
         plan = Plan(queue, entry, args, gsize=gsize, lsize=lsize,

@@ -5,7 +5,7 @@ reference's order of summation, so the tolerance is zero)."""
 import numpy as np
 import pytest
 
-from helpers import RA, to_dev
+from helpers import RA, clone, to_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -40,3 +40,34 @@ def test_convolution_in_single_wave_groups(queue, rng, case):
         mod.plan_conv2d(q, d[[1]], d[[3]], d[[2]], (nxi, nxj, nc), (nyi, nyj, nf), (si, sj),
                         padding=padding, strides=(sti, stj), channels_last=True)()
     assert np.array_equal(dev.buf, data.buf)
+
+
+@pytest.mark.parametrize("rows,cols,per_row", [
+    (1, 1, 1), (17, 64, 12), (64 * 63 + 49, 65, 3), (64 * 256 + 1, 1000, 12), (300, 32768, 64),
+    (300, 32769, 130), (130, 900, 16), (97, 5000, 300)])
+def test_sparse_product_of_spikes_spread_over_the_device(queue, rng, monkeypatch, rows, cols,
+                                                         per_row):
+    """Fewer and more quarters of slices than waves of the device; rows of one quad to several
+    batches of them; the bits of X formed by the groups themselves (up to 32,768 elements) and
+    by a launch of their own; sums that are negative zeros."""
+    import scipy.sparse as sp
+
+    from nengo_ocl_amd import hipra_spmv
+    from oracle import oracle as orc
+
+    monkeypatch.setattr(hipra_spmv, "SKIP_MIN_WIDTH", 0)  # short rows too
+    mat = sp.random(rows, cols, density=min(1.0, per_row / cols), random_state=3, format="csr",
+                    dtype=np.float32)
+    X = RA([np.zeros(3), np.where(rng.uniform(size=cols) < 0.2, rng.normal(size=cols), 0.0)])
+    Y = RA([np.where(np.arange(rows) % 3 == 0, -0.0, rng.normal(size=rows))])
+    dX, dY, Yo = to_dev(queue, X), to_dev(queue, Y), clone(Y)
+    prog = hipra_spmv.plan_sparse_dot_inc(queue, [mat], dX[[1]], dY, inc=True, x_mostly_zero=True)
+    assert prog.plans[0].skips_zero_x
+    oplan = orc.plan_sparse_dot_inc(None, [mat], X[[1]], Yo, inc=True).plans[0]
+    # many values, one value (as spikes of one amplitude have), none, one negative value
+    for x in (X[1], 1000.0 * (X[1] != 0), 0.0 * X[1] + 0.0, -2.5 * (X[1] > 0) + 0.0):
+        X[1] = x
+        dX[1] = x
+        prog.plans[0]()
+        oplan()
+        assert np.array_equal(dY.buf.view(np.uint32), Yo.buf.view(np.uint32))
