@@ -47,6 +47,9 @@ const char *nhip_error_string(int err);
  * per work-group, gcn arch name (copied, NUL-terminated, into `name`). */
 int nhip_device_info(int *n_cu, int *wave_size, int *lds_bytes, char *name, int name_len);
 
+/* `lpr` of small-item launches in which a wave takes one row (see nhip_gemv) */
+#define NHIP_LPR_LONG_ROWS 128
+
 /* ---- ragged gather-GEMV ------------------------------------------------
  * For every output item b:
  *     Y[b] = beta_b * Yin[b] + gamma_b + alpha_b * sum_d  A[b,d] @ X[b,d]
@@ -78,7 +81,10 @@ int nhip_device_info(int *n_cu, int *wave_size, int *lds_bytes, char *name, int 
  * restatement of that kernel.  With lpr 64 (and 16-word task records) the launch is the
  * lpr 1 one with tasks of up to 64 consecutive rows of one item (n_rows <= 64) that a wave
  * takes whole, lane l the row row0 + l: the records are then read once per wave instead
- * of once per row, and the parts of an input sum are fetched by the lanes side by side.  `lpr` = lanes cooperating on one row (1,2,...,64, or
+ * of once per row, and the parts of an input sum are fetched by the lanes side by side.  With lpr
+ * NHIP_LPR_LONG_ROWS (16-word task records, one row each) a wave takes one row, four lanes per
+ * 128-column tile, and with lpr 256 a work-group: for launches of few rows of many columns
+ * (128 or more in every dot product, x_stride0 1).  `lpr` = lanes cooperating on one row (1,2,...,64, or
  * 256 for flavor 0); `vec` = 4 (16-byte loads; needs a_start % 4 == 0 and
  * a_stride0 % 4 == 0 for every dot of the launch) or 1.  `passes` (flavor 0) =
  * rows each lane accumulates at once, i.e. independent loads in flight: 2, 4, 8,

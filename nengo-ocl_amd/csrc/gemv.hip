@@ -301,10 +301,11 @@ int launch_rows_epi(hipStream_t s, int lpr, int task_words, const int* items, co
     if (n_tasks == 0) return 0;
     if (n_tasks < 0 || !items || !coefs || !dots || !tasks || !A || !X || !Yin || !Y)
         return NHIP_E_BADARG;
-    if (lpr != 4 && lpr != 1 && lpr != NHIP_WAVE) return NHIP_E_BADCLASS;
+    if (lpr != 4 && lpr != 1 && lpr != NHIP_WAVE && lpr != NHIP_LPR_LONG_ROWS && lpr != NHIP_WG) return NHIP_E_BADCLASS;
     if (task_words != 4 && task_words != 16) return NHIP_E_BADARG;
-    if (lpr == NHIP_WAVE && task_words != 16) return NHIP_E_BADARG;  // tasks of up to 64 rows
-    const int rows_per_group = (NHIP_WG / NHIP_WAVE) * (NHIP_WAVE / lpr);
+    if (lpr >= NHIP_WAVE && task_words != 16) return NHIP_E_BADARG;  // a wave per task
+    if (lpr >= NHIP_LPR_LONG_ROWS && EPI == EPI_LIF && epi.lif.sum_ranges) return NHIP_E_BADARG;
+    const int rows_per_group = lpr == NHIP_WG ? 1 : (NHIP_WG / NHIP_WAVE) * (lpr >= NHIP_WAVE ? 1 : NHIP_WAVE / lpr);
     side.n_gemv_groups = (n_tasks + rows_per_group - 1) / rows_per_group;
     const dim3 grid(side.n_gemv_groups + side.n_chains);
     auto launch = [&](auto kernel) {
@@ -315,6 +316,8 @@ int launch_rows_epi(hipStream_t s, int lpr, int task_words, const int* items, co
     auto pick = [&](auto side_tag) {
         constexpr bool SD = decltype(side_tag)::value;
         if (lpr == NHIP_WAVE) launch(gemv_rows_ref_epi_kernel<1, EPI, true, SD, true>);
+        else if (lpr == NHIP_LPR_LONG_ROWS) launch(gemv_rows_ref_epi_kernel<NHIP_WAVE, EPI, true, SD>);
+        else if (lpr == NHIP_WG) launch(gemv_rows_ref_epi_kernel<NHIP_WG, EPI, true, SD>);
         else if (lpr == 4 && task_words == 16) launch(gemv_rows_ref_epi_kernel<4, EPI, true, SD>);
         else if (lpr == 4) launch(gemv_rows_ref_epi_kernel<4, EPI, false, SD>);
         else if (task_words == 16) launch(gemv_rows_ref_epi_kernel<1, EPI, true, SD>);
@@ -429,10 +432,11 @@ extern "C" int nhip_gemv(void* stream, int flavor, int lpr, int vec, int passes,
             NHIP_WG_CASE(256)
         }
     } else if (flavor == 2) {
-        if ((lpr != 4 && lpr != 1 && lpr != NHIP_WAVE) || vec != 1) return NHIP_E_BADCLASS;
+        if ((lpr != 4 && lpr != 1 && lpr != NHIP_WAVE && lpr != NHIP_LPR_LONG_ROWS && lpr != NHIP_WG) || vec != 1)
+            return NHIP_E_BADCLASS;
         if (passes != 0 && passes != 16) return NHIP_E_BADARG;  // words of a task record
-        if (lpr == NHIP_WAVE && passes != 16) return NHIP_E_BADARG;  // tasks of up to 64 rows
-        const int rows_per_group = (NHIP_WG / NHIP_WAVE) * (NHIP_WAVE / lpr);
+        if (lpr >= NHIP_WAVE && passes != 16) return NHIP_E_BADARG;  // a wave per task
+        const int rows_per_group = lpr == NHIP_WG ? 1 : (NHIP_WG / NHIP_WAVE) * (lpr >= NHIP_WAVE ? 1 : NHIP_WAVE / lpr);
         side.n_gemv_groups = (n_tasks + rows_per_group - 1) / rows_per_group;
         const dim3 grid(side.n_gemv_groups + side.n_chains);
         auto launch = [&](auto kernel) {
@@ -444,6 +448,8 @@ extern "C" int nhip_gemv(void* stream, int flavor, int lpr, int vec, int passes,
         auto pick = [&](auto side_tag) {
             constexpr bool SD = decltype(side_tag)::value;
             if (lpr == NHIP_WAVE) launch(gemv_rows_ref_kernel<1, true, SD, true>);
+            else if (lpr == NHIP_LPR_LONG_ROWS) launch(gemv_rows_ref_kernel<NHIP_WAVE, true, SD>);
+            else if (lpr == NHIP_WG) launch(gemv_rows_ref_kernel<NHIP_WG, true, SD>);
             else if (lpr == 4 && passes == 16) launch(gemv_rows_ref_kernel<4, true, SD>);
             else if (lpr == 4) launch(gemv_rows_ref_kernel<4, false, SD>);
             else if (passes == 16) launch(gemv_rows_ref_kernel<1, true, SD>);

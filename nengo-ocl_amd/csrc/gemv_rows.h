@@ -15,6 +15,10 @@
 // :1148-1153): per 128-column tile four strided partial sums, one fused multiply-add
 // per element, (s0+s2)+(s1+s3), tiles in order onto beta*y_in, gamma last.
 //   LPR = 4: lane j of a row carries partial sum j; any number of columns.
+//   LPR = 64, 256: a wave, or the whole group, on one row: four lanes per 128-column tile, so
+//            sixteen tiles (64) side by side; the tile sums are then added in order.  For
+//            launches of few rows of many columns, where four lanes (or a wave of the
+//            large-item kernel that walks whole rows) would leave most of the device idle.
 //   LPR = 1: one lane per row, for items whose dot products all have <= 4 columns
 //            (vector sums, "scalar times vector" increments): the four partial sums are
 //            the (up to) four products themselves.
@@ -47,13 +51,13 @@ __device__ __forceinline__ void gemv_rows_ref_block(
     constexpr int TILE = 128;
     constexpr int BATCH = 4;             // dot products whose operands are fetched together
     constexpr int CHUNK = 8;             // steps of a partial sum whose operands are fetched together
-    constexpr int ROWS = NHIP_WAVE / LPR;  // rows (tasks) per wave
-    constexpr int PER_LANE = 4 / LPR;    // elements of a <= 4 column dot product per lane
+    constexpr int ROWS = LPR > NHIP_WAVE ? 1 : NHIP_WAVE / LPR;  // rows (tasks) per wave
+    constexpr int PER_LANE = LPR > 4 ? 1 : 4 / LPR;  // elements of a <= 4 column dot product per lane
     static_assert(!WAVE_TASK || (LPR == 1 && WIDE), "tasks of several rows: one lane per row, wide records");
     const int lane = tid & (NHIP_WAVE - 1);
-    const int lir = lane % LPR;
+    const int lir = LPR > NHIP_WAVE ? tid : lane % LPR;
     const int wave_slot = block * (NHIP_WG / NHIP_WAVE) + __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int slot = WAVE_TASK ? wave_slot : wave_slot * ROWS + lane / LPR;
+    const int slot = LPR > NHIP_WAVE ? block : WAVE_TASK ? wave_slot : wave_slot * ROWS + lane / LPR;
     bool valid = slot < n_tasks;
     GemvTask task;
     GemvItem it;
@@ -170,6 +174,60 @@ __device__ __forceinline__ void gemv_rows_ref_block(
     // the others use; the condition is the same for all of them)
     if (EPI == EPI_LIF && sum_range.y > 0 && (WAVE_TASK ? it.n_dots == 0 : n_dots == 0)) sum = summed(r);
 
+    if (LPR >= NHIP_WAVE) {
+        // Everything but the columns is the same for all lanes.  The operands of a lane's partial
+        // sum (the host has checked: at least 128 columns, stride 1) are 16 bytes apart: 32
+        // loads with constant offsets from one address.  The lanes of the last tile start as
+        // many steps early as it takes to end inside the row, and leave those steps out.
+        constexpr int STEPS = TILE / 4, TILES = NHIP_WAVE / 4;  // per wave and pass
+        constexpr int WAVES = LPR / NHIP_WAVE;                  // on one row
+        __shared__ float s_tiles[WAVES > 1 ? WAVES * TILES : 1];
+        const int my_wave = WAVES > 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) : 0;
+        const int n_dots_u = __builtin_amdgcn_readfirstlane(n_dots);
+        const int row_u = __builtin_amdgcn_readfirstlane(r);
+        const int dot_begin = __builtin_amdgcn_readfirstlane(it.dot_begin);
+        for (int d = 0; d < n_dots_u; ++d) {
+            const GemvDot dot = dots[dot_begin + d];
+            const int n_cols = dot.N;
+            const float* arow = A + dot.a_start + (size_t)row_u * dot.a_stride0;
+            const float* xg = X + dot.x_start;
+#pragma unroll 1
+            for (int c0 = 0; c0 < n_cols; c0 += WAVES * TILES * TILE) {
+                const int start = c0 + (my_wave * TILES + (lane >> 2)) * TILE + (lane & 3);
+                const int early = max((start + TILE - n_cols) >> 2, 0);
+                const int first = early < STEPS ? start - 4 * early : lane & 3;  // (nothing to sum)
+                float s = 0.0f;
+                if (c0 + my_wave * TILES * TILE < n_cols) {  // uniform
+                    float av[STEPS], xv[STEPS];
+#pragma unroll
+                    for (int e = 0; e < STEPS; ++e) {
+                        av[e] = arow[first + 4 * e];
+                        xv[e] = xg[first + 4 * e];
+                    }
+                    if (__any(early > 0)) {
+#pragma unroll
+                        for (int e = 0; e < STEPS; ++e) s = e >= early ? fmaf(av[e], xv[e], s) : s;
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < STEPS; ++e) s = fmaf(av[e], xv[e], s);
+                    }
+                    s = s + __shfl_xor(s, 2, NHIP_WAVE);
+                    s = s + __shfl_xor(s, 1, NHIP_WAVE);
+                }
+                const int n_tiles = min((n_cols - c0 + TILE - 1) / TILE, WAVES * TILES);
+                if (WAVES > 1) {
+                    if ((lane & 3) == 0) s_tiles[my_wave * TILES + (lane >> 2)] = s;
+                    __syncthreads();
+                    s = s_tiles[lane];  // tile `lane` of the pass
+                    __syncthreads();
+                }
+#pragma unroll 1
+                for (int t = 0; t < n_tiles; ++t)
+                    sum = sum + cf.x * __int_as_float(__builtin_amdgcn_readlane(
+                        __float_as_int(s), WAVES > 1 ? t : 4 * t));
+            }
+        }
+    } else
     for (int d0 = 0; __any(d0 < n_dots); d0 += BATCH) {
         GemvDot dot[BATCH];
         bool tiny = true;

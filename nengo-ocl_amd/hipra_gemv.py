@@ -94,6 +94,17 @@ WIDE_TASK_MAX_ROWS = 65536
 # measurements: "0" keeps a task record per row)
 WAVE_TASKS = os.environ.get("NENGO_HIP_WAVE_TASKS", "1") != "0"
 WG, WAVE = 256, 64
+# Launches of few rows of many columns: a wave per row (NHIP_LPR_LONG_ROWS), four lanes per
+# 128-column tile, instead of four lanes per row (up to 512 columns) or a wave that walks
+# whole rows.  Measured (kernel time, this / the other): 64 x 128 3.9 / 3.9 us, 1024 x 200
+# 3.9 / 4.4, 2048 x 384 3.9 / 6.0, 4096 x 384 5.3 / 6.1, 8192 x 256 7.6 / 4.9; 512 x 1000 3.9 / 4.8,
+# 2048 x 2048 6.1 / 7.0, 4096 x 1000 7.1 / 6.0, 1024 x 9216 13.1 / 17.0, 2048 x 4096 10.8 / 10.1.
+LONG_ROWS, LONG_ROW_MIN_COLS = 128, 160
+LONG_ROWS_MAX, LONG_ROWS_MAX_ELEMS, LONG_ROWS_ANY_WIDTH = 2048, 1 << 22, 1024
+# ... and a work-group per row where a row takes a wave several passes and the groups still fit
+# the device at once: 64 x 4096 4.1 us (a wave per row: 6.1), 10 x 9216 7.2 (10.1), 512 x 9216
+# 9.2 (10.8), 1024 x 4096 7.2 (6.5)
+GROUP_ROW_MIN_COLS, GROUP_ROWS_MAX = 2049, 512
 THIN_MIN_ROWS, THIN_ROWS_FOR_LANE_PER_ROW = 32, 65536
 LIF_POP_ENABLED, LIF_POP_DECAY, LIF_POP_NO_J = 1 << 8, 1 << 9, 1 << 10  # flag bits of a population row
 LIF_POP_BITS = 1 << 11  # spikes stored as a bit per neuron (see `store_spikes_as_bits`)
@@ -205,8 +216,11 @@ class gemv_prog:
     force_scalar = False  # one lane per output, 4-byte loads (the plain fallback)
 
     def __init__(self, queue, alpha, A, A_js, X, X_js, beta, Y, Y_in=None, gamma=0.0, tag=None,
-                 tile_items=(), event_items=()):
+                 tile_items=(), event_items=(), learned_items=()):
         self.queue = queue
+        # items whose matrix a learning rule writes: they stay with the large-item kernel, which
+        # can form the change while it streams the matrix (`fuse_learning`)
+        self.learned_items = frozenset(learned_items)
         self.tile_items = frozenset(tile_items)  # items that take the large-item kernel regardless
         # items whose X is mostly zero (spikes) and whose A nothing ever writes: candidates
         # for the launch that only visits the columns with x != 0 (`_event_item`)
@@ -379,6 +393,24 @@ class gemv_prog:
         else:
             lpr = min(WAVE, next_pow2(-(-n_max // vec)))
         return (flavor, lpr, vec)
+
+    def _long_rows(self, members):
+        """Are the items `members` of a launch few rows of many columns?"""
+        geometry = self.geometry
+        rows = sum(geometry[b]["y_len"] for b in members)
+        elems = sum(geometry[b]["y_len"] * d["a_shape1"]
+                    for b in members for d in geometry[b]["dots"])
+        return ((rows <= LONG_ROWS_ANY_WIDTH
+                 or rows <= LONG_ROWS_MAX and elems <= LONG_ROWS_MAX_ELEMS)
+                and not any(b in self.learned_items for b in members)
+                and all(geometry[b]["dots"] and all(
+                    d["a_shape1"] >= LONG_ROW_MIN_COLS and d["x_stride0"] == 1
+                    for d in geometry[b]["dots"]) for b in members))
+
+    def _lanes_of_long_rows(self, members):
+        widest = max(d["a_shape1"] for b in members for d in self.geometry[b]["dots"])
+        rows = sum(self.geometry[b]["y_len"] for b in members)
+        return WG if widest >= GROUP_ROW_MIN_COLS and rows <= GROUP_ROWS_MAX else LONG_ROWS
 
     def _event_item(self, g, any_size=False):
         """Does item `g` take the launch that visits only the columns with x != 0?  One
@@ -571,6 +603,19 @@ class gemv_prog:
             for members in by_class.values():
                 members.sort()
 
+        # a handful of long rows: the tiles of a row side by side over the lanes of a wave, for
+        # all items of the large-item launch, and for those of the small-item launch with them
+        large = [b for c in by_class if c[0] == 3 for b in by_class[c]]
+        small = by_class.get((2, 4, 1), [])
+        if self.force_flavor is None and not self.force_scalar:
+            for members in (large + small, large, small):
+                if members and self._long_rows(members):
+                    by_class = {c: [b for b in m if b not in set(members)]
+                                for c, m in by_class.items()}
+                    by_class = {c: m for c, m in by_class.items() if m}
+                    by_class[(2, self._lanes_of_long_rows(members), 1)] = sorted(members)
+                    break
+
         # the one instance of the compile-time-shape kernel that holds the stage widths of
         # all of them takes the items of several instances
         present = [c for c in by_class if c[0] == 3 and c[1] in STREAM_CLASS_STAGES]
@@ -641,7 +686,7 @@ class gemv_prog:
                 task_tab[:, 2] = 1
                 task_rows = task_tab
             task_tab = np.array(task_rows, dtype=np.int32)
-            if flavor == 2 and (0 < len(task_tab) <= WIDE_TASK_MAX_ROWS or lpr_arg == WAVE):
+            if flavor == 2 and (0 < len(task_tab) <= WIDE_TASK_MAX_ROWS or lpr_arg >= WAVE):
                 which = task_tab[:, 0]
                 wide = np.zeros((len(task_tab), 16), dtype=np.int32)
                 wide[:, 0:4] = task_tab
@@ -666,7 +711,8 @@ class gemv_prog:
             if flavor == 0:
                 n_groups = n_tasks
             elif flavor == 2:
-                n_groups = -(-n_tasks // ((WG // WAVE) * (WAVE // lpr_arg)))
+                n_groups = n_tasks if lpr_arg == WG else -(-n_tasks // (
+                    (WG // WAVE) * max(1, WAVE // lpr_arg)))
             else:
                 n_groups = -(-n_tasks // (WG // WAVE))
             tail = (dev_items.ptr, dev_coefs.ptr, dev_dots.ptr, dev_tasks.ptr, n_tasks, self.A.ptr,
@@ -679,7 +725,10 @@ class gemv_prog:
                 self.queue, kern, args, gsize=(WG * n_groups,), lsize=(WG,),
                 full_args=(dev_items, dev_coefs, dev_dots, dev_tasks, self.A.dev_buf,
                            self.X.dev_buf, self.Y_in.dev_buf, self.Y.dev_buf),
-                name="hipra_gemv.%s" % ("wg", "wave", "wave_ref", "tile")[flavor],
+                # (rows shared by a wave or a group: named after the items' ordinary launch)
+                name="hipra_gemv.%s" % (
+                    "tile" if flavor == 2 and lpr >= LONG_ROWS and not set(members) <= set(small)
+                    else ("wg", "wave", "wave_ref", "tile")[flavor]),
                 tag="%s-lpr%d-v%d" % (self.tag, lpr, vec),
                 bw_per_call=bw_from_geometry(geometry, members),
                 flops_per_call=flops_from_geometry(geometry, members),
@@ -912,7 +961,7 @@ def fuse_lif(prog, lif_plan, unread_currents=()):
             np.concatenate([prog.beta, np.ones(len(idle), np.float32)]),
             _concat([Y, extra]), Y_in=_concat([prog.Y_in, extra]),
             gamma=np.concatenate([prog.gamma, np.zeros(len(idle), np.float32)]), tag=prog.tag,
-            tile_items=range(n_old, n_old + len(idle)))
+            tile_items=range(n_old, n_old + len(idle)), learned_items=prog.learned_items)
         matched = matched + [(p, n_old + k) for k, p in enumerate(idle)]
         Y = prog.Y
 

@@ -222,12 +222,12 @@ def _can_carry(plan, needs=0):
         return getattr(plan, "prelude", None) is None and getattr(plan, "spmv", {}).get("n", 0) > 0
     if cls is None or getattr(plan, "prelude", None) is not None or getattr(plan, "n_tasks", 0) <= 0:
         return False
+    if cls[0] == 2:
+        return name in tuple("hipra_gemv." + k + e for k in ("wave_ref", "tile")
+                             for e in ("", "_lif", "_filter"))
     if name in ("hipra_gemv.tile_lif", "hipra_gemv.tile_filter"):
         return cls[0] == 3 and cls[1] >= 2
-    if name in ("hipra_gemv.events", "hipra_gemv.events_filter"):
-        return cls[0] == 4 and needs == 0
-    return name in ("hipra_gemv.wave_ref", "hipra_gemv.wave_ref_lif",
-                    "hipra_gemv.wave_ref_filter") and cls[0] == 2
+    return name in ("hipra_gemv.events", "hipra_gemv.events_filter") and cls[0] == 4 and needs == 0
 
 
 def carry_sequences(plans):

@@ -1402,6 +1402,12 @@ class Simulator:
         if len(constant_bs) != len(ops):
             raise NotImplementedError("signal-valued beta")
         extra = {}
+        written = {s.base for op2 in self.operators
+                   for s in list(op2.sets) + list(op2.incs) + list(op2.updates)}
+        if hasattr(self.backend, "event_driven_products"):
+            extra["learned_items"] = [
+                k for k, op in enumerate(constant_bs)
+                if any(sig.base in written for sig in self._A_views[op])]
         if getattr(self.backend, "event_driven_products", False) and not self.reference_host_state:
             # products of a constant matrix with the spikes of a population: only the columns
             # of the neurons that spiked need to be visited
@@ -1410,8 +1416,6 @@ class Simulator:
                       and type(op2.neurons).__name__ in SPIKING_NEURON_TYPES}
             # (populations a calibration run saw spiking too densely keep the dense product)
             spikes -= self._spike_sources_read_whole
-            written = {s.base for op2 in self.operators
-                       for s in list(op2.sets) + list(op2.incs) + list(op2.updates)}
             constant = lambda sig: getattr(sig.base, "readonly", False) and sig.base not in written
             extra["event_items"] = [
                 k for k, op in enumerate(constant_bs)

@@ -5,7 +5,7 @@ reference's order of summation, so the tolerance is zero)."""
 import numpy as np
 import pytest
 
-from helpers import RA, clone, to_dev
+from helpers import RA, clone, run_plans, to_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -71,3 +71,30 @@ def test_sparse_product_of_spikes_spread_over_the_device(queue, rng, monkeypatch
         prog.plans[0]()
         oplan()
         assert np.array_equal(dY.buf.view(np.uint32), Yo.buf.view(np.uint32))
+
+
+@pytest.mark.parametrize("widths", [
+    [512, 513, 639, 2047, 2048, 2049, 4095, 4096, 4097, 6145, 9216, 640, 8193],
+    [512, 513, 514, 515, 639, 2047, 2048, 1920, 1921, 1999, 2000, 640, 2046],
+    [160, 161, 162, 163, 255, 256, 257, 383, 384, 385, 511, 512, 200]],
+    ids=["group per row", "wave per row", "short rows"])
+@pytest.mark.parametrize("beta", [0.0, 1.0])
+def test_few_long_rows(queue, rng, beta, widths):
+    """Widths around the 128-column tiles and around the columns of one pass of a wave (2,048)
+    and of a group (8,192)."""
+    from nengo_ocl_amd import hipra_gemv
+    from oracle import oracle as orc
+
+    heights = [33, 1, 2, 17, 10, 3, 5, 40, 1, 2, 10, 70, 1]
+    A = RA([rng.normal(size=(m, n)) for m, n in zip(heights, widths)])
+    X = RA([rng.normal(size=n) for n in widths])
+    Y = RA([rng.normal(size=m) for m in heights])
+    A_js = RA([[k] for k in range(len(widths))], dtype=np.int32)
+    dA, dX, dY, Yo = to_dev(queue, A), to_dev(queue, X), to_dev(queue, Y), clone(Y)
+    args = lambda a, x: (1.5, a, A_js, x, A_js, beta)
+    prog = hipra_gemv.plan_block_gemv(queue, *args(dA, dX), dY, gamma=0.25)
+    long_rows = [p for p in prog.plans if p.kernel_class[:2] in ((2, hipra_gemv.LONG_ROWS), (2, 256))]
+    assert long_rows == prog.plans and len(long_rows) == 1
+    run_plans(prog.plans)
+    orc.plan_block_gemv(None, *args(A, X), Yo, gamma=0.25).plans[0]()
+    assert np.array_equal(dY.buf.view(np.uint32), Yo.buf.view(np.uint32))
