@@ -342,11 +342,10 @@ int nhip_gemv_events(void *stream, const int *items, int n_items, const float *A
 /* The same product for an X that is mostly zero (the spikes of a population; no
  * counterpart in the reference, whose kernels multiply every stored element).  All slices
  * read one X of `n_cols` elements at X + x_start (n_cols <= 1,179,648).  `mask` is a
- * workspace of (n_cols + 127) / 128 * 8 words, 16-byte aligned, that the call may fill with one
- * bit per element of X ("is not +0.0") and the values the others span in a first launch (an X
- * of at most 32,768 elements needs none: the groups of the product form the bits themselves);
- * the product keeps the bits in LDS and takes the constant +0.0 instead of reading X where the
- * bit is clear, and where all the others are one value, that value.  Bit-identical to
+ * workspace of (n_cols + 127) / 128 * 4 words, 16-byte aligned, that the call may fill with one
+ * bit per element of X ("is not +0.0") in a first launch (an X of at most 32,768 elements needs
+ * none: the groups of the product form the bits themselves); the product keeps the bits in LDS
+ * and takes the constant +0.0 instead of reading X where the bit is clear.  Bit-identical to
  * nhip_spmv_sell whatever X and the matrices hold.  NHIP_E_TOOBIG when X is longer than the
  * limit. */
 int nhip_spmv_sell_skip(void *stream, const int *slices, int n_slices, const int *row_len,
@@ -367,6 +366,14 @@ int nhip_spmv_sell_filter(void *stream, const int *slices, int n_slices, const i
                           const int *cols, const float *vals, const float *X, float *Y,
                           const int *slice_epi, const int *targets, float *F, int x_start,
                           int n_cols, unsigned *mask);
+
+/* nhip_spmv_sell_skip (slice_epi NULL) or nhip_spmv_sell_filter for an X whose elements other
+ * than +0.0 are usually all one value (spikes): where they are, that value is used and X is
+ * not read at all.  `ranges`: a second workspace of the size and alignment of `mask`. */
+int nhip_spmv_sell_spikes(void *stream, const int *slices, int n_slices, const int *row_len,
+                          const int *cols, const float *vals, const float *X, float *Y,
+                          const int *slice_epi, const int *targets, float *F, int x_start,
+                          int n_cols, unsigned *mask, unsigned *ranges);
 
 /* ---- neurons -----------------------------------------------------------
  * LIF with refractory state and spike-time interpolation.

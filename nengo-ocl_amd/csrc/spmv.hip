@@ -247,9 +247,10 @@ __device__ __forceinline__ void spmv_wave_range(unsigned& lo, unsigned& hi) {
     }
 }
 
-// n_words words of bits, then {smallest, largest} of every 64 elements
+// a bit per element; with `ranges` also {smallest, largest} bits of the set ones of every 64
 __global__ __launch_bounds__(NHIP_WG) void spmv_mask_kernel(const float* __restrict__ X, int n,
                                                             unsigned* __restrict__ mask,
+                                                            unsigned* __restrict__ ranges,
                                                             int n_words) {
     const int i = blockIdx.x * NHIP_WG + threadIdx.x;
     const unsigned bits = i < n ? __float_as_uint(X[i]) : 0u;
@@ -260,15 +261,18 @@ __global__ __launch_bounds__(NHIP_WG) void spmv_mask_kernel(const float* __restr
         // (words past the last element of X, up to a multiple of 4, are written as zero)
         mask[2 * (i >> 6)] = (unsigned)b;
         mask[2 * (i >> 6) + 1] = (unsigned)(b >> 32);
-        mask[n_words + 2 * (i >> 6)] = lo;
-        mask[n_words + 2 * (i >> 6) + 1] = hi;
+        if (ranges) {
+            ranges[2 * (i >> 6)] = lo;
+            ranges[2 * (i >> 6) + 1] = hi;
+        }
     }
 }
 
 __global__ __launch_bounds__(SPMV_SKIP_WG) void spmv_sell_skip_kernel(
     const SpmvSlice* __restrict__ slices, int n_slices, const int* __restrict__ row_len,
     const int* __restrict__ cols, const float* __restrict__ vals, const float* X, float* Y,
-    const unsigned* __restrict__ mask, int x_start, int n_cols, SpmvEpi epi, SpmvSide side)
+    const unsigned* __restrict__ mask, const unsigned* __restrict__ ranges, int x_start, int n_cols,
+    SpmvEpi epi, SpmvSide side)
 {
     __shared__ __attribute__((aligned(16))) unsigned s_mask[SPMV_MASK_WORDS];
     __shared__ unsigned s_range[2];
@@ -287,10 +291,11 @@ __global__ __launch_bounds__(SPMV_SKIP_WG) void spmv_sell_skip_kernel(
     __syncthreads();
     if (mask) {
         const int n_mask_quads = (n_cols + 127) / 128;
-        const spmv_i4* ranges = reinterpret_cast<const spmv_i4*>(mask) + n_mask_quads;
+        if (!ranges) { lo = 0u; hi = 0xffffffffu; }  // values not known: look-ups
         for (int i = threadIdx.x; i < n_mask_quads; i += SPMV_SKIP_WG) {
             reinterpret_cast<spmv_i4*>(s_mask)[i] = reinterpret_cast<const spmv_i4*>(mask)[i];
-            const spmv_i4 r = ranges[i];
+            if (!ranges) continue;
+            const spmv_i4 r = reinterpret_cast<const spmv_i4*>(ranges)[i];
             lo = min(lo, min((unsigned)r[0], (unsigned)r[2]));
             hi = max(hi, max((unsigned)r[1], (unsigned)r[3]));
         }
@@ -391,7 +396,7 @@ int launch_plain(void* stream, const int* slices, int n_slices, const int* row_l
 // The product, behind a launch for the bits of X where X is long.
 int launch_skip(void* stream, const int* slices, int n_slices, const int* row_len,
                 const int* cols, const float* vals, const float* X, float* Y, int x_start,
-                int n_cols, unsigned* mask, SpmvEpi epi) {
+                int n_cols, unsigned* mask, unsigned* ranges, SpmvEpi epi) {
     SpmvSide side = take_side();
     if (n_slices == 0) return side.n_chains > 0 ? NHIP_E_BADARG : 0;  // nothing to ride in
     if (n_slices < 0 || !slices || !row_len || !cols || !vals || !X || !Y || !mask || x_start < 0 ||
@@ -399,7 +404,7 @@ int launch_skip(void* stream, const int* slices, int n_slices, const int* row_le
         return NHIP_E_BADARG;
     if (n_cols > 32 * SPMV_MASK_WORDS) return NHIP_E_TOOBIG;
     if ((reinterpret_cast<uintptr_t>(cols) | reinterpret_cast<uintptr_t>(vals) |
-         reinterpret_cast<uintptr_t>(mask)) & 15)
+         reinterpret_cast<uintptr_t>(mask) | reinterpret_cast<uintptr_t>(ranges)) & 15)
         return NHIP_E_BADARG;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool bits_in_kernel = n_cols <= SPMV_MASK_INLINE_COLS;
@@ -408,7 +413,8 @@ int launch_skip(void* stream, const int* slices, int n_slices, const int* row_le
         const int n_mask_threads = n_mask_quads * 128;        // one thread per bit, whole quads
         NHIP_LAUNCH_FIRST(spmv_mask_kernel,
                           dim3(n_mask_threads / NHIP_WG + (n_mask_threads % NHIP_WG != 0)),
-                          dim3(NHIP_WG), 0, s, X + x_start, n_cols, mask, 4 * n_mask_quads);
+                          dim3(NHIP_WG), 0, s, X + x_start, n_cols, mask, ranges,
+                          4 * n_mask_quads);
         NHIP_LAUNCH_CHECK();
     }
     static int n_cu = 0;
@@ -427,11 +433,11 @@ int launch_skip(void* stream, const int* slices, int n_slices, const int* row_le
     if (bits_in_kernel)
         NHIP_LAUNCH(spmv_sell_skip_kernel, grid, dim3(SPMV_SKIP_WG), 0, s,
                     reinterpret_cast<const SpmvSlice*>(slices), n_slices, row_len, cols, vals, X, Y,
-                    nullptr, x_start, n_cols, epi, side);
+                    nullptr, nullptr, x_start, n_cols, epi, side);
     else
         NHIP_LAUNCH_LAST(spmv_sell_skip_kernel, grid, dim3(SPMV_SKIP_WG), 0, s,
                          reinterpret_cast<const SpmvSlice*>(slices), n_slices, row_len, cols, vals,
-                         X, Y, mask, x_start, n_cols, epi, side);
+                         X, Y, mask, ranges, x_start, n_cols, epi, side);
     NHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -445,14 +451,30 @@ extern "C" int nhip_spmv_sell(void* stream, const int* slices, int n_slices, con
 
 // The product for an X that is mostly zero.  All slices must read the same X:
 // `n_cols` elements at X + x_start, n_cols <= 32 * SPMV_MASK_WORDS.  `mask` is a workspace
-// of (n_cols + 127) / 128 * 8 words that the call may fill (one bit per element of X, and which
-// values the set ones span) and then read.  One launch, or two where X has more than SPMV_MASK_INLINE_COLS elements.
+// of (n_cols + 127) / 128 * 4 words that the call may fill with one bit per element of X and then
+// read.  One launch, or two where X has more than SPMV_MASK_INLINE_COLS elements.
 extern "C" int nhip_spmv_sell_skip(void* stream, const int* slices, int n_slices,
                                    const int* row_len, const int* cols, const float* vals,
                                    const float* X, float* Y, int x_start, int n_cols,
                                    unsigned* mask) {
     return launch_skip(stream, slices, n_slices, row_len, cols, vals, X, Y, x_start, n_cols, mask,
-                       SpmvEpi{});
+                       nullptr, SpmvEpi{});
+}
+
+// The same, with filters (slice_epi != nullptr) or without, and with `ranges`, a second workspace of
+// the size of `mask`, for the values that the set elements of an X of more than
+// SPMV_MASK_INLINE_COLS elements span: without it such an X is always looked up.
+extern "C" int nhip_spmv_sell_spikes(void* stream, const int* slices, int n_slices,
+                                     const int* row_len, const int* cols, const float* vals,
+                                     const float* X, float* Y, const int* slice_epi,
+                                     const int* targets, float* F, int x_start, int n_cols,
+                                     unsigned* mask, unsigned* ranges) {
+    if (!ranges || (slice_epi && (!targets || !F))) return NHIP_E_BADARG;
+    const SpmvEpi epi = slice_epi ? SpmvEpi{reinterpret_cast<const int4*>(slice_epi),
+                                            reinterpret_cast<const FilterTarget*>(targets), F}
+                                  : SpmvEpi{};
+    return launch_skip(stream, slices, n_slices, row_len, cols, vals, X, Y, x_start, n_cols, mask,
+                       ranges, epi);
 }
 
 // Either product with first-order filters stepped on its fresh rows: `slice_epi` holds
@@ -469,6 +491,6 @@ extern "C" int nhip_spmv_sell_filter(void* stream, const int* slices, int n_slic
                       reinterpret_cast<const FilterTarget*>(targets), F};
     if (mask)
         return launch_skip(stream, slices, n_slices, row_len, cols, vals, X, Y, x_start, n_cols,
-                           mask, epi);
+                           mask, nullptr, epi);
     return launch_plain(stream, slices, n_slices, row_len, cols, vals, X, Y, epi);
 }

@@ -109,7 +109,7 @@ class plan_sparse_dot_inc:
     ``x_mostly_zero`` (one flag, or one per matrix) says that X is zero in most places
     most of the time -- the spikes of a population.  When it holds for every matrix and all
     read the same X of at most `SKIP_MAX_COLS` elements, the launch is
-    `nhip_spmv_sell_skip`: one bit per element of X ("is not +0.0") is made first and kept
+    `nhip_spmv_sell_spikes`: one bit per element of X ("is not +0.0") is made first and kept
     in LDS, and where it is clear the operand is the constant instead of a look-up of X.
     Same bits as the ordinary launch whatever X holds; only faster when X is mostly zero.
     """
@@ -159,10 +159,12 @@ class plan_sparse_dot_inc:
                 and vals.size > SKIP_MIN_WIDTH * WAVE * n)
         if skip:
             n_cols = int(X.shape0s[0])
-            mask = to_device(queue, np.zeros(-(-n_cols // 128) * 8, dtype=np.int32))
-            dev.append(mask)
-            entry = queue.lib.nhip_spmv_sell_skip
-            args = args + (int(X.starts[0]), n_cols, mask.ptr)
+            # a bit per element of X; the values that the set ones span
+            mask, ranges = (to_device(queue, np.zeros(-(-n_cols // 128) * 4, dtype=np.int32))
+                            for _ in range(2))
+            dev += [mask, ranges]
+            entry = queue.lib.nhip_spmv_sell_spikes
+            args = args + (None, None, None, int(X.starts[0]), n_cols, mask.ptr, ranges.ptr)
             gsize, lsize = (1024 * min(queue.n_compute_units, 4 * n),), (1024,)
         else:
             entry, gsize, lsize = queue.lib.nhip_spmv_sell, (WG * n_groups,), (WG,)
@@ -171,7 +173,7 @@ class plan_sparse_dot_inc:
         plan.skips_zero_x = skip
         # what `fuse_linearfilter` needs to rebuild the launch with filters behind its rows
         plan.spmv = dict(X=X, Y=Y, slice_rows=slice_rows, dev=tuple(dev), n=n,
-                         mask=(mask if skip else None),
+                         workspaces=(mask, ranges) if skip else (),
                          x_start=int(X.starts[0]) if skip else 0,
                          n_cols=int(X.shape0s[0]) if skip else 0)
         nnz = int(sum(m.csr.nnz for m in matrices))
@@ -299,10 +301,12 @@ def fuse_linearfilter(spmv_plan, lf_plan):
             slice_epi[k] = (first[item][0], first[item][1], row0, 0)
     dev_epi = to_device(queue, slice_epi)
     dev_targets = to_device(queue, np.array(target_rows, dtype=np.int32))
-    mask = sp["mask"]
-    args = tuple(spmv_plan.args[:7]) + (dev_epi.ptr, dev_targets.ptr, F.ptr, sp["x_start"],
-                                        sp["n_cols"], mask.ptr if mask is not None else None)
-    plan = Plan(queue, queue.lib.nhip_spmv_sell_filter, args, gsize=spmv_plan.gsize,
+    args = tuple(spmv_plan.args[:7]) + (dev_epi.ptr, dev_targets.ptr, F.ptr, sp["x_start"], sp["n_cols"])
+    if sp["workspaces"]:
+        entry, args = queue.lib.nhip_spmv_sell_spikes, args + tuple(w.ptr for w in sp["workspaces"])
+    else:
+        entry, args = queue.lib.nhip_spmv_sell_filter, args + (None,)
+    plan = Plan(queue, entry, args, gsize=spmv_plan.gsize,
                 lsize=spmv_plan.lsize,
                 full_args=tuple(spmv_plan.full_args) + (dev_epi, dev_targets, F.dev_buf),
                 name="hip_spmv_filter", tag=spmv_plan.tag)

@@ -73,6 +73,30 @@ def test_sparse_product_of_spikes_spread_over_the_device(queue, rng, monkeypatch
         assert np.array_equal(dY.buf.view(np.uint32), Yo.buf.view(np.uint32))
 
 
+@pytest.mark.parametrize("cols", [32768, 32769])
+def test_sparse_product_without_ranges(queue, rng, cols):
+    """`nhip_spmv_sell_skip` writes no more than the one bit per element that its workspace holds,
+    and what it gives is the ordinary product."""
+    import scipy.sparse as sp
+
+    from nengo_ocl_amd import hipra_spmv
+    from nengo_ocl_amd.hipraggedarray import to_device
+
+    rows = 300
+    mat = sp.random(rows, cols, density=40 / cols, random_state=3, format="csr", dtype=np.float32)
+    X = RA([np.where(rng.uniform(size=cols) < 0.1, 1000.0, 0.0)])
+    Y = RA([rng.normal(size=rows)])
+    dX, dY, dY2 = to_dev(queue, X), to_dev(queue, Y), to_dev(queue, Y)
+    plan = hipra_spmv.plan_sparse_dot_inc(queue, [mat], dX, dY, inc=True).plans[0]
+    plan()
+    words = -(-cols // 128) * 4
+    mask = to_device(queue, np.full(words + 256, 77, dtype=np.int32))
+    args = plan.args[:6] + (dY2.ptr, int(dX.starts[0]), cols, mask.ptr)
+    assert queue.lib.nhip_spmv_sell_skip(queue.handle, *args) == 0
+    assert np.array_equal(dY.buf.view(np.uint32), dY2.buf.view(np.uint32))
+    assert (mask.get()[words:] == 77).all()
+
+
 @pytest.mark.parametrize("widths", [
     [512, 513, 639, 2047, 2048, 2049, 4095, 4096, 4097, 6145, 9216, 640, 8193],
     [512, 513, 514, 515, 639, 2047, 2048, 1920, 1921, 1999, 2000, 640, 2046],
