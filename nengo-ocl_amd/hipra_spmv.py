@@ -23,7 +23,8 @@ SKIP_MAX_COLS = 32 * 36864  # longest X whose "is not zero" bits fit the LDS (SP
 # ... and slices whose rows hold at least so many elements on average.  Measured (with the launch
 # for the bits / the ordinary one): 100,000 rows of 10 11.9 / 8.7 us, 10,000 of 20 5.2 / 4.0,
 # 30,000 of 50 8.4 / 11.0, 2,000 of 100 6.0 / 13.5, 100,000 of 100 23.8 / 58.4
-SKIP_MIN_WIDTH = 32
+# (steps of a whole network: 20,000 of 26 15.9 / 16.8, 100,000 of 30 17.4 / 18.4, 3,000 of 30 11.0 / 11.6)
+SKIP_MIN_WIDTH = 24
 
 
 def slice_window(columns, n_cols, x_start):
