@@ -122,3 +122,45 @@ def test_few_long_rows(queue, rng, beta, widths):
     run_plans(prog.plans)
     orc.plan_block_gemv(None, *args(A, X), Yo, gamma=0.25).plans[0]()
     assert np.array_equal(dY.buf.view(np.uint32), Yo.buf.view(np.uint32))
+
+
+# rows, columns, elements between rows, of a buffer's start, and pre's stride: four elements of a row
+# at a time or not, rows shorter and longer than a block of 1024, one element, blocks with a rest
+LEARN_SHAPES = [(1, 1, 1, 0, 1), (3, 4, 4, 0, 1), (257, 4, 8, 4, 1), (5, 1028, 1028, 0, 1),
+                (129, 100, 100, 0, 2), (129, 100, 104, 2, 1), (129, 100, 101, 0, 1),
+                (41, 255, 255, 0, 1), (2, 2050, 2052, 0, 1)]
+
+
+@pytest.mark.parametrize("inc", [False, True])
+@pytest.mark.parametrize("rule", ["bcm", "oja", "voja"])
+@pytest.mark.parametrize("shape", LEARN_SHAPES)
+def test_learning_rule_in_quads_of_a_row(queue, rng, rule, inc, shape):
+    """The change of a matrix, stored apart or added to the matrix it is formed from."""
+    from nengo_ocl_amd import hipra_nonlinearities as nl
+    from nengo_ocl_amd.hipraggedarray import HIPRaggedArray
+    from nengo_ocl_amd.raggedarray import RaggedArray
+    from oracle import oracle as orc
+
+    m, n, stride, shift, pre_stride = shape
+    sizes = [4 + m * stride, 4 + m * stride, 4 + n * pre_stride, m, m, 1, m]
+    big = RA([rng.uniform(-2, 9, size=k) for k in sizes])
+    dbig = to_dev(queue, big)
+    s = big.starts
+    at = dict(pre=(s[2] + shift, n, 1, pre_stride), post=(s[3], m, 1, 1), theta=(s[4], m, 1, 1),
+              learn=(s[5], 1, 1, 1), scale=(s[6], m, 1, 1), mat=(s[0] + shift, m, n, stride),
+              delta=(s[0 if inc else 1] + shift, m, n, stride))
+    views = []
+    for d in (False, True):
+        one = lambda *v: [np.int32([x]) for x in v]
+        views.append({k: HIPRaggedArray.from_buffer(queue, dbig.dev_buf, *one(*v, 1)) if d else
+                      RaggedArray.from_buffer(big.buf, *one(*v, 1)) for k, v in at.items()})
+    alpha, beta = np.float32([1e-3]), np.float32([1.5])
+    for mod, q, v in ((orc, None, views[0]), (nl, queue, views[1])):
+        if rule == "bcm":
+            mod.plan_bcm(q, v["pre"], v["post"], v["theta"], v["delta"], alpha, inc=inc)()
+        elif rule == "oja":
+            mod.plan_oja(q, v["pre"], v["post"], v["mat"], v["delta"], alpha, beta, inc=inc)()
+        else:
+            mod.plan_voja(q, v["pre"], v["post"], v["mat"], v["delta"], v["learn"], v["scale"], alpha,
+                          inc=inc)()
+    assert np.array_equal(dbig.buf.view(np.uint32), big.buf.view(np.uint32))
