@@ -106,6 +106,11 @@ LONG_ROWS_MAX, LONG_ROWS_MAX_ELEMS, LONG_ROWS_ANY_WIDTH = 2048, 1 << 22, 1024
 # 9.2 (10.8), 1024 x 4096 7.2 (6.5)
 GROUP_ROW_MIN_COLS, GROUP_ROWS_MAX = 2049, 512
 THIN_MIN_ROWS, THIN_ROWS_FOR_LANE_PER_ROW = 32, 65536
+# ... and below that limit four lanes per row with the small items, also for items of more than
+# SMALL_ITEM_ELEMS, unless a launch of large items stays anyway: launches of up to 21,632 rows of
+# one column 3.0 us instead of 6.2 through LDS; a step of the two convolution layers they feed
+# 47.5 -> 39.3 us, and 41.0 with a lane per row in a launch of their own.  Longer rows keep the LDS
+THIN_CLASS, THIN_MAX_COLS = (2, 4, 1), 4
 LIF_POP_ENABLED, LIF_POP_DECAY, LIF_POP_NO_J = 1 << 8, 1 << 9, 1 << 10  # flag bits of a population row
 LIF_POP_BITS = 1 << 11  # spikes stored as a bit per neuron (see `store_spikes_as_bits`)
 LIF_COMPACT = os.environ.get("NENGO_HIP_LIF_COMPACT", "1") != "0"
@@ -394,6 +399,12 @@ class gemv_prog:
             lpr = min(WAVE, next_pow2(-(-n_max // vec)))
         return (flavor, lpr, vec)
 
+    def _thin_item(self, g):
+        return (bool(g["dots"]) and g["y_len"] >= THIN_MIN_ROWS
+                and g["index"] not in self.tile_items
+                and sum(d["a_shape1"] for d in g["dots"]) <= THIN_MAX_COLS
+                and self._item_class(g)[2] == 1)
+
     def _long_rows(self, members):
         """Are the items `members` of a launch few rows of many columns?"""
         geometry = self.geometry
@@ -602,6 +613,13 @@ class gemv_prog:
             self._events_off = False
             for members in by_class.values():
                 members.sort()
+
+        # large items of a few columns whose rows no 16-byte loads fit: nothing to stage in LDS
+        if self.force_flavor is None and not self.force_scalar:
+            thin = [b for c in by_class if c[0] == 3 for b in by_class[c]]
+            if thin and all(self._thin_item(geometry[b]) for b in thin):
+                by_class = {c: m for c, m in by_class.items() if c[0] != 3}
+                by_class[THIN_CLASS] = sorted(by_class.get(THIN_CLASS, []) + thin)
 
         # a handful of long rows: the tiles of a row side by side over the lanes of a wave, for
         # all items of the large-item launch, and for those of the small-item launch with them

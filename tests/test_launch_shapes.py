@@ -164,3 +164,23 @@ def test_learning_rule_in_quads_of_a_row(queue, rng, rule, inc, shape):
             mod.plan_voja(q, v["pre"], v["post"], v["mat"], v["delta"], v["learn"], v["scale"], alpha,
                           inc=inc)()
     assert np.array_equal(dbig.buf.view(np.uint32), big.buf.view(np.uint32))
+
+
+@pytest.mark.parametrize("heights,cols,four_lanes", [
+    ([8193], 1, True), ([2731, 8192], 3, True), ([65535], 1, True), ([9001, 40, 3], 2, True),
+    ([8193], 5, False), ([65536], 1, False)])
+def test_many_rows_of_few_columns(queue, rng, heights, cols, four_lanes):
+    """Just above the small items' limit, and up to the rows that get a lane each."""
+    from nengo_ocl_amd import hipra_gemv
+    from oracle import oracle as orc
+
+    A = RA([rng.normal(size=(m, cols)) for m in heights])
+    X = RA([rng.normal(size=cols) for _ in heights])
+    Y = RA([rng.normal(size=m) for m in heights])
+    js = RA([[k] for k in range(len(heights))], dtype=np.int32)
+    dA, dX, dY, Yo = to_dev(queue, A), to_dev(queue, X), to_dev(queue, Y), clone(Y)
+    prog = hipra_gemv.plan_block_gemv(queue, 1.5, dA, js, dX, js, 1.0, dY, gamma=0.25)
+    assert ([p.kernel_class[:3] for p in prog.plans] == [(2, 4, 1)]) == four_lanes
+    run_plans(prog.plans)
+    orc.plan_block_gemv(None, 1.5, A, js, X, js, 1.0, Yo, gamma=0.25).plans[0]()
+    assert np.array_equal(dY.buf.view(np.uint32), Yo.buf.view(np.uint32))
