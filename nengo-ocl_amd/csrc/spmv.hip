@@ -166,8 +166,9 @@ constexpr int SPMV_MASK_INLINE_COLS = 32768;
 // still runs through the row element by element: each quad's lane adds its four products to the
 // sum the quad before left, which reaches it by an exchange inside the four lanes.  All the
 // bits of a batch are read first, then all the elements of X that are needed, then it is
-// summed: a batch waits for memory twice and not once per element.  Stored elements past a row's
-// end are +0 times -0, which changes no sum.  (Past the last quad that one again, unused.)
+// summed: a batch waits for memory twice and not once per element.  What is stored past a row's
+// end is not looked at, value or column: such an element counts as +0 times -0, which changes no
+// sum.  (The loads of a batch past the last quad take that one again: past the row's end too.)
 // ONE: every element of X that is not +0.0 is `one` (spikes of one amplitude): the bits are all
 // there is to know, and X is not looked up at all.
 template <int U, bool ONE>
@@ -188,7 +189,10 @@ __device__ __forceinline__ float spmv_skip_rows(const spmv_i4* c, const spmv_f4*
 #pragma unroll
         for (int i = 0; i < U; ++i)
 #pragma unroll
-            for (int u = 0; u < 4; ++u) word[i][u] = s_mask[(unsigned)cq[i][u] >> 5];
+            for (int u = 0; u < 4; ++u) {
+                const bool stored = 4 * (q + 4 * i + j) + u < len;
+                word[i][u] = s_mask[stored ? (unsigned)cq[i][u] >> 5 : 0u];
+            }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < U; ++i)
@@ -205,10 +209,9 @@ __device__ __forceinline__ float spmv_skip_rows(const spmv_i4* c, const spmv_f4*
 #pragma unroll
         for (int i = 0; i < U; ++i) {
             if (q + 4 * i >= n_quads) break;  // uniform
-            const bool mine = q + 4 * i + j < n_quads;  // (else: the last quad's values again)
             float w[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) w[u] = mine ? vq[i][u] : 0.0f;
+            for (int u = 0; u < 4; ++u) w[u] = 4 * (q + 4 * i + j) + u < len ? vq[i][u] : 0.0f;
 #define SPMV_LINK(J, CTRL)                                                               \
             {                                                                            \
                 _Pragma("unroll") for (int u = 0; u < 4; ++u) acc = fmaf(w[u], xi[i][u], acc); \

@@ -97,6 +97,60 @@ def test_sparse_product_without_ranges(queue, rng, cols):
     assert (mask.get()[words:] == 77).all()
 
 
+@pytest.mark.parametrize("padding", ["values", "values and columns"])
+@pytest.mark.parametrize("cols", [900, 40000])
+@pytest.mark.parametrize("longest", [14, 150])
+def test_sparse_product_ignores_what_is_stored_past_a_rows_end(queue, rng, cols, longest, padding):
+    """Rows are padded to the longest of their slice: no entry point may look at what the padding
+    holds, neither as a factor (infinities, NaN, negative numbers, with sums of -0 among the results)
+    nor as an index."""
+    import scipy.sparse as sp
+
+    from nengo_ocl_amd import hipra_spmv
+    from nengo_ocl_amd.hipraggedarray import to_device
+    from oracle import oracle as orc
+
+    rows = 64 * 40 + 21
+    lens = rng.randint(0, longest + 1, size=rows)
+    lens[::64] = longest
+    indptr = np.concatenate([[0], np.cumsum(lens)])
+    mat = sp.csr_matrix((rng.normal(size=indptr[-1]).astype(np.float32),
+                         rng.randint(cols, size=indptr[-1]), indptr), shape=(rows, cols))
+    mat.sum_duplicates()
+    host = hipra_spmv.HostSparseMatrix(mat)
+    slice_rows, row_len, cidx, vals = hipra_spmv.sell_layout([host])
+    padded = np.ones(vals.size, dtype=bool)
+    for _, start, width, len_start, n_rows, _ in slice_rows:
+        for r in range(n_rows):
+            padded[hipra_spmv.sell_index(start, r, np.arange(row_len[len_start + r]))] = False
+    vals[padded] = rng.choice([np.nan, np.inf, -np.inf, -3.0], size=padded.sum())
+    if padding != "values":
+        cidx[padded] = 2 ** 31 - 1
+    X = RA([np.where(rng.uniform(size=cols) < 0.2, rng.normal(size=cols), 0.0)])
+    Y = RA([np.where(np.arange(rows) % 2 == 0, -0.0, rng.normal(size=rows))])
+    dX = to_dev(queue, X)
+    table = np.zeros((len(slice_rows), 8), dtype=np.int32)
+    for k, (_, start, width, len_start, n_rows, row0) in enumerate(slice_rows):
+        table[k] = (start, width, len_start, n_rows, int(dX.starts[0]), row0, 1, -1)
+    d = [to_device(queue, a) for a in (table, row_len, cidx, vals)]
+    words = -(-cols // 128) * 4
+    mask, ranges = (to_device(queue, np.zeros(words, dtype=np.int32)) for _ in range(2))
+    head = (d[0].ptr, len(table), d[1].ptr, d[2].ptr, d[3].ptr, dX.ptr)
+    none, span, lib = (None, None, None), (int(dX.starts[0]), cols), queue.lib
+    calls = {"nhip_spmv_sell": (), "nhip_spmv_sell_skip": span + (mask.ptr,),
+             "nhip_spmv_sell_spikes": none + span + (mask.ptr, ranges.ptr)}
+    for x in (X[0], 1000.0 * (X[0] != 0)):  # many values, one value
+        X[0] = x
+        dX[0] = x
+        Yo = clone(Y)
+        orc.plan_sparse_dot_inc(None, [mat], X, Yo, inc=True).plans[0]()
+        for name, rest in calls.items():
+            dY = to_dev(queue, Y)
+            assert getattr(lib, name)(queue.handle, *head, dY.ptr, *rest) == 0
+            queue.finish()
+            assert np.array_equal(dY.buf.view(np.uint32), Yo.buf.view(np.uint32)), name
+
+
 @pytest.mark.parametrize("widths", [
     [512, 513, 639, 2047, 2048, 2049, 4095, 4096, 4097, 6145, 9216, 640, 8193],
     [512, 513, 514, 515, 639, 2047, 2048, 1920, 1921, 1999, 2000, 640, 2046],
