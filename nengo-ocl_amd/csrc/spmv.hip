@@ -18,6 +18,7 @@
 // column indices (band matrices, rings), the wave first copies that run into LDS and
 // takes the elements inside it from there: only the lanes whose column lies outside
 // go to the cache, which spares it one look-up per line and instruction.
+#include <type_traits>
 #include "nhip_common.h"
 #include "neuron_math.h"
 #include "sequence_ops.h"
@@ -148,12 +149,17 @@ __global__ __launch_bounds__(NHIP_WG) void spmv_sell_kernel(
 // work-group; for a stored element whose bit is clear the operand is the constant +0.0
 // instead of a look-up in the cache.  The sum is formed as above, term by term, so the
 // result has the bits of the kernel above whatever X and the matrix hold.  Groups are
-// persistent: the waves of a group take quarters of slices t, t + (waves of the grid), ... until none
-// is left.  A lane per row, each element's bit and look-up waited for on its own, was bound by
-// that chain: 2,000 rows of 100 took 20.9 us and now take 6.0, 100,000 rows of 100 39.6 us and
-// now 23.8 (4.1 of them the launch for the bits; the rest is 80 MB through the caches at
-// 4 TB/s).  Every group's own copy of the bits made from X costs 400 KB of reads per compute
-// unit at that size (29.3 us in all): hence the limit below.
+// persistent, and their waves take one of two things until none is left:
+//   a quarter of a slice, four lanes per row (spmv_skip_rows), while that is what keeps the waves
+//     busy: 2,000 rows of 100 6.4 us, against 20.4 by whole slices (one lane per row is bound by its chain
+//     of loads, bits and look-ups); 100,000 rows of 100 24.5 against 30.6 (4.1 of them the launch for
+//     the bits).  Quarters are dealt out over the groups first and the waves of a group second.
+//   a whole slice, a lane per row (spmv_skip_slice), where the slices are enough for all waves: a
+//     load is then one run of 1 KiB, and a wave starts a chain of loads once per slice instead
+//     of four times.  1,000,000 rows of 100 139 us (5.9 TB/s), by quarters 161; rows of 20 43 and 52, of 4
+//     21 and 35.  Which one: see `spmv_takes_slices`.
+// Every group's own copy of the bits made from X costs 400 KB of reads per compute unit at
+// 100,000 elements (30.4 us in all instead of 24.5): hence the limit below.
 constexpr int SPMV_SKIP_WG = 1024;
 constexpr int SPMV_MASK_WORDS = 36864;  // 144 KiB of LDS: X of up to 1,179,648 elements
 constexpr int SPMV_MASK_U = 16;
@@ -241,6 +247,84 @@ __device__ __forceinline__ float spmv_skip_rows(const spmv_i4* c, const spmv_f4*
     return acc;
 }
 
+// A slice by one wave, lane r its row r; SPMV_SLICE_U quads of a row are in flight per lane while
+// the ones before are summed.  ONE and what lies past a row's end: as above.
+constexpr int SPMV_SLICE_U = 4;
+template <bool ONE>
+__device__ __forceinline__ float spmv_skip_slice(const spmv_i4* c, const spmv_f4* v, int n_quads,
+                                                 int len, const float* x, const unsigned* s_mask,
+                                                 float one, float acc) {
+    constexpr int U = SPMV_SLICE_U;
+    spmv_i4 ci[U];
+    spmv_f4 vi[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+        ci[i] = spmv_i4{0, 0, 0, 0};
+        vi[i] = spmv_f4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (i < n_quads) {  // the same for all lanes
+            ci[i] = __builtin_nontemporal_load(c + (size_t)i * NHIP_WAVE);
+            vi[i] = __builtin_nontemporal_load(v + (size_t)i * NHIP_WAVE);
+        }
+    }
+    for (int q = 0; q < n_quads; q += U) {
+        // the next U quads are requested before the look-ups of the current ones
+        spmv_i4 cn[U];
+        spmv_f4 vn[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            cn[i] = ci[i];
+            vn[i] = vi[i];
+            if (q + U + i < n_quads) {
+                cn[i] = __builtin_nontemporal_load(c + (size_t)(q + U + i) * NHIP_WAVE);
+                vn[i] = __builtin_nontemporal_load(v + (size_t)(q + U + i) * NHIP_WAVE);
+            }
+        }
+        float xi[U][4];
+#pragma unroll
+        for (int i = 0; i < U; ++i)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const unsigned col = (unsigned)ci[i][u];
+                const bool stored = 4 * (q + i) + u < len;
+                const bool set = stored && ((s_mask[col >> 5] >> (col & 31u)) & 1u);
+                xi[i][u] = 0.0f;
+                if (ONE) xi[i][u] = set ? one : 0.0f;
+                else if (set) xi[i][u] = x[col];
+            }
+#pragma unroll
+        for (int i = 0; i < U; ++i)
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (4 * (q + i) + u < len) acc = fmaf(vi[i][u], xi[i][u], acc);
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            ci[i] = cn[i];
+            vi[i] = vn[i];
+        }
+    }
+    return acc;
+}
+
+// Whole slices or quarters, for a grid of `n_waves` waves.  Measured (kernel time in us, slices /
+// quarters; n rows and columns, rows of 32, 60, 100; 4,096 waves; one amplitude):
+//   n = 160,000 (0.61 slices per wave)  17.5/17.6  24.7/21.8   33.8/32.5
+//       220,000 (0.84)                  18.7/20.3  27.0/27.2   38.1/41.6
+//       260,000 (0.99)                  20.4/22.3  30.2/30.5   43.3/47.3
+//       300,000 (1.14)                  28.0/24.3  40.5/33.3   60.0/52.0   (a second, nearly empty round)
+//       400,000 (1.53)                  30.0/28.7  42.6/42.9   63.6/67.6
+//       500,000 (1.91)                  32.6/34.0  47.9/51.3   73.3/81.3
+//       700,000 (2.67)                  41.5/44.1  63.5/69.2   98.8/112.2
+//     1,000,000 (3.81)                  54.1/60.4  86.7/99.9  138.8/161.1
+// Shorter rows are mostly the start of a task, which quarters pay four times: rows of 12, n =
+// 100,000 12.8/12.4, 150,000 12.1/13.8, 300,000 16.7/18.4; of 24, 100,000 15.2/14.3, 120,000 15.4/15.3,
+// 200,000 16.5/18.7.  (Short: by the width of the first slice.  A choice by one slice is the
+// same for every group, and either form is right for any.)
+constexpr int SPMV_SHORT_WIDTH = 24;
+__device__ __forceinline__ bool spmv_takes_slices(int n_slices, int width, int n_waves) {
+    if (width <= SPMV_SHORT_WIDTH) return 9LL * n_slices >= 4LL * n_waves;
+    return n_slices <= n_waves ? 5LL * n_slices >= 4LL * n_waves : 2LL * n_slices >= 3LL * n_waves;
+}
+
 // smallest and largest bits of the elements of X that are not +0.0
 __device__ __forceinline__ void spmv_wave_range(unsigned& lo, unsigned& hi) {
 #pragma unroll
@@ -278,23 +362,15 @@ __global__ __launch_bounds__(SPMV_SKIP_WG) void spmv_sell_skip_kernel(
     SpmvEpi epi, SpmvSide side)
 {
     __shared__ __attribute__((aligned(16))) unsigned s_mask[SPMV_MASK_WORDS];
-    __shared__ unsigned s_range[2];
+    __shared__ unsigned s_one[SPMV_SKIP_WG / NHIP_WAVE], s_mixed[SPMV_SKIP_WG / NHIP_WAVE];
     if (side.n_chains > 0 && (int)blockIdx.x >= side.n_groups) return spmv_side_chain(side, s_mask);
     const int lane = threadIdx.x & (NHIP_WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr int WAVES = SPMV_SKIP_WG / NHIP_WAVE;
-    // Quarters of slices are dealt out over the groups first and the waves of a group second: a
-    // product that does not fill the grid then keeps every compute unit busy.
     const int stride = side.n_groups * WAVES;
     unsigned lo = 0xffffffffu, hi = 0u;  // smallest and largest bits of a set element
-    if (threadIdx.x == 0) {
-        s_range[0] = lo;
-        s_range[1] = hi;
-    }
-    __syncthreads();
     if (mask) {
         const int n_mask_quads = (n_cols + 127) / 128;
-        if (!ranges) { lo = 0u; hi = 0xffffffffu; }  // values not known: look-ups
         for (int i = threadIdx.x; i < n_mask_quads; i += SPMV_SKIP_WG) {
             reinterpret_cast<spmv_i4*>(s_mask)[i] = reinterpret_cast<const spmv_i4*>(mask)[i];
             if (!ranges) continue;
@@ -327,15 +403,50 @@ __global__ __launch_bounds__(SPMV_SKIP_WG) void spmv_sell_skip_kernel(
             }
         }
     }
-    spmv_wave_range(lo, hi);
-    if (lane == 0) {
-        atomicMin(&s_range[0], lo);
-        atomicMax(&s_range[1], hi);
+    const bool values_known = ranges || !mask;  // (else: look-ups)
+    if (values_known) {
+        // the wave's set elements: one value (0: there are none), or several
+        const unsigned long long some = __ballot(hi != 0u);
+        const unsigned one_w = some ? __builtin_amdgcn_readlane(hi, __ffsll(some) - 1) : 0u;
+        const unsigned long long other = __ballot(hi != 0u && (lo != hi || hi != one_w));
+        if (lane == 0) {
+            s_one[wave] = one_w;
+            s_mixed[wave] = other != 0ull;
+        }
     }
-    __syncthreads();  // every thread reaches it
-    // all set elements have the same bits (or there are none)
-    const bool one_value = s_range[0] >= s_range[1];
-    const float one = __uint_as_float(s_range[1]);
+    const bool whole = spmv_takes_slices(n_slices, slices[0].width, stride);  // uniform over the grid
+    __syncthreads();  // the only barrier; every thread reaches it
+    bool one_value = false;  // all set elements have the same bits (or there are none)
+    float one = 0.0f;
+    if (values_known) {
+        const unsigned w = lane < WAVES ? s_one[lane] : 0u;
+        const unsigned long long some = __ballot(w != 0u);
+        const unsigned first = some ? __builtin_amdgcn_readlane(w, __ffsll(some) - 1) : 0u;
+        one_value = __ballot(lane < WAVES && (s_mixed[lane] != 0u || (w != 0u && w != first))) == 0ull;
+        one = __uint_as_float(first);
+    }
+    auto take_slices = [&](auto one_tag) {
+        for (int s = blockIdx.x * WAVES + wave; s < n_slices; s += stride) {
+            const SpmvSlice sl = slices[s];
+            const bool live = lane < sl.n_rows;
+            const int len = live ? row_len[sl.len_start + lane] : 0;
+            float acc = (live && sl.inc) ? Y[(size_t)sl.y_start + lane] : 0.0f;
+            const spmv_i4* c = reinterpret_cast<const spmv_i4*>(cols + (size_t)sl.data_start) + lane;
+            const spmv_f4* v = reinterpret_cast<const spmv_f4*>(vals + (size_t)sl.data_start) + lane;
+            const float* x = X + sl.x_start;
+            acc = spmv_skip_slice<decltype(one_tag)::value>(c, v, sl.width >> 2, len, x, s_mask, one,
+                                                            acc);
+            if (live) {
+                Y[(size_t)sl.y_start + lane] = acc;
+                if (epi.slice_epi) spmv_filter_rows(epi, s, lane, acc);
+            }
+        }
+    };
+    if (whole) {
+        if (one_value) take_slices(std::true_type());
+        else take_slices(std::false_type());
+        return;
+    }
     for (int t = wave * side.n_groups + blockIdx.x; t < 4 * n_slices; t += stride) {
         const int s = t >> 2, row = 16 * (t & 3) + (lane >> 2), j = lane & 3;
         const SpmvSlice sl = slices[s];

@@ -98,9 +98,12 @@ def test_sparse_product_without_ranges(queue, rng, cols):
 
 
 @pytest.mark.parametrize("padding", ["values", "values and columns"])
-@pytest.mark.parametrize("cols", [900, 40000])
-@pytest.mark.parametrize("longest", [14, 150])
-def test_sparse_product_ignores_what_is_stored_past_a_rows_end(queue, rng, cols, longest, padding):
+@pytest.mark.parametrize("rows,cols,longest", [
+    (64 * 40 + 21, 900, 14), (64 * 40 + 21, 40000, 14), (64 * 40 + 21, 900, 150),
+    (64 * 40 + 21, 40000, 150),
+    (64 * 1830 + 1, 900, 14), (64 * 3300 + 7, 40000, 29)])  # (whole slices)
+def test_sparse_product_ignores_what_is_stored_past_a_rows_end(queue, rng, rows, cols, longest,
+                                                               padding):
     """Rows are padded to the longest of their slice: no entry point may look at what the padding
     holds, neither as a factor (infinities, NaN, negative numbers, with sums of -0 among the results)
     nor as an index."""
@@ -110,7 +113,6 @@ def test_sparse_product_ignores_what_is_stored_past_a_rows_end(queue, rng, cols,
     from nengo_ocl_amd.hipraggedarray import to_device
     from oracle import oracle as orc
 
-    rows = 64 * 40 + 21
     lens = rng.randint(0, longest + 1, size=rows)
     lens[::64] = longest
     indptr = np.concatenate([[0], np.cumsum(lens)])
@@ -121,8 +123,8 @@ def test_sparse_product_ignores_what_is_stored_past_a_rows_end(queue, rng, cols,
     slice_rows, row_len, cidx, vals = hipra_spmv.sell_layout([host])
     padded = np.ones(vals.size, dtype=bool)
     for _, start, width, len_start, n_rows, _ in slice_rows:
-        for r in range(n_rows):
-            padded[hipra_spmv.sell_index(start, r, np.arange(row_len[len_start + r]))] = False
+        at = hipra_spmv.sell_index(start, np.arange(64)[:, None], np.arange(width))
+        padded[at] = np.arange(width) >= row_len[len_start:len_start + 64][:, None]
     vals[padded] = rng.choice([np.nan, np.inf, -np.inf, -3.0], size=padded.sum())
     if padding != "values":
         cidx[padded] = 2 ** 31 - 1
@@ -149,6 +151,52 @@ def test_sparse_product_ignores_what_is_stored_past_a_rows_end(queue, rng, cols,
             assert getattr(lib, name)(queue.handle, *head, dY.ptr, *rest) == 0
             queue.finish()
             assert np.array_equal(dY.buf.view(np.uint32), Yo.buf.view(np.uint32)), name
+
+
+# (on 256 compute units: from 0.8 slices per wave on, not just above one per wave, from 1.5 on; of short
+# rows from 0.45 on)
+@pytest.mark.parametrize("rows,cols,per_row", [
+    (64 * 1821 + 5, 3000, 7), (64 * 3277 + 50, 40000, 40), (64 * 4096, 32768, 26),
+    (64 * 4096 + 1, 70000, 26), (64 * 6144 + 63, 600, 28)])
+def test_sparse_product_of_spikes_in_whole_slices(queue, rng, monkeypatch, rows, cols, per_row):
+    """As many slices as waves, and more: with a filter behind the rows, X of many values and of one."""
+    import scipy.sparse as sp
+
+    from nengo_ocl_amd import hipra_nonlinearities as nl
+    from nengo_ocl_amd import hipra_spmv
+    from oracle import oracle as orc
+
+    monkeypatch.setattr(hipra_spmv, "SKIP_MIN_WIDTH", 0)
+    lens = rng.randint(0, per_row + 1, size=rows)
+    lens[::64] = per_row
+    indptr = np.concatenate([[0], np.cumsum(lens)])
+    mat = sp.csr_matrix((rng.normal(size=indptr[-1]).astype(np.float32),
+                         rng.randint(cols, size=indptr[-1]), indptr), shape=(rows, cols))
+    mat.sum_duplicates()
+    R = RA([np.where(rng.uniform(size=cols) < 0.2, rng.normal(size=cols), 0.0),
+            np.where(np.arange(rows) % 3 == 0, -0.0, rng.normal(size=rows)), rng.normal(size=rows)])
+    den, num = RA([np.array([[-0.8]])]), RA([np.array([[0.2]])])
+    dev, host = to_dev(queue, R), clone(R)
+    bufs = [RA([np.zeros((1, rows))]) for _ in range(2)]
+    plans = []
+    for ra, spmv, mod, q, up, kw in (
+            (dev, hipra_spmv.plan_sparse_dot_inc, nl, queue, lambda a: to_dev(queue, a),
+             dict(x_mostly_zero=True)),
+            (host, orc.plan_sparse_dot_inc, orc, None, clone, {})):
+        plans.append((spmv(q, [mat], ra[[0]], ra[[1]], inc=True, **kw).plans[0],
+                      mod.plan_linearfilter(q, ra[[1]], ra[[2]], up(den), up(num), up(bufs[0]),
+                                            up(bufs[1]))))
+    (plan, lf), (oplan, olf) = plans
+    assert plan.skips_zero_x
+    fused, residual = hipra_spmv.fuse_linearfilter(plan, lf[0])
+    assert [p.name for p in fused] == ["hip_spmv_filter"] and not residual
+    for x in (R[0], 1000.0 * (R[0] != 0)):
+        dev[0] = x
+        host[0] = x
+        run_plans(fused)
+        oplan()
+        run_plans(olf)
+        assert np.array_equal(dev.buf.view(np.uint32), host.buf.view(np.uint32))
 
 
 @pytest.mark.parametrize("widths", [
