@@ -20,12 +20,20 @@ WG, WAVE = 256, 64
 QUAD = 4  # elements of a row stored side by side (one 16-byte access)
 WINDOW = 1024  # consecutive elements of X a wave can keep in LDS (SPMV_WINDOW in csrc/spmv.hip)
 SKIP_MAX_COLS = 32 * 36864  # longest X whose "is not zero" bits fit the LDS (SPMV_MASK_WORDS)
-# ... and slices whose rows hold at least so many elements on average.  Measured (with the launch
-# for the bits / the ordinary one): 100,000 rows of 10 11.9 / 8.7 us, 10,000 of 20 5.2 / 4.0,
-# 30,000 of 50 8.4 / 11.0, 2,000 of 100 6.0 / 13.5, 100,000 of 100 23.8 / 58.4
-# (steps of a whole network: 20,000 of 26 15.9 / 16.8, 100,000 of 30 17.4 / 18.4, 3,000 of 30 11.0 / 11.6)
-SKIP_MIN_WIDTH = 24
-
+# ... and either rows of more than SKIP_MIN_WIDTH stored elements (mean over the slices, padding
+# included), or more than SKIP_MIN_NNZ elements in all: the ordinary launch looks every one of them up
+# in a cache, which gets dearer with the length of X, while the one for spikes has the bits to make
+# and to hand to every group first.  Measured (kernel time in us, spikes / ordinary; n rows and columns):
+#   rows of    n = 2,000    10,000     34,000     70,000     100,000    200,000    300,000    1,000,000
+#       4      5.0/3.9     5.2/4.0   10.1/4.0   11.2/4.0   10.1/4.0   10.6/6.6   13.0/8.6    19.2/32.7
+#      12      5.0/4.0     5.2/4.0   10.5/4.0   11.5/6.3   11.8/9.1   12.4/16.6  16.7/23.4   30.4/85.0
+#      20      5.3/4.9     5.6/4.1   11.2/5.6   13.0/10.9  14.0/14.3  15.4/26.9  22.2/36.1   43.8/130.7
+#      24      5.3/5.4     5.6/4.5   11.3/6.3   13.1/13.0  14.3/16.8  16.4/32.9  25.0/42.0   51.0/155.0
+#      32      5.3/6.4     5.7/5.3   11.6/7.8   13.4/17.5  15.0/21.0  18.2/42.7  24.3/57.8   54.1/201.0
+#     100      6.3/13.7    9.0/11    15.4/21.3  20/43      24.5/58.8  36.3/127   51.8/168    139/582
+# (100,000 rows of 10 on 1,000,000 columns 13.0/11.0, of 50 20.6/37.8; 1,000,000 rows of 10 on
+# 30,000 columns 25.7/58.8, on 1,000 24.9/24.6)
+SKIP_MIN_WIDTH, SKIP_MIN_NNZ = 24, 1750000
 
 def slice_window(columns, n_cols, x_start):
     """First element of the run of `WINDOW` consecutive elements of X that a wave keeps
@@ -109,8 +117,9 @@ class plan_sparse_dot_inc:
 
     ``x_mostly_zero`` (one flag, or one per matrix) says that X is zero in most places
     most of the time -- the spikes of a population.  When it holds for every matrix and all
-    read the same X of at most `SKIP_MAX_COLS` elements, the launch is
-    `nhip_spmv_sell_spikes`: one bit per element of X ("is not +0.0") is made first and kept
+    read the same X of at most `SKIP_MAX_COLS` elements, and the matrices are wide or large
+    (`SKIP_MIN_WIDTH`, `SKIP_MIN_NNZ`), the launch is `nhip_spmv_sell_spikes` (of short rows
+    `nhip_spmv_sell_skip`): one bit per element of X ("is not +0.0") is made first and kept
     in LDS, and where it is clear the operand is the constant instead of a look-up of X.
     Same bits as the ordinary launch whatever X holds; only faster when X is mostly zero.
     """
@@ -156,16 +165,21 @@ class plan_sparse_dot_inc:
         n_groups = max(1, -(-n // (WG // WAVE)))
         flags = np.broadcast_to(np.asarray(x_mostly_zero, dtype=bool), (len(matrices),))
         same_x = len({(int(X.starts[b]), int(X.shape0s[b])) for b in range(len(matrices))}) == 1
+        nnz = int(sum(m.csr.nnz for m in matrices))
+        wide = vals.size > SKIP_MIN_WIDTH * WAVE * n
         skip = (n > 0 and bool(flags.all()) and same_x and int(X.shape0s[0]) <= SKIP_MAX_COLS
-                and vals.size > SKIP_MIN_WIDTH * WAVE * n)
+                and (wide or nnz > SKIP_MIN_NNZ))
+        workspaces = ()
         if skip:
             n_cols = int(X.shape0s[0])
-            # a bit per element of X; the values that the set ones span
-            mask, ranges = (to_device(queue, np.zeros(-(-n_cols // 128) * 4, dtype=np.int32))
-                            for _ in range(2))
-            dev += [mask, ranges]
-            entry = queue.lib.nhip_spmv_sell_spikes
-            args = args + (None, None, None, int(X.starts[0]), n_cols, mask.ptr, ranges.ptr)
+            # a bit per element of X; the values that the set ones span (of short rows nearly as
+            # many words as look-ups that they spare: 1,000,000 rows of 4 19.2 us without, 21.9 with)
+            workspaces = tuple(to_device(queue, np.zeros(-(-n_cols // 128) * 4, dtype=np.int32))
+                               for _ in range(2 if wide else 1))
+            dev += list(workspaces)
+            entry = queue.lib.nhip_spmv_sell_spikes if wide else queue.lib.nhip_spmv_sell_skip
+            args = (args + ((None, None, None) if wide else ()) + (int(X.starts[0]), n_cols)
+                    + tuple(w.ptr for w in workspaces))
             gsize, lsize = (1024 * min(queue.n_compute_units, 4 * n),), (1024,)
         else:
             entry, gsize, lsize = queue.lib.nhip_spmv_sell, (WG * n_groups,), (WG,)
@@ -174,10 +188,9 @@ class plan_sparse_dot_inc:
         plan.skips_zero_x = skip
         # what `fuse_linearfilter` needs to rebuild the launch with filters behind its rows
         plan.spmv = dict(X=X, Y=Y, slice_rows=slice_rows, dev=tuple(dev), n=n,
-                         workspaces=(mask, ranges) if skip else (),
+                         workspaces=workspaces,
                          x_start=int(X.starts[0]) if skip else 0,
                          n_cols=int(X.shape0s[0]) if skip else 0)
-        nnz = int(sum(m.csr.nnz for m in matrices))
         plan.flops_per_call = 2 * nnz
         # reference accounting (clra_gemv.py:1552-1560): values, indices, row pointers, X, Y
         plan.bw_per_call = 8 * nnz + 4 * sum(m.shape[0] + 1 for m in matrices) + X.nbytes + Y.nbytes
@@ -303,10 +316,9 @@ def fuse_linearfilter(spmv_plan, lf_plan):
     dev_epi = to_device(queue, slice_epi)
     dev_targets = to_device(queue, np.array(target_rows, dtype=np.int32))
     args = tuple(spmv_plan.args[:7]) + (dev_epi.ptr, dev_targets.ptr, F.ptr, sp["x_start"], sp["n_cols"])
-    if sp["workspaces"]:
-        entry, args = queue.lib.nhip_spmv_sell_spikes, args + tuple(w.ptr for w in sp["workspaces"])
-    else:
-        entry, args = queue.lib.nhip_spmv_sell_filter, args + (None,)
+    args += tuple(w.ptr for w in sp["workspaces"]) or (None,)
+    entry = (queue.lib.nhip_spmv_sell_spikes if len(sp["workspaces"]) == 2
+             else queue.lib.nhip_spmv_sell_filter)
     plan = Plan(queue, entry, args, gsize=spmv_plan.gsize,
                 lsize=spmv_plan.lsize,
                 full_args=tuple(spmv_plan.full_args) + (dev_epi, dev_targets, F.dev_buf),

@@ -199,6 +199,38 @@ def test_sparse_product_of_spikes_in_whole_slices(queue, rng, monkeypatch, rows,
         assert np.array_equal(dev.buf.view(np.uint32), host.buf.view(np.uint32))
 
 
+# short rows: enough of them in all, or the ordinary launch
+@pytest.mark.parametrize("rows,cols,per_row,skips", [
+    (150000, 150000, 12, True), (440000, 40000, 4, True), (430000, 40000, 4, False),
+    (70000, 70000, 24, False), (3000, 3000, 28, True), (3000, 3000, 24, False)])
+def test_sparse_product_of_spikes_with_short_rows(queue, rng, rows, cols, per_row, skips):
+    import scipy.sparse as sp
+
+    from nengo_ocl_amd import hipra_nonlinearities as nl
+    from nengo_ocl_amd import hipra_spmv
+    from oracle import oracle as orc
+
+    columns = np.sort(rng.randint(cols - per_row, size=(rows, per_row)), axis=1) + np.arange(per_row)
+    mat = sp.csr_matrix((rng.normal(size=columns.size).astype(np.float32), columns.ravel(),
+                         np.arange(0, columns.size + 1, per_row)), shape=(rows, cols))
+    R = RA([np.where(rng.uniform(size=cols) < 0.1, 1000.0, 0.0), rng.normal(size=rows),
+            rng.normal(size=rows)])
+    dev, host = to_dev(queue, R), clone(R)
+    den, num, zero = RA([np.array([[-0.8]])]), RA([np.array([[0.2]])]), RA([np.zeros((1, rows))])
+    plan = hipra_spmv.plan_sparse_dot_inc(queue, [mat], dev[[0]], dev[[1]], inc=True,
+                                          x_mostly_zero=True).plans[0]
+    assert plan.skips_zero_x == skips
+    up = lambda a: to_dev(queue, a)
+    lf = nl.plan_linearfilter(queue, dev[[1]], dev[[2]], up(den), up(num), up(zero), up(zero))
+    fused, residual = hipra_spmv.fuse_linearfilter(plan, lf[0])
+    assert not residual
+    run_plans([plan] + fused)
+    oplan = orc.plan_sparse_dot_inc(None, [mat], host[[0]], host[[1]], inc=True).plans[0]
+    run_plans([oplan, oplan] + orc.plan_linearfilter(None, host[[1]], host[[2]], den, num, clone(zero),
+                                                     clone(zero)))
+    assert np.array_equal(dev.buf.view(np.uint32), host.buf.view(np.uint32))
+
+
 @pytest.mark.parametrize("widths", [
     [512, 513, 639, 2047, 2048, 2049, 4095, 4096, 4097, 6145, 9216, 640, 8193],
     [512, 513, 514, 515, 639, 2047, 2048, 1920, 1921, 1999, 2000, 640, 2046],
