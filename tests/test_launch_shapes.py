@@ -258,6 +258,42 @@ def test_few_long_rows(queue, rng, beta, widths):
     assert np.array_equal(dY.buf.view(np.uint32), Yo.buf.view(np.uint32))
 
 
+@pytest.mark.parametrize("pre,dims,lanes", [(1000, 200, 128), (5000, 2100, 256)],
+                         ids=["wave per row", "group per row"])
+def test_few_long_rows_with_epilogues(queue, pre, dims, lanes):
+    """Encoders of many dimensions and decoders of many neurons: long rows whose launch also updates the
+    neurons or steps the filters, and carries a sequence, bit for bit like the oracle's; the
+    launches have a name of their own."""
+    from nengo_ocl_amd import minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    def make():
+        rng = np.random.RandomState(5)
+        net = mb.Network(seed=4, solver="surrogate")
+        stim = net.Node(mb.WhiteSignal(period=0.5, high=8.0, seed=3), size_out=2)
+        a = net.Ensemble(pre, 2, neuron_type=mb.LIFRate())
+        wide = net.Ensemble(250, dims, radius=3.0)
+        net.Connection(stim, a, synapse=None)
+        net.Connection(stim, wide, synapse=mb.Lowpass(0.01), transform=rng.normal(size=(dims, 2)))
+        out = net.Node(None, size_in=3)
+        net.Connection(a.neurons, out, synapse=mb.Lowpass(0.005),
+                       transform=rng.normal(scale=1e-2 / pre, size=(3, pre)))
+        return net, [net.Probe(out), net.Probe(wide.neurons)]
+
+    (net, probes), (net_o, probes_o) = make(), make()
+    with Simulator(net, seed=1) as gpu, OracleSimulator(net_o, seed=1) as cpu:
+        rows = {p.name: p for p in gpu._plans if p.name.startswith("hipra_gemv.tile_rows")}
+        assert set(rows) == {"hipra_gemv.tile_rows_lif", "hipra_gemv.tile_rows_filter"}
+        assert {p.kernel_class for p in rows.values()} == {(2, lanes, 1)}
+        assert any(getattr(p, "carried", None) is not None for p in rows.values())
+        gpu.run_steps(60)
+        cpu.run_steps(60)
+        for p, q in zip(probes, probes_o):
+            assert np.array_equal(gpu.data[p], cpu.data[q]) and np.any(gpu.data[p] != 0)
+        assert np.array_equal(gpu.signal_buffer(), cpu.signal_buffer())
+
+
 # rows, columns, elements between rows, of a buffer's start, and pre's stride: four elements of a row
 # at a time or not, rows shorter and longer than a block of 1024, one element, blocks with a rest
 LEARN_SHAPES = [(1, 1, 1, 0, 1), (3, 4, 4, 0, 1), (257, 4, 8, 4, 1), (5, 1028, 1028, 0, 1),
