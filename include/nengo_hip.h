@@ -499,6 +499,9 @@ int nhip_learning_rule(void *stream, int rule, int inc, const int *desc, int n_b
  * output is accumulated over channel, kernel row, kernel column in that order with
  * one fused multiply-add per term. */
 int nhip_conv2d(void *stream, const int *geom, const float *X, const float *F, float *Y);
+/* Work-groups that nhip_conv2d launches for `geom`, and the threads of each (256: the tiles above; 64:
+ * where the shape suits it better, one wave per 16 filters x 4 pixels). */
+int nhip_conv2d_groups(const int *geom, int *n_groups, int *group_threads);
 /* Average pooling, channels first; window elements outside the image (bottom /
  * right edge) and NaN inputs are left out of the mean.
  * replaces: `plan_pool2d` (:1972-2079).

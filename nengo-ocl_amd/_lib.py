@@ -60,6 +60,7 @@ SIGNATURES = {
     "nhip_outer_filter": [P, P, c_int, P, P, P, P, P],
     "nhip_learning_rule": [P, c_int, c_int, P, c_int, P, P, P, P, P, P],
     "nhip_conv2d": [P, P, P, P, P],
+    "nhip_conv2d_groups": [P, P, P],
     "nhip_pool2d": [P, P, P, P],
     "nhip_whitenoise": [P, P, c_int, P, c_double, P],
     "nhip_philox4x32": [P, P, P, c_int],

@@ -338,13 +338,17 @@ __global__ __launch_bounds__(NHIP_WG) void pool2d_kernel(const PoolGeom g, const
     Y[g.y_start + e] = __fdiv_rn(out, (float)count);
 }
 
-}  // namespace
-
-extern "C" int nhip_conv2d(void* stream, const int* geom, const float* X, const float* F,
-                           float* Y) {
-    if (!geom || !X || !F || !Y) return NHIP_E_BADARG;
+// What a call with geometry `q` launches.
+struct ConvLaunch {
     ConvGeom g;
-    const int* q = geom;
+    bool waves;  // conv2d_wave_kernel, else conv2d_kernel
+    dim3 grid;
+    int threads;
+    size_t lds;
+};
+
+int conv_launch(const int* q, ConvLaunch& l) {
+    ConvGeom& g = l.g;
     g.nxi = q[0]; g.nxj = q[1]; g.nc = q[2]; g.nyi = q[3]; g.nyj = q[4]; g.nf = q[5];
     g.si = q[6]; g.sj = q[7]; g.sti = q[8]; g.stj = q[9]; g.pi = q[10]; g.pj = q[11];
     g.x_start = q[12]; g.y_start = q[13]; g.f_start = q[14];
@@ -370,28 +374,50 @@ extern "C" int nhip_conv2d(void* stream, const int* geom, const float* X, const 
     g.tiles_j = (g.nyj + g.tile_j - 1) / g.tile_j;
     const int tiles_i = (g.nyi + g.tile_i - 1) / g.tile_i;
     const size_t taps = (size_t)g.si * g.sj;
-    const size_t lds = ((size_t)g.c_chunk * (g.nipatch * g.njpatch + (g.local ? 0 : taps * g.tile_f)) +
-                        taps) * sizeof(float);
-    if (lds > 64 * 1024) return NHIP_E_BADARG;
+    l.lds = ((size_t)g.c_chunk * (g.nipatch * g.njpatch + (g.local ? 0 : taps * g.tile_f)) + taps) *
+            sizeof(float);
+    if (l.lds > 64 * 1024) return NHIP_E_BADARG;
+    l.grid = dim3(g.tiles_j * tiles_i, (g.nf + g.tile_f - 1) / g.tile_f);
+    l.threads = NHIP_WG;
     const long long n_out = (long long)g.nyi * g.nyj * g.nf;
     const size_t n_links = taps * g.nc;
-    if (g.f_fast && !g.local && n_out <= CONV_WAVE_MAX_OUT && n_links >= CONV_WAVE_MIN_LINKS &&
-        n_links <= CONV_WAVE_MAX_LINKS) {
-        const dim3 waves((g.nyi * g.nyj + CONV_WP - 1) / CONV_WP, (g.nf + CONV_WF - 1) / CONV_WF);
-        const size_t words = n_links * (CONV_WF + CONV_WP);
-        const bool vec = !((g.nf | g.f_start) & 3) && !(reinterpret_cast<uintptr_t>(F) & 15);
-        if (vec)
-            NHIP_LAUNCH(conv2d_wave_kernel<true>, waves, dim3(NHIP_WAVE), words * sizeof(float),
-                        NHIP_STREAM(stream), g, X, F, Y);
-        else
-            NHIP_LAUNCH(conv2d_wave_kernel<false>, waves, dim3(NHIP_WAVE), words * sizeof(float),
-                        NHIP_STREAM(stream), g, X, F, Y);
-        NHIP_LAUNCH_CHECK();
-        return 0;
+    l.waves = g.f_fast && !g.local && n_out <= CONV_WAVE_MAX_OUT && n_links >= CONV_WAVE_MIN_LINKS &&
+              n_links <= CONV_WAVE_MAX_LINKS;
+    if (l.waves) {
+        l.grid = dim3((g.nyi * g.nyj + CONV_WP - 1) / CONV_WP, (g.nf + CONV_WF - 1) / CONV_WF);
+        l.threads = NHIP_WAVE;
+        l.lds = n_links * (CONV_WF + CONV_WP) * sizeof(float);
     }
-    const dim3 grid(g.tiles_j * tiles_i, (g.nf + g.tile_f - 1) / g.tile_f);
-    NHIP_LAUNCH(conv2d_kernel, grid, dim3(NHIP_WG), lds, NHIP_STREAM(stream), g, X, F, Y);
+    return 0;
+}
+
+}  // namespace
+
+extern "C" int nhip_conv2d(void* stream, const int* geom, const float* X, const float* F,
+                           float* Y) {
+    if (!geom || !X || !F || !Y) return NHIP_E_BADARG;
+    ConvLaunch l;
+    const int err = conv_launch(geom, l);
+    if (err) return err;
+    const ConvGeom& g = l.g;
+    const dim3 block(l.threads);
+    if (!l.waves)
+        NHIP_LAUNCH(conv2d_kernel, l.grid, block, l.lds, NHIP_STREAM(stream), g, X, F, Y);
+    else if (!((g.nf | g.f_start) & 3) && !(reinterpret_cast<uintptr_t>(F) & 15))
+        NHIP_LAUNCH(conv2d_wave_kernel<true>, l.grid, block, l.lds, NHIP_STREAM(stream), g, X, F, Y);
+    else
+        NHIP_LAUNCH(conv2d_wave_kernel<false>, l.grid, block, l.lds, NHIP_STREAM(stream), g, X, F, Y);
     NHIP_LAUNCH_CHECK();
+    return 0;
+}
+
+extern "C" int nhip_conv2d_groups(const int* geom, int* n_groups, int* group_threads) {
+    if (!geom || !n_groups || !group_threads) return NHIP_E_BADARG;
+    ConvLaunch l;
+    const int err = conv_launch(geom, l);
+    if (err) return err;
+    *n_groups = l.grid.x * l.grid.y;
+    *group_threads = l.threads;
     return 0;
 }
 

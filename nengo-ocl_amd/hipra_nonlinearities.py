@@ -30,6 +30,7 @@ item) at plan time; argument checks raise the same exception types the
 reference's asserts / raises produce (AssertionError, NotImplementedError).
 """
 
+import ctypes
 import logging
 import re
 
@@ -1065,6 +1066,14 @@ def conv2d_tiles(shape_out_ijf, kernel_shape, strides, nc, channels_last):
     return tile_i, tile_j, tile_f, c_chunk
 
 
+def conv2d_groups(lib, geom):
+    """(work-groups, threads per group) of the launch for the geometry record of `plan_conv2d`; no
+    groups for one that the launch would refuse (an empty image)."""
+    n_groups, threads = ctypes.c_int(0), ctypes.c_int(WG)
+    lib.nhip_conv2d_groups(geom.ctypes.data, ctypes.byref(n_groups), ctypes.byref(threads))
+    return n_groups.value, threads.value
+
+
 def plan_conv2d(queue, X, Y, filters, shape_in, shape_out, kernel_shape, conv=True, biases=None,
                 padding=(0, 0), strides=(1, 1), channels_last=True, tag=None, transposed=False):
     """``Y = conv2d(X, filters)`` (``conv``) or local filtering of one image signal;
@@ -1106,9 +1115,9 @@ def plan_conv2d(queue, X, Y, filters, shape_in, shape_out, kernel_shape, conv=Tr
     geom = np.array([nxi, nxj, nc, nyi, nyj, nf, si, sj, sti, stj, pi, pj, x_start, y_start,
                      f_start, int(bool(channels_last)), int(not conv), tile_i, tile_j, tile_f,
                      c_chunk], dtype=np.int32)
-    n_groups = (-(-nyi // tile_i)) * (-(-nyj // tile_j)) * (-(-nf // tile_f))
+    n_groups, threads = conv2d_groups(queue.lib, geom)
     plan = Plan(queue, queue.lib.nhip_conv2d, (geom.ctypes.data, X.ptr, filters.ptr, Y.ptr),
-                gsize=(WG * n_groups,), lsize=(WG,),
+                gsize=(threads * n_groups,), lsize=(threads,),
                 full_args=(geom, X.dev_buf, filters.dev_buf, Y.dev_buf), name="hip_conv2d", tag=tag)
     plan.flops_per_call = 2 * nyi * nyj * nf * nc * si * sj
     plan.bw_per_call = 4 * (x_size + f_size + y_size)
