@@ -181,15 +181,16 @@ __global__ __launch_bounds__(NHIP_WG) void conv2d_kernel(const ConvGeom g, const
 // and no address arithmetic.  Same order, channel, kernel row, kernel column, one fused
 // multiply-add each; taps outside the image multiply a zero, as the padded patch above does.
 // 26 x 26 x 32 -> 12 x 12 x 64 (9,216 outputs of 288 links) 28.4 -> 7.7 us, 46 x 46 x 40 -> 22 x 22 x 80
-// 41.8 -> 13.0, 128 x 128 x 32 -> 126 x 126 x 32 70.1 -> 45.1, 128 x 128 x 8 -> 126 x 126 x 64 (a
-// million outputs) 42.2 -> 41.0; below 64 links the tiles above are as fast or faster (46 x 46 x 3 ->
-// 44 x 44 x 40 6.2 against 8.2).  Bound by the one trip to memory and the chain.
+// 41.8 -> 13.0.  Bound by the one trip to memory and the chain; which launches take it: see
+// `conv_takes_waves`.
 constexpr int CONV_WF = 16, CONV_WP = 4;
 constexpr int CONV_WAVE_PF = 24;          // loads in flight per lane
 constexpr int CONV_WAVE_LINKS = 16;       // chain links whose operands are read together
 constexpr int CONV_WAVE_MAX_LINKS = 800;  // 64,000 bytes of LDS
 constexpr int CONV_WAVE_MIN_LINKS = 64;
 constexpr long long CONV_WAVE_MAX_OUT = 1 << 20;
+// ... resident groups of a launch: the LDS of 256 compute units, at most 8 waves per SIMD
+constexpr int CONV_N_CU = 256, CONV_CU_LDS = 160 * 1024, CONV_CU_WAVES = 32;
 
 // VEC: filters in whole aligned quads
 template <bool VEC>
@@ -338,6 +339,38 @@ __global__ __launch_bounds__(NHIP_WG) void pool2d_kernel(const PoolGeom g, const
     Y[g.y_start + e] = __fdiv_rn(out, (float)count);
 }
 
+// A group of one wave, or a tile?  A group's staging is paid per 4 pixels, a tile's per tile: the groups
+// win while they are all resident at once, and lose in proportion to their rounds after that
+// unless the tiles need several rounds too, or waste their lanes.  Measured (780 shapes, kernel time in
+// us, groups / tiles; kernel, channels, filters; image sides 28, 64, 128, 256):
+//   3 x 3, 32, 16      7.8/20.6    9.8/21.2   26.6/36.7    79.7/108.8
+//   3 x 3, 32, 2      10.8/23.0   13.0/23.6   37.0/24.2   118.5/28.7
+//   3 x 3, 32, 64      9.2/28.8   25.8/45.9   78.7/148.0       -
+//   3 x 3, 88, 64     39.6/74.1  152.8/119.3       -           -
+//   3 x 3,  8, 4       6.1/7.8     7.5/7.9    13.5/8.0     40.9/12.5
+//   1 x 1, 200, 16        -        9.1/42.0        -       58.8/221.1   (no window to share in a tile)
+//   5 x 5 by 2, 3, 16  9.3/7.7         (few channels: the windows load 16 of them side by side)
+//   7 x 7 by 2, 16, 64, side 200   353.9/215.6
+// By the rule below the launch is at most 4 % behind the tiles on those of several taps (of a
+// single tap: two are, by 10 and 25 %), and 0.7 % behind the better of the two on average.
+bool conv_takes_waves(const ConvGeom& g, long long n_tiles, long long n_groups) {
+    const int taps = g.si * g.sj, links = taps * g.nc;
+    if (!g.f_fast || g.local || (long long)g.nyi * g.nyj * g.nf > CONV_WAVE_MAX_OUT ||
+        links < CONV_WAVE_MIN_LINKS || links > CONV_WAVE_MAX_LINKS)
+        return false;
+    const int lds = links * (CONV_WF + CONV_WP) * (int)sizeof(float);
+    const long long resident = (long long)CONV_N_CU * min(CONV_CU_LDS / lds, CONV_CU_WAVES);
+    // n_groups / resident <= rounds * max(1, n_tiles / tiles)
+    auto within = [&](int rounds, int tiles) {
+        return n_groups * tiles <= rounds * resident * max((long long)tiles, n_tiles);
+    };
+    if (taps == 1) return within(2, CONV_N_CU);
+    if (g.nc < 8 || (links < 100 && n_groups > 2000)) return false;
+    const bool cheap_groups = (g.nf >= 24 && !(g.nf & 3)) ||                 // taps in whole quads
+                              (g.nc >= 32 && g.nf >= 4 && taps <= 9);       // full window loads
+    return within(cheap_groups ? 2 : 1, 3 * CONV_N_CU);
+}
+
 // What a call with geometry `q` launches.
 struct ConvLaunch {
     ConvGeom g;
@@ -379,14 +412,12 @@ int conv_launch(const int* q, ConvLaunch& l) {
     if (l.lds > 64 * 1024) return NHIP_E_BADARG;
     l.grid = dim3(g.tiles_j * tiles_i, (g.nf + g.tile_f - 1) / g.tile_f);
     l.threads = NHIP_WG;
-    const long long n_out = (long long)g.nyi * g.nyj * g.nf;
-    const size_t n_links = taps * g.nc;
-    l.waves = g.f_fast && !g.local && n_out <= CONV_WAVE_MAX_OUT && n_links >= CONV_WAVE_MIN_LINKS &&
-              n_links <= CONV_WAVE_MAX_LINKS;
+    const dim3 waves((g.nyi * g.nyj + CONV_WP - 1) / CONV_WP, (g.nf + CONV_WF - 1) / CONV_WF);
+    l.waves = conv_takes_waves(g, (long long)l.grid.x * l.grid.y, (long long)waves.x * waves.y);
     if (l.waves) {
-        l.grid = dim3((g.nyi * g.nyj + CONV_WP - 1) / CONV_WP, (g.nf + CONV_WF - 1) / CONV_WF);
+        l.grid = waves;
         l.threads = NHIP_WAVE;
-        l.lds = n_links * (CONV_WF + CONV_WP) * sizeof(float);
+        l.lds = taps * g.nc * (CONV_WF + CONV_WP) * sizeof(float);
     }
     return 0;
 }

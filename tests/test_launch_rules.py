@@ -26,3 +26,17 @@ def conv_threads(shape_in, filters, kernel, strides=(1, 1), channels_last=True, 
 def test_launch_size_of_a_convolution_is_that_of_its_kernel(channels_last, conv, expected):
     assert conv_threads((26, 26, 32), 64, (3, 3), (2, 2), channels_last, conv) == expected
     assert conv_threads((26, 26, 3), 64, (3, 3), (2, 2), channels_last, conv) == 256  # 27 links
+
+
+# image, filters, kernel, strides; what the other kernel would cost (measured) stands beside the rule
+@pytest.mark.parametrize("shape_in,filters,kernel,strides,expected", [
+    ((46, 46, 40), 80, (3, 3), (2, 2), 64), ((10, 10, 8), 16, (3, 3), (2, 2), 64),
+    ((28, 28, 32), 256, (3, 3), (1, 1), 64), ((64, 64, 32), 2, (3, 3), (1, 1), 64),
+    ((128, 128, 32), 2, (3, 3), (1, 1), 256), ((512, 512, 88), 1, (3, 3), (1, 1), 256),
+    ((256, 256, 8), 4, (3, 3), (1, 1), 256), ((28, 28, 3), 16, (5, 5), (2, 2), 256),
+    ((200, 200, 16), 64, (7, 7), (2, 2), 256), ((64, 64, 88), 64, (3, 3), (1, 1), 256),
+    ((64, 64, 200), 256, (1, 1), (1, 1), 64), ((256, 256, 400), 2, (1, 1), (1, 1), 256),
+    ((20, 20, 801), 2, (1, 1), (1, 1), 256)])
+def test_convolutions_take_single_wave_groups_where_these_are_resident(shape_in, filters, kernel,
+                                                                       strides, expected):
+    assert conv_threads(shape_in, filters, kernel, strides) == expected
