@@ -351,7 +351,7 @@ __global__ __launch_bounds__(NHIP_WG) void pool2d_kernel(const PoolGeom g, const
 //   1 x 1, 200, 16        -        9.1/42.0        -       58.8/221.1   (no window to share in a tile)
 //   5 x 5 by 2, 3, 16  9.3/7.7         (few channels: the windows load 16 of them side by side)
 //   7 x 7 by 2, 16, 64, side 200   353.9/215.6
-// By the rule below the launch is at most 4 % behind the tiles on those of several taps (of a
+// By the rule below the launch is at most 5 % behind the tiles on those of several taps (of a
 // single tap: two are, by 10 and 25 %), and 0.7 % behind the better of the two on average.
 bool conv_takes_waves(const ConvGeom& g, long long n_tiles, long long n_groups) {
     const int taps = g.si * g.sj, links = taps * g.nc;

@@ -273,12 +273,12 @@ def test_few_long_rows_with_epilogues(queue, pre, dims, lanes):
         net = mb.Network(seed=4, solver="surrogate")
         stim = net.Node(mb.WhiteSignal(period=0.5, high=8.0, seed=3), size_out=2)
         a = net.Ensemble(pre, 2, neuron_type=mb.LIFRate())
-        wide = net.Ensemble(250, dims, radius=3.0)
         net.Connection(stim, a, synapse=None)
-        net.Connection(stim, wide, synapse=mb.Lowpass(0.01), transform=rng.normal(size=(dims, 2)))
         out = net.Node(None, size_in=3)
         net.Connection(a.neurons, out, synapse=mb.Lowpass(0.005),
                        transform=rng.normal(scale=1e-2 / pre, size=(3, pre)))
+        wide = net.Ensemble(250, dims, radius=3.0)
+        net.Connection(stim, wide, synapse=mb.Lowpass(0.01), transform=rng.normal(size=(dims, 2)))
         return net, [net.Probe(out), net.Probe(wide.neurons)]
 
     (net, probes), (net_o, probes_o) = make(), make()
@@ -292,6 +292,31 @@ def test_few_long_rows_with_epilogues(queue, pre, dims, lanes):
         for p, q in zip(probes, probes_o):
             assert np.array_equal(gpu.data[p], cpu.data[q]) and np.any(gpu.data[p] != 0)
         assert np.array_equal(gpu.signal_buffer(), cpu.signal_buffer())
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 700), (503, 700), (1, 5000), (300, 5000)])
+def test_few_long_rows_carry_a_sequence(queue, rng, rows, cols):
+    """Two chains in groups of their own beside those of the rows, which have no epilogue."""
+    from nengo_ocl_amd import hipra_gemv, hipra_sequence
+    from nengo_ocl_amd import hipra_nonlinearities as nl
+    from oracle import oracle as orc
+
+    A, X, Y = RA([rng.normal(size=(rows, cols))]), RA([rng.normal(size=cols)]), RA([rng.normal(size=rows)])
+    C = RA([rng.normal(size=50) for _ in range(4)])
+    js = RA([[0]], dtype=np.int32)
+    dA, dX, dY, dC, Yo = *(to_dev(queue, v) for v in (A, X, Y, C)), clone(Y)
+    plan, = hipra_gemv.plan_block_gemv(queue, 1.5, dA, js, dX, js, 1.0, dY).plans
+    copies = [nl.plan_copy(queue, dC[[k]], dC[[k + 2]], [1]) for k in range(2)]
+    plan.reads_mem, plan.writes_mem = {"A", "X"}, {"Y"}
+    for k, p in enumerate(copies):
+        p.reads_mem, p.writes_mem = {k}, {k + 2}
+    carrier, = hipra_sequence.carry_sequences([plan, hipra_sequence.plan_sequence(queue, copies)])
+    assert carrier is plan and plan.name == "hipra_gemv.tile_rows" and plan.carried is not None
+    plan()
+    orc.plan_block_gemv(None, 1.5, A, js, X, js, 1.0, Yo).plans[0]()
+    assert np.array_equal(dY.buf.view(np.uint32), Yo.buf.view(np.uint32))
+    for k in range(2):
+        assert np.array_equal(dC[k + 2], np.float32(C[k]) + np.float32(C[k + 2]))
 
 
 # rows, columns, elements between rows, of a buffer's start, and pre's stride: four elements of a row
