@@ -158,7 +158,7 @@ int nhip_gemv_tile_rows(int n_cols, int blk_words);
  * -expm1(-dt / tau) formed as the kernel would (float quotient, expm1 in double,
  * rounded once to float), allowed when tau is a scalar and upsample == 1: the
  * launch then evaluates transcendental functions only for the few neurons that
- * leave their refractory period or spike in this step; bit 11, with bit 9, scalar amp,
+ * leave their refractory period or spike in this step; bit 11, with pow2_cols != 0, bit 9, scalar amp,
  * s_start even and every task of the item starting at a multiple of 32 rows: the launch
  * leaves the spikes as one BIT per neuron -- bit r % 64 of the 64-bit word r / 64 at
  * S + s_start, set where neuron r spiked -- and writes no float of S for the item; for

@@ -677,7 +677,8 @@ class Simulator:
 
     def _store_spikes_as_bits(self, plans):
         """Spike signals that nothing but launches visiting active columns reads -- no other
-        launch, no probe, no host copy; written by one large-item neuron launch in tasks that
+        launch, no probe, no host copy; written by one large-item neuron launch (not of the kernel
+        for any shape, class (3, 0, .), which stores floats) in tasks that
         start at multiples of 32 rows; one amplitude per population; zero at the start -- are
         kept as one bit per neuron in the first words of their own memory
         (`hipra_gemv.store_spikes_as_bits`): `_spike_bits` maps such a base to
@@ -687,6 +688,7 @@ class Simulator:
         if self.reference_host_state or not getattr(self.backend, "spikes_as_bits", False):
             return
         encs = [p for p in plans if getattr(p, "name", "") == "hipra_gemv.tile_lif"
+                and getattr(p, "kernel_class", (3, 1, 4))[1] != 0
                 and getattr(p, "dev_pops", None) is not None
                 and getattr(p, "host_tasks", None) is not None]
         events = [p for p in plans if getattr(p, "dev_event_table", None) is not None]

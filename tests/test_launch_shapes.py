@@ -379,3 +379,33 @@ def test_many_rows_of_few_columns(queue, rng, heights, cols, four_lanes):
     run_plans(prog.plans)
     orc.plan_block_gemv(None, 1.5, A, js, X, js, 1.0, Yo, gamma=0.25).plans[0]()
     assert np.array_equal(dY.buf.view(np.uint32), Yo.buf.view(np.uint32))
+
+
+# ensembles of as many neurons as make the tasks of every kind of neuron launch start at multiples of
+# 32 rows: rows that no 16-byte loads fit (70, 99), that lie back to back (50), that 16 bytes fit
+@pytest.mark.parametrize("n_ens,neurons,dims,bits", [
+    (6, 4096, 70, False), (12, 2048, 99, False), (8, 2048, 50, True), (8, 2048, 64, True),
+    (2, 7000, 3, False)])
+def test_spikes_are_bits_only_where_the_launch_writes_bits(queue, n_ens, neurons, dims, bits):
+    """Spikes that nothing but launches visiting active columns reads."""
+    from nengo_ocl_amd import minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    def make():
+        net = mb.Network(seed=3, solver="surrogate")
+        stim = net.Node(mb.WhiteSignal(period=0.5, high=6.0, seed=3), size_out=dims)
+        ens = [net.Ensemble(neurons, dims) for _ in range(n_ens)]
+        for k in range(n_ens):
+            net.Connection(stim, ens[k], synapse=mb.Lowpass(0.005))
+            net.Connection(ens[k], ens[k - 1], synapse=mb.Lowpass(0.005))
+        return net, net.Probe(ens[0], synapse=0.01)
+
+    (net, probe), (net_o, probe_o) = make(), make()
+    with Simulator(net, seed=1) as gpu, OracleSimulator(net_o, seed=1) as cpu:
+        assert any(getattr(p, "event_driven", False) for p in gpu._plans)
+        gpu.run_steps(30)
+        cpu.run_steps(30)
+        assert np.any(gpu.data[probe] != 0) and np.array_equal(gpu.data[probe], cpu.data[probe_o])
+        assert np.array_equal(gpu.signal_buffer(), cpu.signal_buffer())
+        assert bool(gpu._spike_bits) == bits
