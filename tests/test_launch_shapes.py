@@ -409,3 +409,42 @@ def test_spikes_are_bits_only_where_the_launch_writes_bits(queue, n_ens, neurons
         assert np.any(gpu.data[probe] != 0) and np.array_equal(gpu.data[probe], cpu.data[probe_o])
         assert np.array_equal(gpu.signal_buffer(), cpu.signal_buffer())
         assert bool(gpu._spike_bits) == bits
+
+
+@pytest.mark.parametrize("what", ["conv", "long rows", "group per row", "oja", "voja", "bcm"])
+def test_infinities_and_nan_reach_the_results_they_reach_in_the_oracle(queue, rng, what):
+    from nengo_ocl_amd import hipra_gemv
+    from nengo_ocl_amd import hipra_nonlinearities as nl
+    from oracle import oracle as orc
+
+    def odd(n, share=0.004):
+        v = rng.normal(size=n)
+        at = rng.uniform(size=n) < share
+        v[at] = rng.choice([np.nan, np.inf, -np.inf, -0.0, np.finfo(np.float32).max], size=at.sum())
+        return v
+
+    if what == "conv":
+        data = RA([odd(9 * 8 * 16), odd(9 * 16 * 20, 0.001), np.zeros(9 * 8 * 20)])
+        run = lambda mod, q, d: [mod.plan_conv2d(q, d[[0]], d[[2]], d[[1]], (9, 8, 16), (9, 8, 20),
+                                                 (3, 3), padding="same", channels_last=True)]
+    elif what in ("long rows", "group per row"):
+        m, n = {"long rows": (90, 700), "group per row": (40, 4100)}[what]
+        data = RA([odd(m * n, 1 / 3000).reshape(m, n), odd(n, 1 / 2000), odd(m, 0.05)])
+        js = RA([[0]], dtype=np.int32)
+        run = lambda mod, q, d: mod.plan_block_gemv(
+            q, 1.0, d[[0]], RA([[0]], dtype=np.int32), d[[1]], js, 1.0, d[[2]]).plans
+    else:
+        data = RA([odd(100), odd(130, 0.05), odd(130 * 100).reshape(130, 100), odd(130), odd(1), odd(130),
+                   odd(130 * 100).reshape(130, 100)])
+        alpha, beta = np.float32([1e-3]), np.float32([1.5])
+        run = lambda mod, q, d: [
+            mod.plan_oja(q, d[[0]], d[[1]], d[[2]], d[[6]], alpha, beta, inc=True) if what == "oja" else
+            mod.plan_bcm(q, d[[0]], d[[1]], d[[3]], d[[6]], alpha, inc=True) if what == "bcm" else
+            mod.plan_voja(q, d[[0]], d[[1]], d[[2]], d[[6]], d[[4]], d[[5]], alpha, inc=True)]
+    dev = to_dev(queue, data)
+    run_plans(run(nl if what in ("conv", "oja", "voja", "bcm") else hipra_gemv, queue, dev))
+    run_plans(run(orc, None, data))
+    got, expected = dev.buf, data.buf
+    nan = np.isnan(expected)
+    assert nan.any() and not nan.all() and np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(got[~nan].view(np.uint32), expected[~nan].view(np.uint32))
