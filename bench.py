@@ -601,14 +601,15 @@ def main():
     roofline = None
     if dom is not None:
         traffic, traffic_source = None, None
-        if args.config == "c3" and args.variant == "shared" and args.scale == 1.0:
+        if (args.config == "c3" and args.variant == "shared" and args.scale == 1.0
+                and "long-rows" not in dom["plan"]):
             traffic, traffic_source = measured_traffic(dom["name"])
         roofline = dict(bound="hbm", achieved=dom["gbs"], peak=HBM_PEAK_GBS, unit="GB/s",
                         frac=dom["gbs"] / HBM_PEAK_GBS, traffic=traffic,
                         traffic_source=traffic_source, kernel=dom["plan"],
                         avg_us=dom["avg_us"], bytes_per_launch=dom["bytes"])
         lif = next((p for p in sim._plans if str(p) == dom["plan"]
-                    and p.name == "hipra_gemv.tile_lif"), None)
+                    and p.name == "hipra_gemv.tile_lif" and p.kernel_class[0] == 3), None)
         if lif is not None:
             # the same traffic through a kernel that does nothing else: rows = neurons of the
             # launch, columns from its matrix bytes

@@ -215,7 +215,7 @@ def _balanced_rows(M, cap):
 class gemv_prog:
     """Geometry + work lists of one ragged GEMV; subclasses pick the kernel classes."""
 
-    # None = reference summation order (kernels "wave_ref", "tile" and "tile_rows"); 0 = work-group
+    # None = reference summation order (kernels "wave_ref" and "tile"); 0 = work-group
     # kernel and 1 = wave kernel with their own, faster-to-reduce order
     force_flavor = None
     force_scalar = False  # one lane per output, 4-byte loads (the plain fallback)
@@ -743,9 +743,13 @@ class gemv_prog:
                 self.queue, kern, args, gsize=(WG * n_groups,), lsize=(WG,),
                 full_args=(dev_items, dev_coefs, dev_dots, dev_tasks, self.A.dev_buf,
                            self.X.dev_buf, self.Y_in.dev_buf, self.Y.dev_buf),
-                name="hipra_gemv.%s" % ("tile_rows" if flavor == 2 and lpr >= LONG_ROWS else
-                                        ("wg", "wave", "wave_ref", "tile")[flavor]),
-                tag="%s-lpr%d-v%d" % (self.tag, lpr, vec),
+                # (rows shared by a wave or a group are named after their items' ordinary launch:
+                # which kernel runs is in `kernel_class`, and in the tag)
+                name="hipra_gemv.%s" % (
+                    "tile" if flavor == 2 and lpr >= LONG_ROWS and not set(members) <= set(small)
+                    else ("wg", "wave", "wave_ref", "tile")[flavor]),
+                tag=("%s-long-rows%d" % (self.tag, lpr) if flavor == 2 and lpr >= LONG_ROWS else
+                     "%s-lpr%d-v%d" % (self.tag, lpr, vec)),
                 bw_per_call=bw_from_geometry(geometry, members),
                 flops_per_call=flops_from_geometry(geometry, members),
             )
@@ -866,8 +870,8 @@ def _subset_param(param, idx):
 
 
 def _takes_epilogue(plan):
-    """Reference-order launches (large or small items, long rows) that do not have an epilogue yet."""
-    return (plan.name in ("hipra_gemv.tile", "hipra_gemv.wave_ref", "hipra_gemv.tile_rows")
+    """Reference-order launches (large or small items) that do not have an epilogue yet."""
+    return (plan.name in ("hipra_gemv.tile", "hipra_gemv.wave_ref")
             and getattr(plan, "kernel_class", (None,))[0] in (2, 3))
 
 

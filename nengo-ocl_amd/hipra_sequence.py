@@ -223,7 +223,7 @@ def _can_carry(plan, needs=0):
     if cls is None or getattr(plan, "prelude", None) is not None or getattr(plan, "n_tasks", 0) <= 0:
         return False
     if cls[0] == 2:
-        return name in tuple("hipra_gemv." + k + e for k in ("wave_ref", "tile_rows")
+        return name in tuple("hipra_gemv." + k + e for k in ("wave_ref", "tile")
                              for e in ("", "_lif", "_filter"))
     if name in ("hipra_gemv.tile_lif", "hipra_gemv.tile_filter"):
         return cls[0] == 3 and cls[1] >= 2

@@ -688,7 +688,8 @@ class Simulator:
         if self.reference_host_state or not getattr(self.backend, "spikes_as_bits", False):
             return
         encs = [p for p in plans if getattr(p, "name", "") == "hipra_gemv.tile_lif"
-                and getattr(p, "kernel_class", (3, 1, 4))[1] != 0
+                and getattr(p, "kernel_class", (3, 1))[0] == 3
+                and getattr(p, "kernel_class", (3, 1))[1] != 0
                 and getattr(p, "dev_pops", None) is not None
                 and getattr(p, "host_tasks", None) is not None]
         events = [p for p in plans if getattr(p, "dev_event_table", None) is not None]

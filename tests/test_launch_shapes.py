@@ -262,8 +262,8 @@ def test_few_long_rows(queue, rng, beta, widths):
                          ids=["wave per row", "group per row"])
 def test_few_long_rows_with_epilogues(queue, pre, dims, lanes):
     """Encoders of many dimensions and decoders of many neurons: long rows whose launch also updates the
-    neurons or steps the filters, and carries a sequence, bit for bit like the oracle's; the
-    launches have a name of their own."""
+    neurons or steps the filters, and carries a sequence, bit for bit like the oracle's; class and
+    tag tell them from large-item launches of the same name."""
     from nengo_ocl_amd import minibuilder as mb
     from nengo_ocl_amd.simulator import Simulator
     from oracle.oracle_sim import OracleSimulator
@@ -283,9 +283,10 @@ def test_few_long_rows_with_epilogues(queue, pre, dims, lanes):
 
     (net, probes), (net_o, probes_o) = make(), make()
     with Simulator(net, seed=1) as gpu, OracleSimulator(net_o, seed=1) as cpu:
-        rows = {p.name: p for p in gpu._plans if p.name.startswith("hipra_gemv.tile_rows")}
-        assert set(rows) == {"hipra_gemv.tile_rows_lif", "hipra_gemv.tile_rows_filter"}
-        assert {p.kernel_class for p in rows.values()} == {(2, lanes, 1)}
+        rows = {p.name: p for p in gpu._plans if getattr(p, "kernel_class", ()) == (2, lanes, 1)}
+        assert set(rows) == {"hipra_gemv.tile_lif", "hipra_gemv.tile_filter"}
+        assert all("long-rows%d" % lanes in p.tag for p in rows.values())
+        assert not any("long-rows" in p.tag for p in gpu._plans if p not in rows.values() and p.tag)
         assert any(getattr(p, "carried", None) is not None for p in rows.values())
         gpu.run_steps(60)
         cpu.run_steps(60)
@@ -311,7 +312,7 @@ def test_few_long_rows_carry_a_sequence(queue, rng, rows, cols):
     for k, p in enumerate(copies):
         p.reads_mem, p.writes_mem = {k}, {k + 2}
     carrier, = hipra_sequence.carry_sequences([plan, hipra_sequence.plan_sequence(queue, copies)])
-    assert carrier is plan and plan.name == "hipra_gemv.tile_rows" and plan.carried is not None
+    assert carrier is plan and plan.kernel_class[0] == 2 and plan.carried is not None
     plan()
     orc.plan_block_gemv(None, 1.5, A, js, X, js, 1.0, Yo).plans[0]()
     assert np.array_equal(dY.buf.view(np.uint32), Yo.buf.view(np.uint32))
