@@ -98,7 +98,9 @@ WG, WAVE = 256, 64
 # 128-column tile, instead of four lanes per row (up to 512 columns) or a wave that walks
 # whole rows.  Measured (kernel time, this / the other): 64 x 128 3.9 / 3.9 us, 1024 x 200
 # 3.9 / 4.4, 2048 x 384 3.9 / 6.0, 4096 x 384 5.3 / 6.1, 8192 x 256 7.6 / 4.9; 512 x 1000 3.9 / 4.8,
-# 2048 x 2048 6.1 / 7.0, 4096 x 1000 7.1 / 6.0, 1024 x 9216 13.1 / 17.0, 2048 x 4096 10.8 / 10.1.
+# 2048 x 2048 6.1 / 7.0, 4096 x 1000 7.1 / 6.0, 1024 x 9216 13.1 / 17.0, 2048 x 4096 10.8 / 10.1; 576
+# shapes inside the limits, up to 64 x 1,000,000 and 1024 x 65,536: at most 0.1 us behind (with the
+# neuron update 1500 and 2048 rows of 512 5.5 / 5.0).
 LONG_ROWS, LONG_ROW_MIN_COLS = 128, 160
 LONG_ROWS_MAX, LONG_ROWS_MAX_ELEMS, LONG_ROWS_ANY_WIDTH = 2048, 1 << 22, 1024
 # ... and a work-group per row where a row takes a wave several passes and the groups still fit
@@ -109,7 +111,9 @@ THIN_MIN_ROWS, THIN_ROWS_FOR_LANE_PER_ROW = 32, 65536
 # ... and below that limit four lanes per row with the small items, also for items of more than
 # SMALL_ITEM_ELEMS, unless a launch of large items stays anyway: launches of up to 21,632 rows of
 # one column 3.0 us instead of 6.2 through LDS; a step of the two convolution layers they feed
-# 47.5 -> 39.3 us, and 41.0 with a lane per row in a launch of their own.  Longer rows keep the LDS
+# 47.5 -> 39.3 us, and 41.0 with a lane per row in a launch of their own.  Longer rows keep the LDS.
+# Up to 65,535 rows of one to three columns: alone, with filters or the neuron update 3.9-4.5 us, through
+# LDS 5.6-9.6; whole steps of 2 x 5,500 x 3 to 2 x 30,000 x 1 LIF neurons 17.1-58.5 us against 22.1-64.3.
 THIN_CLASS, THIN_MAX_COLS = (2, 4, 1), 4
 LIF_POP_ENABLED, LIF_POP_DECAY, LIF_POP_NO_J = 1 << 8, 1 << 9, 1 << 10  # flag bits of a population row
 LIF_POP_BITS = 1 << 11  # spikes stored as a bit per neuron (see `store_spikes_as_bits`)
