@@ -193,6 +193,28 @@ int nhip_gemv_tile_lif_sums(void *stream, int vec, int pow2_cols, int blk_words,
                             int upsample, float *V, float *W, float *S, const float *TAU,
                             const float *REF, const float *AMP, const int *parts);
 
+/* nhip_gemv_tile followed by the update of neurons of another type than the plain LIF, in one
+ * launch: replaces `plan_block_gemv` + `plan_lif` with N, `plan_lif_rate`, `plan_rectified_linear`,
+ * `plan_spiking_rectified_linear` or `plan_sigmoid` (clra_nonlinearities.py:1028-1283).
+ *   pops : int32[n_items][12] {v_start, w_start, out_start, n_start, tau, ref, amp, tau_n (float
+ *          bits), inc_n (float bits), kind, flags, 0}; kind 1 LIF rate, 2 adaptive LIF, 3 adaptive
+ *          LIF rate, 4 rectified linear, 5 spiking rectified linear, 6 sigmoid (its ref); flags as
+ *          bits 8 and 10 of nhip_gemv_tile_lif's pflags.
+ * V, W, N: voltages, refractory times, adaptations (any valid buffer for types without one), S the
+ * outputs.  `parts` as for nhip_gemv_tile_lif_sums, or NULL.  nhip_gemv_rows_neuron: the same for
+ * launches of small items; sum_ranges and parts as for nhip_gemv_rows_lif_sums, or both NULL (the
+ * spare words of 16-word task records are not read).  Results are those of the separate calls. */
+int nhip_gemv_tile_neuron(void *stream, int vec, int pow2_cols, int blk_words, const int *items,
+                          const float *coefs, const int *dots, const int *tasks, int n_tasks,
+                          const float *A, const float *X, const float *Yin, float *Y,
+                          const int *pops, double dt, int upsample, float *V, float *W, float *S,
+                          float *N, const int *parts);
+int nhip_gemv_rows_neuron(void *stream, int lpr, int task_words, const int *items,
+                          const float *coefs, const int *dots, const int *tasks, int n_tasks,
+                          const float *A, const float *X, const float *Yin, float *Y,
+                          const int *pops, double dt, int upsample, float *V, float *W, float *S,
+                          float *N, const int *sum_ranges, const int *parts);
+
 /* nhip_gemv_tile followed by the step of first-order filters on its outputs, in one
  * launch: replaces `plan_block_gemv` (clra_gemv.py:1193-1195) + the simple case of
  * `plan_linearfilter` (clra_nonlinearities.py:577-803, one numerator and at most one

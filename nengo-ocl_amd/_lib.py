@@ -33,6 +33,10 @@ SIGNATURES = {
                            P, ctypes.c_double, c_int, P, P, P, P, P, P],
     "nhip_gemv_tile_lif_sums": [P, c_int, c_int, c_int, P, P, P, P, c_int, P, P, P, P,
                                 P, ctypes.c_double, c_int, P, P, P, P, P, P, P],
+    "nhip_gemv_tile_neuron": [P, c_int, c_int, c_int, P, P, P, P, c_int, P, P, P, P,
+                              P, ctypes.c_double, c_int, P, P, P, P, P],
+    "nhip_gemv_rows_neuron": [P, c_int, c_int, P, P, P, P, c_int, P, P, P, P,
+                              P, ctypes.c_double, c_int, P, P, P, P, P, P],
     "nhip_gemv_tile_filter": [P, c_int, c_int, c_int, P, P, P, P, c_int, P, P, P, P, P, P, P],
     "nhip_gemv_tile_filter_learn": [P, c_int, c_int, c_int, P, P, P, P, c_int, P, P, P, P, P, P, P, P],
     "nhip_gemv_tile_lif_deferred": [P, c_int, c_int, c_int, P, P, P, P, c_int, P, P, P, P,

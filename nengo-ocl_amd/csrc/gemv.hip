@@ -312,7 +312,7 @@ int launch_rows_epi(hipStream_t s, int lpr, int task_words, const int* items, co
     if (lpr != 4 && lpr != 1 && lpr != NHIP_WAVE && lpr != NHIP_LPR_LONG_ROWS && lpr != NHIP_WG) return NHIP_E_BADCLASS;
     if (task_words != 4 && task_words != 16) return NHIP_E_BADARG;
     if (lpr >= NHIP_WAVE && task_words != 16) return NHIP_E_BADARG;  // a wave per task
-    if (lpr >= NHIP_LPR_LONG_ROWS && EPI == EPI_LIF && epi.lif.sum_ranges) return NHIP_E_BADARG;
+    if (lpr >= NHIP_LPR_LONG_ROWS && (EPI == EPI_LIF || EPI == EPI_NEURON) && epi.lif.sum_ranges) return NHIP_E_BADARG;
     const int rows_per_group = lpr == NHIP_WG ? 1 : (NHIP_WG / NHIP_WAVE) * (lpr >= NHIP_WAVE ? 1 : NHIP_WAVE / lpr);
     side.n_gemv_groups = (n_tasks + rows_per_group - 1) / rows_per_group;
     const dim3 grid(side.n_gemv_groups + side.n_chains);
@@ -591,6 +591,32 @@ extern "C" int nhip_gemv_rows_lif_sums(void* stream, int lpr, int task_words, co
     lif.sum_ranges = reinterpret_cast<const int2*>(sum_ranges);
     return launch_rows_epi<EPI_LIF>(static_cast<hipStream_t>(stream), lpr, task_words, items, coefs,
                                     dots, tasks, n_tasks, A, X, Yin, Y, args);
+}
+
+extern "C" int nhip_gemv_rows_neuron(void* stream, int lpr, int task_words, const int* items,
+                                     const float* coefs, const int* dots, const int* tasks,
+                                     int n_tasks, const float* A, const float* X, const float* Yin,
+                                     float* Y, const int* pops, double dt, int upsample, float* V,
+                                     float* W, float* S, float* N, const int* sum_ranges,
+                                     const int* parts) {
+    if (!pops || !V || !W || !S || !N || upsample < 1 || !(dt > 0.0)) return NHIP_E_BADARG;
+    if ((sum_ranges == nullptr) != (parts == nullptr)) return NHIP_E_BADARG;
+    if (parts && static_cast<const float*>(Y) != X) return NHIP_E_BADARG;  // the sums are stored through Y
+    EpilogueArgs args{};
+    LifArgs& lif = args.lif;
+    lif.pops = reinterpret_cast<const LifPop*>(pops);
+    lif.dt = (float)dt;
+    lif.dtu = (float)(dt / (double)upsample);
+    lif.dt_inv = (float)(1.0 / dt);
+    lif.upsample = upsample;
+    lif.V = V;
+    lif.W = W;
+    lif.S = S;
+    lif.N = N;
+    lif.sum_ranges = reinterpret_cast<const int2*>(sum_ranges);
+    lif.parts = reinterpret_cast<const int2*>(parts);
+    return launch_rows_epi<EPI_NEURON>(static_cast<hipStream_t>(stream), lpr, task_words, items, coefs,
+                                       dots, tasks, n_tasks, A, X, Yin, Y, args);
 }
 
 extern "C" int nhip_gemv_rows_filter(void* stream, int lpr, int task_words, const int* items,

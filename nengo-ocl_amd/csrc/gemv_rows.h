@@ -30,8 +30,8 @@
 // value) is requested as soon as the task is known, not after the sums.  Task, item and
 // dot records are per-lane values on purpose (different rows of a wave may belong to
 // different items).
-// EPI: what happens to a finished row besides being stored -- nothing, the LIF update
-// of the neuron whose input current the row is, or the step of the first-order filters
+// EPI: what happens to a finished row besides being stored -- nothing, the update
+// of the neuron whose input current the row is (LIF, or another type), or the step of the first-order filters
 // fed by the row (the same epilogues as the kernel for large items has; small
 // populations and low-dimensional decoded values save a launch the same way).
 // WIDE: the task table holds GemvRowTask records.
@@ -49,6 +49,7 @@ __device__ __forceinline__ void gemv_rows_ref_block(
     const EpilogueArgs* epi = nullptr)
 {
     constexpr int TILE = 128;
+    constexpr bool NEURONS = EPI == EPI_LIF || EPI == EPI_NEURON;
     constexpr int BATCH = 4;             // dot products whose operands are fetched together
     constexpr int CHUNK = 8;             // steps of a partial sum whose operands are fetched together
     constexpr int ROWS = LPR > NHIP_WAVE ? 1 : NHIP_WAVE / LPR;  // rows (tasks) per wave
@@ -83,7 +84,8 @@ __device__ __forceinline__ void gemv_rows_ref_block(
     // epilogue operands, fetched ahead (no branch around the loads: a row without a
     // population or a target reads the first element of the buffer instead)
     LifPop pop = {};
-    float v_old = 0.0f, w_old = 0.0f;
+    NeuronPop npop = {};
+    float v_old = 0.0f, w_old = 0.0f, n_old = 0.0f;
     int2 f_range = make_int2(0, 0);
     FilterTarget f_first = {};
     float f_old = 0.0f;
@@ -95,18 +97,24 @@ __device__ __forceinline__ void gemv_rows_ref_block(
         v_old = epi->lif.V[enabled ? (size_t)(WIDE ? task.pad : pop.v_start) + r : 0];
         w_old = epi->lif.W[enabled ? (size_t)(WIDE ? it.pad : pop.w_start) + r : 0];
     }
+    if (EPI == EPI_NEURON) {
+        npop = reinterpret_cast<const NeuronPop*>(epi->lif.pops)[task.item];
+        v_old = epi->lif.V[neuron_has_v(npop.kind) ? (size_t)npop.v_start + r : 0];
+        w_old = epi->lif.W[neuron_has_w(npop.kind) ? (size_t)npop.w_start + r : 0];
+        n_old = epi->lif.N[neuron_has_n(npop.kind) ? (size_t)npop.n_start + r : 0];
+    }
     if (EPI == EPI_FILTER) {
         f_range = WIDE ? make_int2(task.pad, it.pad) : epi->filter.item_targets[task.item];
         f_first = epi->filter.targets[f_range.y > 0 ? f_range.x : 0];
         f_old = epi->filter.F[f_range.y > 0 ? (size_t)f_first.y_start + r : 0];
     }
     float sum = cf.y * Yin[it.yin_start + (size_t)r * it.yin_stride0];
-    // LIF launches that form input sums themselves: the vector operand of the item's first
+    // Launches with neurons that form input sums themselves: the vector operand of the item's first
     // dot product (at most 4 columns), or the whole row of an item without dot products, is
     // (...(0 + v_0[c] s_0) + v_1[c] s_1) + ..., what this kernel computes for
     // Y = 0 * Y + sum_k v_k s_k as a launch of its own
     int2 sum_range = make_int2(0, 0);
-    if (EPI == EPI_LIF && epi->lif.sum_ranges != nullptr && (WAVE_TASK ? slot < n_tasks : valid))
+    if (NEURONS && epi->lif.sum_ranges != nullptr && (WAVE_TASK ? slot < n_tasks : valid))
         sum_range = epi->lif.sum_ranges[task.item];
     if (WAVE_TASK)  // the same for all lanes of the wave (the lanes past the task's rows take part)
         sum_range = make_int2(__builtin_amdgcn_readfirstlane(sum_range.x),
@@ -172,7 +180,7 @@ __device__ __forceinline__ void gemv_rows_ref_block(
     };
     // (WAVE_TASK: the whole wave forms the sum, also the lanes past the task's rows, whose reads
     // the others use; the condition is the same for all of them)
-    if (EPI == EPI_LIF && sum_range.y > 0 && (WAVE_TASK ? it.n_dots == 0 : n_dots == 0)) sum = summed(r);
+    if (NEURONS && sum_range.y > 0 && (WAVE_TASK ? it.n_dots == 0 : n_dots == 0)) sum = summed(r);
 
     if (LPR >= NHIP_WAVE) {
         // Everything but the columns is the same for all lanes.  The operands of a lane's partial
@@ -246,7 +254,7 @@ __device__ __forceinline__ void gemv_rows_ref_block(
                     const bool live = d0 + k < n_dots && c < dot[k].N;
                     a[k][e] = live ? A[dot[k].a_start + (size_t)r * dot[k].a_stride0 + c] : 0.0f;
                     x[k][e] = live ? X[dot[k].x_start + (size_t)c * dot[k].x_stride0] : 0.0f;
-                    if (WAVE_TASK && EPI == EPI_LIF && k == 0 && d0 == 0 && sum_range.y > 0 &&
+                    if (WAVE_TASK && NEURONS && k == 0 && d0 == 0 && sum_range.y > 0 &&
                         __any(live)) {
                         // (all lanes of the wave run the sum: its reads are spread over them)
                         const float xs = summed_uniform(c);
@@ -254,7 +262,7 @@ __device__ __forceinline__ void gemv_rows_ref_block(
                             x[k][e] = xs;
                             if (r == 0) Y[(size_t)dot[k].x_start + c] = xs;
                         }
-                    } else if (EPI == EPI_LIF && k == 0 && d0 == 0 && live && sum_range.y > 0) {
+                    } else if (NEURONS && k == 0 && d0 == 0 && live && sum_range.y > 0) {
                         x[k][e] = summed(c);
                         // the item's first row also stores the sum in the operand's place
                         if (r == 0) Y[(size_t)dot[k].x_start + c] = x[k][e];
@@ -313,10 +321,13 @@ __device__ __forceinline__ void gemv_rows_ref_block(
     }
     if (lir == 0 && valid) {
         const float y = sum + cf.z;
-        if (!(EPI == EPI_LIF && (pop.pflags & LIF_POP_NO_J)))
+        if (!(EPI == EPI_LIF && (pop.pflags & LIF_POP_NO_J)) &&
+            !(EPI == EPI_NEURON && (npop.flags & LIF_POP_NO_J)))
             Y[it.y_start + (size_t)r * it.y_stride0] = y;
         if (EPI == EPI_LIF && (pop.pflags & LIF_POP_ENABLED))
             lif_epilogue(epi->lif, pop, r, y, v_old, w_old);
+        if (EPI == EPI_NEURON && (npop.flags & LIF_POP_ENABLED))
+            neuron_epilogue(epi->lif, npop, r, y, v_old, w_old, n_old);
         if (EPI == EPI_FILTER && f_range.y > 0) {
             // the first target with what was fetched ahead (the arithmetic of
             // filter_epilogue), further targets of the item from memory

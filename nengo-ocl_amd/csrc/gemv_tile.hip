@@ -316,14 +316,17 @@ __global__ __launch_bounds__(NHIP_WG) void gemv_tile_kernel(
     // current of neuron r of the item's population, which is updated on the spot; with
     // the filter epilogue it is the new input of element r of the item's filters
     LifPop pop = {};
+    NeuronPop npop = {};
     int2 filters = make_int2(0, 0);
     if (EPI == EPI_LIF) pop = epi.lif.pops[task.item];
+    if (EPI == EPI_NEURON) npop = reinterpret_cast<const NeuronPop*>(epi.lif.pops)[task.item];
     if (EPI == EPI_FILTER) filters = make_int2(task.pad, it.pad);  // rides in the task record
     // an item without dot products that would copy Y onto itself unchanged is only
     // there for its epilogue (a constant input current): nothing to store
     const bool store_y = !(it.n_dots == 0 && cf.y == 1.0f && cf.z == 0.0f && Y == Yin &&
                            it.y_start == it.yin_start && it.y_stride0 == it.yin_stride0) &&
-                         !(EPI == EPI_LIF && (pop.pflags & LIF_POP_NO_J));
+                         !(EPI == EPI_LIF && (pop.pflags & LIF_POP_NO_J)) &&
+                         !(EPI == EPI_NEURON && (npop.flags & LIF_POP_NO_J));
 #pragma unroll
     for (int k = 0; k < ROW_SLOTS; ++k) {
         const int r = lane + k * NHIP_WAVE;
@@ -334,6 +337,13 @@ __global__ __launch_bounds__(NHIP_WG) void gemv_tile_kernel(
                 const int i = task.row0 + r;
                 lif_epilogue(epi.lif, pop, i, y, epi.lif.V[(size_t)pop.v_start + i],
                              epi.lif.W[(size_t)pop.w_start + i]);
+            }
+            if (EPI == EPI_NEURON && (npop.flags & LIF_POP_ENABLED)) {
+                const int i = task.row0 + r;
+                neuron_epilogue(epi.lif, npop, i, y,
+                                epi.lif.V[neuron_has_v(npop.kind) ? (size_t)npop.v_start + i : 0],
+                                epi.lif.W[neuron_has_w(npop.kind) ? (size_t)npop.w_start + i : 0],
+                                epi.lif.N[neuron_has_n(npop.kind) ? (size_t)npop.n_start + i : 0]);
             }
             if (EPI == EPI_FILTER) filter_epilogue(epi.filter, filters, task.row0 + r, y);
         }
@@ -521,9 +531,10 @@ template <int EPI, int SLOTS>
 __device__ __forceinline__ void finish_task(const GemvTask& task, const GemvItem& it,
                                             const float4& cf, const float* ys, float* ab,
                                             const float* Yin, float* Y, const EpilogueArgs& epi,
-                                            const LifPop& pop, const float (&v_in)[SLOTS],
-                                            const float (&w_in)[SLOTS],
-                                            const FilterPrefetch& fp, int lane) {
+                                            const LifPop& pop, const NeuronPop& npop,
+                                            const float (&v_in)[SLOTS], const float (&w_in)[SLOTS],
+                                            const float (&n_in)[SLOTS], const FilterPrefetch& fp,
+                                            int lane) {
     const int n_rows = task.n_rows;
     const int2 filters = fp.range;
     const int n_pairs = fp.n_pairs;
@@ -532,7 +543,8 @@ __device__ __forceinline__ void finish_task(const GemvTask& task, const GemvItem
     // there for its epilogue (a constant input current): nothing to store
     const bool store_y = !(it.n_dots == 0 && cf.y == 1.0f && cf.z == 0.0f && Y == Yin &&
                            it.y_start == it.yin_start && it.y_stride0 == it.yin_stride0) &&
-                         !(EPI == EPI_LIF && (pop.pflags & LIF_POP_NO_J));
+                         !(EPI == EPI_LIF && (pop.pflags & LIF_POP_NO_J)) &&
+                         !(EPI == EPI_NEURON && (npop.flags & LIF_POP_NO_J));
     if (EPI == EPI_LIF && (pop.pflags & LIF_POP_DECAY)) {
         lif_task_compacted<SLOTS>(epi.lif, pop, task.row0, n_rows, ys, cf.z,
                            store_y ? Y + it.y_start : nullptr, it.y_stride0, ab, lane, v_in, w_in);
@@ -546,6 +558,8 @@ __device__ __forceinline__ void finish_task(const GemvTask& task, const GemvItem
             if (store_y) Y[it.y_start + (size_t)(task.row0 + r) * it.y_stride0] = y;
             if (EPI == EPI_LIF && (pop.pflags & LIF_POP_ENABLED))
                 lif_epilogue(epi.lif, pop, task.row0 + r, y, v_in[k], w_in[k]);
+            if (EPI == EPI_NEURON && (npop.flags & LIF_POP_ENABLED))
+                neuron_epilogue(epi.lif, npop, task.row0 + r, y, v_in[k], w_in[k], n_in[k]);
         }
     }
     if (EPI == EPI_FILTER) {
@@ -564,6 +578,21 @@ __device__ __forceinline__ void finish_task(const GemvTask& task, const GemvItem
             const FilterTarget t = epi.filter.targets[filters.x + q];
             step(t, r, epi.filter.F[(size_t)t.y_start + task.row0 + r]);
         }
+    }
+}
+
+// EPI_NEURON: the states of the task's neurons (types without one read the buffer's first element)
+template <int SLOTS>
+__device__ __forceinline__ void fetch_states(const LifArgs& a, const NeuronPop& p, int row0, int n_rows,
+                                             int lane, float (&v_in)[SLOTS], float (&w_in)[SLOTS],
+                                             float (&n_in)[SLOTS]) {
+    const bool on = p.flags & LIF_POP_ENABLED;
+#pragma unroll
+    for (int k = 0; k < SLOTS; ++k) {
+        const int i = row0 + min(lane + k * NHIP_WAVE, n_rows - 1);
+        v_in[k] = a.V[on && neuron_has_v(p.kind) ? (size_t)p.v_start + i : 0];
+        w_in[k] = a.W[on && neuron_has_w(p.kind) ? (size_t)p.w_start + i : 0];
+        n_in[k] = a.N[on && neuron_has_n(p.kind) ? (size_t)p.n_start + i : 0];
     }
 }
 
@@ -790,7 +819,12 @@ __global__ __launch_bounds__(NHIP_WG) void gemv_tile_p2_kernel(
     // would stall the wave for a memory round trip with nothing else in flight; read
     // before the matrix loads, the population record would hold those back).
     LifPop pop = {};
-    float v_in[ROW_SLOTS] = {}, w_in[ROW_SLOTS] = {};
+    NeuronPop npop = {};
+    float v_in[ROW_SLOTS] = {}, w_in[ROW_SLOTS] = {}, n_in[ROW_SLOTS] = {};
+    if (EPI == EPI_NEURON) {
+        npop = reinterpret_cast<const NeuronPop*>(epi.lif.pops)[task.item];
+        fetch_states<ROW_SLOTS>(epi.lif, npop, task.row0, n_rows, lane, v_in, w_in, n_in);
+    }
     if (EPI == EPI_LIF) {
         pop = epi.lif.pops[task.item];
         if (pop.pflags & LIF_POP_ENABLED) {
@@ -836,7 +870,7 @@ __global__ __launch_bounds__(NHIP_WG) void gemv_tile_p2_kernel(
         fp.row[k] = f_row[k];
         fp.old[k] = f_old[k];
     }
-    finish_task<EPI, ROW_SLOTS>(task, it, cf, ys, ab, Yin, Y, epi, pop, v_in, w_in, fp, lane);
+    finish_task<EPI, ROW_SLOTS>(task, it, cf, ys, ab, Yin, Y, epi, pop, npop, v_in, w_in, n_in, fp, lane);
 }
 
 
@@ -931,6 +965,7 @@ __global__ __launch_bounds__(NHIP_WG) __attribute__((amdgpu_waves_per_eu((VAR & 
     constexpr bool FLAT = (SET & SET_FLAT) != 0;
     constexpr bool LEARN = EPI == EPI_FILTER && (VAR & VAR_LEARN) != 0;
     constexpr bool DEFER = EPI == EPI_LIF && (VAR & VAR_DEFER) != 0;
+    constexpr bool NEURONS = EPI == EPI_LIF || EPI == EPI_NEURON;
     static_assert(!(LEARN && FLAT), "learned matrices: rows on 16-byte boundaries");
     static_assert(!(FLAT && WIDE), "back-to-back rows: single-stage widths only");
     extern __shared__ __attribute__((aligned(16))) float lds[];
@@ -989,7 +1024,8 @@ __global__ __launch_bounds__(NHIP_WG) __attribute__((amdgpu_waves_per_eu((VAR & 
                             X[(lrn.w & 1) ? (size_t)lrn.x + task.row0 + min(lane, n_rows - 1) : 0]);
     }
     LifPop pop = {};
-    float v_in[SLOTS], w_in[SLOTS];
+    NeuronPop npop = {};
+    float v_in[SLOTS], w_in[SLOTS], n_in[SLOTS];
     // runs once, behind the first matrix loads of the task
     auto after_first_loads = [&]() {
         float y_old[SLOTS];
@@ -1034,6 +1070,10 @@ __global__ __launch_bounds__(NHIP_WG) __attribute__((amdgpu_waves_per_eu((VAR & 
                     }
                 }
             }
+        }
+        if (EPI == EPI_NEURON) {
+            npop = reinterpret_cast<const NeuronPop*>(epi.lif.pops)[task.item];
+            fetch_states<SLOTS>(epi.lif, npop, task.row0, n_rows, lane, v_in, w_in, n_in);
         }
         if (EPI == EPI_FILTER) {
 #pragma unroll
@@ -1261,7 +1301,7 @@ __global__ __launch_bounds__(NHIP_WG) __attribute__((amdgpu_waves_per_eu((VAR & 
 #pragma unroll
             for (int i = 0; i < G::XL; ++i)
                 xq0[i] = x0[(size_t)min(lane + i * NHIP_WAVE, last_cols - 1) * dot.x_stride0];
-            if (EPI == EPI_LIF && decltype(first_tag)::value && G::XL == 1 && it.pad > 0) {
+            if (NEURONS && decltype(first_tag)::value && G::XL == 1 && it.pad > 0) {
                 // X is a sum of vectors that this launch forms itself, element c =
                 // (...(0 + v_0[c] * s_0) + v_1[c] * s_1) + ..., every product rounded on
                 // its own and added in order: what the small-item kernel computes for
@@ -1346,7 +1386,7 @@ __global__ __launch_bounds__(NHIP_WG) __attribute__((amdgpu_waves_per_eu((VAR & 
     auto whole_stages = [&](const GemvDot& dot) { return (dot.N & ((1 << dot.p2) - 1)) == 0; };
     if (it.n_dots == 0) {
         after_first_loads();
-        if (EPI == EPI_LIF && it.pad > 0) {
+        if (NEURONS && it.pad > 0) {
             // an item that is nothing but a sum of vectors times scalars (see the single
             // column stage of a dot product below): row r = (...(0 + v_0[r] s_0) + ...)
 #pragma unroll
@@ -1369,7 +1409,7 @@ __global__ __launch_bounds__(NHIP_WG) __attribute__((amdgpu_waves_per_eu((VAR & 
     }
     GemvTask done = task;
     done.n_rows = n_rows;
-    finish_task<EPI, SLOTS>(done, it, cf, ys, ab, Yin, Y, epi, pop, v_in, w_in, fp, lane);
+    finish_task<EPI, SLOTS>(done, it, cf, ys, ab, Yin, Y, epi, pop, npop, v_in, w_in, n_in, fp, lane);
 }
 
 }  // namespace
@@ -1460,6 +1500,7 @@ int launch_tile(void* stream, int vec, int pow2_cols, int blk_words, const int* 
     };
     if (epilogue == EPI_LIF) launch_epi(std::integral_constant<int, EPI_LIF>{});
     else if (epilogue == EPI_FILTER) launch_epi(std::integral_constant<int, EPI_FILTER>{});
+    else if (epilogue == EPI_NEURON) launch_epi(std::integral_constant<int, EPI_NEURON>{});
     else launch_epi(std::integral_constant<int, EPI_NONE>{});
     NHIP_LAUNCH_CHECK();
     return 0;
@@ -1524,6 +1565,30 @@ extern "C" int nhip_gemv_tile_lif_sums(void* stream, int vec, int pow2_cols, int
     lif.parts = reinterpret_cast<const int2*>(parts);
     return launch_tile(stream, vec, pow2_cols, blk_words, items, coefs, dots, tasks, n_tasks, A, X,
                        Yin, Y, EPI_LIF, args);
+}
+
+extern "C" int nhip_gemv_tile_neuron(void* stream, int vec, int pow2_cols, int blk_words,
+                                     const int* items, const float* coefs, const int* dots,
+                                     const int* tasks, int n_tasks, const float* A, const float* X,
+                                     const float* Yin, float* Y, const int* pops, double dt,
+                                     int upsample, float* V, float* W, float* S, float* N,
+                                     const int* parts) {
+    if (!pops || !V || !W || !S || !N || upsample < 1 || !(dt > 0.0)) return NHIP_E_BADARG;
+    if (parts && (static_cast<const float*>(Y) != X || pow2_cols < 2)) return NHIP_E_BADARG;
+    EpilogueArgs args{};
+    LifArgs& lif = args.lif;
+    lif.pops = reinterpret_cast<const LifPop*>(pops);
+    lif.dt = (float)dt;
+    lif.dtu = (float)(dt / (double)upsample);
+    lif.dt_inv = (float)(1.0 / dt);
+    lif.upsample = upsample;
+    lif.V = V;
+    lif.W = W;
+    lif.S = S;
+    lif.N = N;
+    lif.parts = reinterpret_cast<const int2*>(parts);
+    return launch_tile(stream, vec, pow2_cols, blk_words, items, coefs, dots, tasks, n_tasks, A, X,
+                       Yin, Y, EPI_NEURON, args);
 }
 
 extern "C" int nhip_gemv_tile_filter(void* stream, int vec, int pow2_cols, int blk_words,

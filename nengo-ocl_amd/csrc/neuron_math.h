@@ -52,7 +52,23 @@ struct LifArgs {
     // input is about to be replaced (see nhip_gemv_tile_lif_deferred).  Null: none.
     const int4* deferred;
     float* Fdef;
+    // neuron types other than the plain LIF (EPI_NEURON): `pops` then points at NeuronPop records
+    float* N;            // adaptation states
+    float dt;
 };
+
+// One population of neurons of another type than the plain LIF, driven by one output item of a
+// GEMV: element offsets of its state and float bits of its parameters (one value per population).
+struct NeuronPop {
+    int v_start, w_start, out_start, n_start;  // voltage, refractory time, output (S or R), adaptation
+    int tau, ref, amp, tau_n;
+    int inc_n, kind, flags, pad;               // flags: LIF_POP_ENABLED, LIF_POP_NO_J
+};
+enum { NEURON_LIF_RATE = 1, NEURON_ALIF = 2, NEURON_ALIF_RATE = 3, NEURON_RELU = 4,
+       NEURON_SPIKING_RELU = 5, NEURON_SIGMOID = 6 };
+__device__ __forceinline__ bool neuron_has_v(int kind) { return kind == NEURON_ALIF || kind == NEURON_SPIKING_RELU; }
+__device__ __forceinline__ bool neuron_has_w(int kind) { return kind == NEURON_ALIF; }
+__device__ __forceinline__ bool neuron_has_n(int kind) { return kind == NEURON_ALIF || kind == NEURON_ALIF_RATE; }
 
 __device__ __forceinline__ float lif_param(int word, bool is_vector, const float* data, int i) {
     return is_vector ? data[(size_t)word + i] : nhip_bits(word);
@@ -90,6 +106,68 @@ __device__ __forceinline__ bool lif_step(float j, float& v, float& w, float tau,
     return spiked;
 }
 
+// Adaptive LIF (clra_nonlinearities.py:1086-1133 with `adaptive`): the LIF update with
+// j - n in place of j in the voltage step, then n += (dt / tau_n) (inc_n s - n).  Returns s.
+__device__ __forceinline__ float alif_step(float j, float& v, float& w, float& n, float tau, float ref,
+                                           float amp, float tau_n, float inc_n, float dt, float dtu,
+                                           float dt_inv, int upsample) {
+    bool spiked = false;
+    for (int u = 0; u < upsample; ++u) {
+        w -= dtu;
+        const float delta_t = (w > dtu) ? 0.0f : (w < 0.0f) ? dtu : dtu - w;
+        const float dv = __fmul_rn(-(float)nhip_expm1((double)__fdiv_rn(-delta_t, tau)), (j - n) - v);
+        v = __fadd_rn(v, dv);
+        if (v > 1.0f) {
+            // the spike time interpolates with the unadapted current, as the reference does
+            const float t_spike = __fadd_rn(
+                dtu, __fmul_rn(tau, (float)nhip_log1p((double)__fdiv_rn(-(v - 1.0f), j - 1.0f))));
+            w = ref + t_spike;
+            v = 0.0f;
+            spiked = true;
+        } else if (v < 0.0f) {
+            v = 0.0f;
+        }
+    }
+    const float s = spiked ? __fmul_rn(amp, dt_inv) : 0.0f;
+    n = __fadd_rn(n, __fmul_rn(__fdiv_rn(dt, tau_n), __fsub_rn(__fmul_rn(inc_n, s), n)));
+    return s;
+}
+
+// LIF rate (clra_nonlinearities.py:1174-1184): j <= 1 gives 1/0 = inf, log1p(inf) = inf, amp/inf = 0.
+__device__ __forceinline__ float lif_rate(float current, float tau, float ref, float amp) {
+    const float j = fmaxf(current - 1.0f, 0.0f);
+    const float denom = __fadd_rn(ref, __fmul_rn(tau, (float)nhip_log1p((double)__fdiv_rn(1.0f, j))));
+    return __fdiv_rn(amp, denom);
+}
+
+// Adaptive LIF rate (clra_nonlinearities.py:1174-1188 with `adaptive`).
+__device__ __forceinline__ float alif_rate_step(float current, float& n, float tau, float ref, float amp,
+                                                float tau_n, float inc_n, float dt) {
+    const float r = lif_rate(current - n, tau, ref, amp);
+    n = __fadd_rn(n, __fmul_rn(__fdiv_rn(dt, tau_n), __fsub_rn(__fmul_rn(inc_n, r), n)));
+    return r;
+}
+
+// Rectified linear R = amp max(J, 0) (clra_nonlinearities.py:1238-1258).
+__device__ __forceinline__ float relu(float j, float amp) { return __fmul_rn(amp, fmaxf(j, 0.0f)); }
+
+// Spiking rectified linear (:1200-1235): V += dt max(J, 0), spikes = floor(V), V -= spikes,
+// S = amp spikes / dt.
+__device__ __forceinline__ float spiking_relu_step(float j, float& v, float amp, float dt, float dt_inv) {
+    v = __fadd_rn(v, (j > 0.0f) ? __fmul_rn(dt, j) : 0.0f);
+    const float n_spikes = floorf(v);
+    v = v - n_spikes;
+    return __fmul_rn(__fmul_rn(amp, n_spikes), dt_inv);
+}
+
+// Sigmoid R = 1 / (ref (1 + exp(-J))) with the reference's cut-offs at -88 and 15 (:1261-1283; exp
+// in double, rounded once, so that the value does not depend on the math library).
+__device__ __forceinline__ float sigmoid(float j, float ref) {
+    return (j < -88.0f) ? 0.0f
+           : (j > 15.0f) ? __fdiv_rn(1.0f, ref)
+                         : __fdiv_rn(1.0f, __fmul_rn(ref, __fadd_rn(1.0f, (float)exp((double)-j))));
+}
+
 // Work-list rows of the neuron kernels: a block of <= 512 neurons of one population.
 struct LifDesc {
     int j_start, v_start, w_start, s_start;
@@ -118,7 +196,6 @@ __device__ __forceinline__ void lif_block(const LifDesc d, float dtu, float dt_i
     }
 }
 
-// clra_nonlinearities.py:1174-1184: J <= 1 gives 1/0 = inf, log1p(inf) = inf, amp/inf = 0.
 __device__ __forceinline__ void lif_rate_block(const RateDesc d, const float* J, float* R,
                                                const float* __restrict__ TAU,
                                                const float* __restrict__ REF,
@@ -127,9 +204,7 @@ __device__ __forceinline__ void lif_rate_block(const RateDesc d, const float* J,
         const float tau = lif_param(d.tau, d.pflags & 1, TAU, i);
         const float ref = lif_param(d.ref, d.pflags & 2, REF, i);
         const float amp = lif_param(d.amp, d.pflags & 4, AMP, i);
-        const float j = fmaxf(J[(size_t)d.j_start + i] - 1.0f, 0.0f);
-        const float denom = __fadd_rn(ref, __fmul_rn(tau, (float)nhip_log1p((double)__fdiv_rn(1.0f, j))));
-        R[(size_t)d.r_start + i] = __fdiv_rn(amp, denom);
+        R[(size_t)d.r_start + i] = lif_rate(J[(size_t)d.j_start + i], tau, ref, amp);
     }
 }
 
@@ -144,6 +219,31 @@ __device__ __forceinline__ void lif_epilogue(const LifArgs& a, const LifPop& p, 
     a.V[(size_t)p.v_start + i] = v;
     a.W[(size_t)p.w_start + i] = w;
     a.S[(size_t)p.s_start + i] = spiked ? __fmul_rn(amp, a.dt_inv) : 0.0f;
+}
+
+// Update of neuron i of a population of another type with input current j (GEMV epilogue); v, w and n
+// are its states, read earlier (0 where the type has none).  The same functions as the neuron kernels.
+__device__ __forceinline__ void neuron_epilogue(const LifArgs& a, const NeuronPop& p, int i, float j,
+                                                float v, float w, float n) {
+    const float tau = nhip_bits(p.tau), ref = nhip_bits(p.ref), amp = nhip_bits(p.amp);
+    float out;
+    switch (p.kind) {
+        case NEURON_LIF_RATE: out = lif_rate(j, tau, ref, amp); break;
+        case NEURON_ALIF:
+            out = alif_step(j, v, w, n, tau, ref, amp, nhip_bits(p.tau_n), nhip_bits(p.inc_n), a.dt,
+                            a.dtu, a.dt_inv, a.upsample);
+            break;
+        case NEURON_ALIF_RATE:
+            out = alif_rate_step(j, n, tau, ref, amp, nhip_bits(p.tau_n), nhip_bits(p.inc_n), a.dt);
+            break;
+        case NEURON_RELU: out = relu(j, amp); break;
+        case NEURON_SPIKING_RELU: out = spiking_relu_step(j, v, amp, a.dt, a.dt_inv); break;
+        default: out = sigmoid(j, ref); break;
+    }
+    a.S[(size_t)p.out_start + i] = out;
+    if (neuron_has_v(p.kind)) a.V[(size_t)p.v_start + i] = v;
+    if (neuron_has_w(p.kind)) a.W[(size_t)p.w_start + i] = w;
+    if (neuron_has_n(p.kind)) a.N[(size_t)p.n_start + i] = n;
 }
 
 // First-order filters fed by one output item of a GEMV (a decoded value and the
@@ -175,7 +275,9 @@ __device__ __forceinline__ void filter_epilogue(const FilterArgs& a, int2 range,
 }
 
 // What a GEMV launch does with a finished output row besides storing it.
-enum { EPI_NONE = 0, EPI_LIF = 1, EPI_FILTER = 2 };
+// EPI_NEURON: the update of a neuron of another type than the plain LIF (an instance of its own: the
+// LIF instances keep their registers, and their compacted update of the rare cases).
+enum { EPI_NONE = 0, EPI_LIF = 1, EPI_FILTER = 2, EPI_NEURON = 3 };
 struct EpilogueArgs {
     LifArgs lif;
     FilterArgs filter;

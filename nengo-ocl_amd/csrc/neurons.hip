@@ -35,8 +35,7 @@ struct NeuronDesc {
     int p[8];                                   // tau, ref, amp, tau_n, inc_n
 };
 
-// Adaptive LIF (clra_nonlinearities.py:1086-1133 with `adaptive`): the LIF update with
-// J - N in place of J in the voltage step, then N += (dt / tau_n) (inc_n S - N).
+// Adaptive LIF (`alif_step`).
 __global__ __launch_bounds__(NHIP_WG) void alif_kernel(const NeuronDesc* __restrict__ desc,
                                                        float dt, float dtu, float dt_inv,
                                                        int upsample, const float* J, float* V,
@@ -51,40 +50,21 @@ __global__ __launch_bounds__(NHIP_WG) void alif_kernel(const NeuronDesc* __restr
         const float j = J[(size_t)d.j_start + i];
         float v = V[(size_t)d.v_start + i];
         float w = W[(size_t)d.w_start + i];
-        const float n = N[(size_t)d.n_start + i];
+        float n = N[(size_t)d.n_start + i];
         const float tau = lif_param(d.p[0], d.pflags & 1, TAU, i);
         const float ref = lif_param(d.p[1], d.pflags & 2, REF, i);
         const float amp = lif_param(d.p[2], d.pflags & 4, AMP, i);
         const float tau_n = lif_param(d.p[3], d.pflags & 8, TAU_N, i);
         const float inc_n = lif_param(d.p[4], d.pflags & 16, INC_N, i);
-        bool spiked = false;
-        for (int u = 0; u < upsample; ++u) {
-            w -= dtu;
-            const float delta_t = (w > dtu) ? 0.0f : (w < 0.0f) ? dtu : dtu - w;
-            const float dv =
-                __fmul_rn(-(float)nhip_expm1((double)__fdiv_rn(-delta_t, tau)), (j - n) - v);
-            v = __fadd_rn(v, dv);
-            if (v > 1.0f) {
-                // the spike time interpolates with the unadapted current, as the reference does
-                const float t_spike = __fadd_rn(
-                    dtu, __fmul_rn(tau, (float)nhip_log1p((double)__fdiv_rn(-(v - 1.0f), j - 1.0f))));
-                w = ref + t_spike;
-                v = 0.0f;
-                spiked = true;
-            } else if (v < 0.0f) {
-                v = 0.0f;
-            }
-        }
-        const float s = spiked ? __fmul_rn(amp, dt_inv) : 0.0f;
+        const float s = alif_step(j, v, w, n, tau, ref, amp, tau_n, inc_n, dt, dtu, dt_inv, upsample);
         V[(size_t)d.v_start + i] = v;
         W[(size_t)d.w_start + i] = w;
         S[(size_t)d.out_start + i] = s;
-        N[(size_t)d.n_start + i] =
-            __fadd_rn(n, __fmul_rn(__fdiv_rn(dt, tau_n), __fsub_rn(__fmul_rn(inc_n, s), n)));
+        N[(size_t)d.n_start + i] = n;
     }
 }
 
-// Adaptive LIF rate (clra_nonlinearities.py:1174-1188 with `adaptive`).
+// Adaptive LIF rate (`alif_rate_step`).
 __global__ __launch_bounds__(NHIP_WG) void alif_rate_kernel(const NeuronDesc* __restrict__ desc,
                                                             float dt, const float* J, float* R,
                                                             float* N,
@@ -100,21 +80,15 @@ __global__ __launch_bounds__(NHIP_WG) void alif_rate_kernel(const NeuronDesc* __
         const float amp = lif_param(d.p[2], d.pflags & 4, AMP, i);
         const float tau_n = lif_param(d.p[3], d.pflags & 8, TAU_N, i);
         const float inc_n = lif_param(d.p[4], d.pflags & 16, INC_N, i);
-        const float n = N[(size_t)d.n_start + i];
-        const float j = fmaxf((J[(size_t)d.j_start + i] - n) - 1.0f, 0.0f);
-        const float denom = __fadd_rn(ref, __fmul_rn(tau, (float)nhip_log1p((double)__fdiv_rn(1.0f, j))));
-        const float r = __fdiv_rn(amp, denom);
-        R[(size_t)d.out_start + i] = r;
-        N[(size_t)d.n_start + i] =
-            __fadd_rn(n, __fmul_rn(__fdiv_rn(dt, tau_n), __fsub_rn(__fmul_rn(inc_n, r), n)));
+        float n = N[(size_t)d.n_start + i];
+        R[(size_t)d.out_start + i] =
+            alif_rate_step(J[(size_t)d.j_start + i], n, tau, ref, amp, tau_n, inc_n, dt);
+        N[(size_t)d.n_start + i] = n;
     }
 }
 
-// The stateless and one-state types: kind 0 rectified linear R = amp max(J, 0)
-// (clra_nonlinearities.py:1238-1258); kind 1 spiking rectified linear V += dt max(J, 0),
-// spikes = floor(V), V -= spikes, S = amp spikes / dt (:1200-1235); kind 2 sigmoid
-// R = 1 / (ref (1 + exp(-J))) with the reference's cut-offs at -88 and 15 (:1261-1283;
-// exp in double, rounded once, so that the value does not depend on the math library).
+// The stateless and one-state types: kind 0 rectified linear (`relu`), kind 1 spiking rectified
+// linear (`spiking_relu_step`), kind 2 sigmoid (`sigmoid`).
 __global__ __launch_bounds__(NHIP_WG) void simple_neuron_kernel(
     int kind, const NeuronDesc* __restrict__ desc, float dt, float dt_inv, const float* J,
     float* OUT, float* V, const float* __restrict__ P)
@@ -125,17 +99,13 @@ __global__ __launch_bounds__(NHIP_WG) void simple_neuron_kernel(
         const float p = lif_param(d.p[0], d.pflags & 1, P, i);  // amp (kinds 0, 1) or ref (2)
         float out;
         if (kind == 0) {
-            out = __fmul_rn(p, fmaxf(j, 0.0f));
+            out = relu(j, p);
         } else if (kind == 1) {
             float v = V[(size_t)d.v_start + i];
-            v = __fadd_rn(v, (j > 0.0f) ? __fmul_rn(dt, j) : 0.0f);
-            const float n_spikes = floorf(v);
-            V[(size_t)d.v_start + i] = v - n_spikes;
-            out = __fmul_rn(__fmul_rn(p, n_spikes), dt_inv);
+            out = spiking_relu_step(j, v, p, dt, dt_inv);
+            V[(size_t)d.v_start + i] = v;
         } else {
-            out = (j < -88.0f) ? 0.0f
-                  : (j > 15.0f) ? __fdiv_rn(1.0f, p)
-                                : __fdiv_rn(1.0f, __fmul_rn(p, __fadd_rn(1.0f, (float)exp((double)-j))));
+            out = sigmoid(j, p);
         }
         OUT[(size_t)d.out_start + i] = out;
     }

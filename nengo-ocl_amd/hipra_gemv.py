@@ -907,7 +907,8 @@ def _epilogue_call(lib, plan, kind, extras=None):
 
 def fuse_lif(prog, lif_plan, unread_currents=()):
     """Fewer launches for "J = GEMV(...); LIF(J)" (clra_gemv.py `plan_block_gemv` followed
-    by clra_nonlinearities.py `plan_lif`): the reference-order kernels update the neurons
+    by clra_nonlinearities.py `plan_lif`, or by the planner of another neuron type whose
+    parameters are one value per population): the reference-order kernels update the neurons
     of a row (block) as soon as its currents are final, so the currents are not read
     back and the neuron kernel is not launched.
 
@@ -923,20 +924,27 @@ def fuse_lif(prog, lif_plan, unread_currents=()):
     `unread_currents`: populations (indices into the neuron plan) whose input current the
     caller knows nothing else reads.  Where such a current is formed from operands other
     than itself (``J = bias + E x``, not ``J += ...``), the fused launch does not store it;
-    every fused plan carries ``lazy_currents = (those populations, a plain GEMV over their
-    items)``: running that GEMV puts the currents of the last step into their place, bit
+    every fused plan carries ``lazy_currents = (those populations, a function that plans a GEMV over
+    their items)``: running that GEMV puts the currents of the last step into their place, bit
     for bit what the launch would have stored.
     """
-    from .hipra_nonlinearities import lif_population_table, plan_lif
+    from .hipra_nonlinearities import lif_population_table, neuron_population_table, plan_lif
 
     spec = getattr(lif_plan, "lif_spec", None)
+    other = spec is None  # a neuron type other than the plain LIF
+    spec = getattr(lif_plan, "neuron_spec", None) if other else spec
     if spec is None or not prog.plans:
         return None
     queue, lib = prog.queue, prog.queue.lib
     J, V, W, S = spec["J"], spec["V"], spec["W"], spec["outS"]
+    states = [ra for ra in (V, W, S, spec.get("N")) if ra is not None]
     Y = prog.Y
-    if any(ra.ptr.value != Y.ptr.value for ra in (J, V, W, S)):
+    if any(ra.ptr.value != Y.ptr.value for ra in [J] + states):
         return None  # different device buffers: nothing to match offsets against
+    if other:
+        rows = neuron_population_table(queue, spec)
+        if rows is None:
+            return None  # a parameter per neuron
     large = {}
     for plan in prog.plans:
         if _takes_epilogue(plan):
@@ -955,10 +963,12 @@ def fuse_lif(prog, lif_plan, unread_currents=()):
             rest.append(p)
     if not matched or len({b for _, b in matched}) != len(matched):
         return None
+    if other and rest:
+        return None  # (only the LIF has a launch for what is left over)
 
     # the update must not write what the launch still reads elsewhere
     fused_pops = [p for p, _ in matched] + idle
-    written = [iv for ra in (V, W, S) for iv in (_span(ra, p) for p in fused_pops) if iv]
+    written = [iv for ra in states for iv in (_span(ra, p) for p in fused_pops) if iv]
     read = []
     for g in prog.geometry:
         for d in g["dots"]:
@@ -1000,17 +1010,27 @@ def fuse_lif(prog, lif_plan, unread_currents=()):
                         for d in prog.geometry[b]["dots"])]
     lazy_currents = None
     if lazy:
-        sel = [b for _, b in lazy]
-        lazy_prog = plan_block_gemv(
-            queue, prog.alpha[sel], prog.A, [prog.A_js[b] for b in sel], prog.X,
-            [prog.X_js[b] for b in sel], prog.beta[sel], Y[sel], Y_in=prog.Y_in[sel],
-            gamma=prog.gamma[sel], tag="%s-currents-on-demand" % prog.tag)
+        sel, whole = [b for _, b in lazy], prog
+        lazy_prog = lambda: plan_block_gemv(
+            queue, whole.alpha[sel], whole.A, [whole.A_js[b] for b in sel], whole.X,
+            [whole.X_js[b] for b in sel], whole.beta[sel], whole.Y[sel], Y_in=whole.Y_in[sel],
+            gamma=whole.gamma[sel], tag="%s-currents-on-demand" % whole.tag)
         lazy_currents = ([p for p, _ in lazy], lazy_prog)
     no_store = {p for p, _ in lazy}
 
-    cols, pptrs, keep = lif_population_table(queue, spec)
-    table = np.zeros((len(Y), 8), dtype=np.int32)
-    for p, b in matched:
+    if other:
+        table = np.zeros((len(Y), 12), dtype=np.int32)
+        for p, b in matched:
+            table[b] = rows[p]
+            table[b, 10] = LIF_POP_ENABLED | (LIF_POP_NO_J if p in no_store else 0)
+        keep = ()
+        # (types without a state are handed the outputs' buffer in its place: only its first
+        # element is read, and nothing written)
+        ptr = lambda ra: (S if ra is None else ra).ptr
+    else:
+        cols, pptrs, keep = lif_population_table(queue, spec)
+        table = np.zeros((len(Y), 8), dtype=np.int32)
+    for p, b in (() if other else matched):
         flags = int(cols["pflags"][p]) | LIF_POP_ENABLED | (LIF_POP_NO_J if p in no_store else 0)
         decay_bits = 0
         if not (flags & 1) and spec["upsample"] == 1 and LIF_COMPACT:
@@ -1026,8 +1046,13 @@ def fuse_lif(prog, lif_plan, unread_currents=()):
         table[b] = (cols["v_start"][p], cols["w_start"][p], cols["s_start"][p], decay_bits,
                     cols["tau"][p], cols["ref"][p], cols["amp"][p], flags)
     dev_pops = to_device(queue, table)
-    lif_args = (dev_pops.ptr, spec["dt"], spec["upsample"], V.ptr, W.ptr, S.ptr,
-                pptrs[0], pptrs[1], pptrs[2])
+    if other:
+        lif_args = (dev_pops.ptr, spec["dt"], spec["upsample"], ptr(V), ptr(W), S.ptr, ptr(spec["N"]))
+    else:
+        lif_args = (dev_pops.ptr, spec["dt"], spec["upsample"], V.ptr, W.ptr, S.ptr,
+                    pptrs[0], pptrs[1], pptrs[2])
+    # words per neuron besides its current: states in and out, output out
+    state_words = 2 * (len(states) - 1) + 1
     pop_of = {b: p for p, b in matched}
     out = []
     for plan in prog.plans:
@@ -1038,14 +1063,19 @@ def fuse_lif(prog, lif_plan, unread_currents=()):
         # (currents that are not stored are not traffic)
         unstored = sum(4 * int(J.shape0s[pop_of[b]]) for b in plan.members
                        if b in pop_of and pop_of[b] in no_store)
-        entry, args, kept = _epilogue_call(lib, plan, "lif", lambda items: table[items][:, [0, 1, 7]])
-        fused = Plan(queue, entry, args + lif_args, gsize=plan.gsize,
+        if other:
+            entry, args, kept = _epilogue_call(lib, plan, "neuron",
+                                               lambda items: np.zeros((len(items), 3), np.int32))
+            args += lif_args + ((None,) if plan.kernel_class[0] == 3 else (None, None))  # no input sums
+        else:
+            entry, args, kept = _epilogue_call(lib, plan, "lif", lambda items: table[items][:, [0, 1, 7]])
+            args += lif_args
+        fused = Plan(queue, entry, args, gsize=plan.gsize,
                      lsize=plan.lsize,
-                     full_args=(plan.full_args + (dev_pops, V.dev_buf, W.dev_buf, S.dev_buf)
+                     full_args=(plan.full_args + (dev_pops,) + tuple(ra.dev_buf for ra in states)
                                 + tuple(keep) + kept),
-                     name=plan.name + "_lif", tag=plan.tag,
-                     # V and W in and out, spikes out
-                     bw_per_call=plan.bw_per_call + 5 * lif_bytes - unstored,
+                     name=plan.name + ("_neuron" if other else "_lif"), tag=plan.tag,
+                     bw_per_call=plan.bw_per_call + state_words * lif_bytes - unstored,
                      flops_per_call=plan.flops_per_call)
         fused.description = plan.description
         fused.kernel_class, fused.n_tasks = plan.kernel_class, plan.n_tasks
@@ -1053,7 +1083,7 @@ def fuse_lif(prog, lif_plan, unread_currents=()):
         fused.gemv_bytes = plan.bw_per_call - unstored
         fused.host_pops = table
         fused.dev_pops = dev_pops
-        fused.lif_written = [V, W, S]
+        fused.lif_written = states
         fused.lazy_currents = lazy_currents
         if plan.kernel_class[0] == 3:
             fused.host_tasks = plan.host_tasks
@@ -1089,9 +1119,12 @@ def fuse_input_sums(sum_plan, lif_plan):
     S, E = getattr(sum_plan, "prog", None), getattr(lif_plan, "prog", None)
     if S is None or E is None or sum_plan.name != "hipra_gemv.wave_ref":
         return None
-    large = (lif_plan.name == "hipra_gemv.tile_lif" and lif_plan.kernel_class[0] == 3
+    other = lif_plan.name.endswith("_neuron")  # a neuron type other than the plain LIF
+    large = (lif_plan.name in ("hipra_gemv.tile_lif", "hipra_gemv.tile_neuron")
+             and lif_plan.kernel_class[0] == 3
              and lif_plan.kernel_class[1] >= 2 and getattr(lif_plan, "host_tasks", None) is not None)
-    small = (lif_plan.name == "hipra_gemv.wave_ref_lif" and lif_plan.kernel_class[0] == 2
+    small = (lif_plan.name in ("hipra_gemv.wave_ref_lif", "hipra_gemv.wave_ref_neuron")
+             and lif_plan.kernel_class[0] == 2
              and getattr(lif_plan, "host_tables", None) is not None)
     if not (large or small):
         return None
@@ -1166,7 +1199,8 @@ def fuse_input_sums(sum_plan, lif_plan):
         keep = ()
         if spare:
             # one task each, of an item without dot products and without neurons: Y = the sum
-            pops = np.concatenate([lif_plan.host_pops, np.zeros((1, 8), dtype=np.int32)])
+            pops = np.concatenate([lif_plan.host_pops,
+                                   np.zeros((1, lif_plan.host_pops.shape[1]), dtype=np.int32)])
             extra = np.zeros((len(spare), 24), dtype=np.int32)
             for row, start in zip(extra, spare):
                 first, count = where[start]
@@ -1181,8 +1215,8 @@ def fuse_input_sums(sum_plan, lif_plan):
         tasks = spread_over_dies(tasks)
         dev_tasks = to_device(queue, tasks)
         n_groups = -(-len(tasks) // (WG // WAVE))
-        args = args[:6] + (dev_tasks.ptr, len(tasks)) + args[8:] + (dev_parts.ptr,)
-        entry = lib.nhip_gemv_tile_lif_sums
+        args = args[:6] + (dev_tasks.ptr, len(tasks)) + (args[8:-1] if other else args[8:]) + (dev_parts.ptr,)
+        entry = lib.nhip_gemv_tile_neuron if other else lib.nhip_gemv_tile_lif_sums
         keep = keep + (dev_tasks, dev_parts)
     else:
         # (lpr, task words, items, coefs, dots, tasks, n_tasks, A, X, Yin, Y, pops, ...): the
@@ -1194,7 +1228,7 @@ def fuse_input_sums(sum_plan, lif_plan):
         items = np.concatenate([item_tab, np.zeros((len(spare), 8), dtype=np.int32)])
         coefs = np.concatenate([coef_tab, np.zeros((len(spare), 4), dtype=np.float32)])
         pops = np.concatenate([lif_plan.host_pops[:n_items],
-                               np.zeros((len(spare), 8), dtype=np.int32)])
+                               np.zeros((len(spare), lif_plan.host_pops.shape[1]), dtype=np.int32)])
         ranges = np.zeros((len(items), 2), dtype=np.int32)
         for b in lif_plan.members:
             dots = E.geometry[b]["dots"]
@@ -1222,8 +1256,8 @@ def fuse_input_sums(sum_plan, lif_plan):
         rows_per_group = (WG // WAVE) * (WAVE // lpr)
         n_groups = -(-len(tasks) // rows_per_group)
         args = (lpr, task_words, dev[0].ptr, dev[1].ptr, args[4], dev[2].ptr, len(tasks)) + args[7:11] \
-            + (dev[3].ptr,) + args[12:] + (dev[4].ptr, dev_parts.ptr)
-        entry = lib.nhip_gemv_rows_lif_sums
+            + (dev[3].ptr,) + (args[12:-2] if other else args[12:]) + (dev[4].ptr, dev_parts.ptr)
+        entry = lib.nhip_gemv_rows_neuron if other else lib.nhip_gemv_rows_lif_sums
         keep = tuple(dev) + (dev_parts,)
     fused = Plan(queue, entry, args, gsize=(WG * n_groups,), lsize=lif_plan.lsize,
                  full_args=tuple(lif_plan.full_args) + keep,

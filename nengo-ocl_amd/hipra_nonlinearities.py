@@ -800,10 +800,42 @@ def plan_lif_rate(queue, dt, J, R, ref, tau, amp, N=None, tau_n=None, inc_n=None
                 tag=tag)
     plan.bw_per_call = J.nbytes + R.nbytes + bin(pflags).count("1") * J.nbytes
     plan.description = _description(J)
+    plan.neuron_spec = _neuron_spec(NEURON_LIF_RATE, dt, J, R, tau=tau, ref=ref, amp=amp)
     return plan
 
 
 # ---------------------------------------------------------------- further neuron types
+# kinds of a population row of nhip_gemv_tile_neuron / nhip_gemv_rows_neuron
+NEURON_LIF_RATE, NEURON_ALIF, NEURON_ALIF_RATE, NEURON_RELU = 1, 2, 3, 4
+NEURON_SPIKING_RELU, NEURON_SIGMOID = 5, 6
+
+
+def _neuron_spec(kind, dt, J, out, V=None, W=None, N=None, upsample=1, **params):
+    """What a GEMV that produces J needs to run this update as its epilogue."""
+    return dict(kind=kind, dt=float(dt), upsample=int(upsample), J=J, outS=out, V=V, W=W, N=N,
+                params=params)
+
+
+def neuron_population_table(queue, spec):
+    """int32[n][12] population rows (flags 0) of a neuron plan whose parameters are one value per
+    population, or None where one of them is a vector with a value per neuron."""
+    J = spec["J"]
+    n = len(J)
+    table = np.zeros((n, 12), dtype=np.int32)
+    for word, ra in zip((0, 1, 2, 3), (spec["V"], spec["W"], spec["outS"], spec["N"])):
+        if ra is not None:
+            table[:, word] = ra.starts
+    names = list(spec["params"])
+    cols, pflags, _, _ = _neuron_params(queue, [spec["params"][k] for k in names], J.shape0s,
+                                        np.arange(n), np.zeros(n, dtype=np.int64))
+    if pflags:
+        return None
+    for k, col in zip(names, cols):
+        table[:, {"tau": 4, "ref": 5, "amp": 6, "tau_n": 7, "inc_n": 8}[k]] = col
+    table[:, 9] = spec["kind"]
+    return table
+
+
 def _neuron_table(queue, J, out, params, V=None, W=None, N=None):
     """Work list {j, out, v, w, n offsets, count, pflags, 0, p0..p4, 0, 0, 0} of the neuron
     kernels that share `NeuronDesc` (one row per block of <= 512 neurons)."""
@@ -838,6 +870,8 @@ def _plan_alif(queue, dt, J, V, W, outS, ref, tau, amp, N, tau_n, inc_n, upsampl
     plan.bw_per_call = (J.nbytes + 2 * V.nbytes + 2 * W.nbytes + 2 * N.nbytes + outS.nbytes
                         + n_vec * J.nbytes)
     plan.description = _description(J)
+    plan.neuron_spec = _neuron_spec(NEURON_ALIF, dt, J, outS, V=V, W=W, N=N, upsample=upsample,
+                                    tau=tau, ref=ref, amp=amp, tau_n=tau_n, inc_n=inc_n)
     return plan
 
 
@@ -855,6 +889,8 @@ def _plan_alif_rate(queue, dt, J, R, ref, tau, amp, N, tau_n, inc_n, tag):
                 name="hip_alif_rate", tag=tag)
     plan.bw_per_call = J.nbytes + R.nbytes + 2 * N.nbytes + n_vec * J.nbytes
     plan.description = _description(J)
+    plan.neuron_spec = _neuron_spec(NEURON_ALIF_RATE, dt, J, R, N=N, tau=tau, ref=ref, amp=amp,
+                                    tau_n=tau_n, inc_n=inc_n)
     return plan
 
 
@@ -869,6 +905,7 @@ def plan_rectified_linear(queue, J, R, amp, tag=None, **kwargs):
                 full_args=(table, J.dev_buf, R.dev_buf) + tuple(keep), name="hip_relu", tag=tag)
     plan.bw_per_call = J.nbytes + R.nbytes + n_vec * J.nbytes
     plan.description = _description(J)
+    plan.neuron_spec = _neuron_spec(NEURON_RELU, 1.0, J, R, amp=amp)
     return plan
 
 
@@ -888,6 +925,7 @@ def plan_spiking_rectified_linear(queue, dt, J, V, outS, amp, tag=None, **kwargs
                 name="hip_spikingrelu", tag=tag)
     plan.bw_per_call = J.nbytes + 2 * V.nbytes + outS.nbytes + n_vec * J.nbytes
     plan.description = _description(J)
+    plan.neuron_spec = _neuron_spec(NEURON_SPIKING_RELU, dt, J, outS, V=V, amp=amp)
     return plan
 
 
@@ -902,6 +940,7 @@ def plan_sigmoid(queue, J, R, ref, tag=None, **kwargs):
                 full_args=(table, J.dev_buf, R.dev_buf) + tuple(keep), name="hip_sigmoid", tag=tag)
     plan.bw_per_call = J.nbytes + R.nbytes + n_vec * J.nbytes
     plan.description = _description(J)
+    plan.neuron_spec = _neuron_spec(NEURON_SIGMOID, 1.0, J, R, ref=ref)
     return plan
 
 

@@ -224,8 +224,8 @@ def _can_carry(plan, needs=0):
         return False
     if cls[0] == 2:
         return name in tuple("hipra_gemv." + k + e for k in ("wave_ref", "tile")
-                             for e in ("", "_lif", "_filter"))
-    if name in ("hipra_gemv.tile_lif", "hipra_gemv.tile_filter"):
+                             for e in ("", "_lif", "_filter", "_neuron"))
+    if name in ("hipra_gemv.tile_lif", "hipra_gemv.tile_neuron", "hipra_gemv.tile_filter"):
         return cls[0] == 3 and cls[1] >= 2
     return name in ("hipra_gemv.events", "hipra_gemv.events_filter") and cls[0] == 4 and needs == 0
 

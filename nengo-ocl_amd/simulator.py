@@ -618,7 +618,7 @@ class Simulator:
             if lazy is None:
                 continue
             populations, prog = lazy
-            group = {"prog": prog, "at_step": None}
+            group = {"make": prog, "prog": None, "at_step": None}
             for p in populations:
                 self._lazy_currents[neuron_ops[p].J.base] = group
 
@@ -629,6 +629,8 @@ class Simulator:
         # (before the first step the signal holds its initial value, as in the reference)
         if group is None or self._n_steps == 0 or group["at_step"] == self._n_steps:
             return
+        if group["prog"] is None:  # planned when somebody asks for the first time
+            group["prog"] = group["make"]()
         for plan in group["prog"].plans:
             plan()
         group["at_step"] = self._n_steps

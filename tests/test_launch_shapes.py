@@ -449,3 +449,37 @@ def test_infinities_and_nan_reach_the_results_they_reach_in_the_oracle(queue, rn
     nan = np.isnan(expected)
     assert nan.any() and not nan.all() and np.array_equal(np.isnan(got), nan)
     assert np.array_equal(got[~nan].view(np.uint32), expected[~nan].view(np.uint32))
+
+
+# tasks of the small-item kernel, and of the large-item kernel: rows that lie back to back, four columns,
+# rows that no 16-byte loads fit, 16, 64 and 200 columns
+@pytest.mark.parametrize("neurons,dims", [(41, 2), (701, 50), (2101, 4), (203, 70), (1000, 16), (300, 64),
+                                          (150, 200)])
+@pytest.mark.parametrize("kind", ["LIFRate", "AdaptiveLIF", "AdaptiveLIFRate", "RectifiedLinear",
+                                  "SpikingRectifiedLinear", "Sigmoid"])
+def test_neuron_types_in_the_launch_of_their_currents(queue, kind, neurons, dims):
+    """Every neuron type is updated by the launch that encodes its input, which also forms the sums
+    of decoded values it encodes; an ensemble that nothing feeds rides along."""
+    from nengo_ocl_amd import minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    def make():
+        net = mb.Network(seed=6, solver="surrogate")
+        stim = net.Node(mb.WhiteSignal(period=0.5, high=6.0, seed=3), size_out=dims)
+        kw = dict(neuron_type=getattr(mb, kind)(), radius=2.0)
+        a, b, idle = (net.Ensemble(neurons, dims, **kw) for _ in range(3))
+        net.Connection(stim, a, synapse=mb.Lowpass(0.005))
+        net.Connection(a, b, synapse=mb.Lowpass(0.005))
+        net.Connection(idle, b, synapse=mb.Lowpass(0.005))
+        net.Connection(b, a, synapse=mb.Lowpass(0.005))
+        return net, net.Probe(b, synapse=0.01)
+
+    (net, probe), (net_o, probe_o) = make(), make()
+    with Simulator(net, seed=1) as gpu, OracleSimulator(net_o, seed=1) as cpu:
+        names = [p.name for p in gpu._plans]
+        assert any(n.endswith("_neuron") for n in names), names
+        gpu.run_steps(40)
+        cpu.run_steps(40)
+        assert np.any(gpu.data[probe] != 0) and np.array_equal(gpu.data[probe], cpu.data[probe_o])
+        assert np.array_equal(gpu.signal_buffer().view(np.uint32), cpu.signal_buffer().view(np.uint32))
