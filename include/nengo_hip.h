@@ -33,7 +33,7 @@
 extern "C" {
 #endif
 
-#define NHIP_ABI_VERSION 1
+#define NHIP_ABI_VERSION 2
 
 #define NHIP_E_BADARG (-1)   /* null pointer / negative count / unknown mode   */
 #define NHIP_E_BADCLASS (-2) /* GEMV class (lanes-per-row, vector width) unknown */
@@ -224,6 +224,12 @@ int nhip_gemv_rows_neuron(void *stream, int lpr, int task_words, const int *item
  *   item_targets : int32[n_items][2] {first target, number of targets}
  *   targets      : int32[n][4] {y_start, a0 bits, b0 bits, na}
  *   F[y_start + r] = b0 * y - a0 * F[y_start + r]   (na == 1)   or   b0 * y   (na == 0)
+ * order (1 or 2): 2 if any target has two coefficients on a side (here, in nhip_gemv_rows_filter,
+ * the _learn form and nhip_gemv_events).  Such a target: na = number of denominator coefficients (0..2) + 4 (two numerator
+ * coefficients) + 8 * k, k > 0: rows k and k + 1 of `targets` are {a1 bits, b1 bits, n, 0} and
+ * {address of float state[3][n] (two words), 0, 0}: x[t-1], y[t-1], y[t-2] of the item's n rows,
+ * zero at the start and shifted by the step.
+ *   y[t] = b0 x[t] + b1 x[t-1] - a0 F[y_start + r] - a1 y[t-2], left to right
  * Y is still written.  The filter outputs must not overlap anything the launch reads
  * through A, X or Yin.  Results are bit-identical to the two separate calls.
  * The kernels of this entry point read an item's range of targets from its task
@@ -233,7 +239,7 @@ int nhip_gemv_rows_neuron(void *stream, int lpr, int task_words, const int *item
 int nhip_gemv_tile_filter(void *stream, int vec, int pow2_cols, int blk_words, const int *items,
                           const float *coefs, const int *dots, const int *tasks, int n_tasks,
                           const float *A, const float *X, const float *Yin, float *Y,
-                          const int *item_targets, const int *targets, float *F);
+                          const int *item_targets, const int *targets, float *F, int order);
 
 /* A learning rule's outer-product update done by the launch that streams the learned
  * matrices anyway (reference: `_plan_SimPES`, simulator.py:1334-1345, an outer-product
@@ -252,7 +258,7 @@ int nhip_gemv_tile_filter_learn(void *stream, int vec, int pow2_cols, int blk_wo
                                 const int *items, const float *coefs, const int *dots,
                                 const int *tasks, int n_tasks, float *A, const float *X,
                                 const float *Yin, float *Y, const int *item_targets,
-                                const int *targets, float *F, const int *learn);
+                                const int *targets, float *F, int order, const int *learn);
 
 /* nhip_gemv_tile_lif / nhip_gemv_tile_lif_sums (`parts` may be NULL: no input sums) that
  * also steps first-order filters of the populations' spikes -- the pre-synaptic activities
@@ -313,7 +319,7 @@ int nhip_gemv_rows_filter(void *stream, int lpr, int task_words, const int *item
                           const float *coefs, const int *dots, const int *tasks, int n_tasks,
                           const float *A,
                           const float *X, const float *Yin, float *Y, const int *item_targets,
-                          const int *targets, float *F);
+                          const int *targets, float *F, int order);
 
 /* ---- sparse matrix-vector products -----------------------------------------
  * Y[b] (=|+=) A[b] @ X[b] for many sparse matrices in one launch.
@@ -359,7 +365,7 @@ int nhip_spmv_sell(void *stream, const int *slices, int n_slices, const int *row
  * the launch. */
 int nhip_gemv_events(void *stream, const int *items, int n_items, const float *AT,
                      const float *X, const float *Yin, float *Y, const int *targets, float *F,
-                     int max_cols);
+                     int order, int max_cols);
 
 /* The same product for an X that is mostly zero (the spikes of a population; no
  * counterpart in the reference, whose kernels multiply every stored element).  All slices

@@ -37,8 +37,8 @@ SIGNATURES = {
                               P, ctypes.c_double, c_int, P, P, P, P, P],
     "nhip_gemv_rows_neuron": [P, c_int, c_int, P, P, P, P, c_int, P, P, P, P,
                               P, ctypes.c_double, c_int, P, P, P, P, P, P],
-    "nhip_gemv_tile_filter": [P, c_int, c_int, c_int, P, P, P, P, c_int, P, P, P, P, P, P, P],
-    "nhip_gemv_tile_filter_learn": [P, c_int, c_int, c_int, P, P, P, P, c_int, P, P, P, P, P, P, P, P],
+    "nhip_gemv_tile_filter": [P, c_int, c_int, c_int, P, P, P, P, c_int, P, P, P, P, P, P, P, c_int],
+    "nhip_gemv_tile_filter_learn": [P, c_int, c_int, c_int, P, P, P, P, c_int, P, P, P, P, P, P, P, c_int, P],
     "nhip_gemv_tile_lif_deferred": [P, c_int, c_int, c_int, P, P, P, P, c_int, P, P, P, P,
                                     P, ctypes.c_double, c_int, P, P, P, P, P, P, P, P, P],
     "nhip_gemv_tile_rows": [c_int, c_int],
@@ -46,8 +46,8 @@ SIGNATURES = {
                            P, ctypes.c_double, c_int, P, P, P, P, P, P],
     "nhip_gemv_rows_lif_sums": [P, c_int, c_int, P, P, P, P, c_int, P, P, P, P,
                                 P, ctypes.c_double, c_int, P, P, P, P, P, P, P, P],
-    "nhip_gemv_rows_filter": [P, c_int, c_int, P, P, P, P, c_int, P, P, P, P, P, P, P],
-    "nhip_gemv_events": [P, P, c_int, P, P, P, P, P, P, c_int],
+    "nhip_gemv_rows_filter": [P, c_int, c_int, P, P, P, P, c_int, P, P, P, P, P, P, P, c_int],
+    "nhip_gemv_events": [P, P, c_int, P, P, P, P, P, P, c_int, c_int],
     "nhip_spmv_sell": [P, P, c_int, P, P, P, P, P],
     "nhip_spmv_sell_skip": [P, P, c_int, P, P, P, P, P, c_int, c_int, P],
     "nhip_spmv_sell_filter": [P, P, c_int, P, P, P, P, P, P, P, P, c_int, c_int, P],

@@ -623,12 +623,13 @@ extern "C" int nhip_gemv_rows_filter(void* stream, int lpr, int task_words, cons
                                      const float* coefs, const int* dots, const int* tasks,
                                      int n_tasks,
                                      const float* A, const float* X, const float* Yin, float* Y,
-                                     const int* item_targets, const int* targets, float* F) {
-    if (!item_targets || !targets || !F) return NHIP_E_BADARG;
+                                     const int* item_targets, const int* targets, float* F, int order) {
+    if (!item_targets || !targets || !F || order < 1 || order > 2) return NHIP_E_BADARG;
     EpilogueArgs args{};
     args.filter.item_targets = reinterpret_cast<const int2*>(item_targets);
     args.filter.targets = reinterpret_cast<const FilterTarget*>(targets);
     args.filter.F = F;
-    return launch_rows_epi<EPI_FILTER>(static_cast<hipStream_t>(stream), lpr, task_words, items,
-                                       coefs, dots, tasks, n_tasks, A, X, Yin, Y, args);
+    auto launch = order == 2 ? launch_rows_epi<EPI_FILTER2> : launch_rows_epi<EPI_FILTER>;
+    return launch(static_cast<hipStream_t>(stream), lpr, task_words, items, coefs, dots, tasks, n_tasks, A,
+                  X, Yin, Y, args);
 }

@@ -30,6 +30,8 @@
 // the groups beyond the 256th waited for a compute unit to become free and the launch took
 // one and a half times as long as its groups.
 #define NHIP_SEQ_LEAN  // this kernel runs on 64 registers
+#include <type_traits>
+
 #include "nhip_common.h"
 #include "gemv_types.h"
 #include "neuron_math.h"
@@ -76,10 +78,11 @@ struct EvLds {
     float tile[EV_MAX_TILES][NHIP_WAVE];
 };
 
+// SECOND: some filter is of second order
 // MULTI: some item of the launch has more than EV_MAX_COLS columns
 // CARRY: a sequence rides in extra groups (an instance of its own: the sequence's block
 // functions need more registers than the budget of 64, and spill; the products do not)
-template <bool MULTI, bool CARRY>
+template <bool MULTI, bool CARRY, bool SECOND>
 __global__ __launch_bounds__(EV_WG) __attribute__((amdgpu_waves_per_eu(8, 8))) void gemv_events_kernel(
     const EvItem* __restrict__ items, int n_items, const float* __restrict__ AT, const float* X,
     const float* Yin, float* Y, FilterArgs filter, EvSide side)
@@ -255,11 +258,9 @@ __global__ __launch_bounds__(EV_WG) __attribute__((amdgpu_waves_per_eu(8, 8))) v
         if (it.n_targets > 0) {
             // the first filter from what was requested at the start, the others as usual
             // (the arithmetic of filter_epilogue: rounded products, rounded subtract)
-            const float bx = __fmul_rn(nhip_bits(f_first.b_bits), y);
-            filter.F[(size_t)f_first.y_start + row] =
-                f_first.na ? __fsub_rn(bx, __fmul_rn(nhip_bits(f_first.a_bits), f_old)) : bx;
+            filter.F[(size_t)f_first.y_start + row] = filter_step<SECOND>(filter.targets, f_first, row, y, f_old);
             if (it.n_targets > 1)
-                filter_epilogue(filter, make_int2(it.first_target + 1, it.n_targets - 1), row, y);
+                filter_epilogue<SECOND>(filter, make_int2(it.first_target + 1, it.n_targets - 1), row, y);
         }
     }
 }
@@ -268,14 +269,14 @@ __global__ __launch_bounds__(EV_WG) __attribute__((amdgpu_waves_per_eu(8, 8))) v
 
 extern "C" int nhip_gemv_events(void* stream, const int* items, int n_items, const float* AT,
                                 const float* X, const float* Yin, float* Y,
-                                const int* targets, float* F, int max_cols) {
+                                const int* targets, float* F, int order, int max_cols) {
     // a sequence armed by nhip_gemv_tile_carry is this launch's, whatever becomes of it
     const NhipCarried armed = nhip_carried;
     nhip_carried = NhipCarried{};
     if (n_items == 0) return armed.n_chains > 0 ? NHIP_E_BADARG : 0;  // nothing to ride in
     if (armed.n_chains > 0 && armed.needs != 0) return NHIP_E_BADARG;  // (a lean sequence body)
     if (n_items < 0 || !items || !AT || !X || !Yin || !Y || max_cols <= 0) return NHIP_E_BADARG;
-    if ((targets == nullptr) != (F == nullptr)) return NHIP_E_BADARG;
+    if ((targets == nullptr) != (F == nullptr) || order < 1 || order > 2) return NHIP_E_BADARG;
     EvSide side{};
     if (armed.n_chains > 0) {
         side.ops = static_cast<const NhipSeqOp*>(armed.ops);
@@ -292,8 +293,13 @@ extern "C" int nhip_gemv_events(void* stream, const int* items, int n_items, con
                     n_items, AT, X, Yin, Y, filter, side);
     };
     const bool carry = side.n_chains > 0;
-    if (max_cols > EV_MAX_COLS) carry ? launch(gemv_events_kernel<true, true>) : launch(gemv_events_kernel<true, false>);
-    else carry ? launch(gemv_events_kernel<false, true>) : launch(gemv_events_kernel<false, false>);
+    auto pick = [&](auto second) {
+        constexpr bool S = decltype(second)::value;
+        if (max_cols > EV_MAX_COLS) carry ? launch(gemv_events_kernel<true, true, S>) : launch(gemv_events_kernel<true, false, S>);
+        else carry ? launch(gemv_events_kernel<false, true, S>) : launch(gemv_events_kernel<false, false, S>);
+    };
+    if (order == 2) pick(std::true_type{});
+    else pick(std::false_type{});
     NHIP_LAUNCH_CHECK();
     return 0;
 }

@@ -103,7 +103,7 @@ __device__ __forceinline__ void gemv_rows_ref_block(
         w_old = epi->lif.W[neuron_has_w(npop.kind) ? (size_t)npop.w_start + r : 0];
         n_old = epi->lif.N[neuron_has_n(npop.kind) ? (size_t)npop.n_start + r : 0];
     }
-    if (EPI == EPI_FILTER) {
+    if (epi_filters(EPI)) {
         f_range = WIDE ? make_int2(task.pad, it.pad) : epi->filter.item_targets[task.item];
         f_first = epi->filter.targets[f_range.y > 0 ? f_range.x : 0];
         f_old = epi->filter.F[f_range.y > 0 ? (size_t)f_first.y_start + r : 0];
@@ -328,13 +328,12 @@ __device__ __forceinline__ void gemv_rows_ref_block(
             lif_epilogue(epi->lif, pop, r, y, v_old, w_old);
         if (EPI == EPI_NEURON && (npop.flags & LIF_POP_ENABLED))
             neuron_epilogue(epi->lif, npop, r, y, v_old, w_old, n_old);
-        if (EPI == EPI_FILTER && f_range.y > 0) {
+        if (epi_filters(EPI) && f_range.y > 0) {
             // the first target with what was fetched ahead (the arithmetic of
             // filter_epilogue), further targets of the item from memory
-            const float bx = __fmul_rn(nhip_bits(f_first.b_bits), y);
             epi->filter.F[(size_t)f_first.y_start + r] =
-                f_first.na ? __fsub_rn(bx, __fmul_rn(nhip_bits(f_first.a_bits), f_old)) : bx;
-            filter_epilogue(epi->filter, make_int2(f_range.x + 1, f_range.y - 1), r, y);
+                filter_step<EPI == EPI_FILTER2>(epi->filter.targets, f_first, r, y, f_old);
+            filter_epilogue<EPI == EPI_FILTER2>(epi->filter, make_int2(f_range.x + 1, f_range.y - 1), r, y);
         }
     }
 }

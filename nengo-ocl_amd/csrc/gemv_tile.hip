@@ -320,7 +320,7 @@ __global__ __launch_bounds__(NHIP_WG) void gemv_tile_kernel(
     int2 filters = make_int2(0, 0);
     if (EPI == EPI_LIF) pop = epi.lif.pops[task.item];
     if (EPI == EPI_NEURON) npop = reinterpret_cast<const NeuronPop*>(epi.lif.pops)[task.item];
-    if (EPI == EPI_FILTER) filters = make_int2(task.pad, it.pad);  // rides in the task record
+    if (epi_filters(EPI)) filters = make_int2(task.pad, it.pad);  // rides in the task record
     // an item without dot products that would copy Y onto itself unchanged is only
     // there for its epilogue (a constant input current): nothing to store
     const bool store_y = !(it.n_dots == 0 && cf.y == 1.0f && cf.z == 0.0f && Y == Yin &&
@@ -345,7 +345,7 @@ __global__ __launch_bounds__(NHIP_WG) void gemv_tile_kernel(
                                 epi.lif.W[neuron_has_w(npop.kind) ? (size_t)npop.w_start + i : 0],
                                 epi.lif.N[neuron_has_n(npop.kind) ? (size_t)npop.n_start + i : 0]);
             }
-            if (EPI == EPI_FILTER) filter_epilogue(epi.filter, filters, task.row0 + r, y);
+            if (epi_filters(EPI)) filter_epilogue<EPI == EPI_FILTER2>(epi.filter, filters, task.row0 + r, y);
         }
     }
 }
@@ -562,12 +562,11 @@ __device__ __forceinline__ void finish_task(const GemvTask& task, const GemvItem
                 neuron_epilogue(epi.lif, npop, task.row0 + r, y, v_in[k], w_in[k], n_in[k]);
         }
     }
-    if (EPI == EPI_FILTER) {
+    if (epi_filters(EPI)) {
         // y = b0 x - a0 y, or y = b0 x: the arithmetic of filter_epilogue
         auto step = [&](const FilterTarget& t, int r, float old_value) {
-            const float bx = __fmul_rn(nhip_bits(t.b_bits), ys[r] + cf.z);
             epi.filter.F[(size_t)t.y_start + task.row0 + r] =
-                t.na ? __fsub_rn(bx, __fmul_rn(nhip_bits(t.a_bits), old_value)) : bx;
+                filter_step<EPI == EPI_FILTER2>(epi.filter.targets, t, task.row0 + r, ys[r] + cf.z, old_value);
         };
 #pragma unroll
         for (int k = 0; k < F_SLOTS; ++k)
@@ -649,7 +648,7 @@ __global__ __launch_bounds__(NHIP_WG) void gemv_tile_p2_kernel(
     FilterTarget f_target[F_SLOTS];
     float f_old[F_SLOTS];
     int f_row[F_SLOTS];
-    if (EPI == EPI_FILTER) {
+    if (epi_filters(EPI)) {
         filters = make_int2(task.pad, it.pad);  // the item's range of targets rides in the task record
         n_pairs = filters.y * n_rows;
         // no branch around the loads: an item without targets reads the table's first record
@@ -841,7 +840,7 @@ __global__ __launch_bounds__(NHIP_WG) void gemv_tile_p2_kernel(
         const int r = lane + k * NHIP_WAVE;
         if (r < n_rows) ys[r] = cf.y * y_old[k];
     }
-    if (EPI == EPI_FILTER) {
+    if (epi_filters(EPI)) {
 #pragma unroll
         for (int k = 0; k < F_SLOTS; ++k)
             f_old[k] = epi.filter.F[(size_t)f_target[k].y_start + (n_pairs > 0 ? task.row0 + f_row[k] : 0)];
@@ -963,7 +962,7 @@ __global__ __launch_bounds__(NHIP_WG) __attribute__((amdgpu_waves_per_eu((VAR & 
 {
     constexpr bool WIDE = (SET & (SET_MID | SET_WIDE)) != 0;  // the large LDS layout
     constexpr bool FLAT = (SET & SET_FLAT) != 0;
-    constexpr bool LEARN = EPI == EPI_FILTER && (VAR & VAR_LEARN) != 0;
+    constexpr bool LEARN = epi_filters(EPI) && (VAR & VAR_LEARN) != 0;
     constexpr bool DEFER = EPI == EPI_LIF && (VAR & VAR_DEFER) != 0;
     constexpr bool NEURONS = EPI == EPI_LIF || EPI == EPI_NEURON;
     static_assert(!(LEARN && FLAT), "learned matrices: rows on 16-byte boundaries");
@@ -1003,7 +1002,7 @@ __global__ __launch_bounds__(NHIP_WG) __attribute__((amdgpu_waves_per_eu((VAR & 
     FilterPrefetch fp;
     fp.range = make_int2(0, 0);
     fp.n_pairs = 0;
-    if (EPI == EPI_FILTER) {
+    if (epi_filters(EPI)) {
         fp.range = make_int2(task.pad, it.pad);  // rides in the task record
         fp.n_pairs = fp.range.y * n_rows;
 #pragma unroll
@@ -1075,7 +1074,7 @@ __global__ __launch_bounds__(NHIP_WG) __attribute__((amdgpu_waves_per_eu((VAR & 
             npop = reinterpret_cast<const NeuronPop*>(epi.lif.pops)[task.item];
             fetch_states<SLOTS>(epi.lif, npop, task.row0, n_rows, lane, v_in, w_in, n_in);
         }
-        if (EPI == EPI_FILTER) {
+        if (epi_filters(EPI)) {
 #pragma unroll
             for (int k = 0; k < F_SLOTS; ++k)
                 fp.old[k] = epi.filter.F[(size_t)fp.target[k].y_start +
@@ -1429,7 +1428,7 @@ int launch_tile(void* stream, int vec, int pow2_cols, int blk_words, const int* 
                 int variant = 0) {
     // the variants exist for the shapes they were built for: learned matrices in launches of
     // the wide instance, deferred activity filters in launches of the narrow one
-    if (variant == VAR_LEARN && !(epilogue == EPI_FILTER && pow2_cols == 2)) return NHIP_E_BADCLASS;
+    if (variant == VAR_LEARN && !(epi_filters(epilogue) && pow2_cols == 2)) return NHIP_E_BADCLASS;
     if (variant == VAR_DEFER && !(epilogue == EPI_LIF && pow2_cols == 3)) return NHIP_E_BADCLASS;
     if (variant != 0 && variant != VAR_LEARN && variant != VAR_DEFER) return NHIP_E_BADARG;
     // a sequence armed by nhip_gemv_tile_carry is this launch's, whatever becomes of it
@@ -1485,7 +1484,7 @@ int launch_tile(void* stream, int vec, int pow2_cols, int blk_words, const int* 
                         Y, args, side);
         };
         if (variant == VAR_LEARN) {
-            if constexpr (E == EPI_FILTER) launch_stream(gemv_stream_kernel<E, SET_WIDE, VAR_LEARN>);
+            if constexpr (epi_filters(E)) launch_stream(gemv_stream_kernel<E, SET_WIDE, VAR_LEARN>);
         } else if (variant == VAR_DEFER) {
             if constexpr (E == EPI_LIF) launch_stream(gemv_stream_kernel<E, 0, VAR_DEFER>);
         } else if (pow2_cols == 2) launch_stream(gemv_stream_kernel<E, SET_WIDE>);
@@ -1500,6 +1499,7 @@ int launch_tile(void* stream, int vec, int pow2_cols, int blk_words, const int* 
     };
     if (epilogue == EPI_LIF) launch_epi(std::integral_constant<int, EPI_LIF>{});
     else if (epilogue == EPI_FILTER) launch_epi(std::integral_constant<int, EPI_FILTER>{});
+    else if (epilogue == EPI_FILTER2) launch_epi(std::integral_constant<int, EPI_FILTER2>{});
     else if (epilogue == EPI_NEURON) launch_epi(std::integral_constant<int, EPI_NEURON>{});
     else launch_epi(std::integral_constant<int, EPI_NONE>{});
     NHIP_LAUNCH_CHECK();
@@ -1595,29 +1595,30 @@ extern "C" int nhip_gemv_tile_filter(void* stream, int vec, int pow2_cols, int b
                                      const int* items, const float* coefs, const int* dots,
                                      const int* tasks, int n_tasks, const float* A, const float* X,
                                      const float* Yin, float* Y, const int* item_targets,
-                                     const int* targets, float* F) {
-    if (!item_targets || !targets || !F) return NHIP_E_BADARG;
+                                     const int* targets, float* F, int order) {
+    if (!item_targets || !targets || !F || order < 1 || order > 2) return NHIP_E_BADARG;
     EpilogueArgs args{};
     args.filter.item_targets = reinterpret_cast<const int2*>(item_targets);
     args.filter.targets = reinterpret_cast<const FilterTarget*>(targets);
     args.filter.F = F;
     return launch_tile(stream, vec, pow2_cols, blk_words, items, coefs, dots, tasks, n_tasks, A, X,
-                       Yin, Y, EPI_FILTER, args);
+                       Yin, Y, order == 2 ? EPI_FILTER2 : EPI_FILTER, args);
 }
 
 extern "C" int nhip_gemv_tile_filter_learn(void* stream, int vec, int pow2_cols, int blk_words,
                                            const int* items, const float* coefs, const int* dots,
                                            const int* tasks, int n_tasks, float* A, const float* X,
                                            const float* Yin, float* Y, const int* item_targets,
-                                           const int* targets, float* F, const int* learn) {
-    if (!item_targets || !targets || !F || !learn) return NHIP_E_BADARG;
+                                           const int* targets, float* F, int order,
+                                           const int* learn) {
+    if (!item_targets || !targets || !F || !learn || order < 1 || order > 2) return NHIP_E_BADARG;
     EpilogueArgs args{};
     args.filter.item_targets = reinterpret_cast<const int2*>(item_targets);
     args.filter.targets = reinterpret_cast<const FilterTarget*>(targets);
     args.filter.F = F;
     args.filter.learn = reinterpret_cast<const int4*>(learn);
     return launch_tile(stream, vec, pow2_cols, blk_words, items, coefs, dots, tasks, n_tasks, A, X,
-                       Yin, Y, EPI_FILTER, args, VAR_LEARN);
+                       Yin, Y, order == 2 ? EPI_FILTER2 : EPI_FILTER, args, VAR_LEARN);
 }
 
 extern "C" int nhip_gemv_tile_lif_deferred(void* stream, int vec, int pow2_cols, int blk_words,

@@ -246,9 +246,17 @@ __device__ __forceinline__ void neuron_epilogue(const LifArgs& a, const NeuronPo
     if (neuron_has_n(p.kind)) a.N[(size_t)p.n_start + i] = n;
 }
 
-// First-order filters fed by one output item of a GEMV (a decoded value and the
-// synapses of the connections that carry it): y = b0 x - a0 y, or y = b0 x.
+// Filters fed by one output item of a GEMV (a decoded value and the synapses of the
+// connections that carry it): y = b0 x - a0 y, or y = b0 x; or, with FILTER_SECOND_ORDER bits in
+// `na`, one with two coefficients on either side, whose further coefficients and state are the
+// FilterSecond record in the rows (na >> FILTER_SECOND_SHIFT) of the table of targets.
 struct FilterTarget { int y_start, a_bits, b_bits, na; };
+constexpr int FILTER_NA = 3, FILTER_NB2 = 4, FILTER_SECOND_SHIFT = 3;
+struct FilterSecond {          // two rows of the table of targets
+    int a1_bits, b1_bits, n, pad;
+    float* state;              // x[t-1], y[t-1], y[t-2]: n elements each
+    int pad2, pad3;
+};
 
 struct FilterArgs {
     const int2* item_targets;     // per GEMV item: {first target, number of targets}
@@ -262,22 +270,53 @@ struct FilterArgs {
     const int4* learn;
 };
 
-// Filter step of element i of every target of a GEMV item whose fresh output is x
-// (the arithmetic of the simple case of the linear-filter kernel,
-// clra_nonlinearities.py:630-650: rounded products, rounded subtract).
+// The step of one filter for its element i: x is the fresh input, f_old the output's old value;
+// returns the new one.  Rounded products and sums in the order of the filter kernel
+// (clra_nonlinearities.py:630-711: b0 x [+ b1 x'] [- a0 y] [- a1 y'']).  A second-order filter keeps
+// its two older outputs itself (the ring buffers of the launch it replaces do the same: y[t-2] is
+// what the filter computed, also where somebody has written its output since) and shifts them
+// instead of moving positions: the rows of an item are stepped by many groups, none of which could
+// move a position that the others still read.
+// As a launch of their own, second-order synapses of 48 decoded vectors of 32 took 5.2 us of a step.
+// SECOND: false for launches whose targets are all of first order.
+template <bool SECOND>
+__device__ __forceinline__ float filter_step(const FilterTarget* __restrict__ targets, const FilterTarget& t,
+                                             int i, float x, float f_old) {
+    const float bx = __fmul_rn(nhip_bits(t.b_bits), x);
+    if (!SECOND || (t.na >> FILTER_SECOND_SHIFT) == 0)
+        return t.na ? __fsub_rn(bx, __fmul_rn(nhip_bits(t.a_bits), f_old)) : bx;
+    const FilterSecond e = *reinterpret_cast<const FilterSecond*>(targets + (t.na >> FILTER_SECOND_SHIFT));
+    float* x1 = e.state + i;
+    float* y1 = x1 + e.n;
+    float* y2 = y1 + e.n;
+    const float x_1 = *x1, y_1 = *y1, y_2 = *y2;
+    float y = bx;
+    if (t.na & FILTER_NB2) y = __fadd_rn(y, __fmul_rn(nhip_bits(e.b1_bits), x_1));
+    if (t.na & FILTER_NA) y = __fsub_rn(y, __fmul_rn(nhip_bits(t.a_bits), f_old));
+    if ((t.na & FILTER_NA) > 1) y = __fsub_rn(y, __fmul_rn(nhip_bits(e.a1_bits), y_2));
+    *x1 = x;
+    *y1 = y;
+    *y2 = y_1;
+    return y;
+}
+
+// Filter step of element i of every target of a GEMV item whose fresh output is x.
+template <bool SECOND>
 __device__ __forceinline__ void filter_epilogue(const FilterArgs& a, int2 range, int i, float x) {
     for (int q = 0; q < range.y; ++q) {
         const FilterTarget t = a.targets[range.x + q];
         float* f = a.F + (size_t)t.y_start + i;
-        const float bx = __fmul_rn(nhip_bits(t.b_bits), x);
-        *f = t.na ? __fsub_rn(bx, __fmul_rn(nhip_bits(t.a_bits), *f)) : bx;
+        *f = filter_step<SECOND>(a.targets, t, i, x, *f);
     }
 }
 
 // What a GEMV launch does with a finished output row besides storing it.
 // EPI_NEURON: the update of a neuron of another type than the plain LIF (an instance of its own: the
 // LIF instances keep their registers, and their compacted update of the rare cases).
-enum { EPI_NONE = 0, EPI_LIF = 1, EPI_FILTER = 2, EPI_NEURON = 3 };
+// EPI_FILTER2: EPI_FILTER where a target is of second order (in the instances of EPI_FILTER the code
+// for it cost launches without one 1-3 % of a step).
+enum { EPI_NONE = 0, EPI_LIF = 1, EPI_FILTER = 2, EPI_NEURON = 3, EPI_FILTER2 = 4 };
+constexpr bool epi_filters(int epi) { return epi == EPI_FILTER || epi == EPI_FILTER2; }
 struct EpilogueArgs {
     LifArgs lif;
     FilterArgs filter;

@@ -483,7 +483,7 @@ class gemv_prog:
         dev_items = to_device(queue, table)
         dev_at = to_device(queue, np.concatenate(parts))
         n = len(rows)
-        args = (dev_items.ptr, n, dev_at.ptr, self.X.ptr, self.Y_in.ptr, self.Y.ptr, None, None,
+        args = (dev_items.ptr, n, dev_at.ptr, self.X.ptr, self.Y_in.ptr, self.Y.ptr, None, None, 1,
                 int(table[:, 3].max()))
         plan = Plan(queue, queue.lib.nhip_gemv_events, args, gsize=(1024 * n,), lsize=(1024,),
                     full_args=(dev_items, dev_at, self.X.dev_buf, self.Y_in.dev_buf, self.Y.dev_buf),
@@ -1472,14 +1472,52 @@ def _read_spans(prog, ptr_value):
     return [iv for iv in read if iv]
 
 
-def fuse_linearfilter(gemv_plans, lf_plan):
+def _second_order_targets(queue, rows, second, spec, a_host, b_host):
+    """The table of filter targets with the records of the second-order ones (`second`: filter ->
+    number of its record) behind the `rows` (y_start, a0, b0, na, filter), and the device array of
+    their states (x[t-1], y[t-1], y[t-2] per element; what the ring buffers hold at position 0)."""
+    X, A, B = spec["X"], spec["A"], spec["B"]
+    table = np.zeros((len(rows) + 2 * len(second), 4), dtype=np.int32)
+    table[:len(rows)] = [row[:4] for row in rows]
+    sizes = [int(X.shape0s[i]) for i in second]  # (numbered in the order they were met)
+    starts = np.concatenate([[0], np.cumsum(3 * np.array(sizes, dtype=np.int64))])
+    state = np.zeros(int(starts[-1]), dtype=np.float32)
+    x_host, y_host = spec["Xbuf"].to_host(), spec["Ybuf"].to_host()
+    for i, k in second.items():
+        old = state[starts[k]:starts[k + 1]].reshape(3, -1)
+        if int(B.shape0s[i]) > 1:
+            old[0] = x_host[i][1]
+        if int(A.shape0s[i]) > 1:
+            old[1:] = y_host[i][:2]
+    dev_state = to_device(queue, state)
+    float_bits = lambda v: int(np.float32(v).view(np.int32))
+    for row, (_, _, _, na, i) in zip(table, rows):
+        if i not in second:
+            continue
+        at = len(rows) + 2 * second[i]
+        row[3] = na + (4 if int(B.shape0s[i]) > 1 else 0) + 8 * at
+        table[at, 0] = float_bits(a_host[i][1, 0]) if na > 1 else 0
+        table[at, 1] = float_bits(b_host[i][1, 0]) if int(B.shape0s[i]) > 1 else 0
+        table[at, 2] = int(X.shape0s[i])
+        table[at + 1, :2] = np.array([dev_state.ptr.value + 4 * int(starts[second[i]])],
+                                     dtype=np.uint64).view(np.int32)
+    return table, dev_state
+
+
+def _keep_filter_state(plan, state):
+    if state is not None:
+        plan.full_args = tuple(plan.full_args) + (state,)
+        plan.filter_state = state  # zeroed again by Simulator.reset()
+
+
+def fuse_linearfilter(gemv_plans, lf_plan, second_order=False):
     """Fewer launches for "Y = GEMV(...); filter step on Y" (clra_gemv.py
     `plan_block_gemv` followed by clra_nonlinearities.py `plan_linearfilter`): the
-    reference-order kernels step the first-order filters whose input is one of their
-    output items as soon as a row is final.
+    reference-order kernels step the filters of first and (with `second_order`) second order whose
+    input is one of their output items as soon as a row is final.
 
     `gemv_plans` are the plans of one GEMV (one `gemv_prog`).  A filter item is fused
-    when it has one numerator and at most one denominator coefficient, its input is
+    when it has at most one (two) numerator and one (two) denominator coefficients, its input is
     exactly the output of an item of a reference-order launch without another
     epilogue, and both vectors are contiguous.  Returns ``(plans replacing gemv_plans,
     plans replacing [lf_plan])`` -- the second list holds a filter launch for the items
@@ -1508,8 +1546,10 @@ def fuse_linearfilter(gemv_plans, lf_plan):
     a_host, b_host = A.to_host(), B.to_host()
     targets_of = defaultdict(list)
     rest = []
+    second = {}  # filter -> (b1 or None, a1 or None): two coefficients on a side
     for i in range(len(X)):
-        simple = int(B.shape0s[i]) == 1 and int(A.shape0s[i]) <= 1
+        most = 2 if second_order else 1
+        simple = 1 <= int(B.shape0s[i]) <= most and int(A.shape0s[i]) <= most
         vector = (int(X.shape1s[i]) == 1 and int(X.stride0s[i]) == 1
                   and int(F.shape1s[i]) == 1 and int(F.stride0s[i]) == 1)
         b = large.get((int(X.starts[i]), int(X.shape0s[i]))) if simple and vector else None
@@ -1519,7 +1559,9 @@ def fuse_linearfilter(gemv_plans, lf_plan):
         na = int(A.shape0s[i])
         a0 = np.float32(a_host[i][0, 0]) if na else np.float32(0)
         b0 = np.float32(b_host[i][0, 0])
-        targets_of[b].append((int(F.starts[i]), int(a0.view(np.int32)), int(b0.view(np.int32)), na))
+        if na > 1 or int(B.shape0s[i]) > 1:
+            second[i] = len(second)
+        targets_of[b].append((int(F.starts[i]), int(a0.view(np.int32)), int(b0.view(np.int32)), na, i))
     if not targets_of:
         return None
     fused_filters = [i for i in range(len(X)) if i not in set(rest)]
@@ -1536,8 +1578,12 @@ def fuse_linearfilter(gemv_plans, lf_plan):
         item_targets[b] = (len(target_rows), len(rows))
         target_rows.extend(rows)
     dev_items = to_device(queue, item_targets)
-    dev_targets = to_device(queue, np.array(target_rows, dtype=np.int32))
-    extra = (dev_items.ptr, dev_targets.ptr, F.ptr)
+    targets, filter_state = np.array([row[:4] for row in target_rows], dtype=np.int32), None
+    if second:
+        targets, filter_state = _second_order_targets(queue, target_rows, second, spec, a_host, b_host)
+    dev_targets = to_device(queue, targets)
+    order = 2 if second else 1
+    extra = (dev_items.ptr, dev_targets.ptr, F.ptr, order)
     out = []
     for plan in gemv_plans:
         if not _takes_filters(plan) or not any(b in targets_of for b in plan.members):
@@ -1553,7 +1599,7 @@ def fuse_linearfilter(gemv_plans, lf_plan):
             dev_table = to_device(queue, table)
             fused = Plan(queue, lib.nhip_gemv_events,
                          (dev_table.ptr,) + tuple(plan.args[1:6]) + (dev_targets.ptr, F.ptr,
-                                                                      plan.args[8]),
+                                                                      order, plan.args[9]),
                          gsize=plan.gsize, lsize=plan.lsize,
                          full_args=plan.full_args + (dev_table, dev_targets, F.dev_buf),
                          name=plan.name + "_filter", tag=plan.tag,
@@ -1567,6 +1613,7 @@ def fuse_linearfilter(gemv_plans, lf_plan):
             fused.dev_event_table = dev_table
             fused.event_record_item = plan.event_record_item
             fused.host_tasks = None
+            _keep_filter_state(fused, filter_state)
             out.append(fused)
             continue
         entry, args, keep = _epilogue_call(
@@ -1593,6 +1640,7 @@ def fuse_linearfilter(gemv_plans, lf_plan):
         fused.gemv_bytes = plan.bw_per_call
         if plan.kernel_class[0] == 3:
             fused.host_tasks = tasks
+        _keep_filter_state(fused, filter_state)
         out.append(fused)
     residual = []
     if rest:

@@ -20,6 +20,7 @@ produces the operator graph) or a `minibuilder.Network`; ``model`` may be a
 nengo ``Model`` or an `ir.Model` that already holds operators.
 """
 
+import functools
 import inspect
 import logging
 import os
@@ -91,7 +92,7 @@ class HipBackend:
         if os.environ.get("NENGO_HIP_CARRY_SEQUENCES", "1") != "0":  # switch for measurements
             self.carry_sequences = hipra_sequence.carry_sequences
         self.plans_conflict = hipra_sequence._conflict
-        self.fuse_gemv_filter = hipra_gemv.fuse_linearfilter
+        self.fuse_gemv_filter = functools.partial(hipra_gemv.fuse_linearfilter, second_order=True)
         self.fuse_spmv_filter = hipra_spmv.fuse_linearfilter
         if os.environ.get("NENGO_HIP_OUTER_FILTER", "1") != "0":  # switch for measurements
             self.fuse_outer_filter = hipra_nonlinearities.fuse_outer_filter
@@ -962,6 +963,8 @@ class Simulator:
             for new, old in zip(fused, plans[lo:i + 1]):
                 new.reads_mem = old.reads_mem | fr
                 new.writes_mem = old.writes_mem | fw
+                if getattr(new, "filter_state", None) is not None:
+                    self._filter_positions.append(new.filter_state)
             for p in residual:
                 p.reads_mem, p.writes_mem = rr, rw
                 if ops is not None and len(ops) == len(lf.lf_spec["X"]):
@@ -1692,15 +1695,17 @@ class Simulator:
         python_ops = []
         for process_class, ops in groupby(all_ops, lambda op: type(op.process)):
             for cls in process_class.__mro__:
-                attr = "_plan_" + cls.__name__
-                if hasattr(self, attr):
-                    plan_groups[attr].extend(ops)
+                # (synapses of every class share a planner, and so a launch: a product steps the
+                # filters of one of them in its epilogue)
+                planner = getattr(self, "_plan_" + cls.__name__, None)
+                if planner is not None:
+                    plan_groups[planner].extend(ops)
                     break
             else:
                 python_ops.extend(ops)
         plans = []
-        for attr, ops in plan_groups.items():
-            for p in getattr(self, attr)(ops):
+        for planner, ops in plan_groups.items():
+            for p in planner(ops):
                 p.planned_ops = ops  # each process class touches its own signals only
                 plans.append(p)
         plans += [p for op in python_ops for p in self._plan_python_process(op)]

@@ -483,3 +483,47 @@ def test_neuron_types_in_the_launch_of_their_currents(queue, kind, neurons, dims
         cpu.run_steps(40)
         assert np.any(gpu.data[probe] != 0) and np.array_equal(gpu.data[probe], cpu.data[probe_o])
         assert np.array_equal(gpu.signal_buffer().view(np.uint32), cpu.signal_buffer().view(np.uint32))
+
+
+# the small-item kernel with four lanes and with a wave or a group per row, the large-item kernel, the
+# launch that visits active columns (one and several groups of 64 rows)
+@pytest.mark.parametrize("kind,neurons,dims,ensembles,launch", [
+    ("LIF", 41, 2, 3, "wave_ref_filter"), ("LIFRate", 2000, 32, 4, "tile_filter"),
+    ("LIFRate", 9000, 3, 3, "tile_filter"), ("LIFRate", 701, 64, 40, "tile_filter"),
+    ("LIFRate", 150, 200, 3, None), ("LIF", 1501, 50, 3, "events_filter"),
+    ("LIF", 5000, 130, 3, "events_filter"), ("LIF", 1024, 32, 48, "events_filter")])
+def test_filters_of_second_order_in_the_launch_of_their_input(queue, kind, neurons, dims, ensembles, launch):
+    """Every synapse with at most two coefficients on a side is stepped by the launch that decodes
+    its input, several of one decoded value included; one of third order keeps its launch."""
+    from nengo_ocl_amd import minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    synapses = [mb.Alpha(0.01), mb.LinearFilter([0.3, 0.2], [1.0, -0.5], analog=False),
+                mb.LinearFilter([0.4], [1.0, -0.7, 0.2], analog=False), mb.Lowpass(0.005),
+                mb.LinearFilter([0.4, 0.1], [1.0], analog=False),
+                mb.LinearFilter([0.1], [1.0, -0.7, 0.2, 0.1], analog=False)]
+
+    def make():
+        net = mb.Network(seed=6, solver="surrogate", share_decoded=True)
+        stim = net.Node(mb.WhiteSignal(period=0.5, high=6.0, seed=3), size_out=dims)
+        ens = [net.Ensemble(neurons, dims, neuron_type=getattr(mb, kind)(), radius=2.0)
+               for _ in range(ensembles)]
+        net.Connection(stim, ens[0], synapse=mb.Alpha(0.005))
+        for k in range(ensembles):
+            for u, synapse in enumerate(synapses if k == 0 else synapses[k % 5:k % 5 + 1]):
+                net.Connection(ens[k], ens[(k + u + 1) % ensembles], synapse=synapse, transform=0.3)
+        return net, [net.Probe(ens[1], synapse=mb.Alpha(0.01)), net.Probe(ens[-1], synapse=0.01)]
+
+    (net, probes), (net_o, probes_o) = make(), make()
+    with Simulator(net, seed=1) as gpu, OracleSimulator(net_o, seed=1) as cpu:
+        cpu.run_steps(40)
+        names = [p.name for p in gpu._plans]
+        fused = [p for p in gpu._plans if getattr(p, "filter_state", None) is not None]
+        assert fused and (launch is None or any(p.name == "hipra_gemv." + launch for p in fused)), names
+        for _ in range(2):  # the second time from a reset: the filters' states with it
+            gpu.run_steps(40)
+            for p, p_o in zip(probes, probes_o):
+                assert np.any(gpu.data[p] != 0) and np.array_equal(gpu.data[p], cpu.data[p_o])
+            assert np.array_equal(gpu.signal_buffer().view(np.uint32), cpu.signal_buffer().view(np.uint32))
+            gpu.reset()
