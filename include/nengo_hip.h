@@ -315,6 +315,16 @@ int nhip_gemv_rows_lif_sums(void *stream, int lpr, int task_words, const int *it
                             const int *pops, double dt, int upsample, float *V, float *W,
                             float *S, const float *TAU, const float *REF, const float *AMP,
                             const int *sum_ranges, const int *parts);
+/* nhip_gemv_rows_lif that also leaves the spikes of one population -- the one with bit 12 of its
+ * pflags set; rows of it are tasks in order, the first a multiple of 64 / lanes per row among the
+ * launch's tasks (of 64 rows, from multiples of 64 on, where a task is a wave's) -- as one bit per
+ * neuron in `mask`, 16-byte aligned, for nhip_spmv_sell_bits.  lpr 1, 4 or 64. */
+int nhip_gemv_rows_lif_bits(void *stream, int lpr, int task_words, const int *items,
+                            const float *coefs, const int *dots, const int *tasks, int n_tasks,
+                            const float *A, const float *X, const float *Yin, float *Y,
+                            const int *pops, double dt, int upsample, float *V, float *W,
+                            float *S, const float *TAU, const float *REF, const float *AMP,
+                            unsigned *mask);
 int nhip_gemv_rows_filter(void *stream, int lpr, int task_words, const int *items,
                           const float *coefs, const int *dots, const int *tasks, int n_tasks,
                           const float *A,
@@ -402,6 +412,17 @@ int nhip_spmv_sell_spikes(void *stream, const int *slices, int n_slices, const i
                           const int *cols, const float *vals, const float *X, float *Y,
                           const int *slice_epi, const int *targets, float *F, int x_start,
                           int n_cols, unsigned *mask, unsigned *ranges);
+
+/* The product of an X given as bits -- element c is `one` where bit c of `mask` is set and +0.0
+ * elsewhere (nhip_gemv_rows_lif_bits) --, with filters (slice_epi) or without; n_cols at most
+ * 1,179,520 (NHIP_E_TOOBIG).  `slices` as above (x_start, len_start and window unused), `width` a multiple of
+ * 4 * lanes (lanes 1, 2 or 4); `vals` as above; `cols` of index_bits 24 (or 16, for n_cols <= 65,535) per
+ * element, four elements in three (two) words: quad k of row r of a slice at word
+ * (data_start / 4 + 64 k + r) * 3 (2).  Elements past a row's end have column n_cols and value -0. */
+int nhip_spmv_sell_bits(void *stream, const int *slices, int n_slices, const int *cols,
+                        const float *vals, float *Y, const int *slice_epi, const int *targets,
+                        float *F, int n_cols, const unsigned *mask, float one, int lanes,
+                        int index_bits);
 
 /* ---- neurons -----------------------------------------------------------
  * LIF with refractory state and spike-time interpolation.

@@ -44,6 +44,8 @@ SIGNATURES = {
     "nhip_gemv_tile_rows": [c_int, c_int],
     "nhip_gemv_rows_lif": [P, c_int, c_int, P, P, P, P, c_int, P, P, P, P,
                            P, ctypes.c_double, c_int, P, P, P, P, P, P],
+    "nhip_gemv_rows_lif_bits": [P, c_int, c_int, P, P, P, P, c_int, P, P, P, P,
+                                P, ctypes.c_double, c_int, P, P, P, P, P, P, P],
     "nhip_gemv_rows_lif_sums": [P, c_int, c_int, P, P, P, P, c_int, P, P, P, P,
                                 P, ctypes.c_double, c_int, P, P, P, P, P, P, P, P],
     "nhip_gemv_rows_filter": [P, c_int, c_int, P, P, P, P, c_int, P, P, P, P, P, P, P, c_int],
@@ -52,6 +54,7 @@ SIGNATURES = {
     "nhip_spmv_sell_skip": [P, P, c_int, P, P, P, P, P, c_int, c_int, P],
     "nhip_spmv_sell_filter": [P, P, c_int, P, P, P, P, P, P, P, P, c_int, c_int, P],
     "nhip_spmv_sell_spikes": [P, P, c_int, P, P, P, P, P, P, P, P, c_int, c_int, P, P],
+    "nhip_spmv_sell_bits": [P, P, c_int, P, P, P, P, P, P, c_int, P, c_float, c_int, c_int],
     "nhip_lif": [P, P, c_int, c_double, c_int, P, P, P, P, P, P, P],
     "nhip_lif_rate": [P, P, c_int, P, P, P, P, P],
     "nhip_alif": [P, P, c_int, c_double, c_int, P, P, P, P, P, P, P, P, P, P],

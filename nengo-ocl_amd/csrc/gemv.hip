@@ -312,7 +312,7 @@ int launch_rows_epi(hipStream_t s, int lpr, int task_words, const int* items, co
     if (lpr != 4 && lpr != 1 && lpr != NHIP_WAVE && lpr != NHIP_LPR_LONG_ROWS && lpr != NHIP_WG) return NHIP_E_BADCLASS;
     if (task_words != 4 && task_words != 16) return NHIP_E_BADARG;
     if (lpr >= NHIP_WAVE && task_words != 16) return NHIP_E_BADARG;  // a wave per task
-    if (lpr >= NHIP_LPR_LONG_ROWS && (EPI == EPI_LIF || EPI == EPI_NEURON) && epi.lif.sum_ranges) return NHIP_E_BADARG;
+    if (lpr >= NHIP_LPR_LONG_ROWS && (epi_lif(EPI) || EPI == EPI_NEURON) && epi.lif.sum_ranges) return NHIP_E_BADARG;
     const int rows_per_group = lpr == NHIP_WG ? 1 : (NHIP_WG / NHIP_WAVE) * (lpr >= NHIP_WAVE ? 1 : NHIP_WAVE / lpr);
     side.n_gemv_groups = (n_tasks + rows_per_group - 1) / rows_per_group;
     const dim3 grid(side.n_gemv_groups + side.n_chains);
@@ -324,7 +324,12 @@ int launch_rows_epi(hipStream_t s, int lpr, int task_words, const int* items, co
     auto pick = [&](auto side_tag) {
         constexpr bool SD = decltype(side_tag)::value;
         if (lpr == NHIP_WAVE) launch(gemv_rows_ref_epi_kernel<1, EPI, true, SD, true>);
-        else if (lpr == NHIP_LPR_LONG_ROWS) launch(gemv_rows_ref_epi_kernel<NHIP_WAVE, EPI, true, SD>);
+        else if constexpr (EPI == EPI_LIF_BITS) {  // (no long rows: refused below)
+            if (lpr == 4 && task_words == 16) launch(gemv_rows_ref_epi_kernel<4, EPI, true, SD>);
+            else if (lpr == 4) launch(gemv_rows_ref_epi_kernel<4, EPI, false, SD>);
+            else if (task_words == 16) launch(gemv_rows_ref_epi_kernel<1, EPI, true, SD>);
+            else launch(gemv_rows_ref_epi_kernel<1, EPI, false, SD>);
+        } else if (lpr == NHIP_LPR_LONG_ROWS) launch(gemv_rows_ref_epi_kernel<NHIP_WAVE, EPI, true, SD>);
         else if (lpr == NHIP_WG) launch(gemv_rows_ref_epi_kernel<NHIP_WG, EPI, true, SD>);
         else if (lpr == 4 && task_words == 16) launch(gemv_rows_ref_epi_kernel<4, EPI, true, SD>);
         else if (lpr == 4) launch(gemv_rows_ref_epi_kernel<4, EPI, false, SD>);
@@ -563,6 +568,32 @@ extern "C" int nhip_gemv_rows_lif(void* stream, int lpr, int task_words, const i
     lif.AMP = AMP;
     return launch_rows_epi<EPI_LIF>(static_cast<hipStream_t>(stream), lpr, task_words, items, coefs,
                                     dots, tasks, n_tasks, A, X, Yin, Y, args);
+}
+
+extern "C" int nhip_gemv_rows_lif_bits(void* stream, int lpr, int task_words, const int* items,
+                                       const float* coefs, const int* dots, const int* tasks,
+                                       int n_tasks, const float* A, const float* X, const float* Yin,
+                                       float* Y, const int* pops, double dt, int upsample, float* V,
+                                       float* W, float* S, const float* TAU, const float* REF,
+                                       const float* AMP, unsigned* mask) {
+    if (!pops || !V || !W || !S || upsample < 1 || !(dt > 0.0) || !mask) return NHIP_E_BADARG;
+    if (lpr != 1 && lpr != 4 && lpr != NHIP_WAVE) return NHIP_E_BADCLASS;
+    if (reinterpret_cast<uintptr_t>(mask) & 15u) return NHIP_E_BADARG;
+    EpilogueArgs args{};
+    LifArgs& lif = args.lif;
+    lif.pops = reinterpret_cast<const LifPop*>(pops);
+    lif.dtu = (float)(dt / (double)upsample);
+    lif.dt_inv = (float)(1.0 / dt);
+    lif.upsample = upsample;
+    lif.V = V;
+    lif.W = W;
+    lif.S = S;
+    lif.TAU = TAU;
+    lif.REF = REF;
+    lif.AMP = AMP;
+    lif.mask = mask;
+    return launch_rows_epi<EPI_LIF_BITS>(static_cast<hipStream_t>(stream), lpr, task_words, items, coefs,
+                                         dots, tasks, n_tasks, A, X, Yin, Y, args);
 }
 
 extern "C" int nhip_gemv_rows_lif_sums(void* stream, int lpr, int task_words, const int* items,

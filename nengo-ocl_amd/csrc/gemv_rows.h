@@ -49,7 +49,7 @@ __device__ __forceinline__ void gemv_rows_ref_block(
     const EpilogueArgs* epi = nullptr)
 {
     constexpr int TILE = 128;
-    constexpr bool NEURONS = EPI == EPI_LIF || EPI == EPI_NEURON;
+    constexpr bool NEURONS = epi_lif(EPI) || EPI == EPI_NEURON;
     constexpr int BATCH = 4;             // dot products whose operands are fetched together
     constexpr int CHUNK = 8;             // steps of a partial sum whose operands are fetched together
     constexpr int ROWS = LPR > NHIP_WAVE ? 1 : NHIP_WAVE / LPR;  // rows (tasks) per wave
@@ -89,7 +89,7 @@ __device__ __forceinline__ void gemv_rows_ref_block(
     int2 f_range = make_int2(0, 0);
     FilterTarget f_first = {};
     float f_old = 0.0f;
-    if (EPI == EPI_LIF) {
+    if (epi_lif(EPI)) {
         pop = epi->lif.pops[task.item];
         // where the neuron's state is: from the task record if it says so (the state is
         // then requested together with the population record, not after it)
@@ -319,13 +319,14 @@ __device__ __forceinline__ void gemv_rows_ref_block(
             }
         }
     }
+    bool spiked = false;
     if (lir == 0 && valid) {
         const float y = sum + cf.z;
-        if (!(EPI == EPI_LIF && (pop.pflags & LIF_POP_NO_J)) &&
+        if (!(epi_lif(EPI) && (pop.pflags & LIF_POP_NO_J)) &&
             !(EPI == EPI_NEURON && (npop.flags & LIF_POP_NO_J)))
             Y[it.y_start + (size_t)r * it.y_stride0] = y;
-        if (EPI == EPI_LIF && (pop.pflags & LIF_POP_ENABLED))
-            lif_epilogue(epi->lif, pop, r, y, v_old, w_old);
+        if (epi_lif(EPI) && (pop.pflags & LIF_POP_ENABLED))
+            spiked = lif_epilogue(epi->lif, pop, r, y, v_old, w_old);
         if (EPI == EPI_NEURON && (npop.flags & LIF_POP_ENABLED))
             neuron_epilogue(epi->lif, npop, r, y, v_old, w_old, n_old);
         if (epi_filters(EPI) && f_range.y > 0) {
@@ -334,6 +335,22 @@ __device__ __forceinline__ void gemv_rows_ref_block(
             epi->filter.F[(size_t)f_first.y_start + r] =
                 filter_step<EPI == EPI_FILTER2>(epi->filter.targets, f_first, r, y, f_old);
             filter_epilogue<EPI == EPI_FILTER2>(epi->filter, make_int2(f_range.x + 1, f_range.y - 1), r, y);
+        }
+    }
+    if (EPI == EPI_LIF_BITS) {
+        // The rows of a wave are consecutive rows of the population from a multiple of their number on
+        // (the host's word; a wave at the population's end may hold rows of others behind its own).
+        const bool wanted = valid && (pop.pflags & LIF_POP_MASK);
+        unsigned long long b = __ballot(wanted && lir == 0 && spiked);
+        if (LPR == 4) {  // every fourth lane's bit -> sixteen bits
+            b = (b | b >> 3) & 0x0303030303030303ull;
+            b = (b | b >> 6) & 0x000f000f000f000full;
+            b = (b | b >> 12) & 0x000000ff000000ffull;
+            b = (b | b >> 24) & 0xffffull;
+        }
+        if (lane == 0 && wanted) {
+            if (LPR == 4) reinterpret_cast<unsigned short*>(epi->lif.mask)[r >> 4] = (unsigned short)b;
+            else reinterpret_cast<unsigned long long*>(epi->lif.mask)[r >> 6] = b;
         }
     }
 }

@@ -23,6 +23,10 @@ constexpr int LIF_POP_NO_J = 1 << 10;
 // every task starting at a multiple of 64) -- instead of a float each: a sixteenth of a
 // percent of the bytes, and writes next to a read stream cost about three times theirs
 constexpr int LIF_POP_BITS = 1 << 11;
+// pflags: the small-item launch also leaves the population's spikes as one bit per neuron, in
+// LifArgs::mask, for a sparse product (EPI_LIF_BITS); the floats are stored as always.  A launch of its
+// own for the bits of 100,000 neurons takes 4.6 us of a step of 28.
+constexpr int LIF_POP_MASK = 1 << 12;
 
 // State arrays and constants of a fused LIF update (all populations of a launch).
 struct LifArgs {
@@ -55,6 +59,7 @@ struct LifArgs {
     // neuron types other than the plain LIF (EPI_NEURON): `pops` then points at NeuronPop records
     float* N;            // adaptation states
     float dt;
+    unsigned* mask;      // EPI_LIF_BITS: a bit per neuron of the population with LIF_POP_MASK
 };
 
 // One population of neurons of another type than the plain LIF, driven by one output item of a
@@ -210,7 +215,7 @@ __device__ __forceinline__ void lif_rate_block(const RateDesc d, const float* J,
 
 // LIF update of neuron i of population p with input current j (GEMV epilogue);
 // v and w are the neuron's voltage and refractory time, read earlier
-__device__ __forceinline__ void lif_epilogue(const LifArgs& a, const LifPop& p, int i, float j,
+__device__ __forceinline__ bool lif_epilogue(const LifArgs& a, const LifPop& p, int i, float j,
                                              float v, float w) {
     const float tau = lif_param(p.tau, p.pflags & 1, a.TAU, i);
     const float ref = lif_param(p.ref, p.pflags & 2, a.REF, i);
@@ -219,6 +224,7 @@ __device__ __forceinline__ void lif_epilogue(const LifArgs& a, const LifPop& p, 
     a.V[(size_t)p.v_start + i] = v;
     a.W[(size_t)p.w_start + i] = w;
     a.S[(size_t)p.s_start + i] = spiked ? __fmul_rn(amp, a.dt_inv) : 0.0f;
+    return spiked;
 }
 
 // Update of neuron i of a population of another type with input current j (GEMV epilogue); v, w and n
@@ -315,7 +321,9 @@ __device__ __forceinline__ void filter_epilogue(const FilterArgs& a, int2 range,
 // LIF instances keep their registers, and their compacted update of the rare cases).
 // EPI_FILTER2: EPI_FILTER where a target is of second order (in the instances of EPI_FILTER the code
 // for it cost launches without one 1-3 % of a step).
-enum { EPI_NONE = 0, EPI_LIF = 1, EPI_FILTER = 2, EPI_NEURON = 3, EPI_FILTER2 = 4 };
+// EPI_LIF_BITS: EPI_LIF where a population's spikes are wanted as bits too.
+enum { EPI_NONE = 0, EPI_LIF = 1, EPI_FILTER = 2, EPI_NEURON = 3, EPI_FILTER2 = 4, EPI_LIF_BITS = 5 };
+constexpr bool epi_lif(int epi) { return epi == EPI_LIF || epi == EPI_LIF_BITS; }
 constexpr bool epi_filters(int epi) { return epi == EPI_FILTER || epi == EPI_FILTER2; }
 struct EpilogueArgs {
     LifArgs lif;

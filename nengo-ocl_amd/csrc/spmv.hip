@@ -474,6 +474,200 @@ __global__ __launch_bounds__(SPMV_SKIP_WG) void spmv_sell_skip_kernel(
     }
 }
 
+// ---- spikes that the launch of the neurons has left as bits ------------------------------
+// All spikes have the value `one` (nhip_gemv_rows_lif_bits), so a launch for the bits, look-ups of X and
+// a look at the values it holds fall away.  The layout is one of its own, which leaves a few instructions per
+// stored element (the kernel above is bound by them: 100 elements of a row cost it as much at 6
+// bytes each as at 8):
+//  - column indices of 24 bits, or of 16 where X has fewer than 65,536 elements;
+//  - rows are padded to whole quads for every lane of a row, with a column past X's end, whose bit is
+//    clear, and the value -0: such an element adds -0, which changes no sum, so nothing asks
+//    where a row ends;
+//  - LANES (1, 2, 4) per row, as many as fill the waves: a lane holds every LANES-th quad of its row,
+//    and the sum goes from lane to lane, quad by quad, as in spmv_skip_rows -- which every lane of
+//    the row computes, so fewer lanes are fewer instructions.
+// A wave's record and first elements are on their way before the bits are.
+// A step with its product (the launch of the neurons included; before: bits in a launch of their own,
+// or by every group for itself, 32-bit indices, four lanes per row): 100,000 rows of 100 26.3 -> 18.4 us
+// (the product 18.9 -> 12.6, of 70 MB: 5.6 TB/s), of 20 17.0 -> 10.4; 10,000 rows of 100 11.8 -> 10.6; 2,000 of
+// 30 9.8 -> 9.6; 1,000,000 rows of 20 65.9 -> 50.7.
+template <int BITS> struct SpmvBitCols;
+template <> struct SpmvBitCols<16> {
+    struct quad { int w[2]; };
+    static constexpr int WORDS = 2;
+    static __device__ __forceinline__ unsigned raw(const quad& q, int u) {
+        return (u & 1) ? (unsigned)q.w[u >> 1] >> 16 : (unsigned)q.w[u >> 1];
+    }
+};
+template <> struct SpmvBitCols<24> {
+    struct quad { int w[3]; };
+    static constexpr int WORDS = 3;
+    static __device__ __forceinline__ unsigned raw(const quad& q, int u) {
+        switch (u) {
+            case 0: return (unsigned)q.w[0];
+            case 1: return __builtin_amdgcn_alignbit((unsigned)q.w[1], (unsigned)q.w[0], 24);
+            case 2: return __builtin_amdgcn_alignbit((unsigned)q.w[2], (unsigned)q.w[1], 16);
+            default: return (unsigned)q.w[2] >> 8;
+        }
+    }
+};
+
+template <typename T>
+__device__ __forceinline__ T spmv_uniform(const T* p) {
+    static_assert(sizeof(T) == 16, "four words");
+    typedef const __attribute__((address_space(4))) spmv_i4* scalar;
+    return __builtin_bit_cast(T, *(scalar)reinterpret_cast<uintptr_t>(p));
+}
+
+template <int LANES, int BITS>
+__global__ __launch_bounds__(SPMV_SKIP_WG) void spmv_sell_bits_kernel(
+    const SpmvSlice* __restrict__ slices, int n_slices, const int* __restrict__ cols,
+    const float* __restrict__ vals, float* Y, const unsigned* __restrict__ mask, int n_cols, float one,
+    SpmvEpi epi, SpmvSide side)
+{
+    __shared__ __attribute__((aligned(16))) unsigned s_mask[SPMV_MASK_WORDS];
+    if (side.n_chains > 0 && (int)blockIdx.x >= side.n_groups) return spmv_side_chain(side, s_mask);
+    typedef SpmvBitCols<BITS> Cols;
+    typedef typename Cols::quad quad;
+    constexpr int WAVES = SPMV_SKIP_WG / NHIP_WAVE, U = 4, ROWS = NHIP_WAVE / LANES;
+    const int lane = threadIdx.x & (NHIP_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int j = lane % LANES, stride = side.n_groups * WAVES, n_tasks = LANES * n_slices;
+    const unsigned one_bits = __float_as_uint(one);
+    // quads k .. k + U - 1 of every lane of the row; past the last one: that one again (WHOLE: there are U)
+    auto request = [&](auto whole, const SpmvSlice& sl, int row, int k, quad (&c)[U], spmv_f4 (&v)[U]) {
+        const int m = sl.width / (4 * LANES);  // quads per lane (the host pads the width)
+        const char* cs = reinterpret_cast<const char*>(cols) + (size_t)(sl.data_start >> 2) * sizeof(quad);
+        const char* vs = reinterpret_cast<const char*>(vals + (size_t)sl.data_start);
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const int q = decltype(whole)::value ? k + i : min(k + i, m - 1);
+            const unsigned at = (unsigned)(LANES * q + j) * NHIP_WAVE + row;
+            const int* cp = reinterpret_cast<const int*>(cs + at * (unsigned)sizeof(quad));
+#pragma unroll
+            for (int w = 0; w < Cols::WORDS; ++w) c[i].w[w] = __builtin_nontemporal_load(cp + w);
+            v[i] = __builtin_nontemporal_load(reinterpret_cast<const spmv_f4*>(vs + at * 16u));
+        }
+    };
+    float acc = 0.0f;
+    auto add = [&](auto whole, int n, const quad (&c)[U], const spmv_f4 (&v)[U]) {  // n quads of every lane
+        float x[U][4];
+#pragma unroll
+        for (int i = 0; i < U; ++i)
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                x[i][u] = __uint_as_float(s_mask[(Cols::raw(c[i], u) >> 5) & ((1u << (BITS - 5)) - 1u)]);
+        __builtin_amdgcn_sched_barrier(0);  // (every look-up of the batch before the first is waited for)
+#pragma unroll
+        for (int i = 0; i < U; ++i)
+#pragma unroll
+            for (int u = 0; u < 4; ++u)  // the bit, spread over the word: the value or +0
+                x[i][u] = __uint_as_float((unsigned)__builtin_amdgcn_sbfe((int)__float_as_uint(x[i][u]),
+                                                                          Cols::raw(c[i], u), 1) & one_bits);
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            if (!decltype(whole)::value && i >= n) break;  // uniform
+#define SPMV_LINK(CTRL)                                                                      \
+            {                                                                                \
+                _Pragma("unroll") for (int u = 0; u < 4; ++u) acc = fmaf(v[i][u], x[i][u], acc); \
+                if (LANES > 1)                                                               \
+                    acc = __int_as_float(__builtin_amdgcn_update_dpp(                        \
+                        0, __float_as_int(acc), CTRL, 0xF, 0xF, true));                      \
+            }
+            if (LANES == 4) {  // the sum of lane 0 of the four to all of them, then lane 1's, ...
+                SPMV_LINK(0x00) SPMV_LINK(0x55) SPMV_LINK(0xAA) SPMV_LINK(0xFF)
+            } else if (LANES == 2) {
+                SPMV_LINK(0xA0) SPMV_LINK(0xF5)
+            } else {
+                SPMV_LINK(0xE4)
+            }
+#undef SPMV_LINK
+        }
+    };
+    constexpr std::true_type all{};
+    constexpr std::false_type part{};
+
+    int t = wave * side.n_groups + blockIdx.x;
+    // the bits are asked for first: what they are waited for with is only asked for behind them
+    // (one quad more than the bits: the column of the padding is X's first past its end)
+    const int n_mask_quads = (n_cols + 127) / 128;
+    spmv_i4 bits = {0, 0, 0, 0};
+    if ((int)threadIdx.x < n_mask_quads) bits = reinterpret_cast<const spmv_i4*>(mask)[threadIdx.x];
+    SpmvSlice sl = slices[min(t / LANES, n_slices - 1)];
+    int row = ROWS * (t % LANES) + lane / LANES;
+    quad ca[U], cb[U];
+    spmv_f4 va[U], vb[U];
+    if (sl.width > 0) request(part, sl, row, 0, ca, va);  // (uniform; a wave without a task: of the last slice)
+    // what the row needs at its end is requested now as well: its old sum and its first filter's old value
+    int4 filters = make_int4(0, 0, 0, 0);
+    FilterTarget f_first = {};
+    float y_old = 0.0f, f_old = 0.0f;
+    auto request_ends = [&](int s) {
+        // (tables that no launch writes, at addresses that are the wave's: scalar loads, which
+        // wait for nothing but themselves)
+        if (epi.slice_epi) filters = spmv_uniform(epi.slice_epi + s);
+        if (filters.y > 0) f_first = spmv_uniform(epi.targets + filters.x);
+        y_old = f_old = 0.0f;
+        if (row < sl.n_rows) {
+            if (sl.inc) y_old = Y[(size_t)sl.y_start + row];
+            if (filters.y > 0) f_old = epi.F[(size_t)f_first.y_start + filters.z + row];
+        }
+    };
+    request_ends(min(t / LANES, n_slices - 1));
+    if ((int)threadIdx.x <= n_mask_quads) reinterpret_cast<spmv_i4*>(s_mask)[threadIdx.x] = bits;
+    for (int i = threadIdx.x + SPMV_SKIP_WG; i <= n_mask_quads; i += SPMV_SKIP_WG)
+        reinterpret_cast<spmv_i4*>(s_mask)[i] =
+            i < n_mask_quads ? reinterpret_cast<const spmv_i4*>(mask)[i] : spmv_i4{0, 0, 0, 0};
+    __syncthreads();  // the only barrier; every thread reaches it
+    while (t < n_tasks) {
+        const int m = sl.width / (4 * LANES);
+        const bool live = row < sl.n_rows;
+        acc = y_old;
+        int k = 0;
+#pragma unroll 1
+        for (; k + 3 * U <= m; k += 2 * U) {  // a batch is requested before the one ahead of it is summed
+            request(all, sl, row, k + U, cb, vb);
+            __builtin_amdgcn_sched_barrier(0);
+            add(all, U, ca, va);
+            request(all, sl, row, k + 2 * U, ca, va);
+            __builtin_amdgcn_sched_barrier(0);
+            add(all, U, cb, vb);
+        }
+        for (; k < m; k += 2 * U) {  // up to three batches are left, the last of them in part
+            const bool more = k + U < m, yet_more = k + 2 * U < m;
+            if (more) {
+                request(part, sl, row, k + U, cb, vb);
+                __builtin_amdgcn_sched_barrier(0);
+                add(all, U, ca, va);
+                if (yet_more) {
+                    request(part, sl, row, k + 2 * U, ca, va);
+                    __builtin_amdgcn_sched_barrier(0);
+                    add(all, U, cb, vb);
+                } else {
+                    add(part, m - k - U, cb, vb);
+                }
+            } else {
+                add(part, m - k, ca, va);
+            }
+        }
+        if (live && j == 0) {
+            Y[(size_t)sl.y_start + row] = acc;
+            if (filters.y > 0) {
+                epi.F[(size_t)f_first.y_start + filters.z + row] =
+                    filter_step<false>(epi.targets, f_first, row, acc, f_old);
+                filter_epilogue<false>(FilterArgs{nullptr, epi.targets, epi.F, nullptr},
+                                       make_int2(filters.x + 1, filters.y - 1), filters.z + row, acc);
+            }
+        }
+        t += stride;
+        if (t >= n_tasks) break;
+        sl = slices[t / LANES];
+        row = ROWS * (t % LANES) + lane / LANES;
+        if (sl.width > 0) request(part, sl, row, 0, ca, va);
+        request_ends(t / LANES);
+    }
+}
+
 // a sequence armed by nhip_gemv_tile_carry is the calling launch's, whatever becomes of it
 SpmvSide take_side() {
     SpmvSide side{};
@@ -507,6 +701,23 @@ int launch_plain(void* stream, const int* slices, int n_slices, const int* row_l
     return 0;
 }
 
+// Groups of a product of spikes with so many tasks for waves at most.
+bool skip_groups(SpmvSide& side, int most) {
+    static int n_cu = 0;
+    if (n_cu == 0) {
+        int dev = 0;
+        hipDeviceProp_t prop;
+        if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess)
+            return false;
+        n_cu = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
+    }
+    // a group takes a whole compute unit (its LDS holds the bits of X), so the groups of a
+    // carried sequence need compute units of their own: with one product group per compute
+    // unit they would only start when the product is over
+    side.n_groups = min(n_cu > side.n_chains ? n_cu - side.n_chains : n_cu, most);
+    return true;
+}
+
 // The product, behind a launch for the bits of X where X is long.
 int launch_skip(void* stream, const int* slices, int n_slices, const int* row_len,
                 const int* cols, const float* vals, const float* X, float* Y, int x_start,
@@ -531,18 +742,7 @@ int launch_skip(void* stream, const int* slices, int n_slices, const int* row_le
                           4 * n_mask_quads);
         NHIP_LAUNCH_CHECK();
     }
-    static int n_cu = 0;
-    if (n_cu == 0) {
-        int dev = 0;
-        hipDeviceProp_t prop;
-        if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess)
-            return NHIP_E_BADARG;
-        n_cu = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
-    }
-    // a group takes a whole compute unit (its LDS holds the bits of X), so the groups of a
-    // carried sequence need compute units of their own: with one product group per compute
-    // unit they would only start when the product is over
-    side.n_groups = min(n_cu > side.n_chains ? n_cu - side.n_chains : n_cu, 4 * n_slices);
+    if (!skip_groups(side, 4 * n_slices)) return NHIP_E_BADARG;
     const dim3 grid(side.n_groups + side.n_chains);
     if (bits_in_kernel)
         NHIP_LAUNCH(spmv_sell_skip_kernel, grid, dim3(SPMV_SKIP_WG), 0, s,
@@ -589,6 +789,42 @@ extern "C" int nhip_spmv_sell_spikes(void* stream, const int* slices, int n_slic
                                   : SpmvEpi{};
     return launch_skip(stream, slices, n_slices, row_len, cols, vals, X, Y, x_start, n_cols, mask,
                        ranges, epi);
+}
+
+// The product of spikes whose bits are in `mask` already (nhip_gemv_rows_lif_bits) and all have
+// the value `one`, on the layout of spmv_sell_bits_kernel.
+extern "C" int nhip_spmv_sell_bits(void* stream, const int* slices, int n_slices, const int* cols,
+                                   const float* vals, float* Y, const int* slice_epi, const int* targets,
+                                   float* F, int n_cols, const unsigned* mask, float one, int lanes,
+                                   int index_bits) {
+    SpmvSide side = take_side();
+    if (n_slices == 0) return side.n_chains > 0 ? NHIP_E_BADARG : 0;  // nothing to ride in
+    if (n_slices < 0 || !slices || !cols || !vals || !Y || !mask || n_cols <= 0 ||
+        (slice_epi && (!targets || !F)))
+        return NHIP_E_BADARG;
+    if (n_slices > (1 << 28) || n_cols > 32 * SPMV_MASK_WORDS - 128 || (index_bits == 16 && n_cols > 0xffff))
+        return NHIP_E_TOOBIG;
+    if ((reinterpret_cast<uintptr_t>(vals) | reinterpret_cast<uintptr_t>(mask)) & 15) return NHIP_E_BADARG;
+    const SpmvEpi epi = slice_epi ? SpmvEpi{reinterpret_cast<const int4*>(slice_epi),
+                                            reinterpret_cast<const FilterTarget*>(targets), F}
+                                  : SpmvEpi{};
+    if (!skip_groups(side, lanes * n_slices)) return NHIP_E_BADARG;
+    auto launch = [&](auto kernel) {
+        NHIP_LAUNCH(kernel, dim3(side.n_groups + side.n_chains), dim3(SPMV_SKIP_WG), 0,
+                    static_cast<hipStream_t>(stream), reinterpret_cast<const SpmvSlice*>(slices), n_slices,
+                    cols, vals, Y, mask, n_cols, one, epi, side);
+        return 0;
+    };
+    const int kind = 100 * lanes + index_bits;
+    if (kind == 116) launch(spmv_sell_bits_kernel<1, 16>);
+    else if (kind == 216) launch(spmv_sell_bits_kernel<2, 16>);
+    else if (kind == 416) launch(spmv_sell_bits_kernel<4, 16>);
+    else if (kind == 124) launch(spmv_sell_bits_kernel<1, 24>);
+    else if (kind == 224) launch(spmv_sell_bits_kernel<2, 24>);
+    else if (kind == 424) launch(spmv_sell_bits_kernel<4, 24>);
+    else return NHIP_E_BADCLASS;
+    NHIP_LAUNCH_CHECK();
+    return 0;
 }
 
 // Either product with first-order filters stepped on its fresh rows: `slice_epi` holds

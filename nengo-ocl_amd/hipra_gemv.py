@@ -116,6 +116,7 @@ THIN_MIN_ROWS, THIN_ROWS_FOR_LANE_PER_ROW = 32, 65536
 # LDS 5.6-9.6; whole steps of 2 x 5,500 x 3 to 2 x 30,000 x 1 LIF neurons 17.1-58.5 us against 22.1-64.3.
 THIN_CLASS, THIN_MAX_COLS = (2, 4, 1), 4
 LIF_POP_ENABLED, LIF_POP_DECAY, LIF_POP_NO_J = 1 << 8, 1 << 9, 1 << 10  # flag bits of a population row
+LIF_POP_MASK = 1 << 12
 LIF_POP_BITS = 1 << 11  # spikes stored as a bit per neuron (see `store_spikes_as_bits`)
 LIF_COMPACT = os.environ.get("NENGO_HIP_LIF_COMPACT", "1") != "0"
 
@@ -1314,6 +1315,44 @@ def store_spikes_as_bits(enc_plan, items, event_records, dt):
             plan.dev_event_table.set(plan.event_table.astype(np.int32).ravel())
         enc_plan.tag = "%s + spikes as bits" % enc_plan.tag
     return values
+
+
+def leave_spike_bits(lif_plan, s_start, n):
+    """Make a small-item launch with the LIF epilogue leave the spikes of the population whose
+    output is the `n` elements at `s_start` as bits too (`nhip_gemv_rows_lif_bits`).  Returns
+    ``(device array of the bits, value of a spike)``, or None where the launch cannot: it forms input
+    sums itself, has an amplitude per neuron (or one of zero), or the population's rows do not fill
+    its waves in order from a wave's first row on."""
+    if (getattr(lif_plan.kern, "__name__", "") != "nhip_gemv_rows_lif"
+            or getattr(lif_plan, "host_tables", None) is None or lif_plan.args[0] not in (1, 4, WAVE)):
+        return None
+    queue, pops = lif_plan.queue, lif_plan.host_pops
+    hit = [b for b in lif_plan.members if int(pops[b, 2]) == s_start and int(pops[b, 7]) & LIF_POP_ENABLED
+           and lif_plan.prog.geometry[b]["y_len"] == n]
+    if len(hit) != 1 or int(pops[hit[0], 7]) & (4 | LIF_POP_MASK):
+        return None
+    item = hit[0]
+    one = np.float32(pops[item, 6:7].view(np.float32)[0] * np.float32(1.0 / lif_plan.args[12]))
+    if not np.isfinite(one) or one == 0:
+        return None
+    tasks = lif_plan.host_tables[2]
+    mine = np.flatnonzero(tasks[:, 0] == item)
+    if lif_plan.args[0] == WAVE:  # tasks of 64 rows
+        if np.any(tasks[mine, 1] % WAVE) or int(tasks[mine, 2].sum()) != n:
+            return None
+    else:
+        rows = WAVE // lif_plan.args[0]
+        if (len(mine) != n or mine[0] % rows or np.any(np.diff(mine) != 1)
+                or not np.array_equal(tasks[mine, 1], np.arange(n))):
+            return None
+    pops[item, 7] |= LIF_POP_MASK
+    lif_plan.dev_pops.set(pops.astype(np.int32).ravel())
+    mask = to_device(queue, np.zeros(-(-n // 128) * 4, dtype=np.int32))
+    lif_plan.kern = queue.lib.nhip_gemv_rows_lif_bits
+    lif_plan.args = tuple(lif_plan.args) + (mask.ptr,)
+    lif_plan.full_args = tuple(lif_plan.full_args) + (mask,)
+    lif_plan.tag = "%s + spikes as bits too" % lif_plan.tag
+    return mask, one
 
 
 def fuse_learning(enc_plan, dec_plan, ew_plan, lf_plan):

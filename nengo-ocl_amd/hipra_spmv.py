@@ -107,6 +107,41 @@ def sell_layout(matrices):
     return slice_rows, cat(lens, np.int32), cat(cols, np.int32), cat(vals, np.float32)
 
 
+def bits_lanes(n_slices, n_waves):
+    """Lanes per row of the product that is handed its spikes as bits: as many as fill the waves of
+    the device (`n_waves`); every lane repeats the sum of its row, which a second or fourth lane has to
+    be worth (180,000 rows of 60, one lane: 28.4 us a step before, 19.4 now; 100,000 rows of 100, two:
+    18.4, with four and 16-bit indices 24.4)."""
+    cost = lambda lanes: -(-n_slices * lanes // n_waves) / lanes * (1 + 0.15 * (lanes - 1))
+    return min((1, 2, 4), key=cost)
+
+
+def bits_layout(slice_rows, row_len, cols, vals, n_cols, lanes):
+    """The arrays of `sell_layout` as `nhip_spmv_sell_bits` takes them: ``(start of every slice,
+    width of every slice, cols, vals, bits per index)``.  Rows are padded to whole quads for each of `lanes` lanes with
+    column `n_cols` and value -0; four indices take three words, or two where 16 bits hold `n_cols`."""
+    unit = QUAD * lanes
+    widths = np.array([-(-w // unit) * unit for _, _, w, _, _, _ in slice_rows], dtype=np.int64)
+    starts = np.concatenate([[0], np.cumsum(widths * WAVE)])
+    out_c = np.full(int(starts[-1]), n_cols, dtype=np.uint32)
+    out_v = np.full(int(starts[-1]), -0.0, dtype=np.float32)
+    for (_, start, w, len_start, _, _), at, width in zip(slice_rows, starts, widths):
+        shape = (w // QUAD, WAVE, QUAD)
+        n = w * WAVE
+        stored = (QUAD * np.arange(w // QUAD)[:, None, None] + np.arange(QUAD)
+                  < row_len[len_start:len_start + WAVE][:, None])
+        out_c[at:at + n].reshape(shape)[stored] = cols[start:start + n].reshape(shape)[stored]
+        out_v[at:at + n].reshape(shape)[stored] = vals[start:start + n].reshape(shape)[stored]
+    if n_cols < 65536:
+        return starts[:-1], widths, out_c.astype(np.uint16).view(np.int32), out_v, 16
+    q = out_c.reshape(-1, QUAD)
+    words = np.empty((len(q), 3), dtype=np.uint32)
+    words[:, 0] = q[:, 0] | q[:, 1] << 24
+    words[:, 1] = q[:, 1] >> 8 | q[:, 2] << 16
+    words[:, 2] = q[:, 2] >> 16 | q[:, 3] << 8
+    return starts[:-1], widths, words.view(np.int32).ravel(), out_v, 24
+
+
 class plan_sparse_dot_inc:
     """``Y[b] (=|+=) A[b] @ X[b]``; ``.plans`` holds the one launch.
 
@@ -188,7 +223,7 @@ class plan_sparse_dot_inc:
         plan.skips_zero_x = skip
         # what `fuse_linearfilter` needs to rebuild the launch with filters behind its rows
         plan.spmv = dict(X=X, Y=Y, slice_rows=slice_rows, dev=tuple(dev), n=n,
-                         workspaces=workspaces,
+                         workspaces=workspaces, host=(table, row_len, cols, vals) if skip else None,
                          x_start=int(X.starts[0]) if skip else 0,
                          n_cols=int(X.shape0s[0]) if skip else 0)
         plan.flops_per_call = 2 * nnz
@@ -256,6 +291,31 @@ def spmv_algorithm_heuristic(queue, hA, footprint_hard_limit=0.8, footprint_soft
     if ell_device_ratio < footprint_soft_limit:
         return "ELLPACK"
     return "CSR" if csr_bytes / ell_bytes < soft_limit_ratio else "ELLPACK"
+
+
+def read_spike_bits(plan, mask, one):
+    """Make a launch of the product of spikes read their bits from `mask`, where the launch that
+    updates the neurons leaves them (`hipra_gemv.leave_spike_bits`); `one`: the value of a spike."""
+    sp, queue = plan.spmv, plan.queue
+    table, row_len, cols, vals = sp["host"]
+    lanes = bits_lanes(sp["n"], (1024 // WAVE) * queue.n_compute_units)
+    starts, widths, cols, vals, index_bits = bits_layout(sp["slice_rows"], row_len, cols, vals,
+                                                         sp["n_cols"], lanes)
+    if vals.size >= 2 ** 31:
+        return
+    table = table.copy()
+    table[:sp["n"], 0], table[:sp["n"], 1] = starts, widths
+    dev = tuple(to_device(queue, a if a.size else np.zeros(4, a.dtype)) for a in (table, cols, vals))
+    filters = (None, None, None)
+    if plan.name == "hip_spmv_filter":
+        filters = tuple(plan.args[7:10])  # (slices, n, row_len, cols, vals, X, Y, slice_epi, targets, F, ...)
+    plan.kern = queue.lib.nhip_spmv_sell_bits
+    plan.args = ((dev[0].ptr, sp["n"], dev[1].ptr, dev[2].ptr, plan.args[6]) + filters
+                 + (sp["n_cols"], mask.ptr, float(one), lanes, index_bits))
+    plan.full_args = tuple(a for a in plan.full_args if a not in sp["dev"]) + dev + (mask,)
+    plan.gsize = (1024 * min(queue.n_compute_units, lanes * sp["n"])
+                  + (plan.gsize[0] - 1024 * min(queue.n_compute_units, 4 * sp["n"])),)
+    plan.stored_bytes = 4 * int(cols.size + vals.size)
 
 
 def fuse_linearfilter(spmv_plan, lf_plan):

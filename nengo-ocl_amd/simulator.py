@@ -83,6 +83,7 @@ class HipBackend:
 
         from . import hipra_spmv
 
+        self._spmv = hipra_spmv
         self.plan_sparse_dot_inc = hipra_spmv.plan_sparse_dot_inc
         # switch for measurements: "0" multiplies every stored element of a sparse matrix
         self.skips_zero_operands = os.environ.get("NENGO_HIP_SPMV_SKIP", "1") != "0"
@@ -105,6 +106,16 @@ class HipBackend:
         if self.input_sums_in_launch and hasattr(sum_plan, "prog") and hasattr(lif_plan, "prog"):
             return self._gemv.fuse_input_sums(sum_plan, lif_plan)
         return None
+
+    def share_spike_bits(self, lif_plan, product_plan):
+        """Let the product of a population's spikes read them as bits from the launch that updates
+        its neurons, if that launch can leave them."""
+        sp = product_plan.spmv
+        bits = lif_plan.__dict__.setdefault("spike_bits", {})
+        if sp["x_start"] not in bits:
+            bits[sp["x_start"]] = self._gemv.leave_spike_bits(lif_plan, sp["x_start"], sp["n_cols"])
+        if bits[sp["x_start"]] is not None:
+            self._spmv.read_spike_bits(product_plan, *bits[sp["x_start"]])
 
     def store_spikes_as_bits(self, enc_plan, items, event_records, dt):
         return self._gemv.store_spikes_as_bits(enc_plan, items, event_records, dt)
@@ -515,6 +526,8 @@ class Simulator:
             if fuse and hasattr(self.backend, "carry_sequences"):
                 plans = self.backend.carry_sequences(plans)
         self._store_spikes_as_bits(plans)
+        if fuse and hasattr(self.backend, "share_spike_bits"):
+            self._share_spike_bits(plans)
         logger.info("Plans in %0.3f s", _time.time() - t0)
 
         self._plans = Plans(plans, self.profiling, use_graph=use_graph, branches=branches,
@@ -759,6 +772,31 @@ class Simulator:
                 start = int(pops[b, 2])
                 base = base_at[start]
                 self._spike_bits[base] = (start, int(base.size), np.float32(value))
+
+    def _share_spike_bits(self, plans):
+        """Sparse products of a population's spikes take them as bits from the launch that updates
+        the neurons, where that launch is ahead of them in the step and nothing else writes the
+        spikes (what the host writes there between two steps is overwritten before the product)."""
+        ra = self.all_data
+        for k, product in enumerate(plans):
+            sp = getattr(product, "spmv", None)
+            if sp is None or not product.skips_zero_x:
+                continue
+            spikes = [b for b in self.all_bases
+                      if int(ra.starts[self.sidx[b]]) == sp["x_start"] and int(b.size) == sp["n_cols"]]
+            if len(spikes) != 1:
+                continue
+            # (the launches of a group of neurons all carry the writes of the group; each population
+            # is in one of them)
+            writers = [q for q in plans if spikes[0] in getattr(q, "writes_mem", spikes)]
+            if all(getattr(q, "host_pops", None) is not None and q.name.endswith("_lif") and q in plans[:k]
+                   for q in writers):
+                for q in writers:
+                    if q.name == "hipra_gemv.wave_ref_lif":
+                        self.backend.share_spike_bits(q, product)
+        for plan in plans:
+            if getattr(plan, "spmv", None) is not None:
+                plan.spmv["host"] = None  # (the host arrays have served)
 
     def _spikes_from_bits(self, base):
         """The spike vector of a population whose spikes device memory holds as bits, as an

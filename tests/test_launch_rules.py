@@ -40,3 +40,39 @@ def test_launch_size_of_a_convolution_is_that_of_its_kernel(channels_last, conv,
 def test_convolutions_take_single_wave_groups_where_these_are_resident(shape_in, filters, kernel,
                                                                        strides, expected):
     assert conv_threads(shape_in, filters, kernel, strides) == expected
+
+
+@pytest.mark.parametrize("n_cols", [1, 65535, 65536, 100003, 1179520])
+@pytest.mark.parametrize("lanes", [1, 2, 4])
+def test_layout_of_products_that_are_handed_bits(n_cols, lanes):
+    """Every stored element is found again in the packed indices, everything else is the column past
+    the end with the value -0; rows without elements and a short last slice included."""
+    import scipy.sparse
+
+    from nengo_ocl_amd import hipra_spmv as h
+
+    rng = np.random.RandomState(n_cols)
+    dense_rows = [np.unique(rng.randint(n_cols, size=k)) for k in rng.randint(0, 40, size=130)]
+    dense_rows[0], dense_rows[129] = np.arange(0), np.array([n_cols - 1])
+    mats = []
+    for rows in (dense_rows, dense_rows[::-1][:70]):
+        r = np.repeat(np.arange(len(rows)), [len(c) for c in rows])
+        mats.append(h.HostSparseMatrix(scipy.sparse.csr_matrix(
+            (1.0 + np.arange(len(r)), (r, np.concatenate(rows).astype(int))), shape=(len(rows), n_cols))))
+    slice_rows, row_len, cols, vals = h.sell_layout(mats)
+    starts, widths, packed, values, bits = h.bits_layout(slice_rows, row_len, cols, vals, n_cols, lanes)
+    assert bits == (16 if n_cols < 65536 else 24) and not np.any(widths % (4 * lanes))
+    if bits == 16:
+        index = packed.view(np.uint16).astype(int)
+    else:
+        raw = np.ascontiguousarray(packed).view(np.uint8).reshape(-1, 3).astype(int)
+        index = raw[:, 0] + 256 * raw[:, 1] + 65536 * raw[:, 2]
+    assert len(index) == len(values) == int(np.sum(widths)) * 64
+    used = np.zeros(len(values), dtype=bool)
+    for (item, start, _, len_start, n_rows, row0), at in zip(slice_rows, starts):
+        for r in range(n_rows):
+            k = np.arange(row_len[len_start + r])
+            new, old = h.sell_index(at, r, k), h.sell_index(start, r, k)
+            used[new] = True
+            assert np.array_equal(index[new], cols[old]) and np.array_equal(values[new], vals[old])
+    assert np.all(index[~used] == n_cols) and np.all(np.signbit(values[~used])) and not np.any(values[~used])

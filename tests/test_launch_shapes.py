@@ -527,3 +527,48 @@ def test_filters_of_second_order_in_the_launch_of_their_input(queue, kind, neuro
                 assert np.any(gpu.data[p] != 0) and np.array_equal(gpu.data[p], cpu.data[p_o])
             assert np.array_equal(gpu.signal_buffer().view(np.uint32), cpu.signal_buffer().view(np.uint32))
             gpu.reset()
+
+
+# waves of sixteen rows and of 64, populations that end inside a wave and inside a word; columns on both
+# sides of 65,536, whole slices (120,000 and 140,000 rows), more columns than 17 bits hold
+@pytest.mark.parametrize("n,fan_out,lead,bits", [
+    (65, 30, 0, True), (2001, 40, 0, True), (1000, 30, 48, True), (1000, 30, 50, False), (33000, 60, 0, True),
+    (70001, 30, 0, True), (120000, 15, 0, True), (140000, 14, 0, True)])
+def test_sparse_products_read_the_bits_their_neurons_left(queue, n, fan_out, lead, bits):
+    """A population's spikes reach the sparse products that read them as bits from the launch that
+    updates the neurons (not where another population's rows (`lead`) leave them inside a wave), and
+    the spikes the host sees stay floats that it may write."""
+    from nengo_ocl_amd import configs
+    from nengo_ocl_amd import minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    def make():
+        rng = np.random.RandomState(4)
+        net = mb.Network(seed=2)
+        first = net.Ensemble(lead, 1, neuron_type=mb.LIF(tau_ref=0.001)) if lead else None
+        ens = net.Ensemble(n, 1, neuron_type=mb.LIF(tau_ref=0.001, amplitude=0.7))
+        if lead:  # both in one launch
+            stim = net.Node(mb.WhiteSignal(period=0.5, high=6.0, seed=3), size_out=1)
+            for e in (first, ens):
+                net.Connection(stim, e, synapse=mb.Lowpass(0.005))
+        for _ in range(2):  # two products of the same spikes
+            weights = configs.sparse_ring_weights(n, fan_out, 0.3, rng, scale=2e-4)
+            net.Connection(ens.neurons, ens.neurons, transform=mb.Sparse((n, n), weights),
+                           synapse=mb.Lowpass(0.05))
+        return net, [net.Probe(e.neurons, synapse=0.01) for e in (first, ens) if e is not None]
+
+    (net, probes), (net_o, probes_o) = make(), make()
+    with Simulator(net, seed=1, event_calibration_steps=0) as gpu, OracleSimulator(net_o, seed=1) as cpu:
+        names = [getattr(p.kern, "__name__", "") for p in gpu._plans]
+        assert ("nhip_spmv_sell_bits" in names) == bits, names
+        for _ in range(2):
+            gpu.run_steps(15)
+            cpu.run_steps(15)
+            for p, p_o in zip(probes, probes_o):
+                assert np.any(gpu.data[p] != 0) and np.array_equal(gpu.data[p], cpu.data[p_o])
+            assert np.array_equal(gpu.signal_buffer().view(np.uint32), cpu.signal_buffer().view(np.uint32))
+            for sim in (gpu, cpu):  # what the host puts there is replaced before the product reads it
+                spikes = next(op.output for op in sim.operators if type(op).__name__ == "SimNeurons"
+                              and op.output.size == n)
+                sim.signals[spikes] = np.ones(spikes.shape)
