@@ -1493,6 +1493,126 @@ def fuse_learning(enc_plan, dec_plan, ew_plan, lf_plan):
     return new_enc, new_dec, residual, pending
 
 
+def fuse_hebbian(products, rule_plan, lf_plan=None):
+    """A step that multiplies by matrices which Oja's or the BCM rule then changes in place, from
+    activities that filters then replace -- `products` (plans of one GEMV, with or without the filter
+    epilogue), `rule_plan`, `lf_plan` -- as one launch (``nhip_gemv_learn``): a matrix is read
+    once per step, and the filters need no launch.
+
+    Fused when every item of `products` has one dot product with operands of stride 1, every matrix of the
+    rule is the matrix of one such item (same start, shape and row stride) and its row operand is contiguous.
+    Filters of `lf_plan` with one numerator and at most one denominator coefficient on
+    contiguous vectors move; the caller has checked that nothing between the plans, and nothing the plans
+    read or write themselves, keeps the rule and those filters out of the products' launch.  Returns ``(plan,
+    plans for the filters that stay, filters that moved)`` or None."""
+    from .hipra_nonlinearities import RULE_BCM, RULE_OJA, plan_linearfilter
+
+    spec = rule_plan.rule_spec
+    prog = products[0].prog
+    queue, geometry = prog.queue, prog.geometry
+    pre, post, aux, delta = (spec[k] for k in ("pre", "post", "aux", "delta"))
+    buf = prog.A.ptr.value
+    if spec["rule"] not in (RULE_BCM, RULE_OJA) or not spec["inc"] or any(
+            ra.ptr.value != buf for ra in (prog.X, prog.Y, prog.Y_in, pre, post, aux, delta)):
+        return None
+    members = [b for plan in products for b in plan.members]
+    by_matrix = {}
+    for b in members:
+        dots = geometry[b]["dots"]
+        if len(dots) != 1 or dots[0]["x_stride0"] != 1 or dots[0]["a_shape1"] < 1 or b in by_matrix.values():
+            return None
+        d = dots[0]
+        key = (d["a_start"], geometry[b]["y_len"], d["a_shape1"], d["a_stride0"])
+        if key in by_matrix:
+            return None  # two products with one matrix
+        by_matrix[key] = b
+    rules = np.zeros((len(delta), 8), dtype=np.int32)
+    rule_of = {}
+    for i in range(len(delta)):
+        rows, cols = int(delta.shape0s[i]), int(delta.shape1s[i])
+        key = (int(delta.starts[i]), rows, cols, int(delta.stride0s[i]))
+        b = by_matrix.get(key)
+        contiguous = int(pre.stride0s[i]) == 1 or cols == 1
+        if b is None or b in rule_of or not contiguous or int(delta.stride1s[i]) != 1:
+            return None
+        if spec["rule"] == RULE_OJA and (int(aux.starts[i]), int(aux.stride0s[i])) != (key[0], key[3]):
+            return None
+        rule_of[b] = i
+        theta = spec["rule"] == RULE_BCM
+        rules[i] = (spec["rule"], pre.starts[i], post.starts[i], post.stride0s[i],
+                    aux.starts[i] if theta else 0, aux.stride0s[i] if theta else 0,
+                    np.float32(spec["alpha"][i]).view(np.int32), np.float32(spec["beta"][i]).view(np.int32))
+    item_targets, dev_targets, F = None, None, prog.Y
+    for plan in products:
+        if getattr(plan, "filter_tables", None) is not None:
+            if item_targets is not None and plan.filter_tables[0] is not item_targets:
+                return None
+            item_targets, dev_targets, F = plan.filter_tables
+        elif plan.name.endswith("_filter"):
+            return None
+    if F.ptr.value != buf:
+        return None
+
+    per_group = WG // WAVE
+    tasks = []
+    bits = lambda v: int(np.float32(v).view(np.int32))
+    for b in members:
+        g = geometry[b]
+        d = g["dots"][0]
+        first, n = (0, 0) if item_targets is None else (int(v) for v in item_targets[b])
+        for row0 in range(0, g["y_len"], per_group):
+            tasks.append((d["a_start"], d["a_stride0"], d["a_shape1"], d["x_start"], g["y_start"], g["y_stride0"],
+                          g["y_in_start"], g["y_in_stride0"], bits(prog.alpha[b]), bits(prog.beta[b]),
+                          bits(prog.gamma[b]), row0, min(per_group, g["y_len"] - row0), rule_of.get(b, -1),
+                          first, n))
+    if not tasks:
+        return None
+    filters, moved, rest = [], [], []
+    if lf_plan is not None:
+        S, T, A, B = (lf_plan.lf_spec[k] for k in ("X", "Y", "A", "B"))
+        if S.ptr.value == buf and T.ptr.value == buf:
+            a_host, b_host = A.to_host(), B.to_host()
+            for k in range(len(S)):
+                vector = all(int(r.shape1s[k]) == 1 and int(r.stride0s[k]) == 1 for r in (S, T))
+                if int(B.shape0s[k]) != 1 or int(A.shape0s[k]) > 1 or not vector:
+                    continue
+                na = int(A.shape0s[k])
+                filters.append((S.starts[k], T.starts[k], S.shape0s[k], na,
+                                bits(a_host[k][0, 0]) if na else 0, bits(b_host[k][0, 0]), 0, 0))
+                moved.append(k)
+        rest = [k for k in range(len(S)) if k not in set(moved)]
+    dev_tasks, dev_rules = to_device(queue, np.array(tasks, dtype=np.int32)), to_device(queue, rules)
+    dev_filters = to_device(queue, np.array(filters or [(0,) * 8], dtype=np.int32))
+    arrived = to_device(queue, np.zeros(4, dtype=np.int32))
+    lib = queue.lib
+    targets = dev_targets if dev_targets is not None else dev_rules  # (not read without targets)
+    total = lambda attr: sum(getattr(p, attr) or 0 for p in list(products) + [rule_plan])
+    weights = 4 * int(delta.sizes.sum())
+    plan = Plan(queue, lib.nhip_gemv_learn,
+                (dev_tasks.ptr, len(tasks), dev_rules.ptr, prog.A.ptr, prog.X.ptr, prog.Y_in.ptr, prog.Y.ptr,
+                 targets.ptr, F.ptr, dev_filters.ptr, len(filters), arrived.ptr),
+                gsize=(WG * len(tasks),), lsize=(WG,),
+                full_args=sum((tuple(p.full_args) for p in list(products) + [rule_plan]), ())
+                + (dev_tasks, dev_rules, dev_filters, arrived),
+                name="hipra_gemv.learn", tag=" + ".join([products[0].tag, rule_plan.name]),
+                # the rule's own accounting, less the matrices it need not read again
+                bw_per_call=total("bw_per_call") - (2 if spec["rule"] == RULE_OJA else 1) * weights
+                + sum(12 * int(f[2]) for f in filters),
+                flops_per_call=total("flops_per_call"))
+    plan.description = "; ".join(p.description for p in products)
+    plan.kernel_class, plan.n_tasks = (6, WAVE, 4), len(tasks)
+    plan.members, plan.prog = members, prog
+    plan.gemv_bytes = sum(getattr(p, "gemv_bytes", p.bw_per_call) for p in products)
+    plan.host_tasks = None
+    plan.learned_matrices = len(rule_of)
+    residual = []
+    if lf_plan is not None and rest:
+        residual = plan_linearfilter(queue, S[rest], T[rest], A[rest], B[rest], lf_plan.lf_spec["Xbuf"][rest],
+                                     lf_plan.lf_spec["Ybuf"][rest], tag=lf_plan.tag)
+        residual[0].unfused_items = list(rest)
+    return plan, residual, moved
+
+
 def _read_spans(prog, ptr_value):
     """Element intervals a GEMV reads through A, X and a Y_in that is not its Y, in
     the device buffer at `ptr_value`."""
@@ -1679,6 +1799,7 @@ def fuse_linearfilter(gemv_plans, lf_plan, second_order=False):
         fused.gemv_bytes = plan.bw_per_call
         if plan.kernel_class[0] == 3:
             fused.host_tasks = tasks
+        fused.filter_tables = (item_targets, dev_targets, F)
         _keep_filter_state(fused, filter_state)
         out.append(fused)
     residual = []

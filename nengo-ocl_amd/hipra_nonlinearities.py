@@ -1013,6 +1013,9 @@ def _plan_rule(queue, rule, name, pre, post, aux, delta, alpha, beta=None, learn
     plan.flops_per_call = flops_per_element * int(delta.sizes.sum())
     plan.bw_per_call = (sum(ra.nbytes for _, ra in operands) + alpha.nbytes
                         + (beta.nbytes if rule == RULE_OJA else 0) + (delta.nbytes if inc else 0))
+    # what a product with the matrices that the rule changes needs to run it (`fuse_hebbian`)
+    plan.rule_spec = dict(rule=rule, pre=pre, post=post, aux=aux, delta=delta, alpha=alpha, beta=beta,
+                          inc=bool(inc))
     plan.description = _description(delta)
     return plan
 

@@ -215,9 +215,11 @@ def _can_carry(plan, needs=0):
     """GEMV launches with an epilogue: the large-item kernel with compile-time shapes, the
     launch that visits only the columns with x != 0 (which runs on half the registers of the
     others and holds no unary functions and no higher-order filters: `needs`), the small-item
-    kernel, and the sparse products."""
+    kernel, the sparse products and the products with matrices that a rule changes."""
     cls = getattr(plan, "kernel_class", None)
     name = getattr(plan, "name", "")
+    if name == "hipra_gemv.learn":
+        return getattr(plan, "prelude", None) is None
     if name in ("hip_spmv", "hip_spmv_filter"):  # the sparse products (one or more slices)
         return getattr(plan, "prelude", None) is None and getattr(plan, "spmv", {}).get("n", 0) > 0
     if cls is None or getattr(plan, "prelude", None) is not None or getattr(plan, "n_tasks", 0) <= 0:

@@ -99,6 +99,7 @@ class HipBackend:
             self.fuse_outer_filter = hipra_nonlinearities.fuse_outer_filter
         if os.environ.get("NENGO_HIP_FOLD_LEARNING", "1") != "0":  # switch for measurements
             self.fuse_learning = hipra_gemv.fuse_learning
+            self.fuse_hebbian = hipra_gemv.fuse_hebbian
 
     def fuse_input_sums(self, sum_plan, lif_plan):
         """The plan replacing ``[sum_plan, lif_plan]`` when the first only forms vector
@@ -519,6 +520,8 @@ class Simulator:
             plans = self._fuse_input_sums(plans)
         if fuse and hasattr(self.backend, "fuse_learning"):
             plans = self._fuse_learning(plans)
+        if fuse and hasattr(self.backend, "fuse_hebbian"):
+            plans = self._fuse_hebbian(plans)
         if fuse and hasattr(self.backend, "fuse_outer_filter"):
             plans = self._fuse_outer_filters(plans)
         if merge_small and hasattr(self.backend, "merge_small_plans"):
@@ -897,6 +900,66 @@ class Simulator:
         del plans[r]
         plans[j] = new_dec
         plans[i] = new_enc
+        return plans
+
+    def _fuse_hebbian(self, plans):
+        """Oja's or the BCM rule on matrices that the step multiplies by, and the filters of the
+        activities it reads, as part of the launch of those products (`hipra_gemv.fuse_hebbian`), where
+        no plan between them touches what moves and the products read and write nothing that the rule
+        or the filters need otherwise."""
+        conflict = self.backend.plans_conflict
+        names = tuple("hipra_gemv." + k + e for k in ("tile", "wave_ref") for e in ("", "_filter"))
+        is_product = lambda p: (getattr(p, "name", "") in names and hasattr(p, "prog")
+                                and getattr(p, "kernel_class", (None,))[0] in (2, 3)
+                                and getattr(p, "learned_matrices", 0) == 0)
+        group = lambda r, w: type("Moved", (), {"reads_mem": r, "writes_mem": w})
+        plans = list(plans)
+        r = 0
+        while r < len(plans):
+            rule = plans[r]
+            r += 1
+            if not (getattr(rule, "rule_spec", None) or {}).get("inc"):
+                continue
+            # the products with its matrices: the nearest plans before it that read what it writes
+            j = next((k for k in range(r - 2, -1, -1) if conflict(rule, plans[k])), None)
+            if j is None or not is_product(plans[j]):
+                continue
+            i = j
+            while i > 0 and is_product(plans[i - 1]) and plans[i - 1].prog is plans[j].prog:
+                i -= 1
+            products = plans[i:j + 1]
+            reads = set().union(*(p.reads_mem for p in products))
+            writes = set().union(*(p.writes_mem for p in products))
+            if writes & (rule.reads_mem | rule.writes_mem):
+                continue
+            # the filters behind it that replace what it reads
+            operands = rule.reads_mem - rule.writes_mem
+            f = next((k for k in range(r, len(plans)) if getattr(plans[k], "writes_mem", operands) & operands), None)
+            lf = plans[f] if f is not None else None
+            ops = getattr(lf, "planned_ops", None)
+            movable = (getattr(lf, "lf_spec", None) is not None and ops is not None
+                       and len(ops) == len(lf.lf_spec["X"])
+                       and not any(conflict(lf, q) for q in plans[j + 1:r - 1] + plans[r:f])
+                       and not (writes & (lf.reads_mem | lf.writes_mem)) and not (reads & lf.writes_mem)
+                       and not (rule.writes_mem & (lf.reads_mem | lf.writes_mem)))
+            result = self.backend.fuse_hebbian(products, rule, lf if movable else None)
+            if result is None:
+                continue
+            plan, residual, moved = result
+            plan.reads_mem, plan.writes_mem = reads | rule.reads_mem, writes | rule.writes_mem
+            if moved:
+                kept = [op for k, op in enumerate(ops) if k not in set(moved)]
+                plan.reads_mem |= {ops[k].input.base for k in moved}
+                plan.writes_mem |= {ops[k].output.base for k in moved}
+                for p in residual:
+                    p.reads_mem = {op.input.base for op in kept}
+                    p.writes_mem = {op.output.base for op in kept}
+                    p.planned_ops = kept
+                    self._filter_positions.append(p.bufpos)
+                plans[f:f + 1] = residual
+            del plans[r - 1]
+            plans[i:j + 1] = [plan]
+            r = i + 1
         return plans
 
     @staticmethod

@@ -572,3 +572,49 @@ def test_sparse_products_read_the_bits_their_neurons_left(queue, n, fan_out, lea
                 spikes = next(op.output for op in sim.operators if type(op).__name__ == "SimNeurons"
                               and op.output.size == n)
                 sim.signals[spikes] = np.ones(spikes.shape)
+
+
+# rows of one tile, of a partial one, of whole passes of 2048 columns and a bit more, on 16-byte boundaries
+# and not; groups that end inside their four rows; an infinite and a NaN weight
+@pytest.mark.parametrize("n_pre,n_post", [(4, 3), (50, 60), (301, 90), (128, 1000), (1000, 129), (2048, 66),
+                                          (2049, 70), (2500, 101), (4100, 33)])
+@pytest.mark.parametrize("rule", ["Oja", "BCM"])
+@pytest.mark.parametrize("odd", [False, True])
+def test_rules_between_neurons_in_the_launch_of_their_product(queue, rule, n_pre, n_post, odd):
+    """A matrix that Oja's or the BCM rule changes is read once per step: by the launch that multiplies
+    by it, which also steps the filters of its product and of the activities the rule reads."""
+    from nengo_ocl_amd import minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    def make():
+        rng = np.random.RandomState(8)
+        net = mb.Network(seed=5, solver="surrogate")
+        stim = net.Node(mb.WhiteSignal(period=0.5, high=6.0, seed=3), size_out=2)
+        pre, post = net.Ensemble(n_pre, 2), net.Ensemble(n_post, 2)
+        net.Connection(stim, pre, synapse=mb.Lowpass(0.005))
+        learning = mb.Oja(learning_rate=1e-4, beta=0.7) if rule == "Oja" else mb.BCM(learning_rate=1e-7)
+        synapses = [mb.Lowpass(0.005), mb.Alpha(0.01)] if odd else [mb.Lowpass(0.005)]
+        for synapse in synapses:  # two learned matrices with the same activities
+            weights = rng.normal(scale=1e-1 / n_pre, size=(n_post, n_pre))
+            if odd:
+                weights[n_post // 2, n_pre // 3], weights[1, 0] = np.inf, np.nan
+            net.Connection(pre.neurons, post.neurons, transform=weights, learning_rule=learning, synapse=synapse)
+            learning = mb.Oja(learning_rate=1e-4) if rule == "Oja" else mb.BCM(learning_rate=1e-7)
+        return net, [net.Probe(post, synapse=0.01)]
+
+    (net, probes), (net_o, probes_o) = make(), make()
+    with Simulator(net, seed=1) as gpu, OracleSimulator(net_o, seed=1) as cpu:
+        names = [p.name for p in gpu._plans]
+        assert "hipra_gemv.learn" in names and not {"hip_oja", "hip_bcm"} & set(names), names
+        if not odd:
+            assert "hip_linearfilter" not in names and "hip_sequence" not in names, names
+        for _ in range(2):
+            gpu.run_steps(20)
+            cpu.run_steps(20)
+            got, want = gpu.signal_buffer(), cpu.signal_buffer()
+            nan = np.isnan(want)
+            assert np.array_equal(np.isnan(got), nan) and nan.any() == odd
+            assert np.array_equal(got[~nan].view(np.uint32), want[~nan].view(np.uint32))
+            for p, p_o in zip(probes, probes_o):
+                assert np.array_equal(gpu.data[p], cpu.data[p_o], equal_nan=True)
