@@ -1594,7 +1594,7 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
                 gsize=(WG * len(tasks),), lsize=(WG,),
                 full_args=sum((tuple(p.full_args) for p in list(products) + [rule_plan]), ())
                 + (dev_tasks, dev_rules, dev_filters, arrived),
-                name="hipra_gemv.learn", tag=" + ".join([products[0].tag, rule_plan.name]),
+                name=products[0].name, tag=" + ".join([products[0].tag, rule_plan.name]),
                 # the rule's own accounting, less the matrices it need not read again
                 bw_per_call=total("bw_per_call") - (2 if spec["rule"] == RULE_OJA else 1) * weights
                 + sum(12 * int(f[2]) for f in filters),

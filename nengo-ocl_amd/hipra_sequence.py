@@ -218,7 +218,7 @@ def _can_carry(plan, needs=0):
     kernel, the sparse products and the products with matrices that a rule changes."""
     cls = getattr(plan, "kernel_class", None)
     name = getattr(plan, "name", "")
-    if name == "hipra_gemv.learn":
+    if cls is not None and cls[0] == 6:  # products with matrices that a rule changes
         return getattr(plan, "prelude", None) is None
     if name in ("hip_spmv", "hip_spmv_filter"):  # the sparse products (one or more slices)
         return getattr(plan, "prelude", None) is None and getattr(plan, "spmv", {}).get("n", 0) > 0

@@ -148,6 +148,22 @@ class Plan(BasePlan):
         return "%s{%s %s %s}" % (type(self).__name__, self._label(), self.gsize, self.lsize)
 
 
+class CarriedPlan(BasePlan):
+    """An operation of the step that the launch of another plan does: listed under its own name, and
+    nothing to launch."""
+
+    def __init__(self, queue, **kwargs):
+        super().__init__(**kwargs)
+        self.queue = queue
+        self.reads_mem, self.writes_mem = set(), set()  # (they are those of the launch)
+
+    def enqueue(self, wait_for=None, profiling=False):
+        return self
+
+    def __call__(self, profiling=False):
+        return None
+
+
 def plan_dependencies(plans):
     """For every plan, the earlier plans it has to wait for (indices into `plans`),
     transitively reduced.

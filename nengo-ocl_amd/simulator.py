@@ -34,7 +34,7 @@ import numpy as np
 
 from . import operators as ops_mod
 from .operators import MultiDotInc
-from .plan import BasePlan, Plans, PythonPlan
+from .plan import BasePlan, CarriedPlan, Plans, PythonPlan
 from .planners import batching_planner, greedy_planner  # noqa: F401
 from .raggedarray import RaggedArray
 from .utils import get_closures, groupby, indent, split, stable_unique
@@ -957,7 +957,8 @@ class Simulator:
                     p.planned_ops = kept
                     self._filter_positions.append(p.bufpos)
                 plans[f:f + 1] = residual
-            del plans[r - 1]
+            carried = CarriedPlan(rule.queue, name=rule.name, tag="in %s" % plan.tag)
+            plans[r - 1] = carried
             plans[i:j + 1] = [plan]
             r = i + 1
         return plans

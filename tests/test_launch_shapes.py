@@ -605,10 +605,10 @@ def test_rules_between_neurons_in_the_launch_of_their_product(queue, rule, n_pre
 
     (net, probes), (net_o, probes_o) = make(), make()
     with Simulator(net, seed=1) as gpu, OracleSimulator(net_o, seed=1) as cpu:
-        names = [p.name for p in gpu._plans]
-        assert "hipra_gemv.learn" in names and not {"hip_oja", "hip_bcm"} & set(names), names
+        launches = [getattr(p, "kern").__name__ for p in gpu._plans if hasattr(p, "kern")]
+        assert "nhip_gemv_learn" in launches and "nhip_learning_rule" not in launches, launches
         if not odd:
-            assert "hip_linearfilter" not in names and "hip_sequence" not in names, names
+            assert not {"nhip_linearfilter", "nhip_sequence_chains"} & set(launches), launches
         for _ in range(2):
             gpu.run_steps(20)
             cpu.run_steps(20)
