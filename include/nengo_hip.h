@@ -331,6 +331,20 @@ int nhip_gemv_rows_filter(void *stream, int lpr, int task_words, const int *item
                           const float *X, const float *Yin, float *Y, const int *item_targets,
                           const int *targets, float *F, int order);
 
+/* `n_steps` timesteps of a small network by one work-group, on a copy of its arrays in LDS (at most
+ * 39,936 words): replaces the launch loop of the reference executor (plan.py:137-149) for networks
+ * whose launches cost more than what they do.
+ *   spans : records {uint64 device address, int32 words, int32 word offset in the LDS image, int32
+ *           write_back, 0}: arrays copied in before the first step and, with write_back, out after the
+ *           last; addresses and offsets on 16-byte boundaries
+ *   ops   : records of 112 bytes (csrc/resident.hip: ResOp): the work lists of the entry points above, or
+ *           forms of them for this launch, with word offsets into the image for pointers
+ *   first_op : n_waves + 1 (9) indices: wave w runs ops[first_op[w] .. first_op[w + 1]) in order, every step; a
+ *           record with `last` set ends with a barrier of all waves, and every wave's program has as many --
+ *           operations without a barrier between them touch different memory or belong to one wave */
+int nhip_resident(void *stream, const void *spans, int n_spans, const void *ops, const int *first_op,
+                  int n_waves, int n_steps);
+
 /* Products with matrices that a learning rule (NHIP_RULE_BCM, NHIP_RULE_OJA) changes in the same
  * step, the change, the filters of the products' outputs, and the filters of the activities that the
  * rules read, in one launch: replaces `plan_block_gemv` + `plan_linearfilter` + `plan_bcm` / `plan_oja`

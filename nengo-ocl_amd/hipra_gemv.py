@@ -765,6 +765,7 @@ class gemv_prog:
             plan.prog = self
             plan.host_tasks = task_tab if flavor == 3 or task_tab.shape[1] == 16 else None
             plan.host_tables = (item_tab, coef_tab, task_tab)  # (for plans that extend the launch)
+            self.host_dots = dot_tab
             plans.append(plan)
         return plans
 
@@ -1273,6 +1274,10 @@ def fuse_input_sums(sum_plan, lif_plan):
     fused.input_sums = len(sums)
     fused.lazy_currents = getattr(lif_plan, "lazy_currents", None)
     fused.host_pops = new_pops if large else pops
+    if not large:
+        fused.host_tables, fused.host_ranges = (items, coefs, tasks), ranges
+        fused.host_parts = np.array(part_rows, dtype=np.int32)
+        fused.spare_items = list(range(n_items, len(items)))
     # (the device copy of the table, where it is the one the launch reads: large items)
     fused.dev_pops = (dev_pops if spare else getattr(lif_plan, "dev_pops", None)) if large else None
     return fused
@@ -1547,7 +1552,7 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
         if getattr(plan, "filter_tables", None) is not None:
             if item_targets is not None and plan.filter_tables[0] is not item_targets:
                 return None
-            item_targets, dev_targets, F = plan.filter_tables
+            item_targets, dev_targets, F, _ = plan.filter_tables
         elif plan.name.endswith("_filter"):
             return None
     if F.ptr.value != buf:
@@ -1799,7 +1804,8 @@ def fuse_linearfilter(gemv_plans, lf_plan, second_order=False):
         fused.gemv_bytes = plan.bw_per_call
         if plan.kernel_class[0] == 3:
             fused.host_tasks = tasks
-        fused.filter_tables = (item_targets, dev_targets, F)
+        fused.filter_tables = (item_targets, dev_targets, F, targets)
+        fused.host_tables = plan.host_tables
         _keep_filter_state(fused, filter_state)
         out.append(fused)
     residual = []

@@ -302,7 +302,7 @@ class _GraphSegment:
 class Plans:
     """The ordered plan list of one timestep and its executor."""
 
-    def __init__(self, planlist, profiling, use_graph=True, branches=False, before_last=()):
+    def __init__(self, planlist, profiling, use_graph=True, branches=False, before_last=(), resident=None):
         if branches and use_graph:
             # Switched off: ending a multi-stream recording crashed inside the HIP runtime
             # (segmentation fault in the call that ends the capture) for a step whose
@@ -318,6 +318,9 @@ class Plans:
         self.before_last = list(before_last)
         self.profiling = profiling
         self.use_graph = use_graph
+        # callable that runs n steps of the whole list in one launch (small networks,
+        # `hipra_resident.resident_program`), used where the graph would be
+        self.resident = resident if use_graph and not self.before_last else None
         self._segments = None  # list of _GraphSegment | PythonPlan
 
     def __call__(self):
@@ -358,7 +361,7 @@ class Plans:
     def steps_of_every_graph(self):
         """A step count whose run launches every recorded graph at least once (0 without
         graphs)."""
-        if not self.use_graph:
+        if not self.use_graph or self.resident is not None:
             return 0
         if self._segments is None:
             self._build_segments()
@@ -369,7 +372,7 @@ class Plans:
         """Record all graphs of the executor now (the Simulator calls this once its plan
         list is complete), so that the first `run_steps` -- of any length -- only
         launches.  Does nothing for eager execution."""
-        if self.profiling or not self.use_graph:
+        if self.profiling or not self.use_graph or self.resident is not None:
             return
         if self._segments is None:
             self._build_segments()
@@ -406,6 +409,9 @@ class Plans:
                         plan(profiling=self.profiling)
             return
 
+        if self.resident is not None:
+            self.resident(n)
+            return
         if self._segments is None:
             self._build_segments()
         if len(self._segments) == 1 and isinstance(self._segments[0], _GraphSegment):

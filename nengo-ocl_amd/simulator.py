@@ -84,6 +84,11 @@ class HipBackend:
         from . import hipra_spmv
 
         self._spmv = hipra_spmv
+        from . import hipra_resident
+
+        self._resident = hipra_resident
+        # switch for measurements: "0" replays small networks as graphs too
+        self.runs_resident = os.environ.get("NENGO_HIP_RESIDENT", "1") != "0"
         self.plan_sparse_dot_inc = hipra_spmv.plan_sparse_dot_inc
         # switch for measurements: "0" multiplies every stored element of a sparse matrix
         self.skips_zero_operands = os.environ.get("NENGO_HIP_SPMV_SKIP", "1") != "0"
@@ -110,6 +115,13 @@ class HipBackend:
 
     def share_spike_bits(self, lif_plan, product_plan):
         """Let the product of a population's spikes read them as bits from the launch that updates
+    def resident_program(self, plans, all_data, n_launches):
+        """`hipra_resident.resident_program` for a list of (plan, memory it reads, memory it writes), or
+        None where it is switched off."""
+        if not self.runs_resident:
+            return None
+        return self._resident.resident_program(self.queue, plans, all_data, n_launches)
+
         its neurons, if that launch can leave them."""
         sp = product_plan.spmv
         bits = lif_plan.__dict__.setdefault("spike_bits", {})
@@ -529,15 +541,22 @@ class Simulator:
             if fuse and hasattr(self.backend, "carry_sequences"):
                 plans = self.backend.carry_sequences(plans)
         self._store_spikes_as_bits(plans)
+        # (launches that carry others declare what those touch as well: by now they do not)
+        apart = [(p, getattr(p, "reads_mem", None), getattr(p, "writes_mem", None)) for p in plans]
         if fuse and hasattr(self.backend, "share_spike_bits"):
             self._share_spike_bits(plans)
         logger.info("Plans in %0.3f s", _time.time() - t0)
 
         self._plans = Plans(plans, self.profiling, use_graph=use_graph, branches=branches,
-                            before_last=self._plan_host_view())
+                            before_last=before_last, resident=resident)
         self.rng = None
         self._drain = None
         if hasattr(self.backend, "probe_drain"):
+        before_last = self._plan_host_view()
+        resident = None
+        if (fuse and merge_small and use_graph and not before_last and hasattr(self.backend, "resident_program")
+                and not self._spike_bits):
+            resident = self.backend.resident_program(apart, self.all_data, len(plans))
             self._drain = self.backend.probe_drain(self._probe_plan, self.all_data,
                                                    self.sidx[self.model.step],
                                                    self.sidx[self.model.time])

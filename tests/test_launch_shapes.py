@@ -618,3 +618,46 @@ def test_rules_between_neurons_in_the_launch_of_their_product(queue, rule, n_pre
             assert np.array_equal(got[~nan].view(np.uint32), want[~nan].view(np.uint32))
             for p, p_o in zip(probes, probes_o):
                 assert np.array_equal(gpu.data[p], cpu.data[p_o], equal_nan=True)
+
+
+@pytest.mark.parametrize("kind,neurons,dims,ensembles", [
+    ("LIF", 100, 1, 2), ("LIF", 30, 1, 2), ("LIF", 65, 3, 5), ("LIFRate", 33, 2, 4), ("AdaptiveLIF", 40, 1, 9),
+    ("RectifiedLinear", 17, 4, 3), ("SpikingRectifiedLinear", 130, 2, 3), ("Sigmoid", 9, 6, 3),
+    ("LIF", 300, 4, 3), ("LIF", 7, 2, 5), ("LIFRate", 260, 1, 2), ("LIF", 129, 12, 2)])
+def test_small_networks_run_resident(queue, monkeypatch, kind, neurons, dims, ensembles):
+    """Networks that fit the LDS of a compute unit take all steps of a call in one launch: first- and
+    second-order synapses, sums of inputs, function and table nodes, probes with a period; calls of
+    one and of several steps, a reset between them."""
+    from nengo_ocl_amd import hipra_resident
+    from nengo_ocl_amd import minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    def make():
+        net = mb.Network(seed=6, solver="surrogate")
+        stim = net.Node(mb.WhiteSignal(period=0.05, high=60.0, seed=3), size_out=dims)
+        wave = net.Node(np.sin)
+        ens = [net.Ensemble(neurons, dims, neuron_type=getattr(mb, kind)(), radius=2.0) for _ in range(ensembles)]
+        net.Connection(stim, ens[0], synapse=mb.Alpha(0.005))
+        net.Connection(wave, ens[1], transform=np.ones((dims, 1)), synapse=mb.Lowpass(0.01))
+        for k in range(ensembles):
+            for u, synapse in enumerate((mb.Lowpass(0.005), mb.Alpha(0.01))):
+                net.Connection(ens[k], ens[(k + u + 1) % ensembles], synapse=synapse, transform=0.6)
+        probes = [net.Probe(ens[1], synapse=mb.Alpha(0.01)), net.Probe(ens[-1], synapse=0.01, sample_every=0.003),
+                  net.Probe(ens[0].neurons), net.Probe(wave)]
+        return net, probes
+
+    monkeypatch.setattr(hipra_resident, "GRAPH_LAUNCH", 1e9)  # also where a graph would be shorter
+    (net, probes), (net_o, probes_o) = make(), make()
+    with Simulator(net, seed=1, n_prealloc_probes=32) as gpu, OracleSimulator(net_o, seed=1) as cpu:
+        assert gpu._plans.resident is not None, [p.name for p in gpu._plans]
+        for repeat in range(2):
+            for n in (1, 2, 37, 1, 64):
+                gpu.run_steps(n)
+                if repeat == 0:
+                    cpu.run_steps(n)
+                    assert np.array_equal(gpu.signal_buffer().view(np.uint32), cpu.signal_buffer().view(np.uint32)), n
+            for p, p_o in zip(probes, probes_o):
+                assert np.any(gpu.data[p] != 0) and np.array_equal(gpu.data[p], cpu.data[p_o])
+            assert np.array_equal(gpu.signal_buffer().view(np.uint32), cpu.signal_buffer().view(np.uint32))
+            gpu.reset()
