@@ -583,6 +583,22 @@ int nhip_learning_rule(void *stream, int rule, int inc, const int *desc, int n_b
  * output is accumulated over channel, kernel row, kernel column in that order with
  * one fused multiply-add per term. */
 int nhip_conv2d(void *stream, const int *geom, const float *X, const float *F, float *Y);
+/* nhip_conv2d followed by the filters that its output feeds (`plan_linearfilter`,
+ * clra_nonlinearities.py:577-803): `targets` as for nhip_gemv_tile_filter with order 2, elements in
+ * the order of Y; FO must not overlap anything the call reads. */
+int nhip_conv2d_filter(void *stream, const int *geom, const float *X, const float *F, float *Y,
+                       const int *targets, int n_targets, float *FO);
+/* nhip_conv2d followed by the currents and the neurons that its output drives: replaces
+ * `plan_block_gemv` of one item with at most one dot product of one column, whose Yin or whose A is Y, and the
+ * planner of the neuron type (nhip_gemv_rows_lif / nhip_gemv_rows_neuron on the same item).
+ *   current : host int32[9] {a_start (-1: no dot product, -2: the output), a_stride0, x_start (in A),
+ *             j_start in J (< 0: not stored), alpha, beta, gamma (float bits), yin_start (in A; -2: the
+ *             output), yin_stride0}
+ *   lif     : 1: `pop` is a row of nhip_gemv_tile_lif's pops, 0: of nhip_gemv_tile_neuron's */
+int nhip_conv2d_neuron(void *stream, const int *geom, const float *X, const float *F, float *Y,
+                       const float *A, const int *current, float *J, int lif, const int *pop, double dt,
+                       int upsample, float *V, float *W, float *S, float *N, const float *TAU,
+                       const float *REF, const float *AMP);
 /* Work-groups that nhip_conv2d launches for `geom`, and the threads of each (256: the tiles above; 64:
  * where the shape suits it better, one wave per 16 filters x 4 pixels). */
 int nhip_conv2d_groups(const int *geom, int *n_groups, int *group_threads);

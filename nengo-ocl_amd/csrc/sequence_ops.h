@@ -290,6 +290,23 @@ __device__ __forceinline__ void timeupdate_block(float* step, float* time, doubl
 }
 
 
+// ---------------------------------------------------------------- moves
+// y[i] = x[i], four elements of a lane requested together (past the end: the last one again): a lane
+// waits for memory once per four.
+__device__ __forceinline__ void seq_move(float* y, const float* x, int n, int lane, int L) {
+    constexpr int U = 4;
+#pragma unroll 1
+    for (int i0 = lane; i0 < n; i0 += U * L) {
+        float v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = x[min(i0 + u * L, n - 1)];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (i0 + u * L < n) y[i0 + u * L] = v[u];
+    }
+}
+
+
 // ---------------------------------------------------------------- table playback
 // clra_nonlinearities.py:1694-1730: row index from the float32 step counter.
 struct PiDesc { int y_start, m, t_start, s_start, nt, pt_bits, has_pt, pad; };
@@ -305,10 +322,7 @@ __device__ __forceinline__ void presentinput_block(const PiDesc d, float dt, flo
     } else {
         ti = it % d.nt;
     }
-    float* y = Y + d.y_start;
-    const float* s = S + d.s_start + (size_t)d.m * ti;
-    NHIP_SEQ_LOOP
-    for (int i = lane; i < d.m; i += L) y[i] = s[i];
+    seq_move(Y + d.y_start, S + d.s_start + (size_t)d.m * ti, d.m, lane, L);
 }
 
 
@@ -354,10 +368,14 @@ __device__ __forceinline__ void probes_block(const ProbeDesc d, float* countdown
         const int n_dims = d.shape0 * d.shape1;
         const float* x = X + d.x_start;
         float* y = Y + d.y_start + (size_t)bufpos * n_dims;
-        NHIP_SEQ_LOOP
-        for (int ij = lane; ij < n_dims; ij += L) {
-            const int i = ij / d.shape1, j = ij - i * d.shape1;
-            y[ij] = x[(size_t)i * d.stride0 + (size_t)j * d.stride1];
+        if ((d.shape1 == 1 && d.stride0 == 1) || (d.stride1 == 1 && (d.shape0 == 1 || d.stride0 == d.shape1))) {
+            seq_move(y, x, n_dims, lane, L);  // element ij is x[ij]
+        } else {
+            NHIP_SEQ_LOOP
+            for (int ij = lane; ij < n_dims; ij += L) {
+                const int i = ij / d.shape1, j = ij - i * d.shape1;
+                y[ij] = x[(size_t)i * d.stride0 + (size_t)j * d.stride1];
+            }
         }
     }
     if (L == NHIP_WG) __syncthreads();

@@ -487,7 +487,11 @@ def plan_probes(queue, periods, X, Y, tag=None):
     plan.dev_countdowns = dev_countdowns
     plan.periods = periods
     plan.Y = Y
-    plan.row_iterations = -(-widest // lanes)
+    # (four elements at a time where a signal lies in one piece, and only every `period` steps)
+    whole = ((X.shape1s == 1) & (X.stride0s == 1)) | ((X.stride1s == 1) & (
+        (X.shape0s == 1) | (X.stride0s == X.shape1s)))
+    per_step = X.shape0s * X.shape1s / (np.where(whole, 4, 1) * lanes * np.maximum(periods, 1)) if N else [1]
+    plan.row_iterations = max(1, int(np.ceil(np.max(per_step))))
     plan.bw_per_call = (2 * X.nbytes + dev_periods.nbytes + dev_countdowns.nbytes
                         + dev_bufpositions.nbytes)
     plan.description = _description(X)
@@ -973,7 +977,7 @@ def plan_presentinput(queue, Y, t, signals, dt, pres_t=None, tag=None):
                 gsize=_gsize(n, lanes), lsize=(WG,),
                 full_args=(table, Y.dev_buf, t.dev_buf, signals.dev_buf),
                 name="hip_presentinput", tag=tag)
-    plan.row_iterations = -(-widest // lanes)
+    plan.row_iterations = -(-widest // (4 * lanes))  # (four at a time: seq_move)
     plan.description = _description(Y)
     return plan
 
@@ -1165,6 +1169,118 @@ def plan_conv2d(queue, X, Y, filters, shape_in, shape_out, kernel_shape, conv=Tr
     plan.bw_per_call = 4 * (x_size + f_size + y_size)
     plan.description = "shape_in=%s, shape_out=%s, kernel=%s, conv=%s" % (
         tuple(shape_in), tuple(shape_out), tuple(kernel_shape), conv)
+    plan.conv_spec = dict(Y=Y, y_start=y_start, y_size=y_size)  # what the two functions below need
+    return plan
+
+
+def _conv_with(plan, kern, args, extra, what, bw, flops):
+    fused = Plan(plan.queue, kern, args, gsize=plan.gsize, lsize=plan.lsize,
+                 full_args=tuple(plan.full_args) + tuple(extra), name=plan.name,
+                 tag=" + ".join([plan.tag, what] if plan.tag else [what]), bw_per_call=plan.bw_per_call + (bw or 0), flops_per_call=plan.flops_per_call + (flops or 0))
+    fused.description = plan.description
+    return fused
+
+
+def fuse_conv_filter(conv_plan, lf_plan):
+    """One launch less for "Y = conv(X); filter step on Y": the convolution steps the filters (at most two
+    coefficients on a side) whose input is its whole output (`nhip_conv2d_filter`).  Returns ``(plan replacing
+    conv_plan, plans replacing [lf_plan])`` as `hipra_gemv.fuse_linearfilter` does, or None."""
+    from .hipra_gemv import _second_order_targets
+
+    spec, conv = getattr(lf_plan, "lf_spec", None), getattr(conv_plan, "conv_spec", None)
+    if spec is None or conv is None:
+        return None
+    X, F, A, B = (spec[k] for k in ("X", "Y", "A", "B"))
+    if X.ptr.value != conv["Y"].ptr.value:
+        return None
+    queue = conv_plan.queue
+    a_host, b_host = A.to_host(), B.to_host()
+    rows, second, rest = [], {}, []
+    for i in range(len(X)):
+        vector = all(int(r.shape1s[i]) == 1 and int(r.stride0s[i]) == 1 for r in (X, F))
+        if not (vector and int(X.starts[i]) == conv["y_start"] and int(X.shape0s[i]) == conv["y_size"]
+                and 1 <= int(B.shape0s[i]) <= 2 and int(A.shape0s[i]) <= 2):
+            rest.append(i)
+            continue
+        na = int(A.shape0s[i])
+        if na > 1 or int(B.shape0s[i]) > 1:
+            second[i] = len(second)
+        bits = [int(v) for v in np.array([a_host[i][0, 0] if na else 0, b_host[i][0, 0]],
+                                         dtype=np.float32).view(np.int32)]
+        rows.append((int(F.starts[i]), bits[0], bits[1], na, i))
+    if not rows:
+        return None
+    targets, state = _second_order_targets(queue, rows, second, spec, a_host, b_host)
+    dev_targets = to_device(queue, targets)
+    plan = _conv_with(conv_plan, queue.lib.nhip_conv2d_filter,
+                      tuple(conv_plan.args) + (dev_targets.ptr, len(rows), F.ptr),
+                      (dev_targets, F.dev_buf, state), "filter", 8 * conv["y_size"] * len(rows), 0)
+    if second:
+        plan.filter_state = state
+    residual = []
+    if rest:
+        residual = plan_linearfilter(queue, X[rest], F[rest], A[rest], B[rest], spec["Xbuf"][rest],
+                                     spec["Ybuf"][rest], tag=lf_plan.tag)
+        residual[0].unfused_items = list(rest)
+    return plan, residual
+
+
+def fuse_conv_neurons(conv_plan, rows_plan):
+    """One launch less for "Y = conv(X); J = Y + bias; neurons(J)": the convolution forms the currents and
+    updates the neurons (`nhip_conv2d_neuron`) of a launch of the small-item kernel that does nothing else:
+    one item, with at most one dot product of one column and no input sums, whose old value or whose column is the
+    convolution's whole output.  Returns the plan replacing both, or None."""
+    conv, prog = getattr(conv_plan, "conv_spec", None), getattr(rows_plan, "prog", None)
+    kern = getattr(rows_plan.kern, "__name__", "")
+    if conv is None or prog is None or kern not in ("nhip_gemv_rows_lif", "nhip_gemv_rows_neuron"):
+        return None
+    lif, args = kern == "nhip_gemv_rows_lif", rows_plan.args
+    if len(rows_plan.members) != 1 or (not lif and args[-1] is not None) or any(
+            ra.ptr.value != conv["Y"].ptr.value for ra in (prog.A, prog.X, prog.Y, prog.Y_in)):
+        return None
+    b = rows_plan.members[0]
+    g, pop = prog.geometry[b], np.asarray(rows_plan.host_pops)[b]
+    flags = int(pop[7 if lif else 10])
+    n = conv["y_size"]
+    if not (g["y_len"] == n and g["y_stride0"] == 1 and len(g["dots"]) <= 1 and flags & 256):
+        return None
+    # the output as the old value, or as the column of the dot product (a copy is a product with one)
+    OUT = -2
+    whole = lambda start, stride: start == conv["y_start"] and (stride == 1 or n == 1)
+    a_start, a_stride, x_start = -1, 0, 0
+    yin, yin_stride = g["y_in_start"], g["y_in_stride0"]
+    if whole(yin, yin_stride):
+        yin = OUT
+    if g["dots"]:
+        d = g["dots"][0]
+        if d["a_shape1"] != 1:
+            return None
+        a_start, a_stride, x_start = d["a_start"], d["a_stride0"], d["x_start"]
+        if whole(a_start, a_stride):
+            a_start = OUT
+    if OUT not in (yin, a_start):
+        return None
+    # (what else the current is made of must not be the output, in part or in another order)
+    lo, hi = conv["y_start"], conv["y_start"] + n
+    spans = [(x_start, x_start + 1)] if g["dots"] else []
+    spans += [(start, start + (n - 1) * stride + 1) for start, stride in ((yin, yin_stride), (a_start, a_stride))
+              if start >= 0]
+    if any(a < hi and lo < b for a, b in spans):
+        return None
+    current = np.zeros(9, dtype=np.int32)
+    current[:4] = a_start, a_stride, x_start, -1 if flags & 1024 else g["y_start"]
+    current[7:] = yin, yin_stride
+    current[4:7] = np.array([prog.alpha[b], prog.beta[b], prog.gamma[b]], dtype=np.float32).view(np.int32)
+    queue = conv_plan.queue
+    dev_pop = to_device(queue, pop.astype(np.int32))
+    states = tuple(args[14:17]) + ((args[16],) + tuple(args[17:20]) if lif else (args[17], None, None, None))
+    plan = _conv_with(conv_plan, queue.lib.nhip_conv2d_neuron,
+                      tuple(conv_plan.args) + (prog.A.ptr, current.ctypes.data, prog.Y.ptr, int(lif), dev_pop.ptr,
+                                               args[12], args[13]) + states,
+                      (current, dev_pop) + tuple(rows_plan.full_args), "neurons",
+                      (rows_plan.bw_per_call or 0) - 4 * conv["y_size"], rows_plan.flops_per_call)
+    plan.lif_written = getattr(rows_plan, "lif_written", ())
+    plan.lazy_currents = getattr(rows_plan, "lazy_currents", None)
     return plan
 
 

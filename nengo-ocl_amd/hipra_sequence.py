@@ -232,6 +232,19 @@ def _can_carry(plan, needs=0):
     return name in ("hipra_gemv.events", "hipra_gemv.events_filter") and cls[0] == 4 and needs == 0
 
 
+def _can_carry_more(plan, seq, needs):
+    """Launches whose carried sequence has room for the operations of `seq` (a sequence or one short
+    plan), in a group of their own where they touch nothing that the others do."""
+    carried = getattr(plan, "carried", None)
+    if carried is None or getattr(plan, "prelude", None) is None:
+        return False
+    more = seq.members if seq.name == "hip_sequence" else [seq]
+    ops = carried.members + list(more)
+    if len(ops) > MAX_OPS or sum(_staged_rows(sequence_op(p)) for p in ops) > MAX_STAGED_ROWS:
+        return False
+    return plan.name not in ("hipra_gemv.events", "hipra_gemv.events_filter") or (needs | carried.needs) == 0
+
+
 def carry_sequences(plans):
     """Sequence launches (and single small plans) next to a large-item GEMV launch that
     touches none of their memory ride in that launch, in work-groups of their own
@@ -253,7 +266,7 @@ def carry_sequences(plans):
         for step in (-1, 1):
             q = k + step
             while 0 <= q < len(plans) and hasattr(plans[q], "enqueue") and not _conflict(seq, plans[q]):
-                if _can_carry(plans[q], needs):
+                if _can_carry(plans[q], needs) or (step < 0 and _can_carry_more(plans[q], seq, needs)):
                     j = q
                     break
                 q += step
@@ -262,9 +275,22 @@ def carry_sequences(plans):
         if j is None:
             k += 1
             continue
+        carrier = plans[j]
+        before = getattr(carrier, "carried", None)
+        if before is not None:  # together with what the launch carries already
+            reads, writes = seq.reads_mem, seq.writes_mem
+            more = seq.members if seq.name == "hip_sequence" else [seq]
+            seq = plan_sequence(seq.queue, before.members + list(more))
+            carrier.prelude = (seq.queue.lib.nhip_gemv_tile_carry, tuple(seq.args) + (seq.needs,))
+            carrier.full_args = carrier.full_args + (seq,)
+            carrier.carried = seq
+            carrier.tag = carrier.tag.replace(before.tag, seq.tag)
+            carrier.gsize = (carrier.gsize[0] + seq.gsize[0] - before.gsize[0],)
+            carrier.reads_mem, carrier.writes_mem = carrier.reads_mem | reads, carrier.writes_mem | writes
+            del plans[k]
+            continue
         if seq.name != "hip_sequence":
             seq = plan_sequence(seq.queue, [seq])
-        carrier = plans[j]
         carrier.prelude = (seq.queue.lib.nhip_gemv_tile_carry, tuple(seq.args) + (seq.needs,))
         carrier.full_args = carrier.full_args + (seq,)
         carrier.carried = seq

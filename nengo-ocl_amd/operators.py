@@ -349,6 +349,22 @@ def sparse_products_set_their_target(operators):
     return [replace.get(id(op), op) for op in operators if id(op) not in drop]
 
 
+def convolutions_set_their_target(operators):
+    """``Reset(y); ConvInc(y)`` with no other writer of y: the reset goes away.  The plan of a
+    convolution stores its output, whatever y held before (as the reference's does,
+    clra_nonlinearities.py:1847-1860), so nothing ever sees the value it sets."""
+    sets, incs, _, updates = signal_io_dicts(operators)
+    drop = set()
+    for op in operators:
+        if not _is(op, "ConvInc") or op.Y.is_view:
+            continue
+        base = op.Y.base
+        if (len(sets[base]) == 1 and _is(sets[base][0], "Reset") and not sets[base][0].dst.is_view
+                and len(incs[base]) == 1 and incs[base][0] is op and not updates[base]):
+            drop.add(id(sets[base][0]))
+    return [op for op in operators if id(op) not in drop]
+
+
 def neurons_read_constant_input(operators, keep=()):
     """Neurons whose input current is only ever a copy of a constant (an ensemble
     without incoming connections: J = bias every step) read that constant directly,

@@ -98,6 +98,8 @@ class HipBackend:
         if os.environ.get("NENGO_HIP_CARRY_SEQUENCES", "1") != "0":  # switch for measurements
             self.carry_sequences = hipra_sequence.carry_sequences
         self.plans_conflict = hipra_sequence._conflict
+        self.fuse_conv_neurons = hipra_nonlinearities.fuse_conv_neurons
+        self.fuse_conv_filter = hipra_nonlinearities.fuse_conv_filter
         self.fuse_gemv_filter = functools.partial(hipra_gemv.fuse_linearfilter, second_order=True)
         self.fuse_spmv_filter = hipra_spmv.fuse_linearfilter
         if os.environ.get("NENGO_HIP_OUTER_FILTER", "1") != "0":  # switch for measurements
@@ -113,8 +115,6 @@ class HipBackend:
             return self._gemv.fuse_input_sums(sum_plan, lif_plan)
         return None
 
-    def share_spike_bits(self, lif_plan, product_plan):
-        """Let the product of a population's spikes read them as bits from the launch that updates
     def resident_program(self, plans, all_data, n_launches):
         """`hipra_resident.resident_program` for a list of (plan, memory it reads, memory it writes), or
         None where it is switched off."""
@@ -122,6 +122,8 @@ class HipBackend:
             return None
         return self._resident.resident_program(self.queue, plans, all_data, n_launches)
 
+    def share_spike_bits(self, lif_plan, product_plan):
+        """Let the product of a population's spikes read them as bits from the launch that updates
         its neurons, if that launch can leave them."""
         sp = product_plan.spmv
         bits = lif_plan.__dict__.setdefault("spike_bits", {})
@@ -376,6 +378,7 @@ class Simulator:
         if fuse:
             operators = ops_mod.fuse_into_multidotinc(operators)
             operators = ops_mod.sparse_products_set_their_target(operators)
+            operators = ops_mod.convolutions_set_their_target(operators)
             if not reference_host_state:
                 operators = ops_mod.neurons_read_constant_input(operators, keep=probed)
             if learn_in_place:
@@ -528,6 +531,8 @@ class Simulator:
         plans.extend(probe_plans)
         if fuse and hasattr(self.backend, "fuse_gemv_filter"):
             plans = self._fuse_filter_epilogues(plans)
+        if fuse and hasattr(self.backend, "fuse_conv_neurons"):
+            plans = self._fuse_convolutions(plans)
         if fuse and hasattr(self.backend, "fuse_input_sums"):
             plans = self._fuse_input_sums(plans)
         if fuse and hasattr(self.backend, "fuse_learning"):
@@ -536,27 +541,27 @@ class Simulator:
             plans = self._fuse_hebbian(plans)
         if fuse and hasattr(self.backend, "fuse_outer_filter"):
             plans = self._fuse_outer_filters(plans)
+        # (launches that carry others declare what those touch as well: by now they do not)
+        apart = [(p, getattr(p, "reads_mem", None), getattr(p, "writes_mem", None)) for p in plans]
         if merge_small and hasattr(self.backend, "merge_small_plans"):
             plans = self.backend.merge_small_plans(plans)
             if fuse and hasattr(self.backend, "carry_sequences"):
                 plans = self.backend.carry_sequences(plans)
         self._store_spikes_as_bits(plans)
-        # (launches that carry others declare what those touch as well: by now they do not)
-        apart = [(p, getattr(p, "reads_mem", None), getattr(p, "writes_mem", None)) for p in plans]
         if fuse and hasattr(self.backend, "share_spike_bits"):
             self._share_spike_bits(plans)
         logger.info("Plans in %0.3f s", _time.time() - t0)
 
-        self._plans = Plans(plans, self.profiling, use_graph=use_graph, branches=branches,
-                            before_last=before_last, resident=resident)
-        self.rng = None
-        self._drain = None
-        if hasattr(self.backend, "probe_drain"):
         before_last = self._plan_host_view()
         resident = None
         if (fuse and merge_small and use_graph and not before_last and hasattr(self.backend, "resident_program")
                 and not self._spike_bits):
             resident = self.backend.resident_program(apart, self.all_data, len(plans))
+        self._plans = Plans(plans, self.profiling, use_graph=use_graph, branches=branches,
+                            before_last=before_last, resident=resident)
+        self.rng = None
+        self._drain = None
+        if hasattr(self.backend, "probe_drain"):
             self._drain = self.backend.probe_drain(self._probe_plan, self.all_data,
                                                    self.sidx[self.model.step],
                                                    self.sidx[self.model.time])
@@ -1031,6 +1036,54 @@ class Simulator:
             del plans[i]
             plans.insert(at, fused)
             j -= 1
+        return plans
+
+    def _fuse_convolutions(self, plans):
+        """The neurons that a convolution drives, or the filters that read its output, become part of
+        its launch (`hipra_nonlinearities.fuse_conv_neurons`, `fuse_conv_filter`): where they are the next
+        plan that touches anything of the convolution's, and write nothing that it reads."""
+        conflict = self.backend.plans_conflict
+        plans = list(plans)
+        i = 0
+        while i < len(plans):
+            conv = plans[i]
+            i += 1
+            if getattr(conv, "conv_spec", None) is None:
+                continue
+            j = next((k for k in range(i, len(plans)) if conflict(conv, plans[k])), None)
+            if j is None or not all(hasattr(q, "enqueue") for q in plans[i:j + 1]):
+                continue
+            after = plans[j]
+            output = set(conv.writes_mem)
+            ops = getattr(after, "planned_ops", None)
+            if getattr(after, "lf_spec", None) is not None:
+                if ops is None or len(ops) != len(after.lf_spec["X"]):
+                    continue
+                result = self.backend.fuse_conv_filter(conv, after)
+                if result is None:
+                    continue
+                fused, residual = result
+                rest = set(residual[0].unfused_items) if residual else set()
+                mem = lambda sel: ({op.input.base for k, op in enumerate(ops) if sel(k)},
+                                   {op.output.base for k, op in enumerate(ops) if sel(k)})
+                (reads, writes), (rr, rw) = mem(lambda k: k not in rest), mem(lambda k: k in rest)
+                for p in residual:
+                    p.reads_mem, p.writes_mem = rr, rw
+                    p.planned_ops = [op for k, op in enumerate(ops) if k in rest]
+            else:
+                fused, residual = self.backend.fuse_conv_neurons(conv, after), []
+                reads, writes = after.reads_mem, after.writes_mem
+            if fused is None or writes & (conv.reads_mem | output):
+                continue
+            fused.reads_mem, fused.writes_mem = conv.reads_mem | reads, output | writes
+            if getattr(fused, "filter_state", None) is not None:
+                self._filter_positions.append(fused.filter_state)
+            for p in residual:
+                self._filter_positions.append(p.bufpos)
+            # (nothing between the two touches the convolution's memory: it moves down)
+            plans[j:j + 1] = [fused] + residual
+            del plans[i - 1]
+            i -= 1
         return plans
 
     def _fuse_filter_epilogues(self, plans):

@@ -661,3 +661,49 @@ def test_small_networks_run_resident(queue, monkeypatch, kind, neurons, dims, en
                 assert np.any(gpu.data[p] != 0) and np.array_equal(gpu.data[p], cpu.data[p_o])
             assert np.array_equal(gpu.signal_buffer().view(np.uint32), cpu.signal_buffer().view(np.uint32))
             gpu.reset()
+
+
+# the tiled kernel and the one of a wave per group; layers of every kind of epilogue
+@pytest.mark.parametrize("kind", ["RectifiedLinear", "LIF", "AdaptiveLIF", "LIFRate", "Sigmoid",
+                                  "SpikingRectifiedLinear", "AdaptiveLIFRate"])
+@pytest.mark.parametrize("size,channels,filters,synapse", [(12, 1, 5, "lowpass"), (17, 3, 16, "alpha"),
+                                                           (26, 2, 32, "lowpass")])
+def test_convolutions_update_the_neurons_and_filters_they_feed(queue, kind, size, channels, filters, synapse):
+    """A layer's neurons are updated by the convolution that forms their currents, the synapse behind a
+    convolution is stepped by it, and nothing resets what it overwrites; the image and the samples of a large
+    layer ride in another launch."""
+    from nengo_ocl_amd import minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    def make():
+        rng = np.random.RandomState(3)
+        net = mb.Network(seed=7, solver="surrogate")
+        kw = dict(neuron_type=getattr(mb, kind)(), max_rates=(100, 200), intercepts=(-0.5, 0.5))
+        eye = net.Node(mb.PresentInput(rng.uniform(size=(3, size * size * channels)), 0.004),
+                       size_out=size * size * channels)
+        first = mb.Convolution(filters, (size, size, channels), kernel_size=(3, 3), seed=1)
+        second = mb.Convolution(2 * filters, tuple(first.spec.output_shape.shape), kernel_size=(3, 3),
+                                strides=(2, 2), seed=2,
+                                init=rng.uniform(-1, 1, size=(3, 3, filters, 2 * filters)) / (9.0 * filters))
+        layers = [net.Ensemble(c.size_out, 1, encoders=np.ones((c.size_out, 1)), **kw) for c in (first, second)]
+        net.Connection(eye, layers[0].neurons, transform=first, synapse=None)
+        net.Connection(layers[0].neurons, layers[1].neurons, transform=second,
+                       synapse=mb.Alpha(0.003) if synapse == "alpha" else mb.Lowpass(0.005))
+        out = net.Node(None, size_in=3)
+        net.Connection(layers[1].neurons, out, synapse=mb.Lowpass(0.005),
+                       transform=rng.normal(scale=1e-2 / second.size_out, size=(3, second.size_out)))
+        return net, [net.Probe(out), net.Probe(layers[1].neurons, sample_every=0.004), net.Probe(layers[0].neurons)]
+
+    (net, probes), (net_o, probes_o) = make(), make()
+    with Simulator(net, seed=1) as gpu, OracleSimulator(net_o, seed=1) as cpu:
+        cpu.run_steps(25)
+        launches = [p.kern.__name__ for p in gpu._plans]
+        assert {"nhip_conv2d_neuron", "nhip_conv2d_filter"} <= set(launches), launches
+        assert not {"nhip_conv2d", "nhip_reset", "nhip_linearfilter"} & set(launches), launches
+        for _ in range(2):
+            gpu.run_steps(25)
+            assert np.array_equal(gpu.signal_buffer().view(np.uint32), cpu.signal_buffer().view(np.uint32))
+            for p, p_o in zip(probes, probes_o):
+                assert np.any(gpu.data[p] != 0) and np.array_equal(gpu.data[p], cpu.data[p_o])
+            gpu.reset()
