@@ -115,6 +115,12 @@ THIN_MIN_ROWS, THIN_ROWS_FOR_LANE_PER_ROW = 32, 65536
 # Up to 65,535 rows of one to three columns: alone, with filters or the neuron update 3.9-4.5 us, through
 # LDS 5.6-9.6; whole steps of 2 x 5,500 x 3 to 2 x 30,000 x 1 LIF neurons 17.1-58.5 us against 22.1-64.3.
 THIN_CLASS, THIN_MAX_COLS = (2, 4, 1), 4
+# Neurons that form the sums of their inputs: with four lanes a row each lane reads all parts of the
+# row's sum, with a lane per row the lanes of the wave read one each. Whole steps of small-world graphs
+# (3.9 parts a sum) of 30 x 100 neurons 11.3 us -> 10.45, 64 x 100 11.55 -> 10.54, 1,000 x 10 12.0 -> 11.1,
+# 256 x 100 12.06 -> 10.65, 300 x 150 13.0 -> 10.9, 1,000 x 64 13.4 -> 10.6. Below these rows the launch is
+# a few waves either way.
+SUM_PARTS_FOR_WAVE_TASKS, SUM_MIN_ROWS_FOR_WAVE_TASKS = 3, 3000
 LIF_POP_ENABLED, LIF_POP_DECAY, LIF_POP_NO_J = 1 << 8, 1 << 9, 1 << 10  # flag bits of a population row
 LIF_POP_MASK = 1 << 12
 LIF_POP_BITS = 1 << 11  # spikes stored as a bit per neuron (see `store_spikes_as_bits`)
@@ -215,6 +221,18 @@ def _balanced_rows(M, cap):
     stays 128; M = 100, cap = 64 becomes 50 instead of 64 + 36)."""
     n_tasks = -(-M // cap)
     return -(-M // n_tasks)
+
+
+def wave_tasks(items, lens):
+    """Task rows (item, first row, rows, 0): up to 64 consecutive rows of an item, which a wave takes whole."""
+    lens = np.asarray(lens, dtype=np.int64)
+    per_item = -(-lens // WAVE)  # (built with numpy: there can be millions of rows)
+    first = np.cumsum(per_item) - per_item
+    tasks = np.zeros((int(per_item.sum()), 4), dtype=np.int32)
+    tasks[:, 0] = np.repeat(np.asarray(items, dtype=np.int32), per_item)
+    tasks[:, 1] = (np.arange(len(tasks)) - np.repeat(first, per_item)) * WAVE
+    tasks[:, 2] = np.minimum(WAVE, np.repeat(lens, per_item) - tasks[:, 1])
+    return tasks
 
 
 class gemv_prog:
@@ -693,14 +711,7 @@ class gemv_prog:
                 # a lane per row: tasks of up to 64 consecutive rows of an item that a wave
                 # takes whole, so that the records are the wave's and not each row's
                 lpr_arg = WAVE
-                lens = np.array([geometry[b]["y_len"] for b in members], dtype=np.int64)
-                per_item = -(-lens // WAVE)  # (built with numpy: there can be millions of rows)
-                first = np.cumsum(per_item) - per_item
-                row0 = (np.arange(int(per_item.sum())) - np.repeat(first, per_item)) * WAVE
-                task_rows = np.zeros((len(row0), 4), dtype=np.int32)
-                task_rows[:, 0] = np.repeat(np.array(members, dtype=np.int32), per_item)
-                task_rows[:, 1] = row0
-                task_rows[:, 2] = np.minimum(WAVE, np.repeat(lens, per_item) - row0)
+                task_rows = wave_tasks(members, [geometry[b]["y_len"] for b in members])
             elif flavor == 2:  # built with numpy: there can be millions of rows
                 counts = np.array([geometry[b]["y_len"] for b in members], dtype=np.int64)
                 task_tab = np.zeros((int(counts.sum()), 4), dtype=np.int32)
@@ -1236,6 +1247,15 @@ def fuse_input_sums(sum_plan, lif_plan):
             dots = E.geometry[b]["dots"]
             if dots and dots[0]["x_start"] in where:
                 ranges[b] = where[dots[0]["x_start"]]
+        if (lpr == 4 and WAVE_TASKS and len(tasks) >= SUM_MIN_ROWS_FOR_WAVE_TASKS
+                and len(part_rows) >= SUM_PARTS_FOR_WAVE_TASKS * len(sums)
+                and all(d["a_shape1"] <= THIN_MAX_COLS
+                        for b in lif_plan.members for d in E.geometry[b]["dots"])):
+            lpr, task_words = WAVE, 16
+            rows = wave_tasks(lif_plan.members, [E.geometry[b]["y_len"] for b in lif_plan.members])
+            of = rows[:, 0]
+            tasks = np.concatenate([rows, items[of], coefs[of].view(np.int32)], axis=1)
+            tasks[:, [3, 11, 15]] = 0 if other else pops[of][:, [0, 1, 7]]
         extra = []
         for k, start in enumerate(spare):
             b, n = n_items + k, sums[start][0]
@@ -1268,6 +1288,8 @@ def fuse_input_sums(sum_plan, lif_plan):
                  flops_per_call=(lif_plan.flops_per_call or 0) + (sum_plan.flops_per_call or 0))
     fused.description = lif_plan.description + "; input sums: " + sum_plan.description
     fused.kernel_class, fused.n_tasks = lif_plan.kernel_class, len(tasks)
+    if not large and lpr == WAVE:
+        fused.kernel_class = (2, 1, 1)
     fused.members, fused.prog = lif_plan.members, E
     fused.gemv_bytes = getattr(lif_plan, "gemv_bytes", lif_plan.bw_per_call)
     fused.host_tasks = tasks

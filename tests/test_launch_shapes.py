@@ -707,3 +707,37 @@ def test_convolutions_update_the_neurons_and_filters_they_feed(queue, kind, size
             for p, p_o in zip(probes, probes_o):
                 assert np.any(gpu.data[p] != 0) and np.array_equal(gpu.data[p], cpu.data[p_o])
             gpu.reset()
+
+
+# rows on both sides of the limit for a lane per row; neurons around the 64 rows of a task
+@pytest.mark.parametrize("kind", ["LIF", "LIFRate"])
+@pytest.mark.parametrize("n_ens,neurons,parts,lanes", [(48, 64, 3, 64), (46, 65, 3, 4), (40, 103, 70, 64),
+                                                       (333, 13, 4, 64), (70, 60, 2, 4)])
+def test_waves_form_the_sums_of_many_inputs(queue, kind, n_ens, neurons, parts, lanes):
+    """Neurons in one launch with the sums of their inputs, one to three dimensions, and a sum that no
+    neuron reads."""
+    from nengo_ocl_amd import minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    def make():
+        rng = np.random.RandomState(n_ens)
+        net = mb.Network(seed=2, solver="surrogate")
+        ens = [net.Ensemble(neurons, 1 + i % 3, neuron_type=getattr(mb, kind)()) for i in range(n_ens)]
+        out = net.Node(None, size_in=2)
+        for i, e in enumerate(ens):
+            for j in rng.choice(n_ens, size=parts, replace=parts > n_ens):
+                net.Connection(ens[j], e, synapse=mb.Lowpass(0.005), transform=rng.uniform(
+                    -1, 1, size=(1 + i % 3, 1 + int(j) % 3)))
+        for e in ens[:9:3]:
+            net.Connection(e, out, synapse=mb.Lowpass(0.005), transform=rng.normal(size=(2, 1)))
+        return net, net.Probe(out)
+
+    (net, probe), (net_o, probe_o) = make(), make()
+    with Simulator(net, seed=1) as gpu, OracleSimulator(net_o, seed=1) as cpu:
+        fused = [p for p in gpu._plans if getattr(p, "input_sums", 0)]
+        assert len(fused) == 1 and fused[0].args[0] == lanes, [(p, p.args[0]) for p in fused]
+        cpu.run_steps(20)
+        gpu.run_steps(20)
+        assert np.array_equal(gpu.signal_buffer().view(np.uint32), cpu.signal_buffer().view(np.uint32))
+        assert np.any(gpu.data[probe] != 0) and np.array_equal(gpu.data[probe], cpu.data[probe_o])
