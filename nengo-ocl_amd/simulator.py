@@ -1255,7 +1255,8 @@ class Simulator:
                 if base in sim._host_view_index:
                     # between two steps the reference holds what this signal was before
                     # the last step's update of it
-                    full = np.array(sim._host_view_copy[sim._host_view_index[base]])
+                    copy, k = sim._host_view_copy, sim._host_view_index[base]
+                    full = copy.read_copy(k) if hasattr(copy, "read_copy") else np.array(copy[k])
                     raw = full if base is item else sim._view_of(item, full)
                 elif base in sim._pending_filters:
                     full = sim._with_pending_filter(base, np.array(sim.all_data[sim.sidx[base]]))
