@@ -351,18 +351,18 @@ int nhip_resident(void *stream, const void *spans, int n_spans, const void *ops,
  * with the copy that adds the change (clra_nonlinearities.py:2082-2277) + `plan_linearfilter`, in that
  * order.  One dot product per item, reference order; X may not overlap what the launch writes, except by
  * the outputs of `filters`.
- *   tasks   : int32[n_tasks][16] {a_start, a_stride0, N, x_start, y_start, y_stride0, yin_start,
- *             yin_stride0, alpha, beta, gamma (float bits), row0, n_rows (1..4), rule (row of `rules`,
- *             -1: none), first_target, n_targets}: rows row0 .. row0 + n_rows - 1 of an item
- *   rules   : int32[][8] {kind, pre_start, post_start, post_stride0, theta_start, theta_stride0 (BCM),
- *             alpha, beta (float bits)}: row i of the matrix changes by the rule's element of
- *             X[pre_start + j], X[post_start + i * post_stride0] (and theta, or the old weight); at least one row
+ *   tasks   : int32[n_tasks][24] {a_start, a_stride0, N, x_start, y_start, y_stride0, yin_start,
+ *             yin_stride0, alpha, beta, gamma (float bits), row0, n_rows (1..4), learned (0: the matrix
+ *             stays), first_target, n_targets, then the rule: kind, pre_start, post_start, post_stride0,
+ *             theta_start, theta_stride0 (BCM), alpha, beta (float bits)}: rows row0 .. row0 + n_rows - 1 of an
+ *             item; row i of the matrix changes by the rule's element of X[pre_start + j],
+ *             X[post_start + i * post_stride0] (and theta, or the old weight)
  *   targets, F : filters of the fresh y, as for nhip_gemv_tile_filter (orders 1 and 2)
  *   filters : int32[n_filters][8] {s_start, f_start, n, has_a, a0, b0 (float bits), 0, 0}: stepped on
  *             X[s_start ..], F[f_start ..] when every row has read the old F; F and X one buffer
  *   arrived : one int, zero before the launch and after it (only read with n_filters > 0)
  * Bit-identical to the separate calls. */
-int nhip_gemv_learn(void *stream, const int *tasks, int n_tasks, const int *rules, float *A,
+int nhip_gemv_learn(void *stream, const int *tasks, int n_tasks, float *A,
                     const float *X, const float *Yin, float *Y, const int *targets, float *F,
                     const int *filters, int n_filters, int *arrived);
 

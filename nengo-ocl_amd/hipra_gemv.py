@@ -1590,8 +1590,8 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
         for row0 in range(0, g["y_len"], per_group):
             tasks.append((d["a_start"], d["a_stride0"], d["a_shape1"], d["x_start"], g["y_start"], g["y_stride0"],
                           g["y_in_start"], g["y_in_stride0"], bits(prog.alpha[b]), bits(prog.beta[b]),
-                          bits(prog.gamma[b]), row0, min(per_group, g["y_len"] - row0), rule_of.get(b, -1),
-                          first, n))
+                          bits(prog.gamma[b]), row0, min(per_group, g["y_len"] - row0), int(b in rule_of), first, n)
+                         + (tuple(int(v) for v in rules[rule_of[b]]) if b in rule_of else (0,) * 8))
     if not tasks:
         return None
     filters, moved, rest = [], [], []
@@ -1608,19 +1608,19 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
                                 bits(a_host[k][0, 0]) if na else 0, bits(b_host[k][0, 0]), 0, 0))
                 moved.append(k)
         rest = [k for k in range(len(S)) if k not in set(moved)]
-    dev_tasks, dev_rules = to_device(queue, np.array(tasks, dtype=np.int32)), to_device(queue, rules)
+    dev_tasks = to_device(queue, np.array(tasks, dtype=np.int32))
     dev_filters = to_device(queue, np.array(filters or [(0,) * 8], dtype=np.int32))
     arrived = to_device(queue, np.zeros(4, dtype=np.int32))
     lib = queue.lib
-    targets = dev_targets if dev_targets is not None else dev_rules  # (not read without targets)
+    targets = dev_targets if dev_targets is not None else dev_tasks  # (not read without targets)
     total = lambda attr: sum(getattr(p, attr) or 0 for p in list(products) + [rule_plan])
     weights = 4 * int(delta.sizes.sum())
     plan = Plan(queue, lib.nhip_gemv_learn,
-                (dev_tasks.ptr, len(tasks), dev_rules.ptr, prog.A.ptr, prog.X.ptr, prog.Y_in.ptr, prog.Y.ptr,
+                (dev_tasks.ptr, len(tasks), prog.A.ptr, prog.X.ptr, prog.Y_in.ptr, prog.Y.ptr,
                  targets.ptr, F.ptr, dev_filters.ptr, len(filters), arrived.ptr),
                 gsize=(WG * len(tasks),), lsize=(WG,),
                 full_args=sum((tuple(p.full_args) for p in list(products) + [rule_plan]), ())
-                + (dev_tasks, dev_rules, dev_filters, arrived),
+                + (dev_tasks, dev_filters, arrived),
                 name=products[0].name, tag=" + ".join([products[0].tag, rule_plan.name]),
                 # the rule's own accounting, less the matrices it need not read again
                 bw_per_call=total("bw_per_call") - (2 if spec["rule"] == RULE_OJA else 1) * weights
