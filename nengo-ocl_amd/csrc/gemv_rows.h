@@ -41,6 +41,23 @@
 // row; here the record is the wave's: every lane reads the same addresses for the task, the
 // item's dot products, its population and its input sum, and the parts of an input sum are
 // fetched by the lanes side by side instead of in rounds.
+// Element q of lane p of a quad of lanes and element p of lane q change places (all four lanes are active).
+__device__ __forceinline__ void transpose_quad(float4& v, int lane) {
+    constexpr int XOR1 = 0xB1, XOR2 = 0x4E;  // quad_perm [1,0,3,2] and [2,3,0,1]
+#define NHIP_QUAD(x, ctrl) __int_as_float(__builtin_amdgcn_update_dpp( \
+    0, __float_as_int(x), ctrl, 0xF, 0xF, true))
+    const bool b0 = lane & 1, b1 = lane & 2;
+    // (every exchange before its choice: a lane that is switched off gives nothing)
+    const float x1 = NHIP_QUAD(v.x, XOR1), y1 = NHIP_QUAD(v.y, XOR1), z1 = NHIP_QUAD(v.z, XOR1), w1 = NHIP_QUAD(v.w, XOR1);
+    const float a0 = b0 ? y1 : v.x, a1 = b0 ? v.y : x1, a2 = b0 ? w1 : v.z, a3 = b0 ? v.w : z1;
+    const float x2 = NHIP_QUAD(a0, XOR2), y2 = NHIP_QUAD(a1, XOR2), z2 = NHIP_QUAD(a2, XOR2), w2 = NHIP_QUAD(a3, XOR2);
+    v.x = b1 ? z2 : a0;
+    v.y = b1 ? w2 : a1;
+    v.z = b1 ? a2 : x2;
+    v.w = b1 ? a3 : y2;
+#undef NHIP_QUAD
+}
+
 template <int LPR, int EPI = EPI_NONE, bool WIDE = false, bool WAVE_TASK = false>
 __device__ __forceinline__ void gemv_rows_ref_block(
     const GemvItem* __restrict__ items, const float4* __restrict__ coefs,
@@ -199,13 +216,43 @@ __device__ __forceinline__ void gemv_rows_ref_block(
             const int n_cols = dot.N;
             const float* arow = A + dot.a_start + (size_t)row_u * dot.a_stride0;
             const float* xg = X + dot.x_start;
+            // Rows and vectors of whole aligned quads: a lane loads 16 bytes where it loaded 4, quad 4 i + p
+            // of a tile goes to lane p, and the four lanes transpose what they hold.  64 loads of 16 pieces
+            // of 16 bytes keep a compute unit's address path busy: with as many rows as fill it,
+            // whole steps of rate neurons are faster so (1,026 rows of 1,200 columns 13.0 -> 12.2 us, 1,538
+            // of 2,000 16.9 -> 15.4), but not where a unit has a wave or two (770 rows of 1,000 11.6 both
+            // ways), nor where a group takes a row (160 rows of 3,000 12.8 -> 13.0).
+            const bool quads = LPR == NHIP_WAVE && n_tasks >= 1024 &&
+                               ((n_cols | (int)(reinterpret_cast<uintptr_t>(arow) >> 2) |
+                                 (int)(reinterpret_cast<uintptr_t>(xg) >> 2)) & 3) == 0;
 #pragma unroll 1
             for (int c0 = 0; c0 < n_cols; c0 += WAVES * TILES * TILE) {
                 const int start = c0 + (my_wave * TILES + (lane >> 2)) * TILE + (lane & 3);
                 const int early = max((start + TILE - n_cols) >> 2, 0);
                 const int first = early < STEPS ? start - 4 * early : lane & 3;  // (nothing to sum)
                 float s = 0.0f;
-                if (c0 + my_wave * TILES * TILE < n_cols) {  // uniform
+                if (quads && c0 + my_wave * TILES * TILE < n_cols) {  // uniform
+                    const int tile = c0 + (my_wave * TILES + (lane >> 2)) * TILE;
+                    float4 av[STEPS / 4], xv[STEPS / 4];
+#pragma unroll
+                    for (int i = 0; i < STEPS / 4; ++i) {
+                        const int c = min(tile + 16 * i + 4 * (lane & 3), n_cols - 4);
+                        av[i] = *reinterpret_cast<const float4*>(arow + c);
+                        xv[i] = *reinterpret_cast<const float4*>(xg + c);
+                    }
+                    const int live = (n_cols - tile) >> 2;  // steps inside the row (none: a tile nobody adds)
+#pragma unroll
+                    for (int i = 0; i < STEPS / 4; ++i) {
+                        transpose_quad(av[i], lane);
+                        transpose_quad(xv[i], lane);
+                        s = 4 * i + 0 < live ? fmaf(av[i].x, xv[i].x, s) : s;
+                        s = 4 * i + 1 < live ? fmaf(av[i].y, xv[i].y, s) : s;
+                        s = 4 * i + 2 < live ? fmaf(av[i].z, xv[i].z, s) : s;
+                        s = 4 * i + 3 < live ? fmaf(av[i].w, xv[i].w, s) : s;
+                    }
+                    s = s + __shfl_xor(s, 2, NHIP_WAVE);
+                    s = s + __shfl_xor(s, 1, NHIP_WAVE);
+                } else if (c0 + my_wave * TILES * TILE < n_cols) {
                     float av[STEPS], xv[STEPS];
 #pragma unroll
                     for (int e = 0; e < STEPS; ++e) {

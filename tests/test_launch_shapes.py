@@ -258,6 +258,31 @@ def test_few_long_rows(queue, rng, beta, widths):
     assert np.array_equal(dY.buf.view(np.uint32), Yo.buf.view(np.uint32))
 
 
+@pytest.mark.parametrize("heights,widths,lanes", [
+    ([1, 700, 200, 60, 62], [512, 516, 2048, 2044, 2052], 128), ([400, 624, 1], [1000, 640, 513], 128),
+    ([1024], [2056], 128)])
+@pytest.mark.parametrize("beta", [0.0, 1.0])
+def test_long_rows_in_quads(queue, rng, heights, widths, lanes, beta):
+    """Rows that fill the device and lie on 16-byte boundaries, in whole quads or not, around the tiles and
+    the passes; sums that are or start at -0, and an infinity beside the last tile's end."""
+    from nengo_ocl_amd import hipra_gemv
+    from oracle import oracle as orc
+
+    A = RA([rng.normal(size=(m, n)) for m, n in zip(heights, widths)], align=True)
+    X = RA([rng.normal(size=n) for n in widths], align=True)
+    Y = RA([-0.0 * np.ones(m) for m in heights], align=True)
+    A[0][0, :] = -1e-45
+    X[0][:] = 1e-3
+    A[len(widths) - 1][-1, -1] = np.inf
+    A_js = RA([[k] for k in range(len(widths))], dtype=np.int32)
+    dA, dX, dY, Yo = to_dev(queue, A), to_dev(queue, X), to_dev(queue, Y), clone(Y)
+    prog = hipra_gemv.plan_block_gemv(queue, 1.5, dA, A_js, dX, A_js, beta, dY)
+    assert [p.kernel_class for p in prog.plans] == [(2, lanes, 1)]
+    run_plans(prog.plans)
+    orc.plan_block_gemv(None, 1.5, A, A_js, X, A_js, beta, Yo).plans[0]()
+    assert np.array_equal(dY.buf.view(np.uint32), Yo.buf.view(np.uint32))
+
+
 @pytest.mark.parametrize("pre,dims,lanes", [(1000, 200, 128), (5000, 2100, 256)],
                          ids=["wave per row", "group per row"])
 def test_few_long_rows_with_epilogues(queue, pre, dims, lanes):
