@@ -39,8 +39,11 @@ SHORT_ITEM_ELEMS = 4 * SMALL_ITEM_ELEMS
 REF_ORDER_MAX_COLS = 512
 # float32 words of one wave's LDS block in the reference-order kernel for large items
 TILE_STAGE_WORDS = int(os.environ.get("NENGO_HIP_TILE_WORDS", 2176))
-# the reference-order kernel wants at least this many (wave) tasks per launch
-MIN_TILE_TASKS = int(os.environ.get("NENGO_HIP_TILE_MIN_TASKS", 2048))
+# the reference-order kernel wants at least this many (wave) tasks per launch: six a compute unit. Whole
+# steps with 2,048 / 1,536 / 1,024: 48 x 2000 neurons x 32 dimensions 14.9 / 14.1 / 14.1 us, 100 x 2000 x 48
+# 23.7 / 22.2 / 22.3, 30 x 3000 x 24 16.3 / 15.8 / 15.9, 12 x 4000 x 100 23.2 / 22.6 / 22.7, 20 x 2000 x 64
+# 13.0 / 13.0 / 13.7, 64 learned decoders of 2000 x 32 43.8 / 43.5 / 44.2
+MIN_TILE_TASKS = int(os.environ.get("NENGO_HIP_TILE_MIN_TASKS", 1536))
 TILE_TASK_BLOCKS = tuple(float(v) for v in os.environ.get(
     "NENGO_HIP_TILE_TASK_BLOCKS", "4,3.5,3,2.5,2,1.5,1").split(","))  # row blocks per task, tried in order
 # items of the launch that visits only the columns with x != 0 (csrc/gemv_events.hip)
