@@ -11,7 +11,7 @@
 // alone on its SIMD is bound by the number of instructions (5 clocks each, 13 where one waits for the
 // other): the same arithmetic with everything that can be known beforehand resolved by the host.
 // Two populations of 100 neurons: 8.1 -> 2.8 us a step (2.4 of them the launch; replayed as a graph two
-// launches); of 1000: 8.8 -> 6.9.  16 populations of 20 with 10 inputs each: 11.1 -> 5.7.  An operation costs a wave
+// launches); of 1000: 8.8 -> 6.8.  16 populations of 20 with 10 inputs each: 11.2 -> 5.8.  An operation costs a wave
 // 0.2-0.4 us to fetch, 64 neurons 0.7 us (1.3 with sums of inputs), a row of 100 columns 1.1 us.
 #include <cstdint>
 #include <type_traits>
