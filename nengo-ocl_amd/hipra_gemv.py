@@ -1530,8 +1530,8 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
     once per step, and the filters need no launch.
 
     Fused when every item of `products` has one dot product with operands of stride 1, every matrix of the
-    rule is the matrix of one such item (same start, shape and row stride) and its row operand is contiguous.
-    Filters of `lf_plan` with one numerator and at most one denominator coefficient on
+    rule is the matrix of one such item (same start, shape and row stride), its row operand is contiguous, and
+    nothing else the launch reads or writes lies in such a matrix.  Filters of `lf_plan` with one numerator and at most one denominator coefficient on
     contiguous vectors move; the caller has checked that nothing between the plans, and nothing the plans
     read or write themselves, keeps the rule and those filters out of the products' launch.  Returns ``(plan,
     plans for the filters that stay, filters that moved)`` or None."""
@@ -1581,6 +1581,22 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
         elif plan.name.endswith("_filter"):
             return None
     if F.ptr.value != buf:
+        return None
+    # The launch writes a learned matrix back while other groups still run: nothing else that any of them
+    # reads or writes may lie in it.  (Operands that are views of the matrix -- other rows or columns of
+    # it, a vector in it -- need not have its start and shape.)
+    matrices = {b: _span(delta, i) for b, i in rule_of.items()}
+    vector = lambda start, n, stride: (start, start + (n - 1) * stride + 1)
+    others = [_span(ra, i) for ra in (pre, post) + ((aux,) if spec["rule"] == RULE_BCM else ())
+              for i in range(len(ra))]
+    for b in members:
+        g, d = geometry[b], geometry[b]["dots"][0]
+        others += [vector(d["x_start"], d["a_shape1"], 1), vector(g["y_start"], g["y_len"], g["y_stride0"]),
+                   vector(g["y_in_start"], g["y_len"], g["y_in_stride0"])]
+        if b not in rule_of:
+            others.append((d["a_start"], d["a_start"] + (g["y_len"] - 1) * d["a_stride0"] + d["a_shape1"]))
+    spans = sorted(matrices.values())
+    if _overlaps([iv for iv in others if iv], spans) or any(a[1] > b[0] for a, b in zip(spans, spans[1:])):
         return None
 
     per_group = WG // WAVE

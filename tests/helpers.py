@@ -22,6 +22,34 @@ def to_dev(queue, ra):
     return HIPRaggedArray(queue, ra)
 
 
+def host_queue(monkeypatch):
+    """A queue whose arrays lie in host memory and whose launches do nothing: plans can be made and
+    looked at without a device."""
+    import contextlib
+    import ctypes
+    import types
+
+    import torch
+    from nengo_ocl_amd import _lib, hipraggedarray
+
+    real = _lib.lib()
+    host_functions = ("nhip_gemv_tile_rows", "nhip_gemv_rows_per_task", "nhip_conv2d_groups")
+
+    class Lib:
+        def __getattr__(self, name):
+            if name in host_functions:
+                return getattr(real, name)
+            launch = lambda *args: 0
+            launch.__name__ = getattr(real, name).__name__
+            return launch
+
+    monkeypatch.setattr(hipraggedarray, "_TORCH", torch)
+    return types.SimpleNamespace(
+        lib=Lib(), handle=ctypes.c_void_p(1), device=torch.device("cpu"), arch="gfx950", n_compute_units=256,
+        global_mem_size=288 << 30, stream=types.SimpleNamespace(synchronize=lambda: None),
+        finish=lambda: None, context=contextlib.nullcontext, read=lambda words: words.numpy().copy())
+
+
 def run_plans(plans):
     for p in plans:
         p()

@@ -3,6 +3,8 @@
 import numpy as np
 import pytest
 
+from helpers import RA, host_queue, to_dev
+
 
 def conv_threads(shape_in, filters, kernel, strides=(1, 1), channels_last=True, conv=True):
     """Threads per group for an unpadded convolution, after a look at the number of groups."""
@@ -76,3 +78,66 @@ def test_layout_of_products_that_are_handed_bits(n_cols, lanes):
             used[new] = True
             assert np.array_equal(index[new], cols[old]) and np.array_equal(values[new], vals[old])
     assert np.all(index[~used] == n_cols) and np.all(np.signbit(values[~used])) and not np.any(values[~used])
+
+
+def learned_products(queue, rule, unlearned=(), learned=((0, 300, 300),), aliases=()):
+    """`hipra_gemv.fuse_hebbian` for products with matrices of the rule (`learned`: offset in the matrix
+    buffer, rows, columns) and with others (`unlearned`: the same, or (None, rows, columns) for one of its
+    own); `aliases`: operand ("x", "pre", "post", "y_in") -> its offset in the matrix buffer."""
+    from nengo_ocl_amd import hipra_gemv, hipra_nonlinearities as nl
+    from nengo_ocl_amd.hipraggedarray import HIPRaggedArray
+
+    aliases, items = dict(aliases), list(learned) + list(unlearned)
+    host = RA([np.zeros((300, 400))] + [np.zeros(n) for n in (5000, 5000, 5000)]
+              + [np.zeros((m, n)) for at, m, n in items if at is None] + [np.zeros(m) for _, m, _ in items])
+    dev = to_dev(queue, host)
+    own = iter(range(4, len(host)))
+    starts = [next(own) if at is None else None for at, _, _ in items]
+    outs = [int(host.starts[next(own)]) for _ in items]
+
+    def view(start, m, n, stride=None):
+        one = lambda v: np.array([v], dtype=np.int32)
+        return HIPRaggedArray.from_buffer(queue, dev.dev_buf, one(start), one(m), one(n), one(stride or n), one(1))
+
+    def column(what, k, n):
+        return view(aliases.get(what, int(host.starts[k])), n, 1)
+
+    cat = hipra_gemv._concat
+    matrix = [view(at if at is not None else int(host.starts[s]), m, n, 400 if at is not None else n)
+              for (at, m, n), s in zip(items, starts)]
+    A = cat(matrix)
+    X = cat([column("x" if k else "", 1, n) for k, (_, _, n) in enumerate(items)])
+    Y = cat([view(out, m, 1) for out, (_, m, _) in zip(outs, items)])
+    Y_in = cat([column("y_in", 3, m) if "y_in" in aliases and k == len(items) - 1 else view(out, m, 1)
+                for k, (out, (_, m, _)) in enumerate(zip(outs, items))])
+    js = RA([[k] for k in range(len(items))], dtype=np.int32)
+    prog = hipra_gemv.plan_block_gemv(queue, 1.0, A, js, X, js, 0.0, Y, Y_in=Y_in)
+    pre = cat([column("pre", 1, n) for _, _, n in learned])
+    post = cat([column("post", 2, m) for _, m, _ in learned])
+    delta, ones = cat(matrix[:len(learned)]), np.ones(len(learned), dtype=np.float32)
+    plan = (nl.plan_oja(queue, pre, post, delta, delta, ones, ones, inc=True) if rule == "Oja" else
+            nl.plan_bcm(queue, pre, post, cat([column("theta", 3, m) for _, m, _ in learned]), delta, ones, inc=True))
+    return prog.plans, hipra_gemv.fuse_hebbian(prog.plans, plan)
+
+
+# other rows, other columns and the inside of the learned matrix (300 rows, 400 apart), one row of it, a row
+# that starts behind its columns; vectors and an old output that lie in it; rules of two overlapping matrices
+@pytest.mark.parametrize("rule", ["Oja", "BCM"])
+@pytest.mark.parametrize("unlearned,learned,aliases,fused", [
+    ((), [(0, 300, 300)], {}, True),
+    ([(None, 200, 300)], [(0, 300, 300)], {}, True),
+    ([(None, 200, 300)], [(0, 150, 300), (150 * 400, 150, 300)], {}, True),
+    ([(0, 150, 300)], [(0, 300, 300)], {}, False),
+    ([(0, 300, 200)], [(0, 300, 300)], {}, False),
+    ([(100 * 400 + 100, 150, 200)], [(0, 300, 300)], {}, False),
+    ([(299 * 400, 1, 300)], [(0, 300, 300)], {}, False),
+    ([(149 * 400 + 300, 1, 200)], [(0, 150, 300)], {}, True),
+    ([(None, 200, 300)], [(0, 300, 300)], {"x": 400}, False),
+    ([(None, 200, 300)], [(0, 300, 300)], {"y_in": 400}, False),
+    ((), [(0, 300, 300)], {"pre": 50 * 400}, False),
+    ((), [(0, 300, 300)], {"post": 50 * 400}, False),
+    ((), [(0, 151, 300), (150 * 400, 150, 300)], {}, False)])
+def test_learned_matrices_are_not_written_where_their_launch_reads(monkeypatch, rule, unlearned, learned, aliases,
+                                                                   fused):
+    _, result = learned_products(host_queue(monkeypatch), rule, unlearned, learned, aliases)
+    assert (result is not None) == fused

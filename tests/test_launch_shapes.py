@@ -645,6 +645,40 @@ def test_rules_between_neurons_in_the_launch_of_their_product(queue, rule, n_pre
                 assert np.array_equal(gpu.data[p], cpu.data[p_o], equal_nan=True)
 
 
+@pytest.mark.parametrize("rule", ["Oja", "BCM"])
+@pytest.mark.parametrize("rows,cols", [(slice(0, 150), slice(None)), (slice(None), slice(20, 200)),
+                                       (slice(7, 8), slice(None))])
+def test_products_with_a_part_of_a_learned_matrix_read_it_unchanged(queue, rule, rows, cols):
+    """Another product of the step reads some rows or columns of the matrix that the rule changes."""
+    from nengo_ocl_amd import ir
+    from nengo_ocl_amd import minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    rng = np.random.RandomState(8)
+    net = mb.Network(seed=5, solver="surrogate")
+    stim = net.Node(mb.WhiteSignal(period=0.5, high=6.0, seed=3), size_out=2)
+    pre, post = net.Ensemble(300, 2), net.Ensemble(300, 2)
+    net.Connection(stim, pre, synapse=mb.Lowpass(0.005))
+    learning = mb.Oja(learning_rate=1e-4, beta=0.7) if rule == "Oja" else mb.BCM(learning_rate=1e-7)
+    net.Connection(pre.neurons, post.neurons, transform=rng.normal(scale=1e-3, size=(300, 300)),
+                   learning_rule=learning, synapse=mb.Lowpass(0.005))
+    model = net.build_model()
+    weights = next(op.dst for op in model.operators if isinstance(op, ir.Copy) and op.inc
+                   and op.dst.shape == (300, 300))
+    x = next(op.X for op in model.operators if isinstance(op, ir.DotInc) and op.A is weights)
+    part = weights[rows, cols]
+    y = ir.Signal(np.zeros(part.shape[0]), name="a part of the product")
+    model.add_op(ir.Reset(y))
+    model.add_op(ir.DotInc(part, x[cols], y))
+    with Simulator(None, model=model, seed=1) as gpu, OracleSimulator(None, model=model, seed=1) as cpu:
+        for _ in range(3):
+            gpu.run_steps(20)
+            cpu.run_steps(20)
+            assert np.any(cpu.signals[y] != 0)
+            assert np.array_equal(gpu.signal_buffer().view(np.uint32), cpu.signal_buffer().view(np.uint32))
+
+
 @pytest.mark.parametrize("kind,neurons,dims,ensembles", [
     ("LIF", 100, 1, 2), ("LIF", 30, 1, 2), ("LIF", 65, 3, 5), ("LIFRate", 33, 2, 4), ("AdaptiveLIF", 40, 1, 9),
     ("RectifiedLinear", 17, 4, 3), ("SpikingRectifiedLinear", 130, 2, 3), ("Sigmoid", 9, 6, 3),
