@@ -1385,6 +1385,25 @@ def leave_spike_bits(lif_plan, s_start, n):
     return mask, one
 
 
+def _learned_apart(geometry, members, matrices, operands):
+    """Does a launch over the items `members` that writes the matrices of some of them back (`matrices`: item ->
+    span) read and write nothing else that lies in one of these?  Other groups are still running then, and
+    nothing orders them.  (Views of a learned matrix -- other rows or columns of it, a vector in it -- need not
+    have its start and shape.)  `operands`: spans of what the rule reads."""
+    vector = lambda start, n, stride: (start, start + (n - 1) * stride + 1)
+    others = [iv for iv in operands if iv]
+    for b in members:
+        g = geometry[b]
+        others += [vector(g["y_start"], g["y_len"], g["y_stride0"]),
+                   vector(g["y_in_start"], g["y_len"], g["y_in_stride0"])]
+        for d in g["dots"]:
+            others.append(vector(d["x_start"], d["a_shape1"], d["x_stride0"]))
+            if b not in matrices:
+                others.append((d["a_start"], d["a_start"] + (g["y_len"] - 1) * d["a_stride0"] + d["a_shape1"]))
+    spans = sorted(matrices.values())
+    return not _overlaps(others, spans) and all(a[1] <= b[0] for a, b in zip(spans, spans[1:]))
+
+
 def fuse_learning(enc_plan, dec_plan, ew_plan, lf_plan):
     """A step that ends with an outer-product learning rule -- ``W += (alpha e) (x) f`` and
     then ``f <- filter(spikes)`` (the reference: `_plan_SimPES`, simulator.py:1334-1345, with
@@ -1401,7 +1420,8 @@ def fuse_learning(enc_plan, dec_plan, ew_plan, lf_plan):
       read.  Between steps ``f`` then holds the value from before the pending filter step.
 
     Fused when every outer product's matrix is the only matrix of an item of `dec_plan`
-    (same start, shape and row stride; tasks of at most 64 rows; whole aligned quads), its
+    (same start, shape and row stride; tasks of at most 64 rows; whole aligned quads) and nothing else
+    of that launch lies in it, its
     row and column operands are contiguous vectors, every filter of `lf_plan` whose output is
     such a column operand reads exactly the spikes of a population of `enc_plan` and has one
     numerator and at most one denominator coefficient.  The caller checks what only it knows:
@@ -1434,7 +1454,7 @@ def fuse_learning(enc_plan, dec_plan, ew_plan, lf_plan):
             d = g["dots"][0]
             by_matrix[(d["a_start"], g["y_len"], d["a_shape1"], d["a_stride0"])] = b
     tasks = dec_plan.host_tasks
-    learn_of_item = {}
+    learn_of_item, matrices = {}, {}
     for i in range(len(Wm)):
         rows, cols = int(Wm.shape0s[i]), int(Wm.shape1s[i])
         key = (int(Wm.starts[i]), rows, cols, int(Wm.stride0s[i]) if rows > 1 else cols)
@@ -1450,8 +1470,12 @@ def fuse_learning(enc_plan, dec_plan, ew_plan, lf_plan):
             return _learning_apart(6)
         alpha = np.float32(alphas[i])
         learn_of_item[b] = (int(E.starts[i]), int(Fv.starts[i]), int(alpha.view(np.int32)), 1)
+        matrices[b] = _span(Wm, i)
     if not learn_of_item or int(tasks[np.isin(tasks[:, 0], list(learn_of_item)), 2].max()) > WAVE:
         return _learning_apart(7)
+    if not _learned_apart(D.geometry, dec_plan.members, matrices,
+                          [_span(ra, i) for ra in (E, Fv) for i in range(len(ra))]):
+        return _learning_apart(11)
     learn = np.zeros((len(tasks), 4), dtype=np.int32)
     for t, item in enumerate(tasks[:, 0]):
         if int(item) in learn_of_item:
@@ -1582,21 +1606,9 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
             return None
     if F.ptr.value != buf:
         return None
-    # The launch writes a learned matrix back while other groups still run: nothing else that any of them
-    # reads or writes may lie in it.  (Operands that are views of the matrix -- other rows or columns of
-    # it, a vector in it -- need not have its start and shape.)
-    matrices = {b: _span(delta, i) for b, i in rule_of.items()}
-    vector = lambda start, n, stride: (start, start + (n - 1) * stride + 1)
-    others = [_span(ra, i) for ra in (pre, post) + ((aux,) if spec["rule"] == RULE_BCM else ())
-              for i in range(len(ra))]
-    for b in members:
-        g, d = geometry[b], geometry[b]["dots"][0]
-        others += [vector(d["x_start"], d["a_shape1"], 1), vector(g["y_start"], g["y_len"], g["y_stride0"]),
-                   vector(g["y_in_start"], g["y_len"], g["y_in_stride0"])]
-        if b not in rule_of:
-            others.append((d["a_start"], d["a_start"] + (g["y_len"] - 1) * d["a_stride0"] + d["a_shape1"]))
-    spans = sorted(matrices.values())
-    if _overlaps([iv for iv in others if iv], spans) or any(a[1] > b[0] for a, b in zip(spans, spans[1:])):
+    operands = [_span(ra, i) for ra in (pre, post) + ((aux,) if spec["rule"] == RULE_BCM else ())
+                for i in range(len(ra))]
+    if not _learned_apart(geometry, members, {b: _span(delta, i) for b, i in rule_of.items()}, operands):
         return None
 
     per_group = WG // WAVE

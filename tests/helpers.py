@@ -50,6 +50,17 @@ def host_queue(monkeypatch):
         finish=lambda: None, context=contextlib.nullcontext, read=lambda words: words.numpy().copy())
 
 
+def host_simulators(monkeypatch):
+    """Simulators on queues of that kind: their plan lists can be looked at, steps compute nothing."""
+    import torch
+    from nengo_ocl_amd import hipraggedarray
+
+    monkeypatch.setattr(hipraggedarray, "Queue", lambda device=0: host_queue(monkeypatch))
+    for name in ("empty", "zeros"):
+        make = getattr(torch, name)
+        monkeypatch.setattr(torch, name, lambda *a, pin_memory=False, _make=make, **k: _make(*a, **k))
+
+
 def run_plans(plans):
     for p in plans:
         p()

@@ -3,7 +3,7 @@
 import numpy as np
 import pytest
 
-from helpers import RA, host_queue, to_dev
+from helpers import RA, host_queue, host_simulators, to_dev
 
 
 def conv_threads(shape_in, filters, kernel, strides=(1, 1), channels_last=True, conv=True):
@@ -141,3 +141,24 @@ def test_learned_matrices_are_not_written_where_their_launch_reads(monkeypatch, 
                                                                    fused):
     _, result = learned_products(host_queue(monkeypatch), rule, unlearned, learned, aliases)
     assert (result is not None) == fused
+
+
+@pytest.mark.parametrize("rows,fused", [(None, True), (slice(0, 16), False), (slice(31, 32), False),
+                                        (slice(None), False)])
+def test_learned_decoders_are_not_written_where_their_launch_reads(monkeypatch, rows, fused):
+    """The same for decoders learned from an error signal: a second product with some of their rows or with
+    all of them, of other activities."""
+    from nengo_ocl_amd import configs, ir
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    model = configs.c4_pes(1, n_triples=4, n_neurons=1024, dims=32)[0].build_model()
+    if rows is not None:
+        learned = [op.dst for op in model.operators if isinstance(op, ir.Copy) and op.inc
+                   and op.dst.shape == (32, 1024)]
+        x = next(op.X for op in model.operators if isinstance(op, ir.DotInc) and op.A is learned[1])
+        y = ir.Signal(np.zeros(len(range(32)[rows])), name="part")
+        model.add_op(ir.Reset(y))
+        model.add_op(ir.DotInc(learned[0][rows], x, y))
+    with Simulator(None, model=model, seed=1, event_calibration_steps=0) as sim:
+        assert max(getattr(p, "learned_matrices", 0) for p in sim._plans) == (4 if fused else 0)
