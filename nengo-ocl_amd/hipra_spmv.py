@@ -20,6 +20,9 @@ WG, WAVE = 256, 64
 QUAD = 4  # elements of a row stored side by side (one 16-byte access)
 WINDOW = 1024  # consecutive elements of X a wave can keep in LDS (SPMV_WINDOW in csrc/spmv.hip)
 SKIP_MAX_COLS = 32 * 36864  # longest X whose "is not zero" bits fit the LDS (SPMV_MASK_WORDS)
+# ... and beside them the quad of words past the end that the launch for bits of the neurons looks up for
+# padding (nhip_spmv_sell_bits)
+BITS_MAX_COLS = SKIP_MAX_COLS - 128
 # ... and either rows of more than SKIP_MIN_WIDTH stored elements (mean over the slices, padding
 # included), or more than SKIP_MIN_NNZ elements in all: the ordinary launch looks every one of them up
 # in a cache, which gets dearer with the length of X, while the one for spikes has the bits to make
@@ -293,16 +296,24 @@ def spmv_algorithm_heuristic(queue, hA, footprint_hard_limit=0.8, footprint_soft
     return "CSR" if csr_bytes / ell_bytes < soft_limit_ratio else "ELLPACK"
 
 
+def takes_spike_bits(plan):
+    """Lanes per row of the launch that `read_spike_bits` would make of a product that skips the zeros
+    of X, or 0 where that launch does not hold the product: its bits, or its padded elements."""
+    sp, queue = plan.spmv, plan.queue
+    lanes = bits_lanes(sp["n"], (1024 // WAVE) * queue.n_compute_units)
+    elements = WAVE * sum(-(-w // (QUAD * lanes)) * QUAD * lanes for _, _, w, _, _, _ in sp["slice_rows"])
+    return lanes if sp["n_cols"] <= BITS_MAX_COLS and elements < 2 ** 31 else 0
+
+
 def read_spike_bits(plan, mask, one):
     """Make a launch of the product of spikes read their bits from `mask`, where the launch that
-    updates the neurons leaves them (`hipra_gemv.leave_spike_bits`); `one`: the value of a spike."""
+    updates the neurons leaves them (`hipra_gemv.leave_spike_bits`); `one`: the value of a spike.  For
+    a launch that `takes_spike_bits`."""
     sp, queue = plan.spmv, plan.queue
     table, row_len, cols, vals = sp["host"]
-    lanes = bits_lanes(sp["n"], (1024 // WAVE) * queue.n_compute_units)
+    lanes = takes_spike_bits(plan)
     starts, widths, cols, vals, index_bits = bits_layout(sp["slice_rows"], row_len, cols, vals,
                                                          sp["n_cols"], lanes)
-    if vals.size >= 2 ** 31:
-        return
     table = table.copy()
     table[:sp["n"], 0], table[:sp["n"], 1] = starts, widths
     dev = tuple(to_device(queue, a if a.size else np.zeros(4, a.dtype)) for a in (table, cols, vals))

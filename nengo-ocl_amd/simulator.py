@@ -124,8 +124,10 @@ class HipBackend:
 
     def share_spike_bits(self, lif_plan, product_plan):
         """Let the product of a population's spikes read them as bits from the launch that updates
-        its neurons, if that launch can leave them."""
+        its neurons, if that launch can leave them and the product's can take them."""
         sp = product_plan.spmv
+        if not self._spmv.takes_spike_bits(product_plan):
+            return
         bits = lif_plan.__dict__.setdefault("spike_bits", {})
         if sp["x_start"] not in bits:
             bits[sp["x_start"]] = self._gemv.leave_spike_bits(lif_plan, sp["x_start"], sp["n_cols"])

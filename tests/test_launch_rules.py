@@ -162,3 +162,25 @@ def test_learned_decoders_are_not_written_where_their_launch_reads(monkeypatch, 
         model.add_op(ir.DotInc(learned[0][rows], x, y))
     with Simulator(None, model=model, seed=1, event_calibration_steps=0) as sim:
         assert max(getattr(p, "learned_matrices", 0) for p in sim._plans) == (4 if fused else 0)
+
+
+@pytest.mark.parametrize("n_cols,bits", [(1179520, True), (1179521, False), (1179648, False)])
+def test_spikes_are_handed_on_as_bits_where_the_product_holds_them(monkeypatch, n_cols, bits):
+    """On both sides of the longest X of the launch that is handed bits (nhip_spmv_sell_bits refuses longer
+    ones), up to the longest of the one that forms them."""
+    import scipy.sparse
+    from nengo_ocl_amd import hipra_spmv, minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    monkeypatch.setattr(hipra_spmv, "SKIP_MIN_WIDTH", 0)  # (nearly all rows are empty)
+    net = mb.Network(seed=1, solver="surrogate")
+    ens = net.Ensemble(n_cols, 1)
+    weights = scipy.sparse.csr_matrix((np.ones(320), (np.repeat(np.arange(10), 32), np.arange(320) * 3600)),
+                                      shape=(n_cols, n_cols))
+    net.Connection(ens.neurons, ens.neurons, transform=mb.Sparse((n_cols, n_cols), weights),
+                   synapse=mb.Lowpass(0.01))
+    with Simulator(net, seed=1, event_calibration_steps=0) as sim:
+        kerns = [p.kern.__name__ for p in sim._plans]
+    assert ("nhip_spmv_sell_bits" in kerns) == ("nhip_gemv_rows_lif_bits" in kerns) == bits, kerns
+    assert bits or "nhip_spmv_sell_spikes" in kerns

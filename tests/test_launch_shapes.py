@@ -555,10 +555,12 @@ def test_filters_of_second_order_in_the_launch_of_their_input(queue, kind, neuro
 
 
 # waves of sixteen rows and of 64, populations that end inside a wave and inside a word; columns on both
-# sides of 65,536, whole slices (120,000 and 140,000 rows), more columns than 17 bits hold
+# sides of 65,536, whole slices (120,000 and 140,000 rows), more columns than 17 bits hold, as many bits as
+# the LDS holds and one more
 @pytest.mark.parametrize("n,fan_out,lead,bits", [
     (65, 30, 0, True), (2001, 40, 0, True), (1000, 30, 48, True), (1000, 30, 50, False), (33000, 60, 0, True),
-    (70001, 30, 0, True), (120000, 15, 0, True), (140000, 14, 0, True)])
+    (70001, 30, 0, True), (120000, 15, 0, True), (140000, 14, 0, True), (1179520, 2, 0, True),
+    (1179521, 2, 0, False)])
 def test_sparse_products_read_the_bits_their_neurons_left(queue, n, fan_out, lead, bits):
     """A population's spikes reach the sparse products that read them as bits from the launch that
     updates the neurons (not where another population's rows (`lead`) leave them inside a wave), and
