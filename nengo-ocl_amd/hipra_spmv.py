@@ -324,6 +324,7 @@ def read_spike_bits(plan, mask, one):
     plan.args = ((dev[0].ptr, sp["n"], dev[1].ptr, dev[2].ptr, plan.args[6]) + filters
                  + (sp["n_cols"], mask.ptr, float(one), lanes, index_bits))
     plan.full_args = tuple(a for a in plan.full_args if a not in sp["dev"]) + dev + (mask,)
+    sp["dev"], sp["workspaces"] = dev, ()  # (the arrays of the other layout are given back)
     plan.gsize = (1024 * min(queue.n_compute_units, lanes * sp["n"])
                   + (plan.gsize[0] - 1024 * min(queue.n_compute_units, 4 * sp["n"])),)
     plan.stored_bytes = 4 * int(cols.size + vals.size)

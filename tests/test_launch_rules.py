@@ -184,3 +184,34 @@ def test_spikes_are_handed_on_as_bits_where_the_product_holds_them(monkeypatch, 
         kerns = [p.kern.__name__ for p in sim._plans]
     assert ("nhip_spmv_sell_bits" in kerns) == ("nhip_gemv_rows_lif_bits" in kerns) == bits, kerns
     assert bits or "nhip_spmv_sell_spikes" in kerns
+
+
+@pytest.mark.parametrize("synapse", ["Alpha", "Lowpass"])
+def test_one_copy_of_a_sparse_matrix_stays_on_the_device(monkeypatch, synapse):
+    """A product that is handed bits keeps its own layout of the matrix and gives the other one back."""
+    import gc
+    import weakref
+
+    from nengo_ocl_amd import configs, hipra_spmv, minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    made, upload = [], hipra_spmv.to_device
+
+    def to_device(queue, array):
+        made.append(upload(queue, array))
+        return made[-1]
+
+    monkeypatch.setattr(hipra_spmv, "to_device", to_device)
+    net = mb.Network(seed=1)
+    ens = net.Ensemble(2001, 1)
+    weights = configs.sparse_ring_weights(2001, 40, 0.3, np.random.RandomState(4), scale=2e-4)
+    net.Connection(ens.neurons, ens.neurons, transform=mb.Sparse((2001, 2001), weights),
+                   synapse=getattr(mb, synapse)(0.01))
+    with Simulator(net, seed=1, event_calibration_steps=0) as sim:
+        product, = [p for p in sim._plans if p.kern.__name__ == "nhip_spmv_sell_bits"]
+        made = [weakref.ref(a) for a in made]
+        gc.collect()
+        alive = [r() for r in made if r() is not None]
+        assert alive and len(alive) < len(made)
+        assert all(any(a is kept for kept in product.full_args) for a in alive)
