@@ -45,12 +45,13 @@ class _Image:
         address = ptr if isinstance(ptr, int) else int(ptr.value)
         if address % 16:
             raise _Unfit("an array that does not start on 16 bytes")
+        end = address + 4 * words
         for start, (n, lds, _) in self.spans.items():
-            if start <= address < start + 4 * n:
-                if address + 4 * words > start + 4 * n:
-                    raise _Unfit("overlapping arrays")
+            if start <= address and end <= start + 4 * n and address < start + 4 * n:
                 self.spans[start][2] |= write_back
                 return lds + (address - start) // 4
+            if address < start + 4 * n and start < end:  # (two copies, one of which would go stale)
+                raise _Unfit("overlapping arrays")
         lds = self.words
         self.spans[address] = [int(words), lds, bool(write_back)]
         self.words += -(-int(words) // 4) * 4

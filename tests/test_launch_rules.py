@@ -215,3 +215,20 @@ def test_one_copy_of_a_sparse_matrix_stays_on_the_device(monkeypatch, synapse):
         alive = [r() for r in made if r() is not None]
         assert alive and len(alive) < len(made)
         assert all(any(a is kept for kept in product.full_args) for a in alive)
+
+
+# words before, inside and behind an array of 32 words at word 64
+@pytest.mark.parametrize("first,words,where", [(64, 32, 0), (72, 8, 8), (88, 8, 24), (32, 32, 32), (96, 4, 32),
+                                               (60, 8, None), (32, 33, None), (60, 100, None), (92, 8, None),
+                                               (88, 9, None)])
+def test_arrays_of_a_resident_network_have_one_copy(first, words, where):
+    """An array inside another one is found there, one that reaches over its start or end is refused."""
+    from nengo_ocl_amd import hipra_resident
+
+    image = hipra_resident._Image(None)
+    assert image.add(4 * 64, 32) == 0
+    if where is None:
+        with pytest.raises(hipra_resident._Unfit):
+            image.add(4 * first, words)
+    else:
+        assert image.add(4 * first, words) == where
