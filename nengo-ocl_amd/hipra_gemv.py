@@ -124,6 +124,14 @@ THIN_CLASS, THIN_MAX_COLS = (2, 4, 1), 4
 # 256 x 100 12.06 -> 10.65, 300 x 150 13.0 -> 10.9, 1,000 x 64 13.4 -> 10.6. Below these rows the launch is
 # a few waves either way.
 SUM_PARTS_FOR_WAVE_TASKS, SUM_MIN_ROWS_FOR_WAVE_TASKS = 3, 3000
+# Products beside those with learned matrices in their launch (`fuse_hebbian`): a group of four rows there costs
+# 0.011 us whatever its columns (its LDS holds passes of LEARN_PASS_COLS), a launch of their own 2.7 us for items of
+# at most THIN_MAX_COLS columns, 3.5-4.0 up to 500, 6.7 for 3,000. So they ride up to a group per compute unit, 1.5
+# of wider items, two of items that fill a pass. Whole steps beside Oja's rule on 300 x 300, riding / apart: 1,000 x
+# 4 12.6 / 12.4, 1,500 x 4 13.8 / 12.4, 100,000 x 2 299 / 16; 1,000 x 64 12.2 / 13.6, 1,500 x 64 13.6 / 13.7, 4,000 x 64
+# 20.8 / 13.7; 2,000 x 500 15.0 / 14.1; 2,000 x 3,000 16.5 / 16.6; on 2000 x 2000: 1,500 x 4 22.1 / 20.8, 1,500 x 64
+# 21.7 / 22.5, 4,000 x 64 28.4 / 22.7, 2,000 x 3,000 24.7 / 25.7
+LEARN_RIDING_GROUPS, LEARN_PASS_COLS = 1, 2048
 LIF_POP_ENABLED, LIF_POP_DECAY, LIF_POP_NO_J = 1 << 8, 1 << 9, 1 << 10  # flag bits of a population row
 LIF_POP_MASK = 1 << 12
 LIF_POP_BITS = 1 << 11  # spikes stored as a bit per neuron (see `store_spikes_as_bits`)
@@ -1555,10 +1563,12 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
 
     Fused when every item of `products` has one dot product with operands of stride 1, every matrix of the
     rule is the matrix of one such item (same start, shape and row stride), its row operand is contiguous, and
-    nothing else the launch reads or writes lies in such a matrix.  Filters of `lf_plan` with one numerator and at most one denominator coefficient on
-    contiguous vectors move; the caller has checked that nothing between the plans, and nothing the plans
-    read or write themselves, keeps the rule and those filters out of the products' launch.  Returns ``(plan,
-    plans for the filters that stay, filters that moved)`` or None."""
+    nothing else the launch reads or writes lies in such a matrix.  Items without a learned matrix are part of
+    the launch while they are few (`LEARN_RIDING_GROUPS`).  Filters of `lf_plan` with one numerator and at most
+    one denominator coefficient on contiguous vectors move; the caller has checked that nothing between the
+    plans, and nothing the plans read or write themselves, keeps the rule and those filters out of the
+    products' launch.  Returns ``(plan, plans in front of it for the products that are not part of it, plans
+    for the filters that stay, filters that moved)`` or None."""
     from .hipra_nonlinearities import RULE_BCM, RULE_OJA, plan_linearfilter
 
     spec = rule_plan.rule_spec
@@ -1602,10 +1612,35 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
             if item_targets is not None and plan.filter_tables[0] is not item_targets:
                 return None
             item_targets, dev_targets, F, _ = plan.filter_tables
+            filtered = plan
         elif plan.name.endswith("_filter"):
             return None
     if F.ptr.value != buf:
         return None
+    # What else the GEMV multiplies by rides along while it is little; the rest keeps a launch (in front, where
+    # it reads the matrices as they were).
+    def groups(items):
+        cols = np.array([geometry[b]["dots"][0]["a_shape1"] for b in items])
+        weight = np.where(cols <= THIN_MAX_COLS, 1.0, np.where(cols < LEARN_PASS_COLS, 2 / 3, 0.5))
+        return float(sum(-(-geometry[b]["y_len"] // (WG // WAVE)) * w for b, w in zip(items, weight)))
+
+    limit = LEARN_RIDING_GROUPS * queue.n_compute_units
+    kept, riding = [], []
+    for p in sorted(products, key=lambda p: rule_of.keys().isdisjoint(p.members)):  # those with learned ones first
+        beside = [b for b in p.members if b not in rule_of]
+        if groups(riding) + groups(beside) <= limit:
+            riding += beside
+        elif len(beside) == len(p.members):
+            kept.append(p)
+        else:
+            apart = prog._build(beside)
+            if item_targets is not None:
+                if any(item_targets[q.members, 1].any() and not _takes_filters(q) for q in apart):
+                    return None
+                apart = [filtered.with_filters(q) for q in apart]
+            kept += apart
+    products = [p for p in products if p not in kept]
+    members = [b for p in products for b in p.members if b in rule_of or b in riding]
     operands = [_span(ra, i) for ra in (pre, post) + ((aux,) if spec["rule"] == RULE_BCM else ())
                 for i in range(len(ra))]
     if not _learned_apart(geometry, members, {b: _span(delta, i) for b, i in rule_of.items()}, operands):
@@ -1668,7 +1703,7 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
         residual = plan_linearfilter(queue, S[rest], T[rest], A[rest], B[rest], lf_plan.lf_spec["Xbuf"][rest],
                                      lf_plan.lf_spec["Ybuf"][rest], tag=lf_plan.tag)
         residual[0].unfused_items = list(rest)
-    return plan, residual, moved
+    return plan, kept, residual, moved
 
 
 def _read_spans(prog, ptr_value):
@@ -1801,11 +1836,11 @@ def fuse_linearfilter(gemv_plans, lf_plan, second_order=False):
     dev_targets = to_device(queue, targets)
     order = 2 if second else 1
     extra = (dev_items.ptr, dev_targets.ptr, F.ptr, order)
-    out = []
-    for plan in gemv_plans:
+
+    def with_filters(plan):
+        """A launch over items of the GEMV, with the filters that these items feed"""
         if not _takes_filters(plan) or not any(b in targets_of for b in plan.members):
-            out.append(plan)
-            continue
+            return plan
         f_bytes = sum(8 * int(Y.shape0s[b]) * len(targets_of[b]) for b in plan.members
                       if b in targets_of)  # filter state in and out
         if plan.kernel_class[0] == 4:
@@ -1831,8 +1866,7 @@ def fuse_linearfilter(gemv_plans, lf_plan, second_order=False):
             fused.event_record_item = plan.event_record_item
             fused.host_tasks = None
             _keep_filter_state(fused, filter_state)
-            out.append(fused)
-            continue
+            return fused
         entry, args, keep = _epilogue_call(
             lib, plan, "filter",
             lambda items: np.column_stack([item_targets[items], np.zeros(len(items), np.int32)]))
@@ -1857,10 +1891,12 @@ def fuse_linearfilter(gemv_plans, lf_plan, second_order=False):
         fused.gemv_bytes = plan.bw_per_call
         if plan.kernel_class[0] == 3:
             fused.host_tasks = tasks
-        fused.filter_tables = (item_targets, dev_targets, F, targets)
+        fused.filter_tables, fused.with_filters = (item_targets, dev_targets, F, targets), with_filters
         fused.host_tables = plan.host_tables
         _keep_filter_state(fused, filter_state)
-        out.append(fused)
+        return fused
+
+    out = [with_filters(plan) for plan in gemv_plans]
     residual = []
     if rest:
         residual = plan_linearfilter(queue, X[rest], F[rest], A[rest], B[rest],

@@ -938,7 +938,6 @@ class Simulator:
         is_product = lambda p: (getattr(p, "name", "") in names and hasattr(p, "prog")
                                 and getattr(p, "kernel_class", (None,))[0] in (2, 3)
                                 and getattr(p, "learned_matrices", 0) == 0)
-        group = lambda r, w: type("Moved", (), {"reads_mem": r, "writes_mem": w})
         plans = list(plans)
         r = 0
         while r < len(plans):
@@ -971,22 +970,24 @@ class Simulator:
             result = self.backend.fuse_hebbian(products, rule, lf if movable else None)
             if result is None:
                 continue
-            plan, residual, moved = result
+            plan, kept, residual, moved = result
             plan.reads_mem, plan.writes_mem = reads | rule.reads_mem, writes | rule.writes_mem
+            for p in kept:
+                p.reads_mem, p.writes_mem = reads, writes
             if moved:
-                kept = [op for k, op in enumerate(ops) if k not in set(moved)]
+                rest = [op for k, op in enumerate(ops) if k not in set(moved)]
                 plan.reads_mem |= {ops[k].input.base for k in moved}
                 plan.writes_mem |= {ops[k].output.base for k in moved}
                 for p in residual:
-                    p.reads_mem = {op.input.base for op in kept}
-                    p.writes_mem = {op.output.base for op in kept}
-                    p.planned_ops = kept
+                    p.reads_mem = {op.input.base for op in rest}
+                    p.writes_mem = {op.output.base for op in rest}
+                    p.planned_ops = rest
                     self._filter_positions.append(p.bufpos)
                 plans[f:f + 1] = residual
             carried = CarriedPlan(rule.queue, name=rule.name, tag="in %s" % plan.tag)
             plans[r - 1] = carried
-            plans[i:j + 1] = [plan]
-            r = i + 1
+            plans[i:j + 1] = kept + [plan]  # (what stays reads the matrices before they change)
+            r = i + len(kept) + 1
         return plans
 
     @staticmethod

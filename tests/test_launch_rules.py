@@ -232,3 +232,44 @@ def test_arrays_of_a_resident_network_have_one_copy(first, words, where):
             image.add(4 * first, words)
     else:
         assert image.add(4 * first, words) == where
+
+
+def rule_beside_products(n, extra, rule="Oja", synapses=("Lowpass",)):
+    """Two populations of n neurons with a learned matrix between them; `extra`: (rows, neurons) of products
+    of other populations in the same step."""
+    from nengo_ocl_amd import minibuilder as mb
+
+    rng = np.random.RandomState(1)
+    net = mb.Network(seed=5, solver="surrogate")
+    stim = net.Node(mb.WhiteSignal(period=0.5, high=6.0, seed=3), size_out=2)
+    pre, post = net.Ensemble(n, 2), net.Ensemble(n, 2)
+    net.Connection(stim, pre, synapse=mb.Lowpass(0.005))
+    learning = mb.Oja(learning_rate=1e-6, beta=0.7) if rule == "Oja" else mb.BCM(learning_rate=1e-9)
+    net.Connection(pre.neurons, post.neurons, transform=rng.normal(scale=1e-1 / n, size=(n, n)),
+                   learning_rule=learning, synapse=mb.Lowpass(0.005))
+    for k, (rows, cols) in enumerate(extra):
+        other = net.Ensemble(cols, 2)
+        net.Connection(stim, other, synapse=mb.Lowpass(0.005))
+        net.Connection(other.neurons, net.Node(None, size_in=rows), transform=rng.normal(size=(rows, cols)),
+                       synapse=getattr(mb, synapses[k % len(synapses)])(0.005))
+    return net
+
+
+# rows and columns of the others on both sides of what rides along: at most four columns, more, whole passes;
+# in the class of the learned matrix (300 x 300, 50 x 50) and in another
+@pytest.mark.parametrize("n,extra,rides", [
+    (300, [(1024, 4)], True), (300, [(1028, 4)], False), (300, [(100000, 2)], False), (300, [(1536, 64)], True),
+    (300, [(1540, 64)], False), (300, [(2, 300)] * 16, True), (300, [(2048, 3000)], True),
+    (300, [(2052, 3000)], False), (50, [(20, 50)] * 76, True), (50, [(20, 50)] * 77, False),
+    (300, [(1028, 4), (1536, 64)], None)])
+def test_few_other_products_ride_with_learned_matrices(monkeypatch, n, extra, rides):
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    with Simulator(rule_beside_products(n, extra), seed=1, event_calibration_steps=0) as sim:
+        learn, = [p for p in sim._plans if getattr(p, "learned_matrices", 0)]
+        at = list(sim._plans).index(learn)
+        front = [p for p in list(sim._plans)[:at] if p.name.endswith("_filter")]
+    groups = [-(-rows // 4) for rows, _ in extra]
+    assert learn.n_tasks == -(-n // 4) + (groups[1] if rides is None else sum(groups) if rides else 0)
+    assert len(front) == (0 if rides else 1)

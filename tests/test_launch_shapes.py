@@ -681,6 +681,28 @@ def test_products_with_a_part_of_a_learned_matrix_read_it_unchanged(queue, rule,
             assert np.array_equal(gpu.signal_buffer().view(np.uint32), cpu.signal_buffer().view(np.uint32))
 
 
+@pytest.mark.parametrize("rule", ["Oja", "BCM"])
+@pytest.mark.parametrize("n,extra,synapses", [
+    (300, [(1028, 4)], ["Lowpass"]), (300, [(1540, 64)], ["Lowpass"]), (50, [(20, 50)] * 77, ["Lowpass", "Alpha"]),
+    (301, [(1541, 63), (3, 301)], ["Alpha"]), (300, [(1030, 3), (1024, 64)], ["Lowpass", "Alpha"])])
+def test_products_apart_from_the_launch_of_learned_matrices(queue, rule, n, extra, synapses):
+    """Too many other products for that launch: they keep their filters, of first and second order, in a launch
+    in front of it."""
+    from test_launch_rules import rule_beside_products
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    nets = [rule_beside_products(n, extra, rule, synapses) for _ in range(2)]
+    with Simulator(nets[0], seed=1, event_calibration_steps=0) as gpu, OracleSimulator(nets[1], seed=1) as cpu:
+        learn = next(k for k, p in enumerate(gpu._plans) if getattr(p, "learned_matrices", 0))
+        assert any(p.name.endswith("_filter") for p in list(gpu._plans)[:learn])
+        cpu.run_steps(30)
+        for _ in range(2):  # the second time from a reset: the filters' states with it
+            gpu.run_steps(30)
+            assert np.array_equal(gpu.signal_buffer().view(np.uint32), cpu.signal_buffer().view(np.uint32))
+            gpu.reset()
+
+
 @pytest.mark.parametrize("kind,neurons,dims,ensembles", [
     ("LIF", 100, 1, 2), ("LIF", 30, 1, 2), ("LIF", 65, 3, 5), ("LIFRate", 33, 2, 4), ("AdaptiveLIF", 40, 1, 9),
     ("RectifiedLinear", 17, 4, 3), ("SpikingRectifiedLinear", 130, 2, 3), ("Sigmoid", 9, 6, 3),
