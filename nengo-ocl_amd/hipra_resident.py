@@ -19,8 +19,8 @@ ROWS4, ROWS1, LONG = 16, 32, 48  # kinds of csrc/resident.hip, + epilogue
 LIF, DECODE, FILTER = 64, 65, 66
 EPI_NONE, EPI_LIF, EPI_NEURON, EPI_FILTER = 0, 1, 3, 4
 MAX_STEPS = 4096  # steps of one launch
-# us of a step that one short launch of a replayed graph takes (two launches: 8.1-8.8 us for two populations,
-# 11-13 for networks of a few thousand neurons)
+# us of a step that one short launch of a replayed graph takes (two launches: 8.4-8.9 us for two populations,
+# 10.6-11.5 for networks of a few thousand neurons)
 GRAPH_LAUNCH = 4.2
 
 OP_DTYPE = np.dtype([("kind", "<i4"), ("n_tasks", "<i4"), ("first", "<i4"), ("last", "<i4"),
@@ -178,7 +178,9 @@ def _rows_ops(image, plan, sig_ptr, sig_lds):
         if kind == DECODE:
             cost = 0.5 + 0.006 * max(t[2] for t in tasks)
         elif kind == LIF:
-            cost = 0.75 + (0.6 + 0.03 * max(t[19] for t in tasks) if max(t[19] for t in tasks) else 0.0)
+            # (alone 0.75, without sums; where every wave has some the two of a SIMD slow each other)
+            n_parts = max(t[19] for t in tasks)
+            cost = 1.35 + 0.03 * n_parts if n_parts else 0.93
         else:
             cost = (2.8 if epi == EPI_NEURON else 1.5) if kind == ROWS1 else 1.25
         out.append((row, cost))
@@ -344,8 +346,11 @@ def resident_program(queue, plans, all_data, n_launches):
     """`Resident` for the plan list of a step -- (plan, memory it reads, memory it writes) before short plans
     are merged and carried --, or None where it holds a plan of a kind the resident launch does not hold,
     does not fit the LDS, or would not be shorter than `n_launches` launches of a graph: by the costs
-    of the operations alone in their wave, measured (csrc/resident.hip; the estimates of eight networks between
-    2.4 and 14 us lie within 16 % above and 13 % below what they take)."""
+    of the operations in their wave, measured (csrc/resident.hip; the estimates of 28 networks between
+    2.6 and 12.3 us lie at most 22 % above and 10 % below what they take).  Near the limit, with the launches of
+    a graph beside it: two populations of 1,408 neurons 8.3 us a step (8.5), of 1,500 9.2 (8.8), four of 300 x 2
+    with second-order synapses 8.5 (9.3), of 400 x 2 9.9 (9.7).  What copying the image in and out adds to a
+    call needs no term: a call of one step takes 31 us with 8 KB of it and 40 with 100, a graph's 46-53."""
     memory = [(r, w) for _, r, w in plans]
     plans = [p for p, _, _ in plans]
     if not plans or not all(isinstance(p, Plan) for p in plans):

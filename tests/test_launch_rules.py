@@ -273,3 +273,21 @@ def test_few_other_products_ride_with_learned_matrices(monkeypatch, n, extra, ri
     groups = [-(-rows // 4) for rows, _ in extra]
     assert learn.n_tasks == -(-n // 4) + (groups[1] if rides is None else sum(groups) if rides else 0)
     assert len(front) == (0 if rides else 1)
+
+
+# both sides of the limit: two populations (times beside `resident_program`), many small ones, large ones
+@pytest.mark.parametrize("what,neurons,resident", [
+    ("pair", 30, True), ("pair", 1000, True), ("pair", 1408, True), ("pair", 1500, False), ("pair", 2000, False),
+    ("pair", 2500, False), ("graph", 50, True), ("graph", 150, False)])
+def test_networks_run_resident_where_that_is_shorter(monkeypatch, what, neurons, resident):
+    from nengo_ocl_amd import configs
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    if what == "pair":
+        net = configs.c0_readme(5, n_neurons=neurons)[0]
+    else:
+        net = configs.c2_watts_strogatz(5, n_ens=16, n_neurons=neurons, n_driven=1)[0]
+        net.n_eval_points = 300
+    with Simulator(net, seed=1, event_calibration_steps=0) as sim:
+        assert (sim._plans.resident is not None) == resident
