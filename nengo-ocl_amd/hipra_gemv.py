@@ -1795,34 +1795,35 @@ def fuse_linearfilter(gemv_plans, lf_plan, second_order=False):
                     large[(int(Y.starts[b]), int(Y.shape0s[b]))] = b
     if not large:
         return None
-    a_host, b_host = A.to_host(), B.to_host()
-    targets_of = defaultdict(list)
-    rest = []
-    second = {}  # filter -> (b1 or None, a1 or None): two coefficients on a side
+    item_of = {}
     for i in range(len(X)):
         most = 2 if second_order else 1
         simple = 1 <= int(B.shape0s[i]) <= most and int(A.shape0s[i]) <= most
         vector = (int(X.shape1s[i]) == 1 and int(X.stride0s[i]) == 1
                   and int(F.shape1s[i]) == 1 and int(F.stride0s[i]) == 1)
         b = large.get((int(X.starts[i]), int(X.shape0s[i]))) if simple and vector else None
-        if b is None:
-            rest.append(i)
-            continue
+        if b is not None:
+            item_of[i] = b
+    # (what a filter writes must be nothing that the launch reads or writes: one that does stays behind)
+    touched = _read_spans(prog, F.ptr.value)
+    if F.ptr.value == Y.ptr.value:
+        touched += [iv for iv in (_span(Y, b) for b in range(len(Y))) if iv]
+    written = {i: _span(F, i) for i in item_of if _span(F, i)}
+    if _overlaps(list(written.values()), touched):
+        item_of = {i: b for i, b in item_of.items() if i not in written or not _overlaps([written[i]], touched)}
+    if not item_of:
+        return None
+    rest = [i for i in range(len(X)) if i not in item_of]
+    a_host, b_host = A.to_host(), B.to_host()
+    targets_of = defaultdict(list)
+    second = {}  # filter with two coefficients on a side -> number of its record
+    for i, b in item_of.items():
         na = int(A.shape0s[i])
         a0 = np.float32(a_host[i][0, 0]) if na else np.float32(0)
         b0 = np.float32(b_host[i][0, 0])
         if na > 1 or int(B.shape0s[i]) > 1:
             second[i] = len(second)
         targets_of[b].append((int(F.starts[i]), int(a0.view(np.int32)), int(b0.view(np.int32)), na, i))
-    if not targets_of:
-        return None
-    fused_filters = [i for i in range(len(X)) if i not in set(rest)]
-    written = [iv for iv in (_span(F, i) for i in fused_filters) if iv]
-    if _overlaps(written, _read_spans(prog, F.ptr.value)):
-        return None
-    if F.ptr.value == Y.ptr.value and _overlaps(
-            written, [iv for iv in (_span(Y, b) for b in range(len(Y))) if iv]):
-        return None
 
     item_targets = np.zeros((len(Y), 2), dtype=np.int32)
     target_rows = []

@@ -291,3 +291,15 @@ def test_networks_run_resident_where_that_is_shorter(monkeypatch, what, neurons,
         net.n_eval_points = 300
     with Simulator(net, seed=1, event_calibration_steps=0) as sim:
         assert (sim._plans.resident is not None) == resident
+
+
+def test_synapses_that_their_product_reads_leave_the_others_in_its_launch(monkeypatch):
+    """Among the synapses of one launch are some whose outputs the products read that feed the others."""
+    from nengo_ocl_amd.simulator import Simulator
+    from random_networks import random_network
+
+    host_simulators(monkeypatch)
+    model = random_network(5, big=True, sliced=False, rich=True)[0].build_model()
+    with Simulator(None, model=model, seed=1, event_calibration_steps=0) as sim:
+        launches = [p.kern.__name__ for p in sim._plans if hasattr(p, "kern")]
+    assert {"nhip_gemv_rows_filter", "nhip_gemv_tile_filter"} <= set(launches), launches
