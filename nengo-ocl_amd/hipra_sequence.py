@@ -245,6 +245,22 @@ def _can_carry_more(plan, seq, needs):
     return plan.name not in ("hipra_gemv.events", "hipra_gemv.events_filter") or (needs | carried.needs) == 0
 
 
+def carrier_of(plans, k, seq):
+    """Index of the launch that can take `seq` (a sequence or a short plan, at `plans[k]` or meant for that place):
+    the nearest one, backwards then forwards, over plans that touch none of its memory (moving past those
+    changes nothing); None where there is none, or it is not short."""
+    if getattr(seq, "name", "") != "hip_sequence" and not (hasattr(seq, "enqueue") and is_small(seq)):
+        return None
+    needs = seq.needs if seq.name == "hip_sequence" else sequence_needs([seq])
+    for step in (-1, 1):
+        q = k + step
+        while 0 <= q < len(plans) and hasattr(plans[q], "enqueue") and not _conflict(seq, plans[q]):
+            if _can_carry(plans[q], needs) or (step < 0 and _can_carry_more(plans[q], seq, needs)):
+                return q
+            q += step
+    return None
+
+
 def carry_sequences(plans):
     """Sequence launches (and single small plans) next to a large-item GEMV launch that
     touches none of their memory ride in that launch, in work-groups of their own
@@ -254,24 +270,7 @@ def carry_sequences(plans):
     k = 0
     while k < len(plans):
         seq = plans[k]
-        rides = getattr(seq, "name", "") == "hip_sequence" or (
-            hasattr(seq, "enqueue") and is_small(seq))
-        if not rides:
-            k += 1
-            continue
-        needs = seq.needs if seq.name == "hip_sequence" else sequence_needs([seq])
-        # the nearest launch that can take it, backwards then forwards, over plans that touch
-        # none of its memory (moving past those changes nothing)
-        j = None
-        for step in (-1, 1):
-            q = k + step
-            while 0 <= q < len(plans) and hasattr(plans[q], "enqueue") and not _conflict(seq, plans[q]):
-                if _can_carry(plans[q], needs) or (step < 0 and _can_carry_more(plans[q], seq, needs)):
-                    j = q
-                    break
-                q += step
-            if j is not None:
-                break
+        j = carrier_of(plans, k, seq)
         if j is None:
             k += 1
             continue

@@ -293,6 +293,33 @@ def test_networks_run_resident_where_that_is_shorter(monkeypatch, what, neurons,
         assert (sim._plans.resident is not None) == resident
 
 
+def pes_with_synapses(synapse, n=512, dims=32):
+    """Learned decoders, and a probe with a synapse of second or third order."""
+    from nengo_ocl_amd import configs, minibuilder as mb
+
+    net = configs.c4_pes(1, n_triples=2, n_neurons=n, dims=dims)[0]
+    if synapse == "Alpha":
+        net.Probe(net.ensembles[0].neurons, synapse=mb.Alpha(0.01))
+    else:
+        net.Probe(net.ensembles[0], synapse=mb.LinearFilter([0.1], [1.0, -0.7, 0.2, 0.1], analog=False))
+    return net
+
+
+# spikes of an ensemble behind a second-order synapse (a short launch, which rides, or a long one), a
+# decoded value behind one of third order (which would need a launch)
+@pytest.mark.parametrize("synapse,n,dims,fused", [
+    ("Alpha", 200, 2, True), ("Alpha", 512, 32, True), ("Alpha", 3000, 2, False), ("third order", 512, 32, False)])
+def test_synapses_of_higher_order_leave_the_others_their_launch(monkeypatch, synapse, n, dims, fused):
+    """Synapses of every class share a launch; one of higher order in it does not keep the activities' filters
+    out of the launch of the weights they change, where it finds another to ride in."""
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    with Simulator(pes_with_synapses(synapse, n, dims), seed=1, event_calibration_steps=0) as sim:
+        launches = [p.kern.__name__ for p in sim._plans]
+    assert ("nhip_outer_filter" in launches) == fused and ("nhip_elementwise_inc" in launches) != fused, launches
+
+
 def test_synapses_that_their_product_reads_leave_the_others_in_its_launch(monkeypatch):
     """Among the synapses of one launch are some whose outputs the products read that feed the others."""
     from nengo_ocl_amd.simulator import Simulator

@@ -703,6 +703,26 @@ def test_products_apart_from_the_launch_of_learned_matrices(queue, rule, n, extr
             gpu.reset()
 
 
+@pytest.mark.parametrize("synapse", ["Alpha", "third order"])
+@pytest.mark.parametrize("n,dims", [(200, 2), (512, 32), (1031, 3)])
+def test_synapses_of_every_order_beside_learned_decoders(queue, synapse, n, dims):
+    """The launch of a step's synapses is taken apart: some ride in a product's launch, the activities' in that
+    of the weights, the others keep one; from the start and from a reset."""
+    from test_launch_rules import pes_with_synapses
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    nets = [pes_with_synapses(synapse, n, dims) for _ in range(2)]
+    with Simulator(nets[0], seed=1, event_calibration_steps=0) as gpu, OracleSimulator(nets[1], seed=1) as cpu:
+        cpu.run_steps(40)
+        for _ in range(2):
+            gpu.run_steps(40)
+            for p, p_o in zip(nets[0].probes, nets[1].probes):
+                assert np.array_equal(gpu.data[p], cpu.data[p_o])
+            assert np.array_equal(gpu.signal_buffer().view(np.uint32), cpu.signal_buffer().view(np.uint32))
+            gpu.reset()
+
+
 @pytest.mark.parametrize("kind,neurons,dims,ensembles", [
     ("LIF", 100, 1, 2), ("LIF", 30, 1, 2), ("LIF", 65, 3, 5), ("LIFRate", 33, 2, 4), ("AdaptiveLIF", 40, 1, 9),
     ("RectifiedLinear", 17, 4, 3), ("SpikingRectifiedLinear", 130, 2, 3), ("Sigmoid", 9, 6, 3),
