@@ -350,7 +350,8 @@ int nhip_resident(void *stream, const void *spans, int n_spans, const void *ops,
  * rules read, in one launch: replaces `plan_block_gemv` + `plan_linearfilter` + `plan_bcm` / `plan_oja`
  * with the copy that adds the change (clra_nonlinearities.py:2082-2277) + `plan_linearfilter`, in that
  * order.  One dot product per item, reference order; X may not overlap what the launch writes, except by
- * the outputs of `filters`.
+ * the outputs of `filters`, and nothing but the item and the rule of a learned matrix may read any part of it
+ * here: other groups write it back while theirs still run.
  *   tasks   : int32[n_tasks][24] {a_start, a_stride0, N, x_start, y_start, y_stride0, yin_start,
  *             yin_stride0, alpha, beta, gamma (float bits), row0, n_rows (1..4), learned (0: the matrix
  *             stays), first_target, n_targets, then the rule: kind, pre_start, post_start, post_stride0,

@@ -7,6 +7,23 @@
 #include "gemv_types.h"
 #include "neuron_math.h"
 
+// Element q of lane p of a quad of lanes and element p of lane q change places (all four lanes are active).
+__device__ __forceinline__ void transpose_quad(float4& v, int lane) {
+    constexpr int XOR1 = 0xB1, XOR2 = 0x4E;  // quad_perm [1,0,3,2] and [2,3,0,1]
+#define NHIP_QUAD(x, ctrl) __int_as_float(__builtin_amdgcn_update_dpp( \
+    0, __float_as_int(x), ctrl, 0xF, 0xF, true))
+    const bool b0 = lane & 1, b1 = lane & 2;
+    // (every exchange before its choice: a lane that is switched off gives nothing)
+    const float x1 = NHIP_QUAD(v.x, XOR1), y1 = NHIP_QUAD(v.y, XOR1), z1 = NHIP_QUAD(v.z, XOR1), w1 = NHIP_QUAD(v.w, XOR1);
+    const float a0 = b0 ? y1 : v.x, a1 = b0 ? v.y : x1, a2 = b0 ? w1 : v.z, a3 = b0 ? v.w : z1;
+    const float x2 = NHIP_QUAD(a0, XOR2), y2 = NHIP_QUAD(a1, XOR2), z2 = NHIP_QUAD(a2, XOR2), w2 = NHIP_QUAD(a3, XOR2);
+    v.x = b1 ? z2 : a0;
+    v.y = b1 ? w2 : a1;
+    v.z = b1 ? a2 : x2;
+    v.w = b1 ? a3 : y2;
+#undef NHIP_QUAD
+}
+
 // ---------------------------------------------------------------- reference order, small items
 // One output row per task (task = {item, row, 1, 0}); a wave takes 64 / LPR
 // consecutive tasks, LPR lanes each, whatever items they belong to -- thousands of
@@ -41,23 +58,6 @@
 // row; here the record is the wave's: every lane reads the same addresses for the task, the
 // item's dot products, its population and its input sum, and the parts of an input sum are
 // fetched by the lanes side by side instead of in rounds.
-// Element q of lane p of a quad of lanes and element p of lane q change places (all four lanes are active).
-__device__ __forceinline__ void transpose_quad(float4& v, int lane) {
-    constexpr int XOR1 = 0xB1, XOR2 = 0x4E;  // quad_perm [1,0,3,2] and [2,3,0,1]
-#define NHIP_QUAD(x, ctrl) __int_as_float(__builtin_amdgcn_update_dpp( \
-    0, __float_as_int(x), ctrl, 0xF, 0xF, true))
-    const bool b0 = lane & 1, b1 = lane & 2;
-    // (every exchange before its choice: a lane that is switched off gives nothing)
-    const float x1 = NHIP_QUAD(v.x, XOR1), y1 = NHIP_QUAD(v.y, XOR1), z1 = NHIP_QUAD(v.z, XOR1), w1 = NHIP_QUAD(v.w, XOR1);
-    const float a0 = b0 ? y1 : v.x, a1 = b0 ? v.y : x1, a2 = b0 ? w1 : v.z, a3 = b0 ? v.w : z1;
-    const float x2 = NHIP_QUAD(a0, XOR2), y2 = NHIP_QUAD(a1, XOR2), z2 = NHIP_QUAD(a2, XOR2), w2 = NHIP_QUAD(a3, XOR2);
-    v.x = b1 ? z2 : a0;
-    v.y = b1 ? w2 : a1;
-    v.z = b1 ? a2 : x2;
-    v.w = b1 ? a3 : y2;
-#undef NHIP_QUAD
-}
-
 template <int LPR, int EPI = EPI_NONE, bool WIDE = false, bool WAVE_TASK = false>
 __device__ __forceinline__ void gemv_rows_ref_block(
     const GemvItem* __restrict__ items, const float4* __restrict__ coefs,
@@ -66,6 +66,7 @@ __device__ __forceinline__ void gemv_rows_ref_block(
     const EpilogueArgs* epi = nullptr)
 {
     constexpr int TILE = 128;
+    constexpr int QUAD_MIN_TASKS = 4 * 256;  // rows that give every compute unit of the card four waves
     constexpr bool NEURONS = epi_lif(EPI) || EPI == EPI_NEURON;
     constexpr int BATCH = 4;             // dot products whose operands are fetched together
     constexpr int CHUNK = 8;             // steps of a partial sum whose operands are fetched together
@@ -222,7 +223,7 @@ __device__ __forceinline__ void gemv_rows_ref_block(
             // whole steps of rate neurons are faster so (1,026 rows of 1,200 columns 13.0 -> 12.2 us, 1,538
             // of 2,000 16.9 -> 15.4), but not where a unit has a wave or two (770 rows of 1,000 11.6 both
             // ways), nor where a group takes a row (160 rows of 3,000 12.8 -> 13.0).
-            const bool quads = LPR == NHIP_WAVE && n_tasks >= 1024 &&
+            const bool quads = LPR == NHIP_WAVE && n_tasks >= QUAD_MIN_TASKS &&
                                ((n_cols | (int)(reinterpret_cast<uintptr_t>(arow) >> 2) |
                                  (int)(reinterpret_cast<uintptr_t>(xg) >> 2)) & 3) == 0;
 #pragma unroll 1

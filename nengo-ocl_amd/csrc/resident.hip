@@ -2,7 +2,7 @@
 //
 // A step of a network of a few hundred neurons is a handful of short launches, each a chain of
 // dependent reads of records, states and operands from memory and the start of a launch on top:
-// 8.7 us a step for two populations of 100 neurons, whatever the kernels do inside.  Here one work-group
+// 8.5 us a step for two populations of 100 neurons, whatever the kernels do inside.  Here one work-group
 // copies everything such a network consists of -- signals, work lists, parameters -- into its LDS,
 // runs n steps there, and copies back what the steps wrote.  The host (hipra_resident.py) sorts the
 // operations into phases that touch different memory, with a barrier between them, and gives every wave a
@@ -10,9 +10,10 @@
 // memory; the three that make up most steps of such networks have a form of their own, since a wave
 // alone on its SIMD is bound by the number of instructions (5 clocks each, 13 where one waits for the
 // other): the same arithmetic with everything that can be known beforehand resolved by the host.
-// Two populations of 100 neurons: 8.1 -> 2.8 us a step (2.4 of them the launch; replayed as a graph two
-// launches); of 1000: 8.8 -> 6.8.  16 populations of 20 with 10 inputs each: 11.2 -> 5.8.  An operation costs a wave
-// 0.2-0.4 us to fetch, 64 neurons 0.7 us (1.3 with sums of inputs), a row of 100 columns 1.1 us.
+// Whole steps, two launches replayed as a graph -> this one: two populations of 100 neurons 8.5 -> 2.55 us, of
+// 1000 8.7 -> 6.65; 16 populations of 20 with 10 inputs each 10.9 -> 5.6.  An operation costs a wave 0.2-0.4 us to
+// fetch, 64 neurons 0.75 us (0.93 where both waves of a SIMD have some, 1.35 and more with sums of inputs), a
+// row of 100 columns 1.1 us.
 #include <cstdint>
 #include <type_traits>
 

@@ -487,10 +487,10 @@ __global__ __launch_bounds__(SPMV_SKIP_WG) void spmv_sell_skip_kernel(
 //    and the sum goes from lane to lane, quad by quad, as in spmv_skip_rows -- which every lane of
 //    the row computes, so fewer lanes are fewer instructions.
 // A wave's record and first elements are on their way before the bits are.
-// A step with its product (the launch of the neurons included; before: bits in a launch of their own,
-// or by every group for itself, 32-bit indices, four lanes per row): 100,000 rows of 100 26.3 -> 18.4 us
-// (the product 18.9 -> 12.6, of 70 MB: 5.6 TB/s), of 20 17.0 -> 10.4; 10,000 rows of 100 11.8 -> 10.6; 2,000 of
-// 30 9.8 -> 9.6; 1,000,000 rows of 20 65.9 -> 50.7.
+// A step with its product, in calls of 1,000 (the launch of the neurons included; before: bits in a launch of
+// their own, or by every group for itself, 32-bit indices, four lanes per row): 100,000 rows of 100 25.4 -> 17.3
+// us (the product 18.9 -> 12.6, of 70 MB: 5.6 TB/s), of 20 16.3 -> 9.3; 180,000 of 60 27.9 -> 18.4; 10,000 rows of
+// 100 11.1 -> 10.2; 2,000 of 30 9.1 -> 8.9; 1,000,000 rows of 20 64.9 -> 49.2.
 template <int BITS> struct SpmvBitCols;
 template <> struct SpmvBitCols<16> {
     struct quad { int w[2]; };

@@ -113,8 +113,8 @@ def sell_layout(matrices):
 def bits_lanes(n_slices, n_waves):
     """Lanes per row of the product that is handed its spikes as bits: as many as fill the waves of
     the device (`n_waves`); every lane repeats the sum of its row, which a second or fourth lane has to
-    be worth (180,000 rows of 60, one lane: 28.4 us a step before, 19.4 now; 100,000 rows of 100, two:
-    18.4, with four and 16-bit indices 24.4)."""
+    be worth (180,000 rows of 60, one lane: 27.9 us a step before, 18.4 now; 100,000 rows of 100, two:
+    25.4 and 17.3, with four and 16-bit indices 24.4)."""
     cost = lambda lanes: -(-n_slices * lanes // n_waves) / lanes * (1 + 0.15 * (lanes - 1))
     return min((1, 2, 4), key=cost)
 
