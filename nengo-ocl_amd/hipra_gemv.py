@@ -124,14 +124,24 @@ THIN_CLASS, THIN_MAX_COLS = (2, 4, 1), 4
 # 256 x 100 12.06 -> 10.65, 300 x 150 13.0 -> 10.9, 1,000 x 64 13.4 -> 10.6. Below these rows the launch is
 # a few waves either way.
 SUM_PARTS_FOR_WAVE_TASKS, SUM_MIN_ROWS_FOR_WAVE_TASKS = 3, 3000
-# Products beside those with learned matrices in their launch (`fuse_hebbian`): a group of four rows there costs
-# 0.011 us whatever its columns (its LDS holds passes of LEARN_PASS_COLS), a launch of their own 2.7 us for items of
-# at most THIN_MAX_COLS columns, 3.5-4.0 up to 500, 6.7 for 3,000. So they ride up to a group per compute unit, 1.5
-# of wider items, two of items that fill a pass. Whole steps beside Oja's rule on 300 x 300, riding / apart: 1,000 x
-# 4 12.6 / 12.4, 1,500 x 4 13.8 / 12.4, 100,000 x 2 299 / 16; 1,000 x 64 12.2 / 13.6, 1,500 x 64 13.6 / 13.7, 4,000 x 64
-# 20.8 / 13.7; 2,000 x 500 15.0 / 14.1; 2,000 x 3,000 16.5 / 16.6; on 2000 x 2000: 1,500 x 4 22.1 / 20.8, 1,500 x 64
-# 21.7 / 22.5, 4,000 x 64 28.4 / 22.7, 2,000 x 3,000 24.7 / 25.7
-LEARN_RIDING_GROUPS, LEARN_PASS_COLS = 1, 2048
+# Products beside those with learned matrices in their launch (`fuse_hebbian`): us of a group of four rows there,
+# whatever its columns (its LDS holds passes of 2,048), against a launch of their own (`_own_launch_us`). Whole steps
+# beside Oja's rule on 300 x 300, together / apart: 1,000 x 4 12.6 / 12.4, 1,500 x 4 13.8 / 12.4, 100,000 x 2 299 / 16;
+# 1,000 x 64 12.2 / 13.6, 1,500 x 64 13.6 / 13.7, 4,000 x 64 20.8 / 13.7; 2,000 x 500 15.0 / 14.1; on 2000 x 2000: 1,500 x 4
+# 22.1 / 20.8, 4,000 x 64 28.4 / 22.7; 2,500 x 700 + 1,540 x 700 + 2,500 x 2,500 37.3 / 36.6, 1,028 x 1,000 + 1,028 x 700 +
+# 1,000 x 700 26.7 / 33.6, three of 2,100 x 300 19.3 / 23.3. Of 208 networks drawn at random (up to 1,800 groups of 4
+# to 2,500 columns) one is faster apart
+LEARN_GROUP_US = 0.011
+
+
+def _own_launch_us(kernel_class, n_cols, megabytes):
+    """What a launch of the products of a plan costs a step at most: items of up to `n_cols` columns.  (The
+    least measured are 2.7 us for up to four columns, 3.5 for 50 and 4.0 for 64.)"""
+    if kernel_class[0] == 2:
+        return max(6.0, 4.5 + 0.006 * n_cols)
+    return 10.0 if n_cols <= 64 else 12.0 + megabytes
+
+
 LIF_POP_ENABLED, LIF_POP_DECAY, LIF_POP_NO_J = 1 << 8, 1 << 9, 1 << 10  # flag bits of a population row
 LIF_POP_MASK = 1 << 12
 LIF_POP_BITS = 1 << 11  # spikes stored as a bit per neuron (see `store_spikes_as_bits`)
@@ -1564,7 +1574,7 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
     Fused when every item of `products` has one dot product with operands of stride 1, every matrix of the
     rule is the matrix of one such item (same start, shape and row stride), its row operand is contiguous, and
     nothing else the launch reads or writes lies in such a matrix.  Items without a learned matrix are part of
-    the launch while they are few (`LEARN_RIDING_GROUPS`).  Filters of `lf_plan` with one numerator and at most
+    the launch while they are few (`LEARN_GROUP_US`).  Filters of `lf_plan` with one numerator and at most
     one denominator coefficient on contiguous vectors move; the caller has checked that nothing between the
     plans, and nothing the plans read or write themselves, keeps the rule and those filters out of the
     products' launch.  Returns ``(plan, plans in front of it for the products that are not part of it, plans
@@ -1617,18 +1627,15 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
             return None
     if F.ptr.value != buf:
         return None
-    # What else the GEMV multiplies by rides along while it is little; the rest keeps a launch (in front, where
-    # it reads the matrices as they were).
-    def groups(items):
-        cols = np.array([geometry[b]["dots"][0]["a_shape1"] for b in items])
-        weight = np.where(cols <= THIN_MAX_COLS, 1.0, np.where(cols < LEARN_PASS_COLS, 2 / 3, 0.5))
-        return float(sum(-(-geometry[b]["y_len"] // (WG // WAVE)) * w for b, w in zip(items, weight)))
-
-    limit = LEARN_RIDING_GROUPS * queue.n_compute_units
+    # What else a plan of the GEMV multiplies by rides along where that costs less than a launch of its own, which
+    # the rest keeps (in front, where it reads the matrices as they were).
     kept, riding = [], []
-    for p in sorted(products, key=lambda p: rule_of.keys().isdisjoint(p.members)):  # those with learned ones first
+    for p in products:
         beside = [b for b in p.members if b not in rule_of]
-        if groups(riding) + groups(beside) <= limit:
+        groups = sum(-(-geometry[b]["y_len"] // (WG // WAVE)) for b in beside)
+        cols = [geometry[b]["dots"][0]["a_shape1"] for b in beside]
+        megabytes = 4e-6 * sum(geometry[b]["y_len"] * n for b, n in zip(beside, cols))
+        if LEARN_GROUP_US * groups <= _own_launch_us(p.kernel_class, max(cols + [0]), megabytes):
             riding += beside
         elif len(beside) == len(p.members):
             kept.append(p)

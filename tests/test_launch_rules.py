@@ -255,13 +255,14 @@ def rule_beside_products(n, extra, rule="Oja", synapses=("Lowpass",)):
     return net
 
 
-# rows and columns of the others on both sides of what rides along: at most four columns, more, whole passes;
-# in the class of the learned matrix (300 x 300, 50 x 50) and in another
+# rows and columns of the others on both sides of what rides along: at most four columns, more, many, and rows
+# that no 16-byte loads fit; in the class of the learned matrix (300 x 300, 50 x 50) and in another
 @pytest.mark.parametrize("n,extra,rides", [
-    (300, [(1024, 4)], True), (300, [(1028, 4)], False), (300, [(100000, 2)], False), (300, [(1536, 64)], True),
-    (300, [(1540, 64)], False), (300, [(2, 300)] * 16, True), (300, [(2048, 3000)], True),
-    (300, [(2052, 3000)], False), (50, [(20, 50)] * 76, True), (50, [(20, 50)] * 77, False),
-    (300, [(1028, 4), (1536, 64)], None)])
+    (300, [(2180, 2)], True), (300, [(2184, 2)], False), (300, [(3636, 4)], True), (300, [(3640, 4)], False),
+    (300, [(100000, 2)], False), (300, [(3636, 64)], True),
+    (300, [(3640, 64)], False), (300, [(2, 300)] * 16, True), (300, [(7740, 300)], True),
+    (300, [(7744, 300)], False), (50, [(20, 50)] * 109, True), (50, [(20, 50)] * 110, False),
+    (301, [(7760, 301)], True), (301, [(7764, 301)], False), (300, [(2184, 2), (3636, 64)], None)])
 def test_few_other_products_ride_with_learned_matrices(monkeypatch, n, extra, rides):
     from nengo_ocl_amd.simulator import Simulator
 

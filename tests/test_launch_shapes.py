@@ -683,8 +683,9 @@ def test_products_with_a_part_of_a_learned_matrix_read_it_unchanged(queue, rule,
 
 @pytest.mark.parametrize("rule", ["Oja", "BCM"])
 @pytest.mark.parametrize("n,extra,synapses", [
-    (300, [(1028, 4)], ["Lowpass"]), (300, [(1540, 64)], ["Lowpass"]), (50, [(20, 50)] * 77, ["Lowpass", "Alpha"]),
-    (301, [(1541, 63), (3, 301)], ["Alpha"]), (300, [(1030, 3), (1024, 64)], ["Lowpass", "Alpha"])])
+    (300, [(2300, 2)], ["Lowpass"]), (300, [(3701, 64)], ["Lowpass"]), (50, [(20, 50)] * 115, ["Lowpass", "Alpha"]),
+    (301, [(3700, 63), (3, 301)], ["Alpha"]), (300, [(2301, 3), (1024, 64)], ["Lowpass", "Alpha"]),
+    (300, [(17200, 512), (40, 1024)], ["Lowpass", "Alpha"])])
 def test_products_apart_from_the_launch_of_learned_matrices(queue, rule, n, extra, synapses):
     """Too many other products for that launch: they keep their filters, of first and second order, in a launch
     in front of it."""
