@@ -1012,7 +1012,6 @@ class Simulator:
             self.queue, *(spec[k][which] for k in ("X", "Y", "A", "B", "Xbuf", "Ybuf")), tag=lf.tag)
         plan.planned_ops = ops
         plan.reads_mem, plan.writes_mem = {op.input.base for op in ops}, {op.output.base for op in ops}
-        self._filter_positions.append(plan.bufpos)
         return plan
 
     def _fuse_outer_filters(self, plans):
@@ -1059,6 +1058,8 @@ class Simulator:
                 continue
             fused.reads_mem = ew.reads_mem | lf.reads_mem
             fused.writes_mem = ew.writes_mem | lf.writes_mem
+            if rest:
+                self._filter_positions.append(left.bufpos)
             plans[j - 1:j] = [left] if rest else []
             del plans[i]
             plans.insert(at, fused)

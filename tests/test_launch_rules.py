@@ -316,8 +316,17 @@ def test_synapses_of_higher_order_leave_the_others_their_launch(monkeypatch, syn
     from nengo_ocl_amd.simulator import Simulator
 
     host_simulators(monkeypatch)
+    apart, some_filters = [], Simulator._some_filters
+
+    def record(sim, lf, which):
+        apart.append(some_filters(sim, lf, which))
+        return apart[-1]
+
+    monkeypatch.setattr(Simulator, "_some_filters", record)
     with Simulator(pes_with_synapses(synapse, n, dims), seed=1, event_calibration_steps=0) as sim:
         launches = [p.kern.__name__ for p in sim._plans]
+        # (a launch that was tried and not taken leaves nothing behind)
+        assert any(apart[0].bufpos is pos for pos in sim._filter_positions) == fused
     assert ("nhip_outer_filter" in launches) == fused and ("nhip_elementwise_inc" in launches) != fused, launches
 
 
