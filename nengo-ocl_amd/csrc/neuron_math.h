@@ -111,6 +111,28 @@ __device__ __forceinline__ bool lif_step(float j, float& v, float& w, float tau,
     return spiked;
 }
 
+// The same for one time constant and no sub-steps: the factor of a whole step comes with the population
+// (LIF_POP_DECAY), that of no time is +0, and a wave in which no neuron leaves its refractory period or spikes
+// skips the evaluations in double.
+__device__ __forceinline__ bool lif_step_decay(float j, float& v, float& w, float decay, float tau, float ref,
+                                               float dtu) {
+    w -= dtu;
+    const float delta_t = (w > dtu) ? 0.0f : (w < 0.0f) ? dtu : dtu - w;
+    float factor = delta_t == dtu ? decay : 0.0f;
+    if (delta_t != dtu && delta_t != 0.0f) factor = -(float)nhip_expm1((double)__fdiv_rn(-delta_t, tau));
+    v = __fadd_rn(v, __fmul_rn(factor, j - v));
+    const bool spiked = v > 1.0f;
+    if (spiked) {
+        const float t_spike =
+            __fadd_rn(dtu, __fmul_rn(tau, (float)nhip_log1p((double)__fdiv_rn(-(v - 1.0f), j - 1.0f))));
+        w = ref + t_spike;
+        v = 0.0f;
+    } else if (v < 0.0f) {
+        v = 0.0f;
+    }
+    return spiked;
+}
+
 // Adaptive LIF (clra_nonlinearities.py:1086-1133 with `adaptive`): the LIF update with
 // j - n in place of j in the voltage step, then n += (dt / tau_n) (inc_n s - n).  Returns s.
 __device__ __forceinline__ float alif_step(float j, float& v, float& w, float& n, float tau, float ref,

@@ -198,7 +198,7 @@ N_DIES = 8  # accelerator dies of the device: work-group g runs on die g % 8
 
 
 def spread_over_dies(tasks):
-    """The 24-word task records of a large-item launch in an order that gives every
+    """The task records (24 words and more) of a large-item launch in an order that gives every
     accelerator die the same number of heavy tasks.
 
     Work-groups go to the dies in turn, and the kernels map them so that a die works through
@@ -212,7 +212,7 @@ def spread_over_dies(tasks):
     per_group = WG // WAVE
     n = len(tasks)
     groups = -(-n // per_group)
-    if not SPREAD_OVER_DIES or groups < 2 * N_DIES or tasks.shape[1] != 24:
+    if not SPREAD_OVER_DIES or groups < 2 * N_DIES or tasks.shape[1] < 24:
         return tasks
     weight = tasks[:, 2].astype(np.int64) * np.maximum(tasks[:, 18], 1) * (tasks[:, 9] > 0)
     heavy = weight >= 0.25 * max(int(weight.max()), 1)
@@ -1317,9 +1317,9 @@ def fuse_input_sums(sum_plan, lif_plan):
     fused.input_sums = len(sums)
     fused.lazy_currents = getattr(lif_plan, "lazy_currents", None)
     fused.host_pops = new_pops if large else pops
+    fused.host_parts = np.array(part_rows, dtype=np.int32)
     if not large:
         fused.host_tables, fused.host_ranges = (items, coefs, tasks), ranges
-        fused.host_parts = np.array(part_rows, dtype=np.int32)
         fused.spare_items = list(range(n_items, len(items)))
     # (the device copy of the table, where it is the one the launch reads: large items)
     fused.dev_pops = (dev_pops if spare else getattr(lif_plan, "dev_pops", None)) if large else None
@@ -1359,6 +1359,8 @@ def store_spikes_as_bits(enc_plan, items, event_records, dt):
             enc_plan.bw_per_call -= 4 * n - n // 8
     if values:
         enc_plan.dev_pops.set(pops.astype(np.int32).ravel())
+        if hasattr(enc_plan, "upload_pops"):  # (they ride in the records of its tasks)
+            enc_plan.upload_pops()
         for plan in touched:
             plan.dev_event_table.set(plan.event_table.astype(np.int32).ravel())
         enc_plan.tag = "%s + spikes as bits" % enc_plan.tag
@@ -1394,10 +1396,13 @@ def leave_spike_bits(lif_plan, s_start, n):
                 or not np.array_equal(tasks[mine, 1], np.arange(n))):
             return None
     pops[item, 7] |= LIF_POP_MASK
-    lif_plan.dev_pops.set(pops.astype(np.int32).ravel())
     mask = to_device(queue, np.zeros(-(-n // 128) * 4, dtype=np.int32))
+    lif_plan.dev_pops.set(pops.astype(np.int32).ravel())
     lif_plan.kern = queue.lib.nhip_gemv_rows_lif_bits
     lif_plan.args = tuple(lif_plan.args) + (mask.ptr,)
+    if lif_plan.laid_out is not None:
+        lif_plan.upload_pops()
+        lif_plan.leave_bits(mask.ptr)
     lif_plan.full_args = tuple(lif_plan.full_args) + (mask,)
     lif_plan.tag = "%s + spikes as bits too" % lif_plan.tag
     return mask, one
@@ -1552,11 +1557,12 @@ def fuse_learning(enc_plan, dec_plan, ew_plan, lf_plan):
     for new, old in ((new_dec, dec_plan), (new_enc, enc_plan)):
         for attr in ("description", "kernel_class", "n_tasks", "members", "prog", "gemv_bytes",
                      "host_tasks", "host_pops", "dev_pops", "lif_written", "lazy_currents",
-                     "input_sums"):
+                     "input_sums", "host_parts"):
             if hasattr(old, attr):
                 setattr(new, attr, getattr(old, attr))
     new_dec.learned_matrices = len(learn_of_item)
     new_enc.deferred_filters = len(moved)
+    new_enc.host_deferred = deferred
     residual = []
     if rest:
         residual = plan_linearfilter(queue, S[rest], F[rest], FA[rest], FB[rest],

@@ -167,6 +167,13 @@ def to_device(queue, array, dtype=None):
     return DeviceArray(queue, t, array.dtype)
 
 
+def empty_device(queue, n):
+    """A device array of `n` float32 whose contents are whatever the memory held."""
+    torch = _torch()
+    with queue.context():
+        return DeviceArray(queue, torch.empty(int(n), dtype=torch.float32, device=queue.device), np.float32)
+
+
 class HIPRaggedArray:
     """A linear device buffer partitioned into (possibly aliasing) 2-D sections."""
 

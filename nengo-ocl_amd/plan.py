@@ -80,6 +80,9 @@ class Plan(BasePlan):
         # (function, arguments) of a call that prepares the launch and launches nothing
         # itself, made right before it (a sequence the launch carries)
         self.prelude = None
+        # (function, arguments) of another entry point that does the same work from copies of constant
+        # matrices in its own order (`hipra_lanes.lay_out`); `kern` and `args` stay what the launch was planned as
+        self.laid_out = None
 
     @staticmethod
     def _format_size(size):
@@ -107,7 +110,8 @@ class Plan(BasePlan):
                 _lib.check(lib.nhip_event_record(ev0, handle))
         if self.prelude is not None:
             _lib.check(self.prelude[0](*self.prelude[1]), self.name)
-        _lib.check(self.kern(handle, *self.args), self.name)
+        kern, args = self.laid_out or (self.kern, self.args)
+        _lib.check(kern(handle, *args), self.name)
         if profiling:
             if own and lib.nhip_launch_events_pending():
                 # the entry point returned without launching (an empty work list): the

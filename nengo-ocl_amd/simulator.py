@@ -20,6 +20,7 @@ produces the operator graph) or a `minibuilder.Network`; ``model`` may be a
 nengo ``Model`` or an `ir.Model` that already holds operators.
 """
 
+import bisect
 import functools
 import inspect
 import logging
@@ -87,6 +88,11 @@ class HipBackend:
         from . import hipra_resident
 
         self._resident = hipra_resident
+        from . import hipra_lanes
+
+        self._lanes = hipra_lanes
+        # switch for measurements: "0" reads the matrices of every launch as they lie among the signals
+        self.lays_out_matrices = os.environ.get("NENGO_HIP_LAY_OUT", "1") != "0"
         # switch for measurements: "0" replays small networks as graphs too
         self.runs_resident = os.environ.get("NENGO_HIP_RESIDENT", "1") != "0"
         self.plan_sparse_dot_inc = hipra_spmv.plan_sparse_dot_inc
@@ -134,6 +140,13 @@ class HipBackend:
             bits[sp["x_start"]] = self._gemv.leave_spike_bits(lif_plan, sp["x_start"], sp["n_cols"])
         if bits[sp["x_start"]] is not None:
             self._spmv.read_spike_bits(product_plan, *bits[sp["x_start"]])
+
+    def laid_out_spans(self, plan):
+        """Where the matrices lie that `lay_out_matrices` would give the launch `plan` copies of, or None."""
+        return self._lanes.matrix_spans(plan) if self.lays_out_matrices and hasattr(plan, "prog") else None
+
+    def lay_out_matrices(self, plan):
+        return self._lanes.lay_out(plan)
 
     def store_spikes_as_bits(self, enc_plan, items, event_records, dt):
         return self._gemv.store_spikes_as_bits(enc_plan, items, event_records, dt)
@@ -491,6 +504,7 @@ class Simulator:
         # filter outputs whose last step is pending in device memory (`_fuse_learning`):
         # signal base -> (spike signal base, a0 or None, b0)
         self._pending_filters = {}
+        self._constants_changed = False
         self._n_steps = 0
         self._filter_positions = []
         self._noise_plans = []
@@ -550,16 +564,20 @@ class Simulator:
             plans = self.backend.merge_small_plans(plans)
             if fuse and hasattr(self.backend, "carry_sequences"):
                 plans = self.backend.carry_sequences(plans)
+        before_last = self._plan_host_view()
+        resident = None
+        if (fuse and merge_small and use_graph and not before_last
+                and hasattr(self.backend, "resident_program")):
+            resident = self.backend.resident_program(apart, self.all_data, len(plans))
+        self._laid_out = []  # (base signals of constants, launch that reads copies of them)
+        if fuse and resident is None and hasattr(self.backend, "lay_out_matrices"):
+            self._lay_out_matrices(plans)
         self._store_spikes_as_bits(plans)
         if fuse and hasattr(self.backend, "share_spike_bits"):
             self._share_spike_bits(plans)
+        assert resident is None or not self._spike_bits  # (it holds no launch that reads or writes them)
         logger.info("Plans in %0.3f s", _time.time() - t0)
 
-        before_last = self._plan_host_view()
-        resident = None
-        if (fuse and merge_small and use_graph and not before_last and hasattr(self.backend, "resident_program")
-                and not self._spike_bits):
-            resident = self.backend.resident_program(apart, self.all_data, len(plans))
         self._plans = Plans(plans, self.profiling, use_graph=use_graph, branches=branches,
                             before_last=before_last, resident=resident)
         self.rng = None
@@ -720,6 +738,38 @@ class Simulator:
         self._host_view_plan = plan
         plan()  # nothing has run yet: the copy holds the initial values
         return [plan]
+
+    def _lay_out_matrices(self, plans):
+        """Launches of products with constant matrices (encoders) that update neurons read copies of them in
+        their own order (`hipra_lanes.lay_out`): where nothing of the model writes the matrices.  A write of
+        the host brings the copies up to date (`_constant_written`)."""
+        if self.reference_host_state:
+            return
+        ra = self.all_data
+        written = {s.base for op in self.operators for s in list(op.sets) + list(op.incs) + list(op.updates)}
+        constants = sorted((int(ra.starts[self.sidx[b]]), int(b.size), k) for k, b in enumerate(self.all_bases)
+                           if getattr(b, "readonly", False) and b not in written and b.size)
+        starts = [c[0] for c in constants]
+        for plan in plans:
+            spans = self.backend.laid_out_spans(plan)
+            bases = set()
+            if spans is None:
+                continue
+            for lo, hi in spans:
+                k = bisect.bisect_right(starts, lo) - 1
+                if k < 0 or hi > constants[k][0] + constants[k][1]:
+                    spans = None
+                    break
+                bases.add(self.all_bases[constants[k][2]])
+            if spans is not None and self.backend.lay_out_matrices(plan):
+                self._laid_out.append((bases, plan))
+
+    def _constant_written(self, base):
+        """The host has changed a constant: the copies of it that launches read follow."""
+        for bases, plan in self._laid_out:
+            if base in bases:
+                plan.lay_out_again()
+                self._constants_changed = True
 
     def _store_spikes_as_bits(self, plans):
         """Spike signals that nothing but launches visiting active columns reads -- no other
@@ -1364,6 +1414,7 @@ class Simulator:
                     sim.all_data[sim.sidx[item]] = incoming
                 else:
                     raise NotImplementedError()
+                sim._constant_written(resolved)
 
             def __str__(self):
                 sio = StringIO()
@@ -1503,6 +1554,10 @@ class Simulator:
         if seed is not None:
             raise NotImplementedError("Seed changing not implemented")
         self.backend.write_all(self.all_data, self._initial_buf)
+        if self._constants_changed:  # (what the host had written is gone)
+            for _, plan in self._laid_out:
+                plan.lay_out_again()
+            self._constants_changed = False
         for dev, host in self._raggedarrays_to_reset:
             self.backend.write_all(dev, host.buf)
         for pos in self._filter_positions:

@@ -1,0 +1,120 @@
+"""Launches that update neurons with a lane per neuron (csrc/gemv_lanes.hip), at the sizes where their tasks, column
+quads and passes have edges, against the CPU oracle bit for bit (they keep the reference's order of summation, so the
+tolerance is zero)."""
+
+import numpy as np
+import pytest
+
+from helpers import assert_same_signals, host_simulators
+
+
+def network(n, d, neuron, seed=3):
+    """Populations whose input is a sum of up to nine parts, of one part, a node's value, and nothing."""
+    from nengo_ocl_amd import minibuilder as mb
+
+    net = mb.Network(seed=seed, solver="surrogate")
+    make = lambda n: net.Ensemble(n, d, neuron_type=neuron())
+    ens = [make(n), make(n + 1), make(max(n - 1, 1)), make(n)]
+    stim = net.Node(mb.WhiteSignal(period=0.3, high=8.0, seed=4), size_out=d)
+    net.Connection(stim, ens[0], synapse=mb.Lowpass(0.005))
+    for k in range(8):
+        net.Connection(ens[k % 2], ens[0], transform=0.1 + 0.05 * k, synapse=mb.Lowpass(0.002 + 0.001 * k))
+    net.Connection(ens[0], ens[1], synapse=mb.Alpha(0.01))
+    net.Connection(stim, ens[2], synapse=None)
+    return net, [net.Probe(e, synapse=0.01) for e in ens] + [net.Probe(ens[1].neurons)]
+
+
+def laid_out(sim):
+    return [p for p in sim._plans if getattr(p, "laid_out", None) is not None]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("neuron", ["LIF", "AdaptiveLIF", "LIFRate", "RectifiedLinear", "SpikingRectifiedLinear"])
+# one to four columns are read as they lie; quads of one, two and three columns; 16 quads and one more, 32; tasks of
+# 63, 64 and 65 rows; items of the small and of the large kernel, on 16-byte boundaries and not
+@pytest.mark.parametrize("n,d", [(2, 1), (63, 2), (64, 3), (65, 4), (200, 5), (70, 7), (129, 8), (301, 30), (601, 18),
+                                 (200, 50), (140, 62), (300, 63), (129, 64), (260, 65), (100, 100), (300, 127),
+                                 (65, 128)])
+def test_neurons_a_lane_each(queue, monkeypatch, neuron, n, d):
+    from nengo_ocl_amd import minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    monkeypatch.setenv("NENGO_HIP_RESIDENT", "0")
+    (net, probes), (net_o, probes_o) = (network(n, d, getattr(mb, neuron)) for _ in range(2))
+    with Simulator(net, seed=1, event_calibration_steps=0) as gpu, OracleSimulator(net_o, seed=1) as cpu:
+        assert laid_out(gpu), [str(p) for p in gpu._plans]
+        for steps in (1, 30):
+            gpu.run_steps(steps)
+            cpu.run_steps(steps)
+            for p, p_o in zip(probes, probes_o):
+                assert np.array_equal(gpu.data[p], cpu.data[p_o])
+            assert_same_signals(gpu, cpu)
+
+
+@pytest.mark.gpu
+def test_encoders_that_the_host_changes(queue, monkeypatch):
+    """A write reaches the copy that the launch reads, a reset takes it back."""
+    from nengo_ocl_amd import minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    monkeypatch.setenv("NENGO_HIP_RESIDENT", "0")
+    (net, _), (net_o, _) = (network(200, 50, mb.LIF) for _ in range(2))
+    with Simulator(net, seed=1) as gpu, OracleSimulator(net_o, seed=1) as cpu:
+        for change in (False, True):
+            for sim, ens in ((gpu, net.ensembles[0]), (cpu, net_o.ensembles[0])):
+                if change:
+                    sig = sim.model.sig[ens]["encoders"]
+                    sim.signals[sig] = 1.5 * sim.signals[sig][::-1]
+                sim.run_steps(10)
+            assert_same_signals(gpu, cpu)
+        gpu.reset()
+        with OracleSimulator(network(200, 50, mb.LIF)[0], seed=1) as fresh:
+            for sim in (gpu, fresh):
+                sim.run_steps(10)
+            assert_same_signals(gpu, fresh)
+
+
+@pytest.mark.parametrize("n,d", [(2, 1), (64, 3), (65, 4), (301, 30), (200, 50), (300, 127)])
+def test_tasks_cover_every_neuron_once(monkeypatch, n, d):
+    """Records of at most 64 rows from multiples of 64 on, matrices apart in the copy, groups of four filled
+    up with tasks of no rows."""
+    from nengo_ocl_amd import minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    monkeypatch.setenv("NENGO_HIP_RESIDENT", "0")
+    with Simulator(network(n, d, mb.LIF)[0], seed=1, event_calibration_steps=0) as sim:
+        assert laid_out(sim)
+        for plan in laid_out(sim):
+            tasks, geometry = plan.host_tasks, plan.prog.geometry
+            assert plan.laid_out[1][2] % 4 == 0 and plan.laid_out[1][2] - len(tasks) < 4
+            blocks = []
+            for b in plan.members:
+                mine = tasks[tasks[:, 0] == b]
+                mine = mine[np.argsort(mine[:, 1])]
+                assert not np.any(mine[:, 1] % 64) and mine[:, 2].max() <= 64
+                assert np.array_equal(np.concatenate([r + np.arange(m) for r, m in mine[:, 1:3]]),
+                                      np.arange(geometry[b]["y_len"]))
+                for dot in geometry[b]["dots"][:1]:
+                    if d > 4:
+                        quads = -(-dot["a_shape1"] // 4)
+                        assert set(mine[:, 17]) == {quads} and len(set(mine[:, 16])) == 1
+                        blocks.append((int(mine[0, 16]), -(-geometry[b]["y_len"] // 64) * quads))
+                    else:
+                        assert set(mine[:, 16]) == {dot["a_start"]} and np.all(mine[:, 21] < 0)
+            blocks = sorted(set(blocks))
+            assert all(a + size <= b for (a, size), (b, _) in zip(blocks, blocks[1:]))
+
+
+@pytest.mark.parametrize("groups", [1, 7, 8, 9, 63, 64, 1000])
+def test_groups_of_a_die_are_neighbours_in_the_list(groups):
+    from nengo_ocl_amd import hipra_lanes
+
+    tasks = np.arange(1, 4 * groups)[:, None] * np.ones((1, 3), dtype=np.int32)
+    out = hipra_lanes.for_the_dies(tasks.astype(np.int32))[:, 0].reshape(groups, 4)
+    assert sorted(out.ravel()) == [0] + list(range(1, 4 * groups))
+    for die in range(8):
+        firsts = out[die::8, 0]
+        assert np.all(np.diff(firsts) == 4)
