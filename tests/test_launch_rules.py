@@ -340,3 +340,19 @@ def test_synapses_that_their_product_reads_leave_the_others_in_its_launch(monkey
     with Simulator(None, model=model, seed=1, event_calibration_steps=0) as sim:
         launches = [p.kern.__name__ for p in sim._plans if hasattr(p, "kern")]
     assert {"nhip_gemv_rows_filter", "nhip_gemv_tile_filter"} <= set(launches), launches
+
+
+def test_populations_without_input_ride_with_unaligned_matrices(monkeypatch):
+    """Rows that lie back to back without 16-byte alignment have an instance of their own: a population without
+    input joins it, and the launch forms the input sums of the others."""
+    from nengo_ocl_amd import minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    net = mb.Network(seed=1, solver="surrogate")
+    ens = [net.Ensemble(1501, 50) for _ in range(3)]
+    for k in (1, 1, 2):  # (nothing reaches the first)
+        net.Connection(ens[0], ens[k], synapse=mb.Lowpass(0.005))
+    with Simulator(net, seed=1, event_calibration_steps=0) as sim:
+        neurons = [p for p in sim._plans if p.name.endswith("_lif")]
+        assert len(neurons) == 1 and neurons[0].input_sums == 2, [p.name for p in sim._plans]
