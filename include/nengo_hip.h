@@ -303,6 +303,27 @@ int nhip_gemv_lanes(void *stream, int neurons, const int *tasks, int n_tasks, co
                     float *B, double dt, int upsample, const float *TAU, const float *REF, const float *AMP,
                     const int *parts, int *mask);
 
+/* Products with matrices that nothing writes, one dot product per item, and the filters of order 1 or 2 that their
+ * rows feed: nhip_gemv with flavor 2, nhip_gemv_tile, nhip_gemv_events, nhip_gemv_rows_filter and _tile_filter on
+ * copies of the matrices.  `tiles` of 128 columns are summed side by side, four lanes each.  nhip_lay_out_dots:
+ *   matrices : int32[n][8]  {a_start, a_stride0, M, N, first 64 bytes in At, lanes = 4 * tiles, quads, 64-byte units
+ *              from row to row = ceil(N / (128 * tiles)) * quads * tiles}
+ * Lane l of a row holds columns 128 (l / 4) + l % 4 + 4 e of a pass; e = 4 q .. 4 q + 3 are quad q; the quads q of
+ * all lanes lie side by side; -0 past the row's end.  `max_rows`: the largest M.
+ * nhip_gemv_dots, with `tiles` 1 (`quads` 2, 4 or 8 of 16 columns each) or 2 (8): a record per row, `n_groups` times
+ * 64 / tiles of them:
+ *   records : int32[..][16]  {first 64 bytes of the row in At, x_start, N, number of targets (< 0: no row; its other
+ *             words are a row's), y, y_in, first target, row of its item, alpha, beta, gamma, 0, the first target}
+ * every lane's partial sum having at least `full` and at most `most` elements; with `tiles` 4, 8 or 16 (8 quads; any
+ * N) a record per group of up to 64 / tiles rows of an item:
+ *   records : int32[n_groups][32]  {first 64 bytes of the item's row 0, units from row to row, N, x_start, x_stride0,
+ *             row0, n_rows, number of targets, y_start, y_stride0, yin_start, yin_stride0, alpha, beta, gamma, first
+ *             target, the first target (4), x_bits (as in nhip_gemv_events), 0 ...}
+ * `B` is the buffer of X, Yin, Y and F, which are one here; `targets` as for nhip_gemv_tile_filter. */
+int nhip_lay_out_dots(void *stream, const int *matrices, int n, int max_rows, const float *A, float *At);
+int nhip_gemv_dots(void *stream, int tiles, int quads, int order, const int *records, int n_groups, const float *At,
+                   float *B, const int *targets, int full, int most);
+
 /* The same two epilogues for launches of small items (nhip_gemv with flavor 2, whose
  * `items`, `coefs`, `dots` and `tasks` tables these take; `lpr` 4, 1 or 64): the
  * neuron update / filter step of a row runs in the lane that holds the row's sum.

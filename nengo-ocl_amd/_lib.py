@@ -44,6 +44,8 @@ SIGNATURES = {
     "nhip_gemv_tile_rows": [c_int, c_int],
     "nhip_lay_out_lanes": [P, P, c_int, c_int, P, P],
     "nhip_gemv_lanes": [P, c_int, P, c_int, P, P, P, ctypes.c_double, c_int, P, P, P, P, P],
+    "nhip_lay_out_dots": [P, P, c_int, c_int, P, P],
+    "nhip_gemv_dots": [P, c_int, c_int, c_int, P, c_int, P, P, P, c_int, c_int],
     "nhip_gemv_rows_lif": [P, c_int, c_int, P, P, P, P, c_int, P, P, P, P,
                            P, ctypes.c_double, c_int, P, P, P, P, P, P],
     "nhip_gemv_rows_lif_bits": [P, c_int, c_int, P, P, P, P, c_int, P, P, P, P,

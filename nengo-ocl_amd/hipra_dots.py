@@ -1,0 +1,174 @@
+"""Products with constant matrices, each output row with the filters it feeds, from copies of the matrices in
+the order in which csrc/gemv_dots.hip reads them: decoders, transforms.
+
+`lay_out` has a launch of `hipra_gemv` (small items, long rows, large items, columns of the neurons that spiked; with
+or without the filters of `fuse_linearfilter`) run that kernel instead.  Same sums in the same order (the reference:
+clra_gemv.py:1043-1058, :1148-1153), same results.
+"""
+
+import numpy as np
+
+from .hipra_gemv import GROUP_ROW_MIN_COLS, GROUP_ROWS_MAX, _span
+from .hipraggedarray import empty_device, to_device
+
+WG, TILE = 256, 128
+ROW_COLS = 256  # rows of up to so many columns have a record each, longer ones share one
+# ... but few long rows take a group each elsewhere (`GROUP_ROWS_MAX` of hipra_gemv): 10 rows of 9,216 columns, whole
+# steps 25.9 us; with a group per row and their vector through LDS 26.5
+# Launches that visit active columns only, up to so many bytes of copies: beyond, the columns that count are fewer
+# bytes than the matrices, which the L2 of the dies no longer hold.  Whole steps, active columns / all of them:
+# 20 x 32 x 600 (1.9 MB) 9.5 / 7.9 us, 100 x 16 x 1000 (6.5) 7.6 / 7.6, 37 x 50 x 1501 (15) 10.6 / 10.1,
+# 12 x 64 x 5000 (19; a group per item) 16.7 / 14.1, 60 x 30 x 3000 (30) 14.1 / 16.8
+EVENT_MAX_BYTES = 20 << 20
+GROUPS_FOR_FEW_ROWS = 2048  # of groups that are mostly empty
+
+
+class _Launch:
+    def __init__(self, plan):
+        name, args = getattr(plan.kern, "__name__", ""), plan.args
+        self.known = name in ("nhip_gemv", "nhip_gemv_rows_filter", "nhip_gemv_tile", "nhip_gemv_tile_filter",
+                              "nhip_gemv_events") and hasattr(plan, "prog") and plan.laid_out is None
+        if not self.known:
+            return
+        self.events = name == "nhip_gemv_events"
+        self.order, self.item_targets, self.targets, F = 1, None, None, None
+        if self.events:
+            self.A, (self.X, Yin, Y) = plan.prog.A.ptr, args[3:6]
+            filtered = args[6] is not None
+        else:
+            k = 7 if name == "nhip_gemv_rows_filter" else 8 if "_tile" in name else 9
+            self.A, self.X, Yin, Y = args[k:k + 4]
+            filtered = name.endswith("_filter")
+            self.known = "_tile" in name or name != "nhip_gemv" or args[0] == 2
+        if filtered:
+            tables = getattr(plan, "filter_tables", None)
+            if tables is None:
+                self.known = False
+                return
+            self.item_targets, self.targets, F, self.host_targets = tables
+            self.order = int(args[8] if self.events else args[-1])
+        self.buffers = [self.A, Yin, Y] + ([F.ptr] if F is not None else [])
+
+
+def _shape(plan):
+    """(tiles, quads) of the kernel for a launch, or None where it holds none or has nothing to give."""
+    g = [plan.prog.geometry[b] for b in plan.members]
+    if not g or any(len(item["dots"]) != 1 or item["dots"][0]["a_shape1"] < 1 for item in g):
+        return None
+    dots = [item["dots"][0] for item in g]
+    cols = max(d["a_shape1"] for d in dots)
+    if cols <= ROW_COLS:
+        if any(d["x_stride0"] != 1 and d["a_shape1"] > 1 for d in dots):
+            return None
+        quads = -(-cols // 16)
+        return (2, 8) if cols > TILE else (1, 2 if quads <= 2 else 4 if quads <= 4 else 8)
+    rows = sum(item["y_len"] for item in g)
+    tiles = 4 if cols <= 4 * TILE else 8 if cols <= 8 * TILE else 16
+    if cols >= GROUP_ROW_MIN_COLS and rows <= GROUP_ROWS_MAX:
+        return None
+    per_group = WG // (4 * tiles)
+    groups = sum(-(-item["y_len"] // per_group) for item in g)
+    if groups > GROUPS_FOR_FEW_ROWS and 4 * rows < groups * per_group:
+        return None
+    return tiles, 8
+
+
+def _copy_units(plan, tiles, quads):
+    """{matrix: 64-byte units of its copy}"""
+    out = {}
+    for b in plan.members:
+        g = plan.prog.geometry[b]
+        d = g["dots"][0]
+        passes = -(-d["a_shape1"] // (tiles * TILE))
+        out[d["a_start"], d["a_stride0"], g["y_len"], d["a_shape1"]] = (passes * quads * tiles, d["a_j"])
+    return out
+
+
+def matrix_spans(plan):
+    """Intervals of the signal buffer that hold the matrices `lay_out` would copy, or None where the launch does not
+    qualify."""
+    launch = _Launch(plan)
+    if not launch.known or any(ptr is None or ptr.value != launch.X.value for ptr in launch.buffers):
+        return None
+    shape = _shape(plan)
+    if shape is None:
+        return None
+    mats = _copy_units(plan, *shape)
+    size = sum(64 * key[2] * units for key, (units, _) in mats.items())
+    if size >= 2 ** 33 or launch.events and size > EVENT_MAX_BYTES:
+        return None
+    return sorted({_span(plan.prog.A, a_j) for _, a_j in mats.values()} - {None})
+
+
+def lay_out(plan):
+    """Make `plan` (for which `matrix_spans` gave spans, of constants) run the kernel that reads copies of its
+    matrices.  The plan gets `lay_out_again`, for when the host has changed a matrix."""
+    from . import _lib
+
+    queue, lib, prog = plan.queue, plan.queue.lib, plan.prog
+    launch = _Launch(plan)
+    tiles, quads = _shape(plan)
+    mats, at, rows, cursor = _copy_units(plan, tiles, quads), {}, [], 0
+    for key, (units, _) in mats.items():
+        at[key] = (cursor, units)
+        rows.append(key + (cursor, 4 * tiles, quads, units))
+        cursor += key[2] * units
+    dev_mats = to_device(queue, np.array(rows, dtype=np.int32))
+    dev_at = empty_device(queue, 16 * cursor)
+    max_rows = max(r[2] for r in rows)
+    bits = lambda v: int(np.float32(v).view(np.int32))
+    per_group = WG // (4 * tiles)
+    records, item_of = [], []
+    full, most = 32, 0
+    for b in plan.members:
+        g, d = prog.geometry[b], prog.geometry[b]["dots"][0]
+        M, N = g["y_len"], d["a_shape1"]
+        start, units = at[d["a_start"], d["a_stride0"], M, N]
+        first, n_targets = (0, 0) if launch.item_targets is None else (int(v) for v in launch.item_targets[b])
+        target = [int(v) for v in launch.host_targets[first][:4]] if n_targets else [0] * 4
+        coefs = [bits(v) for v in (prog.alpha[b], prog.beta[b], prog.gamma[b])]
+        if tiles <= 2:
+            full = min([full] + [max(0, min(TILE, N - TILE * t) // 4) for t in range(tiles)])
+            most = max(most, -(-min(N, TILE) // 4))
+            for r in range(M):
+                records.append([start + r * units, d["x_start"], N, n_targets, g["y_start"] + r * g["y_stride0"],
+                                g["y_in_start"] + r * g["y_in_stride0"], first, r] + coefs + [0] + target)
+                item_of.append(b)
+        else:
+            for r in range(0, M, per_group):
+                records.append([start, units, N, d["x_start"], d["x_stride0"], r, min(per_group, M - r), n_targets,
+                                g["y_start"], g["y_stride0"], g["y_in_start"], g["y_in_stride0"]]
+                               + coefs + [first] + target + [0] * 12)
+                item_of.append(b)
+    if tiles <= 2:  # whole groups: more of the last row, that store nothing
+        pad = list(records[-1])
+        pad[3] = -1
+        records += [pad] * (-len(records) % per_group)
+    records, item_of = np.array(records, dtype=np.int32), np.array(item_of)
+    n_groups = len(records) // per_group if tiles <= 2 else len(records)
+    dev_records = to_device(queue, records)
+
+    def again():
+        _lib.check(lib.nhip_lay_out_dots(queue.handle, dev_mats.ptr, len(rows), max_rows, launch.A, dev_at.ptr),
+                   "laying out matrices")
+
+    again()
+    plan.lay_out_again = again
+    carried = getattr(plan, "carried", None)
+    plan.laid_out = (lib.nhip_gemv_dots, (
+        tiles, quads, launch.order, dev_records.ptr, n_groups, dev_at.ptr, launch.X,
+        launch.targets.ptr if launch.targets is not None else dev_records.ptr, full if tiles <= 2 else 0, most))
+    plan.full_args = tuple(plan.full_args) + (dev_mats, dev_at, dev_records)
+    plan.gsize = (WG * n_groups + (carried.gsize[0] if carried is not None else 0),)
+    plan.lsize = (WG,)
+    plan.tag = "%s, laid out" % plan.tag
+    plan.host_records = records
+
+    def upload_x_bits():
+        """The spikes of some items are bits now (`hipra_gemv.store_spikes_as_bits`)."""
+        value = dict(zip(plan.event_record_item.tolist(), plan.event_table[:, 15].tolist()))
+        records[:, 20] = [value[b] for b in item_of.tolist()]
+        dev_records.set(records.ravel())
+
+    plan.upload_x_bits = upload_x_bits
+    return True

@@ -1367,6 +1367,8 @@ def store_spikes_as_bits(enc_plan, items, event_records, dt):
             enc_plan.upload_pops()
         for plan in touched:
             plan.dev_event_table.set(plan.event_table.astype(np.int32).ravel())
+            if getattr(plan, "laid_out", None) is not None:
+                plan.upload_x_bits()
         enc_plan.tag = "%s + spikes as bits" % enc_plan.tag
     return values
 
@@ -1882,6 +1884,7 @@ def fuse_linearfilter(gemv_plans, lf_plan, second_order=False):
             fused.event_table, fused.event_driven = table, True
             fused.dev_event_table = dev_table
             fused.event_record_item = plan.event_record_item
+            fused.filter_tables = (item_targets, dev_targets, F, targets)
             fused.host_tasks = None
             _keep_filter_state(fused, filter_state)
             return fused

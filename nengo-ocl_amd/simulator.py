@@ -88,9 +88,9 @@ class HipBackend:
         from . import hipra_resident
 
         self._resident = hipra_resident
-        from . import hipra_lanes
+        from . import hipra_dots, hipra_lanes
 
-        self._lanes = hipra_lanes
+        self._lanes, self._dots = hipra_lanes, hipra_dots
         # switch for measurements: "0" reads the matrices of every launch as they lie among the signals
         self.lays_out_matrices = os.environ.get("NENGO_HIP_LAY_OUT", "1") != "0"
         # switch for measurements: "0" replays small networks as graphs too
@@ -143,10 +143,13 @@ class HipBackend:
 
     def laid_out_spans(self, plan):
         """Where the matrices lie that `lay_out_matrices` would give the launch `plan` copies of, or None."""
-        return self._lanes.matrix_spans(plan) if self.lays_out_matrices and hasattr(plan, "prog") else None
+        if not self.lays_out_matrices or not hasattr(plan, "prog"):
+            return None
+        spans = self._lanes.matrix_spans(plan)
+        return self._dots.matrix_spans(plan) if spans is None else spans
 
     def lay_out_matrices(self, plan):
-        return self._lanes.lay_out(plan)
+        return (self._dots if self._lanes.matrix_spans(plan) is None else self._lanes).lay_out(plan)
 
     def store_spikes_as_bits(self, enc_plan, items, event_records, dt):
         return self._gemv.store_spikes_as_bits(enc_plan, items, event_records, dt)
@@ -740,8 +743,8 @@ class Simulator:
         return [plan]
 
     def _lay_out_matrices(self, plans):
-        """Launches of products with constant matrices (encoders) that update neurons read copies of them in
-        their own order (`hipra_lanes.lay_out`): where nothing of the model writes the matrices.  A write of
+        """Launches of products with constant matrices (encoders, decoders) read copies of them in their own order
+        (`hipra_lanes.lay_out`, `hipra_dots.lay_out`): where nothing of the model writes the matrices.  A write of
         the host brings the copies up to date (`_constant_written`)."""
         if self.reference_host_state:
             return

@@ -25,7 +25,7 @@ def network(n, d, neuron, seed=3):
 
 
 def laid_out(sim):
-    return [p for p in sim._plans if getattr(p, "laid_out", None) is not None]
+    return [p for p in sim._plans if getattr(p, "laid_out", None) is not None and hasattr(p, "host_pops")]
 
 
 @pytest.mark.gpu
