@@ -301,3 +301,53 @@ def carry_sequences(plans):
         carrier.writes_mem = carrier.writes_mem | seq.writes_mem
         del plans[k]  # (the same index now holds the next plan)
     return plans
+
+
+# us of an operation inside a carried chain (a trip to memory and back behind the barrier; table playback looks up
+# the step before it reads), for dividing chains over launches
+OP_US, PLAYBACK_US = 0.9, 1.2
+
+
+def divide_chains(plans):
+    """What the longest chain of a carried sequence begins with moves to an earlier launch, where the one that carries
+    it is short.
+
+    An operation of a chain waits for the one before it: clock, input playback and the input's filter take 4.6 us
+    in a launch whose rows take 2.1 (34 x 16 rows of 1,000 columns) to 2.9 (50 x 32 of 2,000). The first
+    ones run in the launch before as well: 32 x 1000 x 16 adaptive neurons 9.4 -> 7.4 us a step, 256 x 100 in a small
+    world 9.5 -> 7.7, 48 x 2000 x 32 rate neurons 10.3 -> 9.5. Launches of large matrices (256 x 4096 x 64: 12 us, learned
+    decoders: 20) hide the chain."""
+    for j, carrier in enumerate(plans):
+        seq = getattr(carrier, "carried", None)
+        if seq is None or not (getattr(carrier, "laid_out", None) is not None
+                               or getattr(carrier, "kernel_class", (None,))[0] == 2):
+            continue
+        chain = max(chains_of(seq.members), key=len)
+        if len(chain) < 2:
+            continue
+        cost = [PLAYBACK_US if sequence_op(p)[0] == SEQ_PRESENTINPUT else OP_US for p in chain]
+        best = min(range(1, len(chain)), key=lambda n: (max(sum(cost[:n]), sum(cost[n:])), -n))
+        for n in range(best, 0, -1):
+            first = chain[:n]
+            # (they move past the launch that carried them and past what is between the two)
+            q = j
+            while q >= 0 and hasattr(plans[q], "enqueue") and not any(_conflict(p, plans[q]) for p in first if q != j):
+                if q < j and _can_carry(plans[q], sequence_needs(first)) and plans[q].divided is None:
+                    break
+                q -= 1
+            else:
+                continue
+            if q < 0:
+                continue
+            head = plan_sequence(seq.queue, first)
+            rest = [p for p in seq.members if p not in first]
+            tail = plan_sequence(seq.queue, rest) if rest else None
+            arm = lambda s: () if s is None else (
+                (s.queue.lib.nhip_gemv_tile_carry, tuple(s.args) + (s.needs,)),)
+            plans[q].divided, carrier.divided = arm(head), arm(tail)
+            for plan, part in ((plans[q], head), (carrier, tail)):
+                plan.full_args, plan.runs = tuple(plan.full_args) + (part,), part
+                plan.tag = "%s [runs %s]" % (plan.tag, part.tag if part is not None else "nothing else")
+            plans[q].reads_mem = plans[q].reads_mem | head.reads_mem
+            plans[q].writes_mem = plans[q].writes_mem | head.writes_mem
+            break

@@ -83,6 +83,9 @@ class Plan(BasePlan):
         # (function, arguments) of another entry point that does the same work from copies of constant
         # matrices in its own order (`hipra_lanes.lay_out`); `kern` and `args` stay what the launch was planned as
         self.laid_out = None
+        # the calls made instead of `prelude` where the sequence that the launch was to carry is divided over
+        # several launches (`hipra_sequence.divide_chains`)
+        self.divided = None
 
     @staticmethod
     def _format_size(size):
@@ -108,8 +111,9 @@ class Plan(BasePlan):
                 _lib.check(lib.nhip_time_next_launch(ev0, ev1))
             else:
                 _lib.check(lib.nhip_event_record(ev0, handle))
-        if self.prelude is not None:
-            _lib.check(self.prelude[0](*self.prelude[1]), self.name)
+        preludes = self.divided if self.divided is not None else (self.prelude,) if self.prelude else ()
+        for call, arguments in preludes:
+            _lib.check(call(*arguments), self.name)
         kern, args = self.laid_out or (self.kern, self.args)
         _lib.check(kern(handle, *args), self.name)
         if profiling:

@@ -103,6 +103,7 @@ class HipBackend:
         self.merge_small_plans = hipra_sequence.merge_small_plans
         if os.environ.get("NENGO_HIP_CARRY_SEQUENCES", "1") != "0":  # switch for measurements
             self.carry_sequences = hipra_sequence.carry_sequences
+            self.divide_chains = hipra_sequence.divide_chains
             self.carrier_of = hipra_sequence.carrier_of
         self.plans_conflict = hipra_sequence._conflict
         self.fuse_conv_neurons = hipra_nonlinearities.fuse_conv_neurons
@@ -575,6 +576,8 @@ class Simulator:
         self._laid_out = []  # (base signals of constants, launch that reads copies of them)
         if fuse and resident is None and hasattr(self.backend, "lay_out_matrices"):
             self._lay_out_matrices(plans)
+            if merge_small and hasattr(self.backend, "carry_sequences"):
+                self.backend.divide_chains(plans)
         self._store_spikes_as_bits(plans)
         if fuse and hasattr(self.backend, "share_spike_bits"):
             self._share_spike_bits(plans)

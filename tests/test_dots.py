@@ -115,3 +115,18 @@ def test_records_cover_every_row_once(monkeypatch, n, m):
                 assert len(records) == n_groups and records[:, 6].max() <= 64 // tiles
                 assert sorted(y + (r + k) * stride for y, stride, r, count in records[:, [8, 9, 5, 6]].tolist()
                               for k in range(count)) == rows
+
+
+def test_chains_divided_over_launches(monkeypatch):
+    """What a chain of short operations begins with rides in the launch before the one that carries the rest."""
+    from nengo_ocl_amd import configs
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    net = configs.c2_watts_strogatz(1, n_ens=64, n_neurons=100, n_driven=2)[0]
+    with Simulator(net, seed=1, event_calibration_steps=0) as sim:
+        runs = [[p.name for p in q.runs.members] for q in sim._plans if getattr(q, "runs", None) is not None]
+        assert len(runs) == 2 and runs[0] == ["hip_timeupdate", "hip_presentinput"], runs
+        assert "hip_linearfilter" in runs[1]
+        whole, = [q.carried for q in sim._plans if getattr(q, "carried", None) is not None]
+        assert sorted(runs[0] + runs[1]) == sorted(p.name for p in whole.members)
