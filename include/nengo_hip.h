@@ -33,7 +33,7 @@
 extern "C" {
 #endif
 
-#define NHIP_ABI_VERSION 2
+#define NHIP_ABI_VERSION 3
 
 #define NHIP_E_BADARG (-1)   /* null pointer / negative count / unknown mode   */
 #define NHIP_E_BADCLASS (-2) /* GEMV class (lanes-per-row, vector width) unknown */
@@ -394,16 +394,17 @@ int nhip_resident(void *stream, const void *spans, int n_spans, const void *ops,
  * order.  One dot product per item, reference order; X may not overlap what the launch writes, except by
  * the outputs of `filters`, and nothing but the item and the rule of a learned matrix may read any part of it
  * here: other groups write it back while theirs still run.
- *   tasks   : int32[n_tasks][24] {a_start, a_stride0, N, x_start, y_start, y_stride0, yin_start,
+ *   tasks   : int32[n_tasks][32] (on a 64-byte boundary) {a_start, a_stride0, N, x_start, y_start, y_stride0, yin_start,
  *             yin_stride0, alpha, beta, gamma (float bits), row0, n_rows (1..4), learned (0: the matrix
  *             stays), first_target, n_targets, then the rule: kind, pre_start, post_start, post_stride0,
- *             theta_start, theta_stride0 (BCM), alpha, beta (float bits)}: rows row0 .. row0 + n_rows - 1 of an
+ *             theta_start, theta_stride0 (BCM), alpha, beta (float bits), then the item's first target (4
+ *             words) and four zeros}: rows row0 .. row0 + n_rows - 1 of an
  *             item; row i of the matrix changes by the rule's element of X[pre_start + j],
  *             X[post_start + i * post_stride0] (and theta, or the old weight)
  *   targets, F : filters of the fresh y, as for nhip_gemv_tile_filter (orders 1 and 2)
- *   filters : int32[n_filters][8] {s_start, f_start, n, has_a, a0, b0 (float bits), 0, 0}: stepped on
+ *   filters : int32[max(n_filters, 2)][8] (on a 64-byte boundary) {s_start, f_start, n, has_a, a0, b0 (float bits), 0, 0}: stepped on
  *             X[s_start ..], F[f_start ..] when every row has read the old F; F and X one buffer
- *   arrived : one int, zero before the launch and after it (only read with n_filters > 0)
+ *   arrived : int32[33 * 32], zero before the launch and after it (only read with n_filters > 0)
  * Bit-identical to the separate calls. */
 int nhip_gemv_learn(void *stream, const int *tasks, int n_tasks, float *A,
                     const float *X, const float *Yin, float *Y, const int *targets, float *F,

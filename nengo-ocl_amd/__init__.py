@@ -11,7 +11,7 @@ import logging
 
 from .version import version as __version__
 
-ABI_VERSION = 2  # must equal NHIP_ABI_VERSION in include/nengo_hip.h
+ABI_VERSION = 3  # must equal NHIP_ABI_VERSION in include/nengo_hip.h
 
 logging.getLogger(__name__).addHandler(logging.NullHandler())
 

@@ -1633,7 +1633,7 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
         if getattr(plan, "filter_tables", None) is not None:
             if item_targets is not None and plan.filter_tables[0] is not item_targets:
                 return None
-            item_targets, dev_targets, F, _ = plan.filter_tables
+            item_targets, dev_targets, F, host_targets = plan.filter_tables
             filtered = plan
         elif plan.name.endswith("_filter"):
             return None
@@ -1672,11 +1672,13 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
         g = geometry[b]
         d = g["dots"][0]
         first, n = (0, 0) if item_targets is None else (int(v) for v in item_targets[b])
+        target = tuple(int(v) for v in host_targets[first][:4]) if n else (0,) * 4
         for row0 in range(0, g["y_len"], per_group):
             tasks.append((d["a_start"], d["a_stride0"], d["a_shape1"], d["x_start"], g["y_start"], g["y_stride0"],
                           g["y_in_start"], g["y_in_stride0"], bits(prog.alpha[b]), bits(prog.beta[b]),
                           bits(prog.gamma[b]), row0, min(per_group, g["y_len"] - row0), int(b in rule_of), first, n)
-                         + (tuple(int(v) for v in rules[rule_of[b]]) if b in rule_of else (0,) * 8))
+                         + (tuple(int(v) for v in rules[rule_of[b]]) if b in rule_of else (0,) * 8)
+                         + target + (0,) * 4)
     if not tasks:
         return None
     filters, moved, rest = [], [], []
@@ -1694,8 +1696,8 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
                 moved.append(k)
         rest = [k for k in range(len(S)) if k not in set(moved)]
     dev_tasks = to_device(queue, np.array(tasks, dtype=np.int32))
-    dev_filters = to_device(queue, np.array(filters or [(0,) * 8], dtype=np.int32))
-    arrived = to_device(queue, np.zeros(4, dtype=np.int32))
+    dev_filters = to_device(queue, np.array((filters + [(0,) * 8] * 2)[:max(2, len(filters))], dtype=np.int32))
+    arrived = to_device(queue, np.zeros(33 * 32, dtype=np.int32))
     lib = queue.lib
     targets = dev_targets if dev_targets is not None else dev_tasks  # (not read without targets)
     total = lambda attr: sum(getattr(p, attr) or 0 for p in list(products) + [rule_plan])

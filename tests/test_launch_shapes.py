@@ -647,6 +647,14 @@ def test_rules_between_neurons_in_the_launch_of_their_product(queue, rule, n_pre
                 assert np.array_equal(gpu.data[p], cpu.data[p_o], equal_nan=True)
 
 
+# fewer columns than a quad and one behind it, one group more than there are counters of arrivals, an odd
+# remainder behind a whole pass
+@pytest.mark.parametrize("n_pre,n_post", [(1, 5), (2, 9), (3, 129), (5, 133), (2051, 7)])
+@pytest.mark.parametrize("rule", ["Oja", "BCM"])
+def test_learned_rows_that_do_not_end_with_a_quad(queue, rule, n_pre, n_post):
+    test_rules_between_neurons_in_the_launch_of_their_product(queue, rule, n_pre, n_post, False)
+
+
 @pytest.mark.parametrize("rule", ["Oja", "BCM"])
 @pytest.mark.parametrize("rows,cols", [(slice(0, 150), slice(None)), (slice(None), slice(20, 200)),
                                        (slice(7, 8), slice(None))])
