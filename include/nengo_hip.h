@@ -410,6 +410,21 @@ int nhip_gemv_learn(void *stream, const int *tasks, int n_tasks, float *A,
                     const float *X, const float *Yin, float *Y, const int *targets, float *F,
                     const int *filters, int n_filters, int *arrived);
 
+/* The same without filters of activities, for the rule of kind 16 too, W += (alpha post) (x) pre with every product
+ * and sum rounded on its own, and with further items whose matrices nothing writes and whose vectors are mostly
+ * zero: only the columns whose x is not zero are visited.
+ *   items   : int32[n_items][32] (on a 64-byte boundary) {at_start, mp, M (<= 64), N, x_start, y_start, y_stride0,
+ *             yin_start, yin_stride0, alpha, beta, gamma (float bits), first_target, n_targets, row0 (first of the
+ *             record's M rows), all (not zero: every column is visited), the first target (4 words), 12 zeros}
+ *   AT      : columns of their matrices (nhip_lay_out_columns): element (r, c) at AT[at_start + c * mp + r] */
+int nhip_gemv_learn_events(void *stream, const int *tasks, int n_tasks, float *A, const float *X, const float *Yin,
+                           float *Y, const int *targets, float *F, const int *items, int n_items, const float *AT);
+/* matrices: int32[n][8] {a_start, a_stride0, M, N, out, mp, first_record, n_records}: column c to AT[out + c * mp ..],
+ * mp >= M a multiple of 16; where a matrix holds an infinity or a NaN `all` of the records first_record .. is set.
+ * max_cols: the largest N. */
+int nhip_lay_out_columns(void *stream, const int *matrices, int n, int max_cols, const float *A, float *AT,
+                         int *records);
+
 /* ---- sparse matrix-vector products -----------------------------------------
  * Y[b] (=|+=) A[b] @ X[b] for many sparse matrices in one launch.
  * replaces: `plan_sparse_dot_inc` / `spmv_csr_impl` / `spmv_ellpack_impl`

@@ -1,4 +1,4 @@
-// Products with matrices that Oja's or the BCM rule changes in the same step.
+// Products with matrices that a learning rule (Oja's, the BCM rule, an outer product: PES) changes in the same step.
 //
 // As launches of their own, a step of such a matrix reads it for the product, reads and writes it for the
 // rule, and a third launch steps the filters of the activities the rule reads (2000 x 2000: 8.0 + 10.4 + 4.7
@@ -51,6 +51,7 @@ struct LearnFilter {
 };
 static_assert(sizeof(LearnTask) == 128 && sizeof(LearnFilter) == 32, "tables");
 
+constexpr int LEARN_OUTER = 16;                // kind of rule besides NHIP_RULE_*: W += (alpha post) (x) pre
 constexpr int LROWS = NHIP_WG / NHIP_WAVE;     // rows of a group
 constexpr int LTILE = 128, LTILES = 16;        // columns of a tile, tiles of a pass
 constexpr int LSTRIDE = LTILE + 4;             // words between tiles in LDS
@@ -60,6 +61,13 @@ typedef float learn_f4 __attribute__((ext_vector_type(4)));
 typedef float learn_q4 __attribute__((ext_vector_type(4), aligned(4)));  // at any element of a row
 typedef int learn_i16 __attribute__((ext_vector_type(16)));
 #define LEARN_INLINE __attribute__((always_inline))
+
+// LDS written by some lanes of a wave is read by others
+__device__ __forceinline__ void learn_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 __device__ __forceinline__ int learn_lds(int c) { return (c >> 7) * LSTRIDE + (c & (LTILE - 1)); }
 
@@ -140,7 +148,9 @@ __device__ __forceinline__ void learn_rows(const LearnTask& task, const float* s
         }
         if (c0 + LCOLS >= task.N) read();
         if (mine) {
+            const float scale = __fmul_rn(rule.alpha, post);  // (the outer product's)
             auto changed = [&](float p, float e) LEARN_INLINE {
+                if constexpr (RULE == LEARN_OUTER) return __fadd_rn(e, __fmul_rn(scale, p));
                 if constexpr (RULE == NHIP_RULE_BCM || RULE == NHIP_RULE_OJA)
                     return __fadd_rn(e, learn_element<RULE>(rule.alpha, rule.beta, 0.0f, 0.0f, p, post,
                                                             RULE == NHIP_RULE_BCM ? theta : e));
@@ -164,9 +174,7 @@ __device__ __forceinline__ void learn_rows(const LearnTask& task, const float* s
                 if (lane < 4) lds.w[wave][learn_lds(tail)] = tail < n ? wt : -0.0f;
                 if (LEARNED && tail < n) arow[c0 + tail] = changed(pt, wt);
             }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            learn_wave_sync();
             const int at = (lane >> 2) * LSTRIDE + (lane & 3);  // partial sum lane & 3 of tile lane >> 2
             float s = 0.0f;
 #pragma unroll
@@ -182,10 +190,159 @@ __device__ __forceinline__ void learn_rows(const LearnTask& task, const float* s
     } while (c0 < task.N);
 }
 
+// Up to 64 rows of an item whose matrix nothing writes and whose vector is mostly zero (spikes): only the columns whose
+// x is not zero are read, from a copy of the columns.  (A column left out would add zeros to its partial sum.)
+struct ColumnsItem {
+    int at_start, mp;              // column c: AT[at_start + c * mp ..], mp a multiple of 16
+    int M, N, x_start;
+    int y_start, y_stride0, yin_start, yin_stride0;  // of the item's first row
+    float alpha, beta, gamma;
+    int first_target, n_targets;
+    int row0;                      // first row of this record (at_start is that of row 0)
+    int all;                       // not zero: the columns whose x is zero count too (the matrix holds an infinity or a NaN)
+    FilterTarget target;
+    int pad[12];
+};
+static_assert(sizeof(ColumnsItem) == 128, "table");
+struct LearnEvents {
+    const ColumnsItem* items;
+    const float* AT;
+    int n_items;
+};
+
+constexpr int CTILES = 32, CCOLS = CTILES * LTILE;  // tiles and columns of a pass
+constexpr int CBATCH = 20, CPART = 4;               // columns of a tile requested together; added together
+struct ColumnsLds {
+    uint2 list[CTILES][LTILE];     // active columns of a tile in order: byte offset | column % 4, x
+    float tile[CTILES][NHIP_WAVE];
+    int count[CTILES];
+};
+
+// A group per record.  A wave lists the active columns of its tiles; then 16, 32 or 64 lanes (as many as there are
+// rows) take a tile, and request 20 columns each of two tiles together: 128 neurons of which 8 % spike have
+// ten.  192 such items of 32 x 2000 beside 2,048 learned rows of 2,000: the launch 11.0 us, 16.6 with the walk of
+// csrc/gemv_events.hip (a column a wave at a time) in groups of this size, 12.8 with these groups behind those
+// of rows, whose requests theirs then wait behind; 22.0 with every column read (gemv_stream_kernel).  From the first
+// group's start: lists at 2.2 us, columns requested at 4.3 (behind the rows' on their way), there at 4.6, added at 6.4,
+// done at 7.3; the rows beside them at 6.0.
+__device__ __forceinline__ void columns_group(const ColumnsItem& it, const float* __restrict__ AT, const float* X,
+                                              const float* Yin, float* Y, const FilterArgs& filter, ColumnsLds& lds,
+                                              int wave, int lane) {
+    const int lg = it.M <= 16 ? 4 : it.M <= 32 ? 5 : 6, workers = NHIP_WAVE >> lg;  // lanes of a tile; tiles at once
+    const int me = lane >> lg, at_row = lane & ((1 << lg) - 1);
+    const char* at = reinterpret_cast<const char*>(AT + it.at_start + it.row0 + min(at_row, it.M - 1));
+    const unsigned col_bytes = 4u * (unsigned)it.mp;
+    const int row = it.row0 + min(lane, it.M - 1);
+    const float* y_at = Yin + it.yin_start + (size_t)row * it.yin_stride0;
+    const float* f_at = filter.F + (it.n_targets > 0 ? (size_t)it.target.y_start + row : 0);
+    float y_old = 0.0f, f_old = 0.0f, sum = 0.0f;
+    int base = 0;
+    do {
+        const int n_cols = min(it.N - base, CCOLS), n_tiles = (n_cols + LTILE - 1) / LTILE;
+        const int per_wave = (n_tiles + LROWS - 1) / LROWS;
+        const int t_lo = min(wave * per_wave, n_tiles), t_hi = min(t_lo + per_wave, n_tiles);
+        for (int t0 = t_lo; t0 < t_hi; t0 += 4) {  // (up to 2,048 columns: once)
+            float xv[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                xv[u] = X[it.x_start + base + min(t0 * LTILE + u * NHIP_WAVE + lane, n_cols - 1)];
+            y_old = *y_at;  // (the first wave's, which has tiles)
+            f_old = *f_at;
+            int found = 0;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int t = t0 + (u >> 1), c = t0 * LTILE + u * NHIP_WAVE + lane;
+                if (t >= t_hi) break;  // uniform
+                const bool active = c < n_cols && (it.all || (__float_as_uint(xv[u]) & 0x7fffffffu) != 0u);
+                const unsigned long long b = __ballot(active);
+                if ((u & 1) == 0) found = 0;
+                const int before = found + __builtin_amdgcn_mbcnt_hi((unsigned)(b >> 32),
+                                                                     __builtin_amdgcn_mbcnt_lo((unsigned)b, 0));
+                if (active)
+                    lds.list[t][before] = make_uint2((unsigned)(base + c) * col_bytes | (unsigned)(c & 3),
+                                                     __float_as_uint(xv[u]));
+                found += __popcll(b);
+                if ((u & 1) && lane == 0) lds.count[t] = found;
+            }
+        }
+        learn_wave_sync();
+        for (int t0 = t_lo; t0 < t_hi; t0 += 2 * workers) {
+            const int ta = t0 + me, tb = ta + workers;
+            const int na = ta < t_hi ? lds.count[ta] : 0, nb = tb < t_hi ? lds.count[tb] : 0;
+            const uint2* la = lds.list[min(ta, CTILES - 1)];
+            const uint2* lb = lds.list[min(tb, CTILES - 1)];
+            float a[CBATCH], b[CBATCH];
+            // (entries that are not there: the first column, and no sum takes it)
+            auto request = [&](const uint2* list, int n, int k, float (&v)[CBATCH]) LEARN_INLINE {
+#pragma unroll
+                for (int u = 0; u < CBATCH; ++u) {
+                    const unsigned off = list[min(k + u, LTILE - 1)].x & ~3u;  // (read whether it is there or not)
+                    v[u] = *reinterpret_cast<const float*>(at + (k + u < n ? off : 0u));
+                }
+            };
+            float s[4];
+            auto add = [&](const uint2* list, int n, int k, const float (&v)[CBATCH]) LEARN_INLINE {
+#pragma unroll
+                for (int p = 0; p < CBATCH; p += CPART)
+                    if (__any(k + p < n))
+#pragma unroll
+                        for (int u = p; u < p + CPART; ++u) {
+                            const uint2 e = list[min(k + u, LTILE - 1)];
+                            const int j = k + u < n ? (int)(e.x & 3u) : 4;
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) {
+                                const float next = fmaf(v[u], __uint_as_float(e.y), s[q]);
+                                s[q] = j == q ? next : s[q];
+                            }
+                        }
+            };
+            auto finish = [&](int t, const uint2* list, int n, float (&v)[CBATCH]) LEARN_INLINE {
+                s[0] = s[1] = s[2] = s[3] = 0.0f;
+                add(list, n, 0, v);
+                for (int k = CBATCH; __any(k < n); k += CBATCH) {
+                    request(list, n, k, v);
+                    add(list, n, k, v);
+                }
+                if (t < t_hi) lds.tile[t][at_row] = it.alpha * ((s[0] + s[2]) + (s[1] + s[3]));
+            };
+            request(la, na, 0, a);
+            request(lb, nb, 0, b);
+            finish(ta, la, na, a);
+            finish(tb, lb, nb, b);
+        }
+        __syncthreads();
+        if (wave == 0) {
+            if (base == 0) sum = it.beta * y_old;
+#pragma unroll
+            for (int h = 0; h < CTILES; h += 16) {
+                float v[16];
+#pragma unroll
+                for (int t = 0; t < 16; ++t) v[t] = lds.tile[h + t][lane];  // (16 reads at once)
+#pragma unroll
+                for (int t = 0; t < 16; ++t)
+                    if (h + t < n_tiles) sum = sum + v[t];
+            }
+        }
+        base += CCOLS;
+        if (base < it.N) __syncthreads();  // read, before the next pass
+    } while (base < it.N);
+    if (wave == 0 && lane < it.M) {
+        const float y = sum + it.gamma;
+        Y[it.y_start + (size_t)row * it.y_stride0] = y;
+        if (it.n_targets > 0) {
+            filter.F[(size_t)it.target.y_start + row] = filter_step<true>(filter.targets, it.target, row, y, f_old);
+            filter_epilogue<true>(filter, make_int2(it.first_target + 1, it.n_targets - 1), row, y);
+        }
+    }
+}
+
+// EVENTS: there are such items (their groups before those of rows: they take longer)
+template <bool EVENTS>
 __global__ __launch_bounds__(NHIP_WG) void gemv_learn_kernel(
     const LearnTask* tasks, float* A, const float* X, const float* Yin, float* Y,
-    FilterArgs filter, const LearnFilter* filters, int n_filters, int* arrived, RowsSide side)
+    FilterArgs filter, const LearnFilter* filters, int n_filters, int* arrived, LearnEvents events, RowsSide side)
 {
+    static_assert(sizeof(ColumnsLds) <= sizeof(LearnLds), "one piece of LDS for both");
     __shared__ LearnLds lds;
     const int tid = threadIdx.x, lane = tid & (NHIP_WAVE - 1);
     if ((int)blockIdx.x < side.n_chains) {  // a carried sequence first: it takes longer than a group's rows
@@ -199,7 +356,20 @@ __global__ __launch_bounds__(NHIP_WG) void gemv_learn_kernel(
         return;
     }
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int group = (int)blockIdx.x - side.n_chains;
+    int group = (int)blockIdx.x - side.n_chains;
+    if (EVENTS && group < events.n_items) {
+        typedef const __attribute__((address_space(4))) learn_i16 const_i16;
+        const const_i16* at = reinterpret_cast<const const_i16*>(
+            reinterpret_cast<uintptr_t>(events.items + group));
+        learn_i16 w0 = at[0], w1 = at[1];
+        asm volatile("" : "+s"(w0), "+s"(w1));
+        struct Words { learn_i16 a, b; };
+        const Words words = {w0, w1};
+        columns_group(__builtin_bit_cast(ColumnsItem, words), events.AT, X, Yin, Y, filter,
+                      *reinterpret_cast<ColumnsLds*>(&lds), wave, lane);
+        return;
+    }
+    if (EVENTS) group -= events.n_items;
     // (constant address space: the whole record, and those of the filters, at once)
     typedef const __attribute__((address_space(4))) learn_i16 const_i16;
     const const_i16* at = reinterpret_cast<const const_i16*>(reinterpret_cast<uintptr_t>(tasks + group));
@@ -227,7 +397,7 @@ __global__ __launch_bounds__(NHIP_WG) void gemv_learn_kernel(
     // the word behind them.
     auto read = [&]() LEARN_INLINE {
         if (n_filters > 0 && tid == 0) {
-            const int n_groups = (int)gridDim.x - side.n_chains, mine = group % LCOUNTERS;
+            const int n_groups = side.n_gemv_groups, mine = group % LCOUNTERS;
             auto tell = [&](int counter, int expected) {  // the last of `expected`? (it clears the word for the next launch)
                 int* word = arrived + counter * LCOUNTER_WORDS;
                 if (__hip_atomic_fetch_add(word, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != expected - 1) return 0;
@@ -243,6 +413,7 @@ __global__ __launch_bounds__(NHIP_WG) void gemv_learn_kernel(
                                           f_at, f_first, sum, read);
     };
     if (!task.learned) rows(std::integral_constant<int, 0>{});
+    else if (task.rule.kind == LEARN_OUTER) rows(std::integral_constant<int, LEARN_OUTER>{});
     else if (task.rule.kind == NHIP_RULE_BCM) rows(std::integral_constant<int, NHIP_RULE_BCM>{});
     else rows(std::integral_constant<int, NHIP_RULE_OJA>{});
     if (mine) {
@@ -311,11 +482,39 @@ __global__ __launch_bounds__(NHIP_WG) void gemv_learn_kernel(
     }
 }
 
-}  // namespace
+// Matrix a_start, a_stride0, M x N of A -> its columns, mp floats apart, from `out` of AT on; the records of the items
+// first_record .. are told where it holds an infinity or a NaN (products of those with zeros count)
+struct LearnColumns { int a_start, a_stride0, M, N, out, mp, first_record, n_records; };
 
-extern "C" int nhip_gemv_learn(void* stream, const int* tasks, int n_tasks, float* A,
-                               const float* X, const float* Yin, float* Y, const int* targets, float* F,
-                               const int* filters, int n_filters, int* arrived) {
+__global__ __launch_bounds__(NHIP_WG) void lay_out_columns_kernel(const LearnColumns* __restrict__ mats, const float* A,
+                                                                  float* AT, ColumnsItem* records) {
+    constexpr int T = NHIP_WAVE;  // rows and columns of a block
+    __shared__ float block[T][T + 1];
+    const LearnColumns m = mats[blockIdx.y];
+    const int lane = threadIdx.x & (T - 1), wave = threadIdx.x >> 6;
+    bool odd = false;
+    for (int c0 = blockIdx.x * T; c0 < m.N; c0 += gridDim.x * T)
+        for (int r0 = 0; r0 < m.mp; r0 += T) {
+            __syncthreads();
+            for (int r = wave; r < T; r += NHIP_WG / T) {
+                const bool inside = r0 + r < m.M && c0 + lane < m.N;
+                const float v = inside ? A[m.a_start + (size_t)(r0 + r) * m.a_stride0 + c0 + lane] : 0.0f;
+                odd |= (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u;
+                block[r][lane] = v;
+            }
+            __syncthreads();
+            for (int c = wave; c < T; c += NHIP_WG / T)
+                if (c0 + c < m.N && r0 + lane < m.mp)
+                    AT[(size_t)m.out + (size_t)(c0 + c) * m.mp + r0 + lane] = block[lane][c];
+        }
+    if (odd)
+        for (int i = 0; i < m.n_records; ++i) records[m.first_record + i].all = 1;
+}
+
+template <typename Launch>
+int learn_launch(void* stream, const int* tasks, int n_tasks, float* A, const float* X, const float* Yin, float* Y,
+                 const int* targets, float* F, const int* filters, int n_filters, int* arrived, int n_more,
+                 Launch&& launch) {
     RowsSide side;
     if (take_carried(side) && n_tasks <= 0) return NHIP_E_BADARG;  // an empty launch cannot carry it
     if (n_tasks == 0) return 0;
@@ -327,10 +526,48 @@ extern "C" int nhip_gemv_learn(void* stream, const int* tasks, int n_tasks, floa
     FilterArgs filter{};
     filter.targets = reinterpret_cast<const FilterTarget*>(targets);
     filter.F = F;
-    NHIP_LAUNCH(gemv_learn_kernel, dim3(n_tasks + side.n_chains), dim3(NHIP_WG), 0,
-                static_cast<hipStream_t>(stream), reinterpret_cast<const LearnTask*>(tasks),
-                A, X, Yin, Y, filter,
-                reinterpret_cast<const LearnFilter*>(filters), n_filters, arrived, side);
+    launch(dim3(n_tasks + n_more + side.n_chains), filter, side);
+    NHIP_LAUNCH_CHECK();
+    return 0;
+}
+
+}  // namespace
+
+extern "C" int nhip_gemv_learn(void* stream, const int* tasks, int n_tasks, float* A,
+                               const float* X, const float* Yin, float* Y, const int* targets, float* F,
+                               const int* filters, int n_filters, int* arrived) {
+    return learn_launch(stream, tasks, n_tasks, A, X, Yin, Y, targets, F, filters, n_filters, arrived, 0,
+                        [&](dim3 grid, const FilterArgs& filter, const RowsSide& side) {
+        NHIP_LAUNCH(gemv_learn_kernel<false>, grid, dim3(NHIP_WG), 0, static_cast<hipStream_t>(stream),
+                    reinterpret_cast<const LearnTask*>(tasks), A, X, Yin, Y, filter,
+                    reinterpret_cast<const LearnFilter*>(filters), n_filters, arrived, LearnEvents{}, side);
+    });
+}
+
+extern "C" int nhip_gemv_learn_events(void* stream, const int* tasks, int n_tasks, float* A, const float* X,
+                                      const float* Yin, float* Y, const int* targets, float* F, const int* items,
+                                      int n_items, const float* AT) {
+    if (n_items < 0 || (n_items > 0 && (!items || !AT)) || (reinterpret_cast<uintptr_t>(items) & 63)) {
+        RowsSide none;
+        take_carried(none);  // (whatever becomes of the launch)
+        return NHIP_E_BADARG;
+    }
+    return learn_launch(stream, tasks, n_tasks, A, X, Yin, Y, targets, F, nullptr, 0, nullptr, n_items,
+                        [&](dim3 grid, const FilterArgs& filter, const RowsSide& side) {
+        NHIP_LAUNCH(gemv_learn_kernel<true>, grid, dim3(NHIP_WG), 0, static_cast<hipStream_t>(stream),
+                    reinterpret_cast<const LearnTask*>(tasks), A, X, Yin, Y, filter, nullptr, 0, nullptr,
+                    (LearnEvents{reinterpret_cast<const ColumnsItem*>(items), AT, n_items}), side);
+    });
+}
+
+extern "C" int nhip_lay_out_columns(void* stream, const int* matrices, int n, int max_cols, const float* A, float* AT,
+                                    int* records) {
+    if (n == 0) return 0;
+    if (n < 0 || n > 65535 || max_cols < 1 || !matrices || !A || !AT || !records) return NHIP_E_BADARG;
+    const int blocks = (max_cols + NHIP_WAVE - 1) / NHIP_WAVE;
+    NHIP_LAUNCH(lay_out_columns_kernel, dim3(blocks < 1024 ? blocks : 1024, n), dim3(NHIP_WG), 0,
+                static_cast<hipStream_t>(stream), reinterpret_cast<const LearnColumns*>(matrices), A, AT,
+                reinterpret_cast<ColumnsItem*>(records));
     NHIP_LAUNCH_CHECK();
     return 0;
 }

@@ -1563,10 +1563,10 @@ def fuse_learning(enc_plan, dec_plan, ew_plan, lf_plan):
     for new, old in ((new_dec, dec_plan), (new_enc, enc_plan)):
         for attr in ("description", "kernel_class", "n_tasks", "members", "prog", "gemv_bytes",
                      "host_tasks", "host_pops", "dev_pops", "lif_written", "lazy_currents",
-                     "input_sums", "host_parts"):
+                     "input_sums", "host_parts", "filter_tables"):
             if hasattr(old, attr):
                 setattr(new, attr, getattr(old, attr))
-    new_dec.learned_matrices = len(learn_of_item)
+    new_dec.learned_matrices, new_dec.learn_of_item = len(learn_of_item), learn_of_item
     new_enc.deferred_filters = len(moved)
     new_enc.host_deferred = deferred
     residual = []

@@ -315,8 +315,8 @@ def divide_chains(plans):
     An operation of a chain waits for the one before it: clock, input playback and the input's filter take 4.6 us
     in a launch whose rows take 2.1 (34 x 16 rows of 1,000 columns) to 2.9 (50 x 32 of 2,000). The first
     ones run in the launch before as well: 32 x 1000 x 16 adaptive neurons 9.4 -> 7.4 us a step, 256 x 100 in a small
-    world 9.5 -> 7.7, 48 x 2000 x 32 rate neurons 10.3 -> 9.5. Launches of large matrices (256 x 4096 x 64: 12 us, learned
-    decoders: 20) hide the chain."""
+    world 9.5 -> 7.7, 48 x 2000 x 32 rate neurons 10.3 -> 9.5. Launches of large matrices (256 x 4096 x 64:
+    12 us) hide the chain."""
     for j, carrier in enumerate(plans):
         seq = getattr(carrier, "carried", None)
         if seq is None or not (getattr(carrier, "laid_out", None) is not None

@@ -88,9 +88,9 @@ class HipBackend:
         from . import hipra_resident
 
         self._resident = hipra_resident
-        from . import hipra_dots, hipra_lanes
+        from . import hipra_dots, hipra_lanes, hipra_learned
 
-        self._lanes, self._dots = hipra_lanes, hipra_dots
+        self._layouts = (hipra_lanes, hipra_dots, hipra_learned)
         # switch for measurements: "0" reads the matrices of every launch as they lie among the signals
         self.lays_out_matrices = os.environ.get("NENGO_HIP_LAY_OUT", "1") != "0"
         # switch for measurements: "0" replays small networks as graphs too
@@ -146,11 +146,10 @@ class HipBackend:
         """Where the matrices lie that `lay_out_matrices` would give the launch `plan` copies of, or None."""
         if not self.lays_out_matrices or not hasattr(plan, "prog"):
             return None
-        spans = self._lanes.matrix_spans(plan)
-        return self._dots.matrix_spans(plan) if spans is None else spans
+        return next((s for s in (layout.matrix_spans(plan) for layout in self._layouts) if s is not None), None)
 
     def lay_out_matrices(self, plan):
-        return (self._dots if self._lanes.matrix_spans(plan) is None else self._lanes).lay_out(plan)
+        return next(layout for layout in self._layouts if layout.matrix_spans(plan) is not None).lay_out(plan)
 
     def store_spikes_as_bits(self, enc_plan, items, event_records, dt):
         return self._gemv.store_spikes_as_bits(enc_plan, items, event_records, dt)

@@ -1,0 +1,128 @@
+"""Decoders that PES changes in the launch that decodes with them and with others (csrc/gemv_learn.hip): whole networks
+against the CPU oracle bit for bit (the reference's order of summation), and the kernel alone, where quads, passes,
+records and batches of columns have edges, on whole numbers whose sums are exact in any order."""
+
+import numpy as np
+import pytest
+
+from helpers import assert_same_signals, host_simulators
+
+
+def learning_launch(sim):
+    plan, = [p for p in sim._plans if getattr(p, "laid_out", None) is not None
+             and p.laid_out[0].__name__ == "nhip_gemv_learn_events"]
+    return plan
+
+
+def network(n, dims):
+    from nengo_ocl_amd import configs
+
+    net, probes, _ = configs.c4_pes(1, n_triples=2, n_neurons=n, dims=dims, learning_rate=1e-3)
+    return net, list(probes.values())
+
+
+# whole and partial tiles, one to three passes of rows, two of columns
+SIZES = [(1024, 32), (1500, 20), (2048, 64), (2052, 32), (4100, 20)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,dims", SIZES)
+def test_learned_decoders_and_others_in_one_launch(queue, n, dims):
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    (net, probes), (net_o, probes_o) = (network(n, dims) for _ in range(2))
+    with Simulator(net, seed=1) as gpu, OracleSimulator(net_o, seed=1) as cpu:
+        assert learning_launch(gpu).laid_out[1][9] > 0
+        for steps in (1, 40):
+            gpu.run_steps(steps)
+            cpu.run_steps(steps)
+            for p, p_o in zip(probes, probes_o):
+                assert np.array_equal(gpu.data[p], cpu.data[p_o])
+            assert_same_signals(gpu, cpu)
+
+
+@pytest.mark.gpu
+def test_matrices_that_the_host_changes(queue):
+    """... to others with an infinity, and back."""
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    (net, _), (net_o, _) = (network(1024, 32) for _ in range(2))
+    with Simulator(net, seed=1) as gpu, OracleSimulator(net_o, seed=1) as cpu:
+        plan = learning_launch(gpu)
+        base = sorted((b for bases, p in gpu._laid_out if p is plan for b in bases
+                       if b not in gpu._shared), key=gpu.all_bases.index)[0]
+        for value in (2.5e-3, np.inf, 5e-4):
+            for sim in (gpu, cpu):
+                sig = sim.all_bases[gpu.all_bases.index(base)]  # (the two lay their signals out in the same order)
+                new = np.linspace(-1e-3, 1e-3, 32 * 1024).reshape(32, 1024)
+                new[3, 7] = value
+                sim.signals[sig] = new
+                sim.run_steps(5)
+            got, want = gpu.signal_buffer(), cpu.signal_buffer()
+            assert np.isnan(want).any() == (value != 2.5e-3)
+            assert np.array_equal(got, want, equal_nan=True)
+
+
+# rows: 16, 32 and 64 lanes, two records; columns: less than a tile and more, one to three passes
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 64, 70])
+@pytest.mark.parametrize("N", [5, 128, 1003, 2049, 4096, 8200])
+def test_columns_beside_a_learned_row(queue, M, N):
+    """No, some (more of a tile than a batch holds) and all columns with x != 0; a matrix with an infinity."""
+    from nengo_ocl_amd import _lib
+    from nengo_ocl_amd.hipraggedarray import empty_device, to_device
+
+    rng = np.random.RandomState(M + N)
+    lib, bits = queue.lib, lambda v: int(np.float32(v).view(np.int32))
+    for share, odd in ((0.0, False), (0.08, False), (0.3, True), (1.0, False)):
+        fixed = rng.randint(-4, 5, size=(M, N)).astype(np.float32)
+        learned, rows = rng.randint(-4, 5, size=(3, N)).astype(np.float32), 3
+        x = (rng.uniform(size=N) < share) * rng.randint(1, 4, size=N).astype(np.float32)
+        f, e = (rng.randint(-3, 4, size=k).astype(np.float32) for k in (N, rows))
+        if odd:
+            fixed[M // 2, N - 1] = np.inf
+        y, y_in, old = (rng.randint(-9, 10, size=k).astype(np.float32) for k in (M + rows, M + rows, M))
+        parts = [fixed.ravel(), learned.ravel(), x, f, e, y, y_in, old]
+        at = np.concatenate([[0], np.cumsum([p.size for p in parts])])
+        B = to_device(queue, np.concatenate(parts))
+        mp = -(-M // 16) * 16
+        target = [int(at[7]), bits(-0.5), bits(2.0), 1]
+        items = np.zeros((-(-M // 64), 32), dtype=np.int32)
+        for k in range(len(items)):
+            items[k, :20] = ([0, mp, min(64, M - 64 * k), N, at[2], at[5], 1, at[6], 1, bits(2.0), bits(0.5), bits(3.0),
+                              0, 1, 64 * k, 0] + target)
+        task = np.zeros((1, 32), dtype=np.int32)
+        task[0, :24] = [at[1], N, N, at[2], at[5] + M, 1, at[6] + M, 1, bits(1.0), bits(1.0), bits(0.0), 0, rows, 1, 0, 0,
+                        16, at[3], at[4], 1, 0, 0, bits(0.5), 0]
+        dev = [to_device(queue, a) for a in (task, items, np.array([target], dtype=np.int32),
+                                             np.array([[0, N, M, N, 0, mp, 0, len(items)]], dtype=np.int32))]
+        columns = empty_device(queue, N * mp)
+        _lib.check(lib.nhip_lay_out_columns(queue.handle, dev[3].ptr, 1, N, B.ptr, columns.ptr, dev[1].ptr), "")
+        _lib.check(lib.nhip_gemv_learn_events(queue.handle, dev[0].ptr, 1, B.ptr, B.ptr, B.ptr, B.ptr, dev[2].ptr, B.ptr,
+                                              dev[1].ptr, len(items), columns.ptr), "")
+        got = np.split(np.asarray(B.get()), at[1:-1])
+        with np.errstate(invalid="ignore"):
+            want = 2 * (fixed.astype(np.float64) @ x) + 0.5 * y_in[:M] + 3
+        assert np.array_equal(got[5][:M], want.astype(np.float32), equal_nan=True), (share, odd)
+        assert np.array_equal(got[7], (2 * want + 0.5 * old).astype(np.float32), equal_nan=True)
+        assert np.array_equal(got[5][M:], (learned @ x + y_in[M:]).astype(np.float32))
+        assert np.array_equal(got[1].reshape(rows, N), learned + 0.5 * np.outer(e, f))
+
+
+@pytest.mark.parametrize("n,dims", SIZES)
+def test_records_cover_every_row_once(monkeypatch, n, dims):
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    with Simulator(network(n, dims)[0], seed=1) as sim:
+        plan = learning_launch(sim)
+        tasks, records = plan.host_learned
+        assert len(tasks) == plan.laid_out[1][1] and len(records) == plan.laid_out[1][9]
+        covered = [y + (r + k) * s for y, s, r, c in tasks[:, [4, 5, 11, 12]].tolist() for k in range(c)]
+        covered += [y + (r + k) * s for y, s, r, c in records[:, [5, 6, 14, 2]].tolist() for k in range(c)]
+        assert sorted(covered) == sorted(
+            g["y_start"] + r * g["y_stride0"] for g in (plan.prog.geometry[b] for b in plan.members)
+            for r in range(g["y_len"]))
+        assert tasks[:, 12].max() <= 4 and records[:, 2].max() <= 64 and not (records[:, 1] % 16).any()
