@@ -294,11 +294,17 @@ void gemv_lanes_kernel(const LaneTask* tasks, const lane_f4* At, float* B, const
     } else {
         auto before = [&]() LANE_INLINE {
             fetch_state();
-            if (it.pad > 0) {  // (at most 64 columns)
+            if (it.pad > 0) {
                 const float x = input_sum(min(lane, ft.dot0.N - 1));
                 xb[lane] = x;
                 // the task with the item's first rows stores the sum in the operand's place
                 if (row0 == 0 && lane < ft.dot0.N) Y[(size_t)ft.dot0.x_start + lane] = x;
+                if (ft.dot0.N > LANE_HALF) {
+                    const int c = lane + LANE_HALF;
+                    const float more = input_sum(min(c, ft.dot0.N - 1));
+                    xb[c] = more;
+                    if (row0 == 0 && c < ft.dot0.N) Y[(size_t)ft.dot0.x_start + c] = more;
+                }
                 lane_sync();
             } else {
                 gather(ft.dot0);

@@ -148,8 +148,13 @@ class HipBackend:
             return None
         return next((s for s in (layout.matrix_spans(plan) for layout in self._layouts) if s is not None), None)
 
-    def lay_out_matrices(self, plan):
-        return next(layout for layout in self._layouts if layout.matrix_spans(plan) is not None).lay_out(plan)
+    def lay_out_matrices(self, plan, before=None):
+        """... and does.  What the launch before it does besides may become part of the new one: returns whether it
+        has been laid out, and whether `before` is not needed any more."""
+        layout = next(layout for layout in self._layouts if layout.matrix_spans(plan) is not None)
+        formed = layout.sums_in_front(before, plan) if layout is self._layouts[0] and before is not None else None
+        done = layout.lay_out(plan) if formed is None else layout.lay_out(plan, formed)
+        return done, done and formed is not None
 
     def store_spikes_as_bits(self, enc_plan, items, event_records, dt):
         return self._gemv.store_spikes_as_bits(enc_plan, items, event_records, dt)
@@ -755,7 +760,7 @@ class Simulator:
         constants = sorted((int(ra.starts[self.sidx[b]]), int(b.size), k) for k, b in enumerate(self.all_bases)
                            if getattr(b, "readonly", False) and b not in written and b.size)
         starts = [c[0] for c in constants]
-        for plan in plans:
+        for plan in list(plans):
             spans = self.backend.laid_out_spans(plan)
             bases = set()
             if spans is None:
@@ -766,8 +771,21 @@ class Simulator:
                     spans = None
                     break
                 bases.add(self.all_bases[constants[k][2]])
-            if spans is not None and self.backend.lay_out_matrices(plan):
+            if spans is None:
+                continue
+            k = plans.index(plan)
+            before = plans[k - 1] if k > 0 and hasattr(plans[k - 1], "enqueue") else None
+            done, alone = self.backend.lay_out_matrices(plan, before)
+            if done:
                 self._laid_out.append((bases, plan))
+            if alone:
+                plan.reads_mem = plan.reads_mem | before.reads_mem
+                plan.writes_mem = plan.writes_mem | before.writes_mem
+                plan.full_args = tuple(plan.full_args) + tuple(before.full_args)
+                plan.tag = "%s + input sums" % plan.tag
+                plan.bw_per_call = (plan.bw_per_call or 0) + (before.bw_per_call or 0)
+                plan.flops_per_call = (plan.flops_per_call or 0) + (before.flops_per_call or 0)
+                del plans[k - 1]
 
     def _constant_written(self, base):
         """The host has changed a constant: the copies of it that launches read follow."""

@@ -118,3 +118,62 @@ def test_groups_of_a_die_are_neighbours_in_the_list(groups):
     for die in range(8):
         firsts = out[die::8, 0]
         assert np.all(np.diff(firsts) == 4)
+
+
+def populations(n, dims, neuron="LIF", idle=True):
+    """Populations that send decoded vectors to each other and to a node of nobody's, one (`idle`) without input."""
+    from nengo_ocl_amd import minibuilder as mb
+
+    net = mb.Network(seed=4, solver="surrogate")
+    stim = net.Node(mb.WhiteSignal(period=0.3, high=8.0, seed=4), size_out=dims)
+    ens = [net.Ensemble(n + k, dims, neuron_type=getattr(mb, neuron)()) for k in range(4)]
+    for k, post in enumerate(ens[:3] if idle else ens):
+        net.Connection(stim, post, synapse=mb.Lowpass(0.005))
+        for pre in (ens[3], ens[(k + 1) % 3], ens[(k + 2) % 3]):
+            net.Connection(pre, post, transform=0.3, synapse=mb.Lowpass(0.005))
+    spare = net.Node(None, size_in=dims)
+    for pre in ens[:2]:
+        net.Connection(pre, spare, synapse=mb.Lowpass(0.005))
+    return net, [net.Probe(ens[0], synapse=0.01), net.Probe(spare), net.Probe(ens[3], synapse=0.01)]
+
+
+# four lanes or one per row of small matrices, large ones of any shape, of quads and back to back; sums of up to 64
+# elements and of more, part of them in a node's place
+POPULATIONS = [(60, 1), (150, 4), (90, 7), (250, 37), (220, 64), (210, 65), (214, 86), (130, 128), (900, 94), (700, 3)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("neuron", ["LIF", "Sigmoid"])
+@pytest.mark.parametrize("idle", [False, True])
+@pytest.mark.parametrize("n,dims", POPULATIONS)
+def test_input_sums_and_populations_without_input(queue, monkeypatch, n, dims, idle, neuron):
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    monkeypatch.setenv("NENGO_HIP_RESIDENT", "0")
+    (net, probes), (net_o, probes_o) = (populations(n, dims, neuron, idle) for _ in range(2))
+    with Simulator(net, seed=1) as gpu, OracleSimulator(net_o, seed=1) as cpu:
+        names = [p.laid_out[0].__name__ if p.laid_out else p.kern.__name__ for p in gpu._plans
+                 if getattr(p, "kern", None)]
+        assert "nhip_gemv_lanes" in names and "nhip_gemv" not in names and len(names) <= 3, names
+        for steps in (1, 25):
+            gpu.run_steps(steps)
+            cpu.run_steps(steps)
+            for p, p_o in zip(probes, probes_o):
+                assert np.array_equal(gpu.data[p], cpu.data[p_o])
+            assert_same_signals(gpu, cpu)
+
+
+@pytest.mark.parametrize("n,dims", POPULATIONS)
+def test_input_sums_are_formed_once(monkeypatch, n, dims):
+    """Every sum belongs to a record of the neurons' launch, also one that no population reads."""
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    monkeypatch.setenv("NENGO_HIP_RESIDENT", "0")
+    with Simulator(populations(n, dims)[0], seed=1) as sim:
+        plan, = [p for p in sim._plans if p.laid_out and p.laid_out[0].__name__ == "nhip_gemv_lanes"]
+        tasks = plan.host_tasks
+        parts = tasks[(tasks[:, 11] > 0) & (tasks[:, 1] == 0)][:, 11]
+        assert sorted(parts.tolist()) == [1, 1, 2, 4, 4, 4]  # (two of probes)
+        assert sorted(set(tasks[tasks[:, 9] == 0][:, 11].tolist())) == [0, 1, 2]
