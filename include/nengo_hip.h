@@ -398,27 +398,30 @@ int nhip_resident(void *stream, const void *spans, int n_spans, const void *ops,
  *             yin_stride0, alpha, beta, gamma (float bits), row0, n_rows (1..4), learned (0: the matrix
  *             stays), first_target, n_targets, then the rule: kind, pre_start, post_start, post_stride0,
  *             theta_start, theta_stride0 (BCM), alpha, beta (float bits), then the item's first target (4
- *             words) and four zeros}: rows row0 .. row0 + n_rows - 1 of an
+ *             words), own_groups, own_filter, two zeros}: rows row0 .. row0 + n_rows - 1 of an
  *             item; row i of the matrix changes by the rule's element of X[pre_start + j],
  *             X[post_start + i * post_stride0] (and theta, or the old weight)
  *   targets, F : filters of the fresh y, as for nhip_gemv_tile_filter (orders 1 and 2)
  *   filters : int32[max(n_filters, 2)][8] (on a 64-byte boundary) {s_start, f_start, n, has_a, a0, b0 (float bits), 0, 0}: stepped on
  *             X[s_start ..], F[f_start ..] when every row has read the old F; F and X one buffer
- *   arrived : int32[33 * 32], zero before the launch and after it (only read with n_filters > 0)
+ *             A record with own_groups > 0 (in launches with n_filters 0) stands instead for one of so many groups that
+ *             read the F that filters[own_filter] replaces: when they have, that one is stepped.
+ *   arrived : int32[(33 + own filters) * 32], zero before the launch and after it (only read with filters)
  * Bit-identical to the separate calls. */
 int nhip_gemv_learn(void *stream, const int *tasks, int n_tasks, float *A,
                     const float *X, const float *Yin, float *Y, const int *targets, float *F,
                     const int *filters, int n_filters, int *arrived);
 
-/* The same without filters of activities, for the rule of kind 16 too, W += (alpha post) (x) pre with every product
- * and sum rounded on its own, and with further items whose matrices nothing writes and whose vectors are mostly
+/* The same (both take the rule of kind 16 too, W += (alpha post) (x) pre with every product
+ * and sum rounded on its own) with further items whose matrices nothing writes and whose vectors are mostly
  * zero: only the columns whose x is not zero are visited.
  *   items   : int32[n_items][32] (on a 64-byte boundary) {at_start, mp, M (<= 64), N, x_start, y_start, y_stride0,
  *             yin_start, yin_stride0, alpha, beta, gamma (float bits), first_target, n_targets, row0 (first of the
  *             record's M rows), all (not zero: every column is visited), the first target (4 words), 12 zeros}
  *   AT      : columns of their matrices (nhip_lay_out_columns): element (r, c) at AT[at_start + c * mp + r] */
 int nhip_gemv_learn_events(void *stream, const int *tasks, int n_tasks, float *A, const float *X, const float *Yin,
-                           float *Y, const int *targets, float *F, const int *items, int n_items, const float *AT);
+                           float *Y, const int *targets, float *F, const int *filters, int n_filters, int *arrived,
+                           const int *items, int n_items, const float *AT);
 /* matrices: int32[n][8] {a_start, a_stride0, M, N, out, mp, first_record, n_records}: column c to AT[out + c * mp ..],
  * mp >= M a multiple of 16; where a matrix holds an infinity or a NaN `all` of the records first_record .. is set.
  * max_cols: the largest N. */

@@ -57,7 +57,7 @@ SIGNATURES = {
     "nhip_conv2d_neuron": [P, P, P, P, P, P, P, P, c_int, P, ctypes.c_double, c_int, P, P, P, P, P, P, P],
     "nhip_resident": [P, P, c_int, P, P, c_int, c_int],
     "nhip_gemv_learn": [P, P, c_int, P, P, P, P, P, P, P, c_int, P],
-    "nhip_gemv_learn_events": [P, P, c_int, P, P, P, P, P, P, P, c_int, P],
+    "nhip_gemv_learn_events": [P, P, c_int, P, P, P, P, P, P, P, c_int, P, P, c_int, P],
     "nhip_lay_out_columns": [P, P, c_int, c_int, P, P, P],
     "nhip_gemv_events": [P, P, c_int, P, P, P, P, P, P, c_int, c_int],
     "nhip_spmv_sell": [P, P, c_int, P, P, P, P, P],

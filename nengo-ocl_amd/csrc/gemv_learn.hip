@@ -41,7 +41,8 @@ struct LearnTask {
         float alpha, beta;
     } rule;
     FilterTarget target;                 // the item's first filter
-    int pad[4];
+    int own_groups, own_filter;          // not zero: so many groups read the activities that this filter replaces
+    int pad[2];
 };
 // A filter stepped when no group reads its output any more: F[f + i] = b S[s + i] - a F[f + i] (or b S[s + i])
 struct LearnFilter {
@@ -396,7 +397,7 @@ __global__ __launch_bounds__(NHIP_WG) void gemv_learn_kernel(
     // 13.9 -> 9.8 us).  So a group tells one of LCOUNTERS words, each in a line of its own; the last there tells
     // the word behind them.
     auto read = [&]() LEARN_INLINE {
-        if (n_filters > 0 && tid == 0) {
+        if ((n_filters > 0 || task.own_groups > 0) && tid == 0) {
             const int n_groups = side.n_gemv_groups, mine = group % LCOUNTERS;
             auto tell = [&](int counter, int expected) {  // the last of `expected`? (it clears the word for the next launch)
                 int* word = arrived + counter * LCOUNTER_WORDS;
@@ -404,8 +405,9 @@ __global__ __launch_bounds__(NHIP_WG) void gemv_learn_kernel(
                 __hip_atomic_store(word, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 return 1;
             };
-            lds.last = tell(mine, (n_groups - mine + LCOUNTERS - 1) / LCOUNTERS) &&
-                       tell(LCOUNTERS, min(n_groups, LCOUNTERS));
+            lds.last = task.own_groups > 0 ? tell(LCOUNTERS + 1 + task.own_filter, task.own_groups)
+                                           : tell(mine, (n_groups - mine + LCOUNTERS - 1) / LCOUNTERS) &&
+                                                 tell(LCOUNTERS, min(n_groups, LCOUNTERS));
         }
     };
     auto rows = [&](auto rule) LEARN_INLINE {
@@ -426,15 +428,13 @@ __global__ __launch_bounds__(NHIP_WG) void gemv_learn_kernel(
         for (int q = lane + NHIP_WAVE; q < task.n_targets; q += NHIP_WAVE)
             filter_epilogue<true>(filter, make_int2(task.first_target + q, 1), row, y);
     }
-    if (n_filters == 0) return;
+    const bool own = task.own_groups > 0;  // activities of its item's groups alone: their last one replaces those
+    if (!own && n_filters == 0) return;
     __syncthreads();
     if (lds.last == 0) return;
     struct TwoFilters { LearnFilter a, b; };
     const TwoFilters here = __builtin_bit_cast(TwoFilters, fw);
-    for (int k = 0; k < n_filters; k += 2) {  // two at a time (the activities of both sides), in quads
-        const LearnFilter fa = k == 0 ? here.a : filters[k];
-        LearnFilter fb = k == 0 ? here.b : filters[min(k + 1, n_filters - 1)];
-        if (k + 1 >= n_filters) fb.n = 0;
+    auto step = [&](const LearnFilter& fa, const LearnFilter& fb) LEARN_INLINE {  // in quads
         constexpr int U = 2;  // quads of a thread requested together, of each filter
         const auto stepped = [](const LearnFilter& f, float s, float old) LEARN_INLINE {
             const float bx = __fmul_rn(f.b, s);
@@ -479,6 +479,15 @@ __global__ __launch_bounds__(NHIP_WG) void gemv_learn_kernel(
         }
         element(fa);
         element(fb);
+    };
+    if (own) {
+        step(filters[task.own_filter], LearnFilter{});
+        return;
+    }
+    for (int k = 0; k < n_filters; k += 2) {  // two at a time (the activities of both sides)
+        LearnFilter fb = k == 0 ? here.b : filters[min(k + 1, n_filters - 1)];
+        if (k + 1 >= n_filters) fb.n = 0;
+        step(k == 0 ? here.a : filters[k], fb);
     }
 }
 
@@ -545,17 +554,18 @@ extern "C" int nhip_gemv_learn(void* stream, const int* tasks, int n_tasks, floa
 }
 
 extern "C" int nhip_gemv_learn_events(void* stream, const int* tasks, int n_tasks, float* A, const float* X,
-                                      const float* Yin, float* Y, const int* targets, float* F, const int* items,
-                                      int n_items, const float* AT) {
+                                      const float* Yin, float* Y, const int* targets, float* F, const int* filters,
+                                      int n_filters, int* arrived, const int* items, int n_items, const float* AT) {
     if (n_items < 0 || (n_items > 0 && (!items || !AT)) || (reinterpret_cast<uintptr_t>(items) & 63)) {
         RowsSide none;
         take_carried(none);  // (whatever becomes of the launch)
         return NHIP_E_BADARG;
     }
-    return learn_launch(stream, tasks, n_tasks, A, X, Yin, Y, targets, F, nullptr, 0, nullptr, n_items,
+    return learn_launch(stream, tasks, n_tasks, A, X, Yin, Y, targets, F, filters, n_filters, arrived, n_items,
                         [&](dim3 grid, const FilterArgs& filter, const RowsSide& side) {
         NHIP_LAUNCH(gemv_learn_kernel<true>, grid, dim3(NHIP_WG), 0, static_cast<hipStream_t>(stream),
-                    reinterpret_cast<const LearnTask*>(tasks), A, X, Yin, Y, filter, nullptr, 0, nullptr,
+                    reinterpret_cast<const LearnTask*>(tasks), A, X, Yin, Y, filter,
+                    reinterpret_cast<const LearnFilter*>(filters), n_filters, arrived,
                     (LearnEvents{reinterpret_cast<const ColumnsItem*>(items), AT, n_items}), side);
     });
 }

@@ -132,6 +132,12 @@ SUM_PARTS_FOR_WAVE_TASKS, SUM_MIN_ROWS_FOR_WAVE_TASKS = 3, 3000
 # 1,000 x 700 26.7 / 33.6, three of 2,100 x 300 19.3 / 23.3. Of 208 networks drawn at random (up to 1,800 groups of 4
 # to 2,500 columns) one is faster apart
 LEARN_GROUP_US = 0.011
+# Outer products of fewer columns keep a launch for the rule and its filters (its tests are at 300 columns; nothing is
+# won by it). Whole steps with and without, us: 3 triples of 300 x 8 13.5 / 9.0, 20 of 250 x 14 16.2 / 9.7, 30 of 500 x 4
+# 17.1 / 9.1, 10 of 500 x 10 17.4 / 9.1, 4 of 1000 x 4 11.3 / 9.6, 372 x 36 16.2 / 9.3, 40 of 1028 x 7 14.3 / 10.6, 2 of
+# 2000 x 50 16.4 / 12.3
+OUTER_MIN_COLS = 320
+RULE_OUTER = 16  # of csrc/gemv_learn.hip, besides `RULE_*` of hipra_nonlinearities
 
 
 def _own_launch_us(kernel_class, n_cols, megabytes):
@@ -1595,8 +1601,14 @@ def fuse_learning(enc_plan, dec_plan, ew_plan, lf_plan):
     return new_enc, new_dec, residual, pending
 
 
-def fuse_hebbian(products, rule_plan, lf_plan=None):
-    """A step that multiplies by matrices which Oja's or the BCM rule then changes in place, from
+def _spikes_item(prog, b):
+    """Does `hipra_learned` give item `b` a group that visits active columns?"""
+    d = prog.geometry[b]["dots"][0]
+    return b in prog.event_items and EVENT_MIN_COLS <= d["a_shape1"] <= EVENT_MAX_COLS
+
+
+def fuse_hebbian(products, rule_plan, lf_plan=None, lays_out=False):
+    """A step that multiplies by matrices which Oja's or the BCM rule or an outer product then changes in place, from
     activities that filters then replace -- `products` (plans of one GEMV, with or without the filter
     epilogue), `rule_plan`, `lf_plan` -- as one launch (``nhip_gemv_learn``): a matrix is read
     once per step, and the filters need no launch.
@@ -1611,12 +1623,21 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
     for the filters that stay, filters that moved)`` or None."""
     from .hipra_nonlinearities import RULE_BCM, RULE_OJA, plan_linearfilter
 
-    spec = rule_plan.rule_spec
+    spec = getattr(rule_plan, "rule_spec", None)
+    if spec is None:  # an outer product (PES): W += (alpha e) (x) f
+        ew = rule_plan.ew_spec
+        spec = dict(rule=RULE_OUTER, inc=True, pre=ew["X"], post=ew["A"], aux=ew["Y"], delta=ew["Y"],
+                    alpha=ew["alphas"], beta=np.zeros(len(ew["Y"])))
+        if any(int(n) != 1 for ra in (ew["X"], ew["A"]) for n in ra.shape1s) or any(
+                (int(ew["A"].shape0s[i]), int(ew["X"].shape0s[i])) != (int(ew["Y"].shape0s[i]), int(ew["Y"].shape1s[i]))
+                for i in range(len(ew["Y"]))):
+            return None
     prog = products[0].prog
     queue, geometry = prog.queue, prog.geometry
     pre, post, aux, delta = (spec[k] for k in ("pre", "post", "aux", "delta"))
     buf = prog.A.ptr.value
-    if spec["rule"] not in (RULE_BCM, RULE_OJA) or not spec["inc"] or any(
+    outer = spec["rule"] == RULE_OUTER
+    if spec["rule"] not in (RULE_BCM, RULE_OJA, RULE_OUTER) or not spec["inc"] or any(
             ra.ptr.value != buf for ra in (prog.X, prog.Y, prog.Y_in, pre, post, aux, delta)):
         return None
     members = [b for plan in products for b in plan.members]
@@ -1665,6 +1686,8 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
         groups = sum(-(-geometry[b]["y_len"] // (WG // WAVE)) for b in beside)
         cols = [geometry[b]["dots"][0]["a_shape1"] for b in beside]
         megabytes = 4e-6 * sum(geometry[b]["y_len"] * n for b, n in zip(beside, cols))
+        if outer and lays_out:  # (products with spikes visit active columns only there: `hipra_learned`)
+            groups -= sum(-(-geometry[b]["y_len"] // (WG // WAVE)) for b in beside if _spikes_item(prog, b))
         if LEARN_GROUP_US * groups <= _own_launch_us(p.kernel_class, max(cols + [0]), megabytes):
             riding += beside
         elif len(beside) == len(p.members):
@@ -1678,13 +1701,16 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
             kept += apart
     products = [p for p in products if p not in kept]
     members = [b for p in products for b in p.members if b in rule_of or b in riding]
+    if outer and (any(geometry[b]["dots"][0]["a_shape1"] < OUTER_MIN_COLS for b in rule_of) or (
+            lf_plan is not None and any(int(n) > 1 for k in ("A", "B") for n in lf_plan.lf_spec[k].shape0s))):
+        return None  # (synapses of higher order beside the activities' keep a launch with them: `_fuse_outer_filters`)
     operands = [_span(ra, i) for ra in (pre, post) + ((aux,) if spec["rule"] == RULE_BCM else ())
                 for i in range(len(ra))]
     if not _learned_apart(geometry, members, {b: _span(delta, i) for b, i in rule_of.items()}, operands):
         return None
 
     per_group = WG // WAVE
-    tasks = []
+    tasks, item_of = [], []
     bits = lambda v: int(np.float32(v).view(np.int32))
     for b in members:
         g = geometry[b]
@@ -1692,14 +1718,20 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
         first, n = (0, 0) if item_targets is None else (int(v) for v in item_targets[b])
         target = tuple(int(v) for v in host_targets[first][:4]) if n else (0,) * 4
         for row0 in range(0, g["y_len"], per_group):
-            tasks.append((d["a_start"], d["a_stride0"], d["a_shape1"], d["x_start"], g["y_start"], g["y_stride0"],
+            tasks.append([d["a_start"], d["a_stride0"], d["a_shape1"], d["x_start"], g["y_start"], g["y_stride0"],
                           g["y_in_start"], g["y_in_stride0"], bits(prog.alpha[b]), bits(prog.beta[b]),
-                          bits(prog.gamma[b]), row0, min(per_group, g["y_len"] - row0), int(b in rule_of), first, n)
-                         + (tuple(int(v) for v in rules[rule_of[b]]) if b in rule_of else (0,) * 8)
-                         + target + (0,) * 4)
+                          bits(prog.gamma[b]), row0, min(per_group, g["y_len"] - row0), int(b in rule_of), first, n]
+                         + ([int(v) for v in rules[rule_of[b]]] if b in rule_of else [0] * 8)
+                         + list(target) + [0] * 4)
+            item_of.append(b)
     if not tasks:
         return None
     filters, moved, rest = [], [], []
+    # (an outer product's activities belong to few items each: their groups' last one replaces them)
+    readers = {}
+    for row in tasks:
+        if outer and row[13]:
+            readers.setdefault((row[17], row[2]), []).append(row)
     if lf_plan is not None:
         S, T, A, B = (lf_plan.lf_spec[k] for k in ("X", "Y", "A", "B"))
         if S.ptr.value == buf and T.ptr.value == buf:
@@ -1709,26 +1741,30 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
                 if int(B.shape0s[k]) != 1 or int(A.shape0s[k]) > 1 or not vector:
                     continue
                 na = int(A.shape0s[k])
+                if outer and (int(T.starts[k]), int(T.shape0s[k])) not in readers:
+                    continue
+                for row in readers.get((int(T.starts[k]), int(T.shape0s[k])), ()):
+                    row[28:30] = len(readers[int(T.starts[k]), int(T.shape0s[k])]), len(filters)
                 filters.append((S.starts[k], T.starts[k], S.shape0s[k], na,
                                 bits(a_host[k][0, 0]) if na else 0, bits(b_host[k][0, 0]), 0, 0))
                 moved.append(k)
         rest = [k for k in range(len(S)) if k not in set(moved)]
     dev_tasks = to_device(queue, np.array(tasks, dtype=np.int32))
     dev_filters = to_device(queue, np.array((filters + [(0,) * 8] * 2)[:max(2, len(filters))], dtype=np.int32))
-    arrived = to_device(queue, np.zeros(33 * 32, dtype=np.int32))
+    arrived = to_device(queue, np.zeros((33 + (len(filters) if outer else 0)) * 32, dtype=np.int32))
     lib = queue.lib
     targets = dev_targets if dev_targets is not None else dev_tasks  # (not read without targets)
     total = lambda attr: sum(getattr(p, attr) or 0 for p in list(products) + [rule_plan])
     weights = 4 * int(delta.sizes.sum())
     plan = Plan(queue, lib.nhip_gemv_learn,
                 (dev_tasks.ptr, len(tasks), prog.A.ptr, prog.X.ptr, prog.Y_in.ptr, prog.Y.ptr,
-                 targets.ptr, F.ptr, dev_filters.ptr, len(filters), arrived.ptr),
+                 targets.ptr, F.ptr, dev_filters.ptr, 0 if outer else len(filters), arrived.ptr),
                 gsize=(WG * len(tasks),), lsize=(WG,),
                 full_args=sum((tuple(p.full_args) for p in list(products) + [rule_plan]), ())
                 + (dev_tasks, dev_filters, arrived),
                 name=products[0].name, tag=" + ".join([products[0].tag, rule_plan.name]),
                 # the rule's own accounting, less the matrices it need not read again
-                bw_per_call=total("bw_per_call") - (2 if spec["rule"] == RULE_OJA else 1) * weights
+                bw_per_call=total("bw_per_call") - (1 if spec["rule"] == RULE_BCM else 2) * weights
                 + sum(12 * int(f[2]) for f in filters),
                 flops_per_call=total("flops_per_call"))
     plan.description = "; ".join(p.description for p in products)
@@ -1737,6 +1773,10 @@ def fuse_hebbian(products, rule_plan, lf_plan=None):
     plan.gemv_bytes = sum(getattr(p, "gemv_bytes", p.bw_per_call) for p in products)
     plan.host_tasks = None
     plan.learned_matrices = len(rule_of)
+    if outer:  # (the other rules' launches have few decoders beside them: two rows of 2,000 columns in a group of
+        # `hipra_learned`, 2000 x 2000 by Oja's rule 9.4 -> 10.1 us)
+        plan.host_learn = (np.array(tasks, dtype=np.int32), np.array(item_of), item_targets,
+                           host_targets if item_targets is not None else None)
     residual = []
     if lf_plan is not None and rest:
         residual = plan_linearfilter(queue, S[rest], T[rest], A[rest], B[rest], lf_plan.lf_spec["Xbuf"][rest],

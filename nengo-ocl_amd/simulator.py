@@ -152,7 +152,9 @@ class HipBackend:
         """... and does.  What the launch before it does besides may become part of the new one: returns whether it
         has been laid out, and whether `before` is not needed any more."""
         layout = next(layout for layout in self._layouts if layout.matrix_spans(plan) is not None)
-        formed = layout.sums_in_front(before, plan) if layout is self._layouts[0] and before is not None else None
+        formed = None
+        if layout is self._layouts[0] and before is not None and self.input_sums_in_launch:
+            formed = layout.sums_in_front(before, plan)
         done = layout.lay_out(plan) if formed is None else layout.lay_out(plan, formed)
         return done, done and formed is not None
 
@@ -1003,7 +1005,7 @@ class Simulator:
         return plans
 
     def _fuse_hebbian(self, plans):
-        """Oja's or the BCM rule on matrices that the step multiplies by, and the filters of the
+        """Oja's or the BCM rule, or an outer product, on matrices that the step multiplies by, and the filters of the
         activities it reads, as part of the launch of those products (`hipra_gemv.fuse_hebbian`), where
         no plan between them touches what moves and the products read and write nothing that the rule
         or the filters need otherwise."""
@@ -1013,11 +1015,17 @@ class Simulator:
                                 and getattr(p, "kernel_class", (None,))[0] in (2, 3)
                                 and getattr(p, "learned_matrices", 0) == 0)
         plans = list(plans)
+        resident = getattr(self.backend, "_resident", None)
+        may_be_resident = resident is not None and sum(int(b.size) for b in self.all_bases) <= resident.LDS_WORDS
         r = 0
         while r < len(plans):
             rule = plans[r]
             r += 1
-            if not (getattr(rule, "rule_spec", None) or {}).get("inc"):
+            outer = getattr(rule, "ew_spec", None) or {}
+            # (what may fit the resident launch, which holds no such products, keeps its launches)
+            outer = outer.get("outer") and outer.get("inc") and not may_be_resident and hasattr(
+                self.backend, "fuse_learning")
+            if not outer and not (getattr(rule, "rule_spec", None) or {}).get("inc"):
                 continue
             # the products with its matrices: the nearest plans before it that read what it writes
             j = next((k for k in range(r - 2, -1, -1) if conflict(rule, plans[k])), None)
@@ -1041,7 +1049,8 @@ class Simulator:
                        and not any(conflict(lf, q) for q in plans[j + 1:r - 1] + plans[r:f])
                        and not (writes & (lf.reads_mem | lf.writes_mem)) and not (reads & lf.writes_mem)
                        and not (rule.writes_mem & (lf.reads_mem | lf.writes_mem)))
-            result = self.backend.fuse_hebbian(products, rule, lf if movable else None)
+            result = self.backend.fuse_hebbian(products, rule, lf if movable else None,
+                                               getattr(self.backend, "lays_out_matrices", False))
             if result is None:
                 continue
             plan, kept, residual, moved = result

@@ -33,7 +33,7 @@ def test_learned_decoders_and_others_in_one_launch(queue, n, dims):
 
     (net, probes), (net_o, probes_o) = (network(n, dims) for _ in range(2))
     with Simulator(net, seed=1) as gpu, OracleSimulator(net_o, seed=1) as cpu:
-        assert learning_launch(gpu).laid_out[1][9] > 0
+        assert learning_launch(gpu).laid_out[1][12] > 0
         for steps in (1, 40):
             gpu.run_steps(steps)
             cpu.run_steps(steps)
@@ -101,7 +101,7 @@ def test_columns_beside_a_learned_row(queue, M, N):
         columns = empty_device(queue, N * mp)
         _lib.check(lib.nhip_lay_out_columns(queue.handle, dev[3].ptr, 1, N, B.ptr, columns.ptr, dev[1].ptr), "")
         _lib.check(lib.nhip_gemv_learn_events(queue.handle, dev[0].ptr, 1, B.ptr, B.ptr, B.ptr, B.ptr, dev[2].ptr, B.ptr,
-                                              dev[1].ptr, len(items), columns.ptr), "")
+                                              None, 0, None, dev[1].ptr, len(items), columns.ptr), "")
         got = np.split(np.asarray(B.get()), at[1:-1])
         with np.errstate(invalid="ignore"):
             want = 2 * (fixed.astype(np.float64) @ x) + 0.5 * y_in[:M] + 3
@@ -119,10 +119,33 @@ def test_records_cover_every_row_once(monkeypatch, n, dims):
     with Simulator(network(n, dims)[0], seed=1) as sim:
         plan = learning_launch(sim)
         tasks, records = plan.host_learned
-        assert len(tasks) == plan.laid_out[1][1] and len(records) == plan.laid_out[1][9]
+        assert len(tasks) == plan.laid_out[1][1] and len(records) == plan.laid_out[1][12]
         covered = [y + (r + k) * s for y, s, r, c in tasks[:, [4, 5, 11, 12]].tolist() for k in range(c)]
         covered += [y + (r + k) * s for y, s, r, c in records[:, [5, 6, 14, 2]].tolist() for k in range(c)]
         assert sorted(covered) == sorted(
             g["y_start"] + r * g["y_stride0"] for g in (plan.prog.geometry[b] for b in plan.members)
             for r in range(g["y_len"]))
         assert tasks[:, 12].max() <= 4 and records[:, 2].max() <= 64 and not (records[:, 1] % 16).any()
+
+
+# rows that are read whole beside learned ones, no quad at the end, few groups to an item and one
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,dims,triples", [(330, 36, 1), (513, 3, 4), (1050, 19, 3), (1028, 7, 5), (2999, 66, 2), (4099, 1, 2)])
+def test_activities_replaced_by_their_last_reader(queue, n, dims, triples):
+    """Filters of activities that few groups read are stepped by the last of these, in the launch that read them."""
+    from nengo_ocl_amd import configs
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    (net, probes, _), (net_o, probes_o, _) = (
+        configs.c4_pes(1, n_triples=triples, n_neurons=n, dims=dims, learning_rate=1e-3) for _ in range(2))
+    with Simulator(net, seed=1) as gpu, OracleSimulator(net_o, seed=1) as cpu:
+        plan, = [p for p in gpu._plans if getattr(p, "host_learn", None) is not None]
+        own = plan.host_learn[0][:, 28:30]
+        assert sorted(set(own[own[:, 0] > 0, 1].tolist())) == list(range(triples))
+        for steps in (1, 20, 37):
+            gpu.run_steps(steps)
+            cpu.run_steps(steps)
+            for key in probes:
+                assert np.array_equal(gpu.data[probes[key]], cpu.data[probes_o[key]])
+            assert_same_signals(gpu, cpu)
