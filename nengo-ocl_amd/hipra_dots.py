@@ -20,6 +20,10 @@ ROW_COLS = 256  # rows of up to so many columns have a record each, longer ones 
 # 20 x 32 x 600 (1.9 MB) 9.5 / 7.9 us, 100 x 16 x 1000 (6.5) 7.6 / 7.6, 37 x 50 x 1501 (15) 10.6 / 10.1,
 # 12 x 64 x 5000 (19; a group per item) 16.7 / 14.1, 60 x 30 x 3000 (30) 14.1 / 16.8
 EVENT_MAX_BYTES = 20 << 20
+# Other launches, up to so many: beyond, encoders and decoders of a step no longer stay in the memory-side cache (256 MB),
+# and non-temporal rows in long runs come faster. Rate neurons, whole steps, this kernel / csrc/gemv_tile.hip:
+# 84 MB of decoders (80 x 64 x 4096) 32.0 / 34.6 us, 134 MB 48.0 / 53.3, 168 MB 65.5 / 59.1, 268 MB 101 / 89
+MAX_BYTES = 144 << 20
 GROUPS_FOR_FEW_ROWS = 2048  # of groups that are mostly empty
 
 
@@ -95,7 +99,7 @@ def matrix_spans(plan):
         return None
     mats = _copy_units(plan, *shape)
     size = sum(64 * key[2] * units for key, (units, _) in mats.items())
-    if size >= 2 ** 33 or launch.events and size > EVENT_MAX_BYTES:
+    if size > (EVENT_MAX_BYTES if launch.events else MAX_BYTES):
         return None
     return sorted({_span(plan.prog.A, a_j) for _, a_j in mats.values()} - {None})
 

@@ -130,3 +130,15 @@ def test_chains_divided_over_launches(monkeypatch):
         assert "hip_linearfilter" in runs[1]
         whole, = [q.carried for q in sim._plans if getattr(q, "carried", None) is not None]
         assert sorted(runs[0] + runs[1]) == sorted(p.name for p in whole.members)
+
+
+def test_launches_of_more_than_the_memory_side_cache_holds_read_matrices_as_they_lie(monkeypatch):
+    from nengo_ocl_amd import hipra_dots
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    monkeypatch.setenv("NENGO_HIP_RESIDENT", "0")
+    for limit, expected in ((1 << 30, True), (100 * 16 * 40 * 4, False)):
+        monkeypatch.setattr(hipra_dots, "MAX_BYTES", limit)
+        with Simulator(network(1500, 50)[0], seed=1) as sim:
+            assert bool(laid_out(sim)) == expected
