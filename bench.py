@@ -196,7 +196,7 @@ def config_summary(config, steps, warmup, profile_steps, max_regions, cpu_budget
     return out
 
 
-KERNEL_SOURCES = ("gemv_tile.hip", "gemv_types.h", "gemv_rows.h", "neuron_math.h", "nhip_common.h",
+KERNEL_SOURCES = ("gemv_lanes.hip", "gemv_types.h", "neuron_math.h", "nhip_common.h", "rows_side.h",
                   "sequence_ops.h", "small_arg_math.h")
 
 
@@ -218,8 +218,7 @@ def measured_traffic(plan_name):
     from.  The summary names the hash of the kernel sources it was taken with; when the
     sources in this tree hash differently the figure is stale and None is returned in its
     place.  (None, None) for other workloads."""
-    kernel = {"hipra_gemv.tile_lif": "gemv_stream_kernel<1,0,0>",
-              "hipra_gemv.tile_filter": "gemv_stream_kernel<2,4,0>"}.get(plan_name)
+    kernel = {"hipra_gemv.tile_lif": "gemv_lanes_kernel<1,false>"}.get(plan_name)
     rel = os.path.join("profiles", "c3_shared_step.txt")
     path = os.path.join(ROOT, rel)
     if kernel is None or not os.path.exists(path):
