@@ -884,18 +884,19 @@ class plan_ref_gemv(gemv_prog):
     force_scalar = True
 
 
+def _overlapping(a, b):
+    """Which half-open intervals of `a` overlap one of `b`?  (lists of (lo, hi))"""
+    if not len(a) or not len(b):
+        return np.zeros(len(a), dtype=bool)
+    (lo, hi), (los, his) = (np.asarray(v, dtype=np.int64).T for v in (a, b))
+    order = np.argsort(los, kind="stable")
+    before = np.searchsorted(los[order], hi, side="left")  # intervals of b starting before hi
+    return (before > 0) & (np.maximum.accumulate(his[order])[before - 1] > lo)
+
+
 def _overlaps(a, b):
     """Does any half-open interval of `a` overlap one of `b`?  (lists of (lo, hi))"""
-    if not a or not b:
-        return False
-    b = sorted(b)
-    los = np.array([lo for lo, _ in b])
-    his = np.maximum.accumulate(np.array([hi for _, hi in b]))
-    for lo, hi in a:
-        k = np.searchsorted(los, hi, side="left")  # intervals of b starting before hi
-        if k > 0 and his[k - 1] > lo:
-            return True
-    return False
+    return bool(_overlapping(a, b).any())
 
 
 def _span(ra, i):
@@ -1727,7 +1728,9 @@ def fuse_hebbian(products, rule_plan, lf_plan=None, lays_out=False):
     if not tasks:
         return None
     filters, moved, rest = [], [], []
-    # (an outer product's activities belong to few items each: their groups' last one replaces them)
+    # (an outer product's activities belong to few items each: their groups' last one replaces them, where these
+    # are all that read any of them, as the rule's column operand: readers of other parts, and of single
+    # elements (row operands), are not counted)
     readers = {}
     for row in tasks:
         if outer and row[13]:
@@ -1735,13 +1738,18 @@ def fuse_hebbian(products, rule_plan, lf_plan=None, lays_out=False):
     if lf_plan is not None:
         S, T, A, B = (lf_plan.lf_spec[k] for k in ("X", "Y", "A", "B"))
         if S.ptr.value == buf and T.ptr.value == buf:
+            replaced = [_span(T, k) or (0, 0) for k in range(len(T))]
+            others = [iv for ra in (post, S) for iv in (_span(ra, i) for i in range(len(ra))) if iv]
+            begins, ends = np.sort([key[0] for key in readers]), np.sort([sum(key) for key in readers])
+            uncounted = [lo < hi and (odd or begins.searchsorted(hi) - ends.searchsorted(lo, side="right") > 1)
+                         for (lo, hi), odd in zip(replaced, _overlapping(replaced, others))]
             a_host, b_host = A.to_host(), B.to_host()
             for k in range(len(S)):
                 vector = all(int(r.shape1s[k]) == 1 and int(r.stride0s[k]) == 1 for r in (S, T))
                 if int(B.shape0s[k]) != 1 or int(A.shape0s[k]) > 1 or not vector:
                     continue
                 na = int(A.shape0s[k])
-                if outer and (int(T.starts[k]), int(T.shape0s[k])) not in readers:
+                if outer and (uncounted[k] or (int(T.starts[k]), int(T.shape0s[k])) not in readers):
                     continue
                 for row in readers.get((int(T.starts[k]), int(T.shape0s[k])), ()):
                     row[28:30] = len(readers[int(T.starts[k]), int(T.shape0s[k])]), len(filters)

@@ -149,3 +149,68 @@ def test_activities_replaced_by_their_last_reader(queue, n, dims, triples):
             for key in probes:
                 assert np.array_equal(gpu.data[probes[key]], cpu.data[probes_o[key]])
             assert_same_signals(gpu, cpu)
+
+
+def rules_on_one_activity(rows, shared, n=1050, dims=20):
+    """A decoder learned from the filtered activities of a population, and a matrix of `rows` rows learned from some of
+    the same: `shared` "part", the first 700 of them, "all" or "rows", all of them as the column operand of the rule
+    and `rows` of them as its row operand too."""
+    from nengo_ocl_amd import configs, ir
+
+    net, probes, _ = configs.c4_pes(1, n_triples=1, n_neurons=n, dims=dims, learning_rate=1e-3)
+    model = net.build_model(dt=0.001)
+    rule, = [op for op in model.operators if isinstance(op, ir.SimPES)]
+    spikes, = [op.input for op in model.operators if isinstance(op, ir.SimProcess) and op.output is rule.pre_filtered]
+    pre, acts = (rule.pre_filtered[:700], spikes[:700]) if shared == "part" else (rule.pre_filtered, spikes)
+    rng = np.random.RandomState(rows)
+    weights = ir.Signal(rng.normal(scale=1e-3, size=(rows, pre.size)), name="more.weights")
+    delta = ir.Signal(np.zeros(weights.shape), name="more.Delta")
+    out = ir.Signal(np.zeros(rows), name="more.out")
+    error = (rule.pre_filtered[:rows] if shared == "rows" else
+             ir.Signal(rng.normal(size=rows), name="more.error", readonly=True))
+    for op in (ir.Reset(out), ir.DotInc(weights, acts, out), ir.SimPES(pre, error, delta, 1e-3),
+               ir.Copy(delta, weights, inc=True)):
+        model.add_op(op)
+    return model, probes
+
+
+SHARED = [("part", False), ("rows", False), ("all", True)]
+
+
+@pytest.mark.parametrize("shared,moves", SHARED)
+def test_activities_that_others_read_too_are_replaced_behind_the_launch(monkeypatch, shared, moves):
+    """The last reader of a filter's output replaces it in the launch only where all readers there read all of it, as
+    the rules' column operand: the readers of anything else are not counted."""
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    with Simulator(None, model=rules_on_one_activity(64, shared)[0], seed=1) as sim:
+        plan, = [p for p in sim._plans if getattr(p, "host_learn", None) is not None]
+        tasks = plan.host_learn[0]
+        learned = tasks[tasks[:, 13] != 0]
+        assert plan.learned_matrices == 2 and len(learned) == 5 + 16
+        assert set(learned[:, 28].tolist()) == ({5 + 16} if moves else {0})
+        filters = [p for p in sim._plans if p.name == "hip_linearfilter"]
+        assert bool(filters) != moves
+        if filters:
+            order = list(sim._plans)
+            assert order.index(filters[0]) > order.index(plan)
+
+
+# more groups than run at once: the last ones read long after the first rule's are through
+@pytest.mark.gpu
+@pytest.mark.parametrize("shared", [s for s, _ in SHARED])
+def test_rules_that_share_activities(queue, shared):
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    rows = 1000 if shared == "rows" else 12000
+    (model, probes), (model_o, probes_o) = (rules_on_one_activity(rows, shared) for _ in range(2))
+    with Simulator(None, model=model, seed=1) as gpu, OracleSimulator(None, model=model_o, seed=1) as cpu:
+        assert any(getattr(p, "learned_matrices", 0) == 2 for p in gpu._plans)
+        for steps in (1, 20):
+            gpu.run_steps(steps)
+            cpu.run_steps(steps)
+            for key in probes:
+                assert np.array_equal(gpu.data[probes[key]], cpu.data[probes_o[key]])
+            assert_same_signals(gpu, cpu)
