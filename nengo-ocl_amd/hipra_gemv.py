@@ -896,6 +896,9 @@ def _overlapping(a, b):
 
 def _overlaps(a, b):
     """Does any half-open interval of `a` overlap one of `b`?  (lists of (lo, hi))"""
+    if len(a) == len(b) == 1:
+        (lo, hi), (b_lo, b_hi) = a[0], b[0]
+        return b_lo < hi and lo < b_hi
     return bool(_overlapping(a, b).any())
 
 
@@ -1174,21 +1177,21 @@ def formed_sums(sum_plan, lif_plan, max_cols):
     # launch, reads the whole sum with stride 1, and has a single column stage
     used = set()
     members = set(lif_plan.members)
-    for g in E.geometry:
-        for k, d in enumerate(g["dots"]):
-            span = (d["x_start"], d["x_start"] + (d["a_shape1"] - 1) * d["x_stride0"] + 1)
-            if not _overlaps([span], sum_spans):
-                continue
-            want = sums.get(d["x_start"])
-            if (k != 0 or g["index"] not in members or want is None or want[0] != d["a_shape1"]
-                    or (d["x_stride0"] != 1 and d["a_shape1"] > 1)
-                    or (max_cols <= 64 and stream_stage(d["a_shape1"])[0] > 6)):
-                return None
-            used.add(d["x_start"])
-        # (matrices and old outputs that overlap a sum would be read while it is written)
-        if _overlaps([(g["y_in_start"], g["y_in_start"] + (g["y_len"] - 1) * g["y_in_stride0"] + 1)],
-                     sum_spans) and E.Y_in.ptr.value == buf:
+    dots = [(g, k, d) for g in E.geometry for k, d in enumerate(g["dots"])]
+    touch = _overlapping([(d["x_start"], d["x_start"] + (d["a_shape1"] - 1) * d["x_stride0"] + 1) for _, _, d in dots],
+                         sum_spans)
+    for g, k, d in (dots[i] for i in np.flatnonzero(touch)):
+        want = sums.get(d["x_start"])
+        if (k != 0 or g["index"] not in members or want is None or want[0] != d["a_shape1"]
+                or (d["x_stride0"] != 1 and d["a_shape1"] > 1)
+                or (max_cols <= 64 and stream_stage(d["a_shape1"])[0] > 6)):
             return None
+        used.add(d["x_start"])
+    # (matrices and old outputs that overlap a sum would be read while it is written)
+    if E.Y_in.ptr.value == buf and _overlaps(
+            [(g["y_in_start"], g["y_in_start"] + (g["y_len"] - 1) * g["y_in_stride0"] + 1) for g in E.geometry],
+            sum_spans):
+        return None
     spare = sorted(set(sums) - used)  # sums nothing here reads: tasks of their own, below
     if not used:
         return None

@@ -356,3 +356,31 @@ def test_populations_without_input_ride_with_unaligned_matrices(monkeypatch):
     with Simulator(net, seed=1, event_calibration_steps=0) as sim:
         neurons = [p for p in sim._plans if p.name.endswith("_lif")]
         assert len(neurons) == 1 and neurons[0].input_sums == 2, [p.name for p in sim._plans]
+
+
+def test_planning_of_many_populations_looks_at_each_a_few_times(monkeypatch):
+    """What a launch with input sums must not overlap is looked up for all of its items at once."""
+    from nengo_ocl_amd import hipra_gemv, minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    monkeypatch.setenv("NENGO_HIP_RESIDENT", "0")
+    looked_at, overlapping = [0], hipra_gemv._overlapping
+
+    def counted(a, b):
+        looked_at[0] += len(a) + len(b)
+        return overlapping(a, b)
+
+    monkeypatch.setattr(hipra_gemv, "_overlapping", counted)
+    counts = []
+    for n in (40, 160):
+        net = mb.Network(seed=0, solver="surrogate")
+        ens = [net.Ensemble(4, 5) for _ in range(n)]
+        for a, b in zip(ens, ens[1:] + ens[:1]):
+            net.Connection(a, b, synapse=mb.Lowpass(0.005))
+            net.Connection(b, a, synapse=mb.Lowpass(0.01))
+        looked_at[0] = 0
+        with Simulator(net, seed=1, event_calibration_steps=0) as sim:
+            assert any("input sums" in p.tag for p in sim._plans)
+        counts.append(looked_at[0])
+    assert counts[1] <= 5 * counts[0], counts
