@@ -288,7 +288,7 @@ int nhip_gemv_tile_lif_deferred(void *stream, int vec, int pow2_cols, int blk_wo
  *   matrices : int32[n][8]  {a_start, a_stride0, M, N, first KB in At, quads = ceil(N / 4), 0, 0}
  * 64 rows by four columns are 1 KB of At (row r % 64, column c % 4 at 16 (r % 64) + 4 (c % 4) bytes), blocks of
  * columns side by side, ceil(M / 64) * quads KB in all; rows and columns past the end are zeros.
- * `max_blocks`: the largest ceil(M / 64).
+ * `max_blocks`: the largest ceil(M / 64); n is 65,535 at most (a grid's limit), here and below.
  *   tasks : int32[n_tasks][40]  the 24 words of nhip_gemv_tile's records (row0 a multiple of 64, at most 64 rows; word 3 and
  *           11: first part and number of parts of the input sum, for a first dot product of at most 64 columns), the
  *           item's row of `pops` (8 words, or 12 for other neuron types; padded to 12), its row of `deferred` (4)

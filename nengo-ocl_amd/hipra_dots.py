@@ -8,7 +8,7 @@ clra_gemv.py:1043-1058, :1148-1153), same results.
 
 import numpy as np
 
-from .hipra_gemv import GROUP_ROW_MIN_COLS, GROUP_ROWS_MAX, _span
+from .hipra_gemv import GROUP_ROW_MIN_COLS, GROUP_ROWS_MAX, _span, lay_out_matrices
 from .hipraggedarray import empty_device, to_device
 
 WG, TILE = 256, 128
@@ -107,8 +107,6 @@ def matrix_spans(plan):
 def lay_out(plan):
     """Make `plan` (for which `matrix_spans` gave spans, of constants) run the kernel that reads copies of its
     matrices.  The plan gets `lay_out_again`, for when the host has changed a matrix."""
-    from . import _lib
-
     queue, lib, prog = plan.queue, plan.queue.lib, plan.prog
     launch = _Launch(plan)
     tiles, quads = _shape(plan)
@@ -153,8 +151,7 @@ def lay_out(plan):
     dev_records = to_device(queue, records)
 
     def again():
-        _lib.check(lib.nhip_lay_out_dots(queue.handle, dev_mats.ptr, len(rows), max_rows, launch.A, dev_at.ptr),
-                   "laying out matrices")
+        lay_out_matrices(lib.nhip_lay_out_dots, queue, dev_mats, len(rows), max_rows, launch.A, dev_at)
 
     again()
     plan.lay_out_again = again

@@ -16,6 +16,7 @@ signature, same ``.plans`` attribute; what differs is the work decomposition:
 For each item b:  ``Y[b] = beta[b]*Y_in[b] + gamma[b] + alpha[b] * sum_j A[A_js[b][j]] @ X[X_js[b][j]]``.
 """
 
+import ctypes
 import logging
 import os
 from collections import defaultdict
@@ -882,6 +883,16 @@ class plan_ref_gemv(gemv_prog):
     """One lane per output element, scalar loads: the plain fallback kernel."""
 
     force_scalar = True
+
+
+LAY_OUT_MATRICES = 65535  # of a launch: its grid has one row each
+
+
+def lay_out_matrices(entry, queue, matrices, n, largest, A, out):
+    """Copies of the `n` matrices of a table of nhip_lay_out_lanes or nhip_lay_out_dots (`entry`)."""
+    for first in range(0, n, LAY_OUT_MATRICES):
+        _lib.check(entry(queue.handle, ctypes.c_void_p(matrices.ptr.value + 32 * first), min(n - first, LAY_OUT_MATRICES),
+                         largest, A, out.ptr), "laying out matrices")
 
 
 def _overlapping(a, b):

@@ -8,7 +8,7 @@ the same order (the reference: clra_gemv.py:1043-1058, :1148-1153), same results
 
 import numpy as np
 
-from .hipra_gemv import N_DIES, _span, formed_sums, spread_over_dies
+from .hipra_gemv import N_DIES, _span, formed_sums, lay_out_matrices, spread_over_dies
 from .hipra_sequence import _conflict
 from .hipraggedarray import empty_device, to_device
 
@@ -212,12 +212,7 @@ def lay_out(plan, formed=None):
     dev_tasks, dev_dots = to_device(queue, tasks), to_device(queue, dots)
 
     def again():
-        lib_check(lib.nhip_lay_out_lanes(queue.handle, dev_mats.ptr, len(rows), max_blocks, launch.A, dev_at.ptr))
-
-    def lib_check(err):
-        from . import _lib
-
-        _lib.check(err, "laying out matrices")
+        lay_out_matrices(lib.nhip_lay_out_lanes, queue, dev_mats, len(rows), max_blocks, launch.A, dev_at)
 
     again()
     plan.lay_out_again = again

@@ -177,3 +177,71 @@ def test_input_sums_are_formed_once(monkeypatch, n, dims):
         parts = tasks[(tasks[:, 11] > 0) & (tasks[:, 1] == 0)][:, 11]
         assert sorted(parts.tolist()) == [1, 1, 2, 4, 4, 4]  # (two of probes)
         assert sorted(set(tasks[tasks[:, 9] == 0][:, 11].tolist())) == [0, 1, 2]
+
+
+def many_matrices(neuron):
+    """Encoders and decoders of seven populations of one launch each."""
+    from nengo_ocl_amd import minibuilder as mb
+
+    net = mb.Network(seed=2, solver="surrogate")
+    stim = net.Node(mb.WhiteSignal(period=0.3, high=8.0, seed=4), size_out=6)
+    probes = []
+    for k in range(7):
+        ens = net.Ensemble(70 + k, 6, neuron_type=neuron())
+        net.Connection(stim, ens, synapse=mb.Lowpass(0.005))
+        probes.append(net.Probe(ens, synapse=0.01))
+    return net, probes
+
+
+@pytest.mark.parametrize("limit", [1, 3, 7])
+def test_matrices_are_laid_out_in_launches_that_hold_them(monkeypatch, limit):
+    from nengo_ocl_amd import hipra_gemv, hipraggedarray, minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    monkeypatch.setenv("NENGO_HIP_RESIDENT", "0")
+    monkeypatch.setattr(hipra_gemv, "LAY_OUT_MATRICES", limit)
+    calls, make = {}, hipraggedarray.Queue
+
+    def queue(device=0):
+        q = make(device)
+
+        class Lib:
+            def __getattr__(self, name, lib=q.lib):
+                entry = getattr(lib, name)
+                if name not in ("nhip_lay_out_lanes", "nhip_lay_out_dots"):
+                    return entry
+
+                def lay_out(handle, matrices, n, *rest):
+                    calls.setdefault(name, []).append((matrices.value, n))
+                    return -1 if n > limit else 0
+
+                return lay_out
+
+        q.lib = Lib()
+        return q
+
+    monkeypatch.setattr(hipraggedarray, "Queue", queue)
+    with Simulator(many_matrices(mb.LIFRate)[0], seed=1):
+        assert set(calls) == {"nhip_lay_out_lanes", "nhip_lay_out_dots"}
+        for made in calls.values():
+            assert sum(n for _, n in made) == 7 and [at - made[0][0] for at, _ in made] == [
+                32 * limit * k for k in range(-(-7 // limit))]
+
+
+@pytest.mark.gpu
+def test_matrices_that_several_launches_lay_out(queue, monkeypatch):
+    from nengo_ocl_amd import hipra_gemv, minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    monkeypatch.setenv("NENGO_HIP_RESIDENT", "0")
+    monkeypatch.setattr(hipra_gemv, "LAY_OUT_MATRICES", 3)
+    (net, probes), (net_o, probes_o) = (many_matrices(mb.LIFRate) for _ in range(2))
+    with Simulator(net, seed=1) as gpu, OracleSimulator(net_o, seed=1) as cpu:
+        assert len([p for p in gpu._plans if p.laid_out is not None]) == 2
+        gpu.run_steps(20)
+        cpu.run_steps(20)
+        for p, p_o in zip(probes, probes_o):
+            assert np.array_equal(gpu.data[p], cpu.data[p_o])
+        assert_same_signals(gpu, cpu)
