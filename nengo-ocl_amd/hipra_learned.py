@@ -144,4 +144,7 @@ def lay_out(plan):
     plan.gsize = (WG * (len(tasks) + n_records) + (carried.gsize[0] if carried is not None else 0),)
     plan.lsize = (WG,)
     plan.tag = "%s, laid out" % plan.tag
+    # (where populations spike densely, listing columns costs more than reading rows: their products are planned
+    # again without, `Simulator._calibrate_event_launches`)
+    plan.event_driven = n_records > 0
     return True

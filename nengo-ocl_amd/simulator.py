@@ -606,12 +606,15 @@ class Simulator:
     # share of a population's neurons that may spike per step before the launch that visits
     # only their columns loses to the dense product (measured on MI355X: 4.4 us with no spikes,
     # 8.7 us at 8 %, 20.3 us at 30 %, 50.3 us at 100 % against 45 us dense, for 256 matrices of
-    # 64 x 4096)
+    # 64 x 4096).  Beside learned rows (`hipra_learned`) the two cross at 0.26 for 3 PES triples of 2000 x 32, 0.28
+    # for 16 and 32 of them, 0.2 for 128, 0.7 for 64; 0.12 for 2 and 16 of 4000 x 64, 0.3 for 100 of 1050 x 20, 0.45
+    # for 64 of 1028 x 32.  Whole steps at 90 %, columns / all of it: 3 x 2000 x 32 25.6 / 14.1 us, 2 x 4000 x 64 78.4 /
+    # 20.6, 64 x 2000 x 32 41.0 / 37.6; the latter at 32 % 30.2 / 38.0
     EVENT_MAX_SPIKING_SHARE = 0.25
 
     def _calibrate_event_launches(self, n_steps):
         """Runs `n_steps` steps, reads the spikes of the populations whose products visit
-        active columns only after each quarter of them, resets; populations that spiked
+        active columns only (in a launch of their own or beside learned rows) after each quarter of them, resets; populations that spiked
         above `EVENT_MAX_SPIKING_SHARE` per step get dense products (the simulator is built
         again around the same model).  Skipped when a plan is a host callback: running the
         model before the user does would show in whatever the callback keeps."""

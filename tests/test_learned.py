@@ -214,3 +214,36 @@ def test_rules_that_share_activities(queue, shared):
             for key in probes:
                 assert np.array_equal(gpu.data[probes[key]], cpu.data[probes_o[key]])
             assert_same_signals(gpu, cpu)
+
+
+def test_launches_that_list_columns_are_looked_at_by_the_calibration(monkeypatch):
+    """... and products of populations that spike densely are not among these columns."""
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    for n in (1050, 2048):  # (either way into the launch)
+        model = network(n, 32)[0].build_model(dt=0.001)
+        with Simulator(None, model=model, seed=1) as sim:
+            assert learning_launch(sim).event_driven and sim.event_calibration is not None
+            sources = sim._event_spike_sources
+        with Simulator(None, model=model, seed=1, _spike_sources_read_whole=sources) as sim:
+            assert not any(getattr(p, "event_driven", False) for p in sim._plans)
+            assert not any(p.laid_out[1][12] for p in sim._plans if getattr(p, "laid_out", None) is not None
+                           and p.laid_out[0].__name__ == "nhip_gemv_learn_events")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1050, 2048])
+def test_populations_that_spike_densely_beside_learned_rows(queue, n):
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    (net, probes), (net_o, probes_o) = (network(n, 32) for _ in range(2))
+    with Simulator(net, dt=0.008, seed=1) as gpu, OracleSimulator(net_o, dt=0.008, seed=1) as cpu:
+        assert gpu.event_calibration["populations_switched_to_dense_products"] > 0, gpu.event_calibration
+        for steps in (1, 20):
+            gpu.run_steps(steps)
+            cpu.run_steps(steps)
+            for p, p_o in zip(probes, probes_o):
+                assert np.array_equal(gpu.data[p], cpu.data[p_o])
+            assert_same_signals(gpu, cpu)
