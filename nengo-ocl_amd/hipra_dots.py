@@ -8,7 +8,7 @@ clra_gemv.py:1043-1058, :1148-1153), same results.
 
 import numpy as np
 
-from .hipra_gemv import GROUP_ROW_MIN_COLS, GROUP_ROWS_MAX, _span, lay_out_matrices
+from .hipra_gemv import GROUP_ROW_MIN_COLS, GROUP_ROWS_MAX, STREAM_FLAT, _span, lay_out_matrices
 from .hipraggedarray import empty_device, to_device
 
 WG, TILE = 256, 128
@@ -25,6 +25,19 @@ EVENT_MAX_BYTES = 20 << 20
 # 84 MB of decoders (80 x 64 x 4096) 32.0 / 34.6 us, 134 MB 48.0 / 53.3, 168 MB 65.5 / 59.1, 268 MB 101 / 89
 MAX_BYTES = 144 << 20
 GROUPS_FOR_FEW_ROWS = 2048  # of groups that are mostly empty
+# Rows of up to 256 columns are padded to 32, 64, 128 or 256 of them, as the launch's widest, and have records of 64
+# bytes.  `_reads_little` says where that pays; what it says no to reads its matrices as they lie.  Whole steps, as
+# they lie / laid out:
+# - small items (four lanes or one per row), up to four columns: 90,000 x 2 11.9 / 11.9 us, 130,000 x 1 11.7 / 12.4,
+#   200,000 x 2 12.6 / 17.2, 1,000,000 x 2 20.8 / 42.1; from five columns on 4,000 of 50 x 5 18.4 / 17.3, 8,000 of
+#   50 x 32 38.7 / 28.2; rows widened by others of the launch: 100 of 50 x 2 beside 10 x 100 11.0 / 11.7, 1,000 of them
+#   12.8 / 14.8 (beside 10 x 250 14.2 / 22.1; 100 of them 12.9 / 11.9)
+# - large items: what is read fits the L2 of the dies (32 MB): 65,000 x 16 12.3 / 8.8, 130,000 x 32 15.9 / 12.7; beyond,
+#   200,000 x 8 14.4 / 17.3, x 32 17.2 / 19.8, x 64 19.2 / 18.2, x 100 28.7 / 25.9, 400,000 x 40 26.9 / 28.3, 130,000 x
+#   68 19.1 / 20.2, x 132 26.6 / 31.5; rows that are not on 16-byte boundaries 200,000 x 15 16.2 / 17.5, x 50 20.4 /
+#   18.0, x 66 41.8 / 26.1
+# Longer rows of up to 144 MB (250 to 1,700 columns, padded to twice that at most) are faster laid out throughout
+SMALL_ITEMS_BYTES, L2_BYTES = 20 << 20, 32 << 20
 
 
 class _Launch:
@@ -88,6 +101,26 @@ def _copy_units(plan, tiles, quads):
     return out
 
 
+def _reads_little(plan, tiles, quads, mats):
+    """Is what the kernel reads of its copies and records little enough, against the matrices as they lie?"""
+    if tiles > 2:
+        return True
+    kind, cols = tuple(plan.kernel_class), max(key[3] for key in mats)
+    read = sum(64 * key[2] * (units + 1) for key, (units, _) in mats.items())
+    useful = sum(4 * key[2] * key[3] for key in mats)
+    if kind[0] == 2:
+        own = sum(64 * key[2] * ((2 if key[3] <= 32 else 4 if key[3] <= 64 else 8 if key[3] <= TILE else 16) + 1)
+                  for key in mats)
+        if read > 2 * own:
+            return cols > TILE and read <= SMALL_ITEMS_BYTES
+        return read <= max(10 * useful, SMALL_ITEMS_BYTES)
+    if read <= L2_BYTES or kind == (3, 0, 1):
+        return True
+    if kind == (3, STREAM_FLAT, 4):
+        return cols > 16
+    return cols > 32 and (2 * read <= 3 * useful or (read - useful <= L2_BYTES and 2 * read <= 5 * useful))
+
+
 def matrix_spans(plan):
     """Intervals of the signal buffer that hold the matrices `lay_out` would copy, or None where the launch does not
     qualify."""
@@ -99,7 +132,7 @@ def matrix_spans(plan):
         return None
     mats = _copy_units(plan, *shape)
     size = sum(64 * key[2] * units for key, (units, _) in mats.items())
-    if size > (EVENT_MAX_BYTES if launch.events else MAX_BYTES):
+    if size > (EVENT_MAX_BYTES if launch.events else MAX_BYTES) or not _reads_little(plan, *shape, mats):
         return None
     return sorted({_span(plan.prog.A, a_j) for _, a_j in mats.values()} - {None})
 

@@ -142,3 +142,33 @@ def test_launches_of_more_than_the_memory_side_cache_holds_read_matrices_as_they
         monkeypatch.setattr(hipra_dots, "MAX_BYTES", limit)
         with Simulator(network(1500, 50)[0], seed=1) as sim:
             assert bool(laid_out(sim)) == expected
+
+
+# rows x columns (x items) of a launch: lane or four lanes per row, streamed on 16-byte boundaries and not, any shape;
+# what its widest matrix makes of the others; on both sides of each limit
+@pytest.mark.parametrize("shapes,expected", [
+    ([(50, 2, 20)], True), ([(105000, 2, 1)], True), ([(115000, 2, 1)], False), ([(2000, 4, 60)], False),
+    ([(50, 5, 3000)], True), ([(100, 2, 10), (10, 30, 1)], True), ([(100, 2, 10), (10, 100, 1)], False),
+    ([(100, 2, 10), (10, 250, 1)], True), ([(500, 2, 50), (10, 250, 1)], False), ([(170000, 8, 1)], True),
+    ([(180000, 8, 1)], False), ([(180000, 32, 1)], False), ([(180000, 15, 1)], False), ([(180000, 31, 1)], True),
+    ([(180000, 40, 1)], True), ([(300000, 40, 1)], False), ([(120000, 68, 1)], False), ([(150000, 100, 1)], True),
+    ([(60000, 132, 1)], False), ([(110000, 66, 1)], True), ([(9000, 520, 1)], True)])
+def test_copies_that_read_much_more_than_their_matrices_are_not_made(monkeypatch, shapes, expected):
+    from nengo_ocl_amd import minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    monkeypatch.setenv("NENGO_HIP_RESIDENT", "0")
+    net = mb.Network(seed=4, solver="surrogate")
+    stim = net.Node(mb.WhiteSignal(period=0.3, high=8.0, seed=4), size_out=1)
+    for m, n, items in shapes:
+        for k in range(items):
+            ens, out = net.Ensemble(n, 1, neuron_type=mb.LIFRate()), net.Node(None, size_in=m)
+            net.Connection(stim, ens, synapse=None)
+            weights = np.broadcast_to(np.float64(k + 1.0), (m, n))
+            net.Connection(ens.neurons, out, transform=weights, synapse=mb.Lowpass(0.005))
+    with Simulator(net, seed=1) as sim:
+        plan, = [p for p in sim._plans if hasattr(p, "prog") and any(
+            d["a_shape1"] == shapes[0][1] and p.prog.geometry[b]["y_len"] == shapes[0][0]
+            for b in p.members for d in p.prog.geometry[b]["dots"])]
+        assert (plan in laid_out(sim)) == expected, (plan.kernel_class, str(plan))
