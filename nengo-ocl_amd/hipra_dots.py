@@ -165,21 +165,23 @@ def lay_out(plan):
         if tiles <= 2:
             full = min([full] + [max(0, min(TILE, N - TILE * t) // 4) for t in range(tiles)])
             most = max(most, -(-min(N, TILE) // 4))
-            for r in range(M):
-                records.append([start + r * units, d["x_start"], N, n_targets, g["y_start"] + r * g["y_stride0"],
-                                g["y_in_start"] + r * g["y_in_stride0"], first, r] + coefs + [0] + target)
-                item_of.append(b)
+            r = np.arange(M)
+            mine = np.empty((M, 16), dtype=np.int32)
+            mine[:] = [start, d["x_start"], N, n_targets, g["y_start"], g["y_in_start"], first, 0] + coefs + [0] + target
+            mine[:, [0, 4, 5, 7]] += np.stack([r * units, r * g["y_stride0"], r * g["y_in_stride0"], r], 1).astype(np.int32)
         else:
-            for r in range(0, M, per_group):
-                records.append([start, units, N, d["x_start"], d["x_stride0"], r, min(per_group, M - r), n_targets,
-                                g["y_start"], g["y_stride0"], g["y_in_start"], g["y_in_stride0"]]
-                               + coefs + [first] + target + [0] * 12)
-                item_of.append(b)
+            r = np.arange(0, M, per_group)
+            mine = np.empty((len(r), 32), dtype=np.int32)
+            mine[:] = [start, units, N, d["x_start"], d["x_stride0"], 0, 0, n_targets, g["y_start"], g["y_stride0"],
+                       g["y_in_start"], g["y_in_stride0"]] + coefs + [first] + target + [0] * 12
+            mine[:, 5], mine[:, 6] = r, np.minimum(per_group, M - r)
+        records.append(mine)
+        item_of.append(np.full(len(mine), b))
     if tiles <= 2:  # whole groups: more of the last row, that store nothing
-        pad = list(records[-1])
-        pad[3] = -1
-        records += [pad] * (-len(records) % per_group)
-    records, item_of = np.array(records, dtype=np.int32), np.array(item_of)
+        pad = np.repeat(records[-1][-1:], -sum(map(len, records)) % per_group, axis=0)
+        pad[:, 3] = -1
+        records.append(pad)
+    records, item_of = np.concatenate(records), np.concatenate(item_of)
     n_groups = len(records) // per_group if tiles <= 2 else len(records)
     dev_records = to_device(queue, records)
 
