@@ -304,6 +304,15 @@ class HIPRaggedArray:
         isz = self.dtype.itemsize
         return np.lib.stride_tricks.as_strided(span, shape=(m, n), strides=(sm * isz, sn * isz))
 
+    def read_vectors(self, items):
+        """Items of one column that lie in whole runs of memory, as host arrays, in one transfer."""
+        if any(int(self.shape1s[i]) != 1 or (int(self.stride0s[i]) != 1 and int(self.shape0s[i]) > 1) for i in items):
+            return [self.read_copy(i).ravel() for i in items]
+        flat, sizes = self.dev_buf.tensor.view(-1), [int(self.shape0s[i]) for i in items]
+        with self.queue.context():
+            both = _torch().cat([flat[int(self.starts[i]):int(self.starts[i]) + n] for i, n in zip(items, sizes)])
+        return np.split(self.queue.read(both), np.cumsum(sizes)[:-1])
+
     def read_copy(self, i):
         """Item ``i`` as a host array of its own that may be written."""
         out = self._read_item(int(i))

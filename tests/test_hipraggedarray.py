@@ -99,3 +99,12 @@ def test_bounds_are_checked_on_the_host(queue, rng):
     bad = HIPRaggedArray.from_buffer(queue, dA.dev_buf, [A.buf.size - 4], [3], [3], [3], [1])
     with pytest.raises(ValueError):
         bad.check_bounds("bad")
+
+
+@pytest.mark.parametrize("items", [[1], [2, 0, 3], [0, 1, 2, 3]])
+def test_vectors_read_together(queue, items):
+    """Vectors in one transfer, and one at a time where one of them is a matrix."""
+    host = RA([np.arange(5.0), np.arange(10.0, 11.0), np.arange(20.0, 27.0), np.arange(6.0).reshape(2, 3)])
+    dev = to_dev(queue, host)
+    for got, i in zip(dev.read_vectors(items), items):
+        assert np.array_equal(got, np.asarray(host[i]).ravel())
