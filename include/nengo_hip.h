@@ -290,14 +290,16 @@ int nhip_gemv_tile_lif_deferred(void *stream, int vec, int pow2_cols, int blk_wo
  * columns side by side, ceil(M / 64) * quads KB in all; rows and columns past the end are zeros.
  * `max_blocks`: the largest ceil(M / 64); n is 65,535 at most (a grid's limit), here and below.
  *   tasks : int32[n_tasks][40]  the 24 words of nhip_gemv_tile's records (row0 a multiple of 64, at most 64 rows; word 3 and
- *           11: first part and number of parts of the input sum, for a first dot product of at most 64 columns), the
+ *           11: first part and number of parts of the input sum, for a first dot product of any of these widths), the
  *           item's row of `pops` (8 words, or 12 for other neuron types; padded to 12), its row of `deferred` (4)
  *   dots  : as for nhip_gemv_tile; here and in the records a_start is the first KB in At, a_stride0 the quads
  * Task 4 g + w is run by wave w of group g; `n_tasks` is a multiple of 4 (tasks of no rows do nothing).  `B` is the
  * buffer of X, Yin, Y, the states and the filters' outputs, which are one here.
- * `neurons`: 1 = LIF, 3 = the types of nhip_gemv_tile_neuron (TAU, REF, AMP are not read).
+ * `neurons`: 1 = LIF, 3 = the types of nhip_gemv_tile_neuron (TAU, REF, AMP are not read); + NHIP_LANES_PAST_CACHE:
+ * matrices are read with non-temporal loads (a step that moves more than the memory-side cache keeps).
  * `parts` (or NULL) as for nhip_gemv_tile_lif_sums, every range padded to a multiple of four with its last part;
  * `mask` as for nhip_gemv_rows_lif_bits. */
+#define NHIP_LANES_PAST_CACHE 16
 int nhip_lay_out_lanes(void *stream, const int *matrices, int n, int max_blocks, const float *A, float *At);
 int nhip_gemv_lanes(void *stream, int neurons, const int *tasks, int n_tasks, const int *dots, const float *At,
                     float *B, double dt, int upsample, const float *TAU, const float *REF, const float *AMP,

@@ -15,9 +15,12 @@
 // Whole steps before (gemv_stream_kernel, gemv_rows_ref_epi_kernel) -> with this kernel: 256 x 4096 x 64 63.9 -> 57.8 us
 // (encoders and neurons: 272 MB in 46 us), 64 triples of 2000 x 32 with learning 44.3 -> 42.5, 48 x 2000 x 32 rate neurons
 // 14.4 -> 11.0, 37 x 1501 x 50 14.5 -> 10.4, 32 x 1000 x 16 adaptive neurons 12.3 -> 9.4, 256 x 100 in a small world
-// 10.7 -> 9.65, 100,000 x 1 with bits for a sparse product 17.7 -> 16.7.  The large ones are bound by what memory gives
-// (loads are ordinary ones: with non-temporal ones, which keep nothing in the memory-side cache, 272 MB of encoders
-// take 3.6 us longer), the others by the chain record -> parts -> x -> update: 2.3 us behind the launch's 0.9.  Two row
+// 10.7 -> 9.65, 100,000 x 1 with bits for a sparse product 17.7 -> 16.7.  The large ones are bound by what memory gives:
+// ordinary loads while the memory-side cache keeps much of the matrices from step to step (whole steps with 268 MB of
+// encoders, 256 x 4096 x 64: 57.7 us, non-temporal 61.1), non-temporal ones (PAST) where a step moves more (302 MB,
+// 288 x 4096 x 64: 71.8 / 67.8, before this kernel 71.9; 512 x 4096 x 64 126.4 / 111.4, 115.4; 2000 x 1000 x 64 129.7 /
+// 116.3, 116.4; 2000 x 4096 x 16 186.5 / 165.2, 196.6; the rule: `hipra_lanes.read_past_the_cache`).  The others
+// are bound by the chain record -> parts -> x -> update: 2.3 us behind the launch's 0.9.  Two row
 // blocks a wave were as fast for 272 MB (58.5) and slower where the launch is short (48 x 2000 x 32 13.1).
 //
 // A wave's task is up to 64 rows of one item.  Everything it needs to start is in its record (item,
@@ -84,7 +87,8 @@ __device__ __forceinline__ void lane_sync() {
 // Task 4 g + w is wave w's of group g (behind the carried chains); the host has put the list into that order for the
 // accelerator dies, and filled the last group up with tasks of no rows.  (With the number of tasks and the grid
 // among the arguments, and those read where they are used, a wave made five dependent reads before its record.)
-template <int EPI, bool SIDE>
+// PAST: matrices are read past the memory-side cache.
+template <int EPI, bool SIDE, bool PAST>
 __global__ __launch_bounds__(NHIP_WG) __attribute__((amdgpu_waves_per_eu(4)))
 void gemv_lanes_kernel(const LaneTask* tasks, const lane_f4* At, float* B, const int2* parts_table, LaneArgs la,
                        RowsSide side)
@@ -208,7 +212,8 @@ void gemv_lanes_kernel(const LaneTask* tasks, const lane_f4* At, float* B, const
 #pragma unroll
             for (int i = 0; i < NQ; ++i) {  // (uniform base, the lane's own 32-bit offset)
                 const int q = i < NQ - 1 ? i : min(i, quads - 1);
-                a[i] = *reinterpret_cast<const lane_f4*>(a0 + ((size_t)(q0 + q) << 10) + lane_off);
+                const lane_f4* at_quad = reinterpret_cast<const lane_f4*>(a0 + ((size_t)(q0 + q) << 10) + lane_off);
+                a[i] = PAST ? __builtin_nontemporal_load(at_quad) : *at_quad;
             }
             first();
             auto step = [&](int i, auto n_cols) LANE_INLINE {
@@ -439,6 +444,8 @@ extern "C" int nhip_gemv_lanes(void* stream, int neurons, const int* tasks, int 
     const int waves = NHIP_WG / NHIP_WAVE;
     if (n_tasks < 0 || n_tasks % waves || !tasks || !dots || !At || !B || upsample < 1 || !(dt > 0.0))
         return NHIP_E_BADARG;
+    const bool past = neurons & NHIP_LANES_PAST_CACHE;
+    neurons &= ~NHIP_LANES_PAST_CACHE;
     if (neurons != EPI_LIF && neurons != EPI_NEURON) return NHIP_E_BADCLASS;
     if (reinterpret_cast<uintptr_t>(At) & 15) return NHIP_E_BADARG;
     LaneArgs args{};
@@ -459,8 +466,8 @@ extern "C" int nhip_gemv_lanes(void* stream, int neurons, const int* tasks, int 
     };
     auto of_type = [&](auto epi) {
         constexpr int E = decltype(epi)::value;
-        if (side.n_chains > 0) launch(gemv_lanes_kernel<E, true>);
-        else launch(gemv_lanes_kernel<E, false>);
+        if (side.n_chains > 0) past ? launch(gemv_lanes_kernel<E, true, true>) : launch(gemv_lanes_kernel<E, true, false>);
+        else past ? launch(gemv_lanes_kernel<E, false, true>) : launch(gemv_lanes_kernel<E, false, false>);
     };
     if (neurons == EPI_LIF) of_type(std::integral_constant<int, EPI_LIF>{});
     else of_type(std::integral_constant<int, EPI_NEURON>{});

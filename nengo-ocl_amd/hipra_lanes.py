@@ -18,6 +18,13 @@ RAW_COLS = 4        # matrices of so many columns are read as they lie in the si
 PARTS = 4           # of an input sum are read together
 TASK_WORDS = 40
 _LIF, _NEURON = 1, 3  # EPI_LIF, EPI_NEURON
+PAST_CACHE = 16     # NHIP_LANES_PAST_CACHE
+# Bytes that the launches of a step move, from which on matrices are read with non-temporal loads: the memory-side
+# cache (256 MB) keeps too little of them until the next step.  Both sides stand at the kernel; they cross between
+# 313 MB (256 x 4096 x 64) and 340 (1000 x 4096 x 16: 94.5 / 86.8 us a step), with a decoder matrix for each of four
+# connections between 297 (192 ensembles: 55.8 / 59.5) and 397 (256: 80.9 / 75.0).  Launches that visit active
+# columns only count a tenth (populations spike in 8 to 11 % of the steps)
+STEP_BYTES, ACTIVE_SHARE = 330e6, 0.1
 _KERNELS = {"nhip_gemv_%s_%s" % k: _NEURON if k[1] == "neuron" else _LIF
             for k in [("tile", "lif"), ("tile", "lif_sums"), ("tile", "lif_deferred"), ("tile", "neuron"),
                       ("rows", "lif"), ("rows", "lif_sums"), ("rows", "neuron")]}
@@ -237,6 +244,17 @@ def lay_out(plan, formed=None):
 
     plan.upload_pops, plan.leave_bits = upload_pops, leave_bits
     return True
+
+
+def read_past_the_cache(plans):
+    """Launches of `lay_out` among the `plans` of a step that moves more than the memory-side cache keeps read their
+    matrices past it."""
+    moved = sum((getattr(p, "bw_per_call", None) or 0) * (ACTIVE_SHARE if getattr(p, "event_driven", False) else 1.0)
+                for p in plans)
+    for plan in plans if moved > STEP_BYTES else ():
+        if getattr(plan, "laid_out", None) is not None and plan.laid_out[0].__name__ == "nhip_gemv_lanes":
+            entry, args = plan.laid_out
+            plan.laid_out = (entry, (args[0] | PAST_CACHE,) + args[1:])
 
 
 def for_the_dies(tasks):

@@ -158,6 +158,9 @@ class HipBackend:
         done = layout.lay_out(plan) if formed is None else layout.lay_out(plan, formed)
         return done, done and formed is not None
 
+    def read_past_the_cache(self, plans):
+        self._layouts[0].read_past_the_cache(plans)
+
     def store_spikes_as_bits(self, enc_plan, items, event_records, dt):
         return self._gemv.store_spikes_as_bits(enc_plan, items, event_records, dt)
 
@@ -795,6 +798,7 @@ class Simulator:
                 plan.bw_per_call = (plan.bw_per_call or 0) + (before.bw_per_call or 0)
                 plan.flops_per_call = (plan.flops_per_call or 0) + (before.flops_per_call or 0)
                 del plans[k - 1]
+        self.backend.read_past_the_cache(plans)
 
     def _constant_written(self, base):
         """The host has changed a constant: the copies of it that launches read follow."""

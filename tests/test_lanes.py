@@ -245,3 +245,43 @@ def test_matrices_that_several_launches_lay_out(queue, monkeypatch):
         for p, p_o in zip(probes, probes_o):
             assert np.array_equal(gpu.data[p], cpu.data[p_o])
         assert_same_signals(gpu, cpu)
+
+
+@pytest.mark.parametrize("limit,past", [(330e6, False), (1e3, True)])
+def test_steps_that_move_more_than_the_cache_keeps_read_past_it(monkeypatch, limit, past):
+    """... all that moves in the step counts, of launches that visit active columns only a part."""
+    from nengo_ocl_amd import configs, hipra_lanes, minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    monkeypatch.setattr(hipra_lanes, "STEP_BYTES", limit)
+    for net in (network(300, 30, mb.LIF)[0], configs.c3_large(n_ens=3, n_neurons=1024, dims=16, fan_out=2)[0]):
+        with Simulator(net, seed=1, event_calibration_steps=0) as sim:
+            kinds = [p.laid_out[1][0] for p in laid_out(sim)]
+            assert kinds and all(k == (1 | 16 if past else 1) for k in kinds)
+            moved = sum((p.bw_per_call or 0) * (0.1 if getattr(p, "event_driven", False) else 1) for p in sim._plans)
+        for share, expected in ((0.5, True), (2.0, False)):
+            monkeypatch.setattr(hipra_lanes, "STEP_BYTES", share * moved)
+            with Simulator(net, seed=1, event_calibration_steps=0) as sim:
+                assert all(bool(p.laid_out[1][0] & 16) == expected for p in laid_out(sim))
+        monkeypatch.setattr(hipra_lanes, "STEP_BYTES", limit)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("neuron", ["LIF", "LIFRate"])
+@pytest.mark.parametrize("n,d", [(65, 4), (200, 5), (129, 8), (301, 30), (129, 64), (260, 65), (65, 128)])
+def test_neurons_whose_encoders_are_read_past_the_cache(queue, monkeypatch, neuron, n, d):
+    from nengo_ocl_amd import hipra_lanes, minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    monkeypatch.setenv("NENGO_HIP_RESIDENT", "0")
+    monkeypatch.setattr(hipra_lanes, "STEP_BYTES", 0)
+    (net, probes), (net_o, probes_o) = (network(n, d, getattr(mb, neuron)) for _ in range(2))
+    with Simulator(net, seed=1) as gpu, OracleSimulator(net_o, seed=1) as cpu:
+        assert laid_out(gpu) and all(p.laid_out[1][0] & 16 for p in laid_out(gpu))
+        gpu.run_steps(25)
+        cpu.run_steps(25)
+        for p, p_o in zip(probes, probes_o):
+            assert np.array_equal(gpu.data[p], cpu.data[p_o])
+        assert_same_signals(gpu, cpu)
