@@ -1616,10 +1616,17 @@ def fuse_learning(enc_plan, dec_plan, ew_plan, lf_plan):
     return new_enc, new_dec, residual, pending
 
 
+# Rows of an item from which on `hipra_learned` visits its active columns: fewer are read whole, four to a group, as
+# learned ones are. Whole steps of PES triples, without that launch / from one row on / from five on: 230 of 1202 x 1
+# 22.3 / 23.3 / 18.9 us, 400 of 1000 x 2 34.4 / 30.8 / 28.0, 60 of 2000 x 4 17.8 / 13.9 / 13.2; 100 of 1500 x 8 20.4 /
+# 16.5 / 16.4, and 19.5 with none of them
+SPIKES_MIN_ROWS = 5
+
+
 def _spikes_item(prog, b):
     """Does `hipra_learned` give item `b` a group that visits active columns?"""
     d = prog.geometry[b]["dots"][0]
-    return b in prog.event_items and EVENT_MIN_COLS <= d["a_shape1"] <= EVENT_MAX_COLS
+    return b in prog.event_items and prog.geometry[b]["y_len"] >= SPIKES_MIN_ROWS and EVENT_MIN_COLS <= d["a_shape1"] <= EVENT_MAX_COLS
 
 
 def fuse_hebbian(products, rule_plan, lf_plan=None, lays_out=False):

@@ -216,6 +216,27 @@ def test_rules_that_share_activities(queue, shared):
             assert_same_signals(gpu, cpu)
 
 
+@pytest.mark.parametrize("dims,columns", [(1, 0), (4, 0), (5, 3), (8, 3)])
+def test_few_rows_are_read_whole(monkeypatch, dims, columns):
+    """... in the groups of learned rows, each of them once."""
+    from nengo_ocl_amd import configs
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    net = configs.c4_pes(1, n_triples=3, n_neurons=1024, dims=dims)[0]
+    with Simulator(net, seed=1, event_calibration_steps=0) as sim:
+        plan, = [p for p in sim._plans if getattr(p, "learned_matrices", 0)]
+        name, args = plan.laid_out[0].__name__ if plan.laid_out else plan.kern.__name__, (plan.laid_out or (0, plan.args))[1]
+        assert name == ("nhip_gemv_learn_events" if columns else "nhip_gemv_learn")
+        # (the others that are applied to spikes: of the errors' inputs and the probes, see `configs.c4_pes`)
+        assert (args[12] if columns else 0) >= columns
+        if not columns:
+            covered = [y + (r + k) * s for y, s, r, c in plan.host_learn[0][:, [4, 5, 11, 12]].tolist() for k in range(c)]
+            assert sorted(covered) == sorted(
+                g["y_start"] + r * g["y_stride0"] for g in (plan.prog.geometry[b] for b in plan.members)
+                for r in range(g["y_len"]))
+
+
 def test_launches_that_list_columns_are_looked_at_by_the_calibration(monkeypatch):
     """... and products of populations that spike densely are not among these columns."""
     from nengo_ocl_amd.simulator import Simulator
