@@ -19,11 +19,14 @@ PARTS = 4           # of an input sum are read together
 TASK_WORDS = 40
 _LIF, _NEURON = 1, 3  # EPI_LIF, EPI_NEURON
 PAST_CACHE = 16     # NHIP_LANES_PAST_CACHE
-# Bytes that the launches of a step move, from which on matrices are read with non-temporal loads: the memory-side
-# cache (256 MB) keeps too little of them until the next step.  Both sides stand at the kernel; they cross between
-# 313 MB (256 x 4096 x 64) and 340 (1000 x 4096 x 16: 94.5 / 86.8 us a step), with a decoder matrix for each of four
-# connections between 297 (192 ensembles: 55.8 / 59.5) and 397 (256: 80.9 / 75.0).  Launches that visit active
-# columns only count a tenth (populations spike in 8 to 11 % of the steps)
+# Bytes that the launches of a step move through the memory-side cache (256 MB), from which on it keeps too little of
+# the matrices until the next step: they are read with non-temporal loads then.  Both sides stand at the kernel; they
+# cross between 317 MB (256 x 4096 x 64: 57.7 / 61.1 us a step) and 350 (1000 x 4096 x 16: 94.5 / 86.8; 288 x 4096 x
+# 64: 71.8 / 67.8), with a decoder for each of four connections between 303 (192 ensembles: 55.8 / 59.5) and 401 (256:
+# 80.9 / 75.0).  Launches that visit active columns only count a tenth (populations spike in 8 to 11 % of the steps),
+# those of csrc/gemv_tile.hip, whose loads are non-temporal, only where they write matrices: every column of 256 x
+# 4096 x 64 multiplied 92.1 / 96.6, 320 of them 124.2 / 118.2; rate neurons 272 x 4096 x 64 94.6 / 96.3, 330 of them 122.0 /
+# 114.7; PES 300 of 2000 x 32 128.1 / 119.0
 STEP_BYTES, ACTIVE_SHARE = 330e6, 0.1
 _KERNELS = {"nhip_gemv_%s_%s" % k: _NEURON if k[1] == "neuron" else _LIF
             for k in [("tile", "lif"), ("tile", "lif_sums"), ("tile", "lif_deferred"), ("tile", "neuron"),
@@ -249,8 +252,10 @@ def lay_out(plan, formed=None):
 def read_past_the_cache(plans):
     """Launches of `lay_out` among the `plans` of a step that moves more than the memory-side cache keeps read their
     matrices past it."""
-    moved = sum((getattr(p, "bw_per_call", None) or 0) * (ACTIVE_SHARE if getattr(p, "event_driven", False) else 1.0)
-                for p in plans)
+    share = lambda p: (ACTIVE_SHARE if getattr(p, "event_driven", False) else
+                       0.0 if getattr(getattr(p, "kern", None), "__name__", "").startswith("nhip_gemv_tile")
+                       and getattr(p, "laid_out", None) is None and not getattr(p, "learned_matrices", 0) else 1.0)
+    moved = sum((getattr(p, "bw_per_call", None) or 0) * share(p) for p in plans)
     for plan in plans if moved > STEP_BYTES else ():
         if getattr(plan, "laid_out", None) is not None and plan.laid_out[0].__name__ == "nhip_gemv_lanes":
             entry, args = plan.laid_out

@@ -267,6 +267,27 @@ def test_steps_that_move_more_than_the_cache_keeps_read_past_it(monkeypatch, lim
         monkeypatch.setattr(hipra_lanes, "STEP_BYTES", limit)
 
 
+def test_matrices_read_past_the_cache_do_not_count(monkeypatch):
+    """Decoders of rate neurons that keep the launch with non-temporal loads."""
+    from nengo_ocl_amd import hipra_dots, hipra_lanes, minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    monkeypatch.setattr(hipra_dots, "MAX_BYTES", 0)
+    net = mb.Network(seed=2, solver="surrogate")
+    ens = [net.Ensemble(1024, 64, neuron_type=mb.LIFRate()) for _ in range(40)]
+    for a, b in zip(ens, ens[1:] + ens[:1]):
+        net.Connection(a, b, synapse=mb.Lowpass(0.005))
+    with Simulator(net, seed=1) as sim:
+        own = sum(p.bw_per_call for p in laid_out(sim))
+        others = sum(p.bw_per_call for p in sim._plans if p.name == "hipra_gemv.tile_filter" and p.laid_out is None)
+    assert others > 0.5 * own > 0
+    for limit, expected in ((1.4 * own, False), (0.9 * own, True)):
+        monkeypatch.setattr(hipra_lanes, "STEP_BYTES", limit)
+        with Simulator(net, seed=1) as sim:
+            assert all(bool(p.laid_out[1][0] & 16) == expected for p in laid_out(sim))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("neuron", ["LIF", "LIFRate"])
 @pytest.mark.parametrize("n,d", [(65, 4), (200, 5), (129, 8), (301, 30), (129, 64), (260, 65), (65, 128)])
