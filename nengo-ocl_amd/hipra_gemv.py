@@ -133,8 +133,9 @@ SUM_PARTS_FOR_WAVE_TASKS, SUM_MIN_ROWS_FOR_WAVE_TASKS = 3, 3000
 # 1,000 x 700 26.7 / 33.6, three of 2,100 x 300 19.3 / 23.3. Of 208 networks drawn at random (up to 1,800 groups of 4
 # to 2,500 columns) one is faster apart
 LEARN_GROUP_US = 0.011
-# Outer products of fewer columns keep a launch for the rule and its filters (its tests are at 300 columns; nothing is
-# won by it). Whole steps with and without, us: 3 triples of 300 x 8 13.5 / 9.0, 20 of 250 x 14 16.2 / 9.7, 30 of 500 x 4
+# Outer products of fewer columns keep the launches that they had (`fuse_learning`, `_fuse_outer_filters`).  The two do
+# not cross here: one launch is shorter at every size measured, and the line could lie lower.  Whole steps with and
+# without launches of their own, us: 3 triples of 300 x 8 13.5 / 9.0, 20 of 250 x 14 16.2 / 9.7, 30 of 500 x 4
 # 17.1 / 9.1, 10 of 500 x 10 17.4 / 9.1, 4 of 1000 x 4 11.3 / 9.6, 372 x 36 16.2 / 9.3, 40 of 1028 x 7 14.3 / 10.6, 2 of
 # 2000 x 50 16.4 / 12.3
 OUTER_MIN_COLS = 320

@@ -1033,7 +1033,8 @@ class Simulator:
             rule = plans[r]
             r += 1
             outer = getattr(rule, "ew_spec", None) or {}
-            # (what may fit the resident launch, which holds no such products, keeps its launches)
+            # (networks of the resident launch's size keep the launches they had; none of them is resident: their
+            # matrices have a copy for the host, `_plan_host_view`)
             outer = outer.get("outer") and outer.get("inc") and not may_be_resident and hasattr(
                 self.backend, "fuse_learning")
             if not outer and not (getattr(rule, "rule_spec", None) or {}).get("inc"):
