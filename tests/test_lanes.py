@@ -306,3 +306,26 @@ def test_neurons_whose_encoders_are_read_past_the_cache(queue, monkeypatch, neur
         for p, p_o in zip(probes, probes_o):
             assert np.array_equal(gpu.data[p], cpu.data[p_o])
         assert_same_signals(gpu, cpu)
+
+
+@pytest.mark.parametrize("several,others,expected", [(1, 4, True), (2, 2, True), (3, 2, False), (4, 0, False)])
+def test_small_items_with_several_products_keep_their_launch(monkeypatch, several, others, expected):
+    from nengo_ocl_amd import minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+
+    host_simulators(monkeypatch)
+    monkeypatch.setenv("NENGO_HIP_RESIDENT", "0")
+    net = mb.Network(seed=1, solver="surrogate")
+    stim = net.Node(mb.WhiteSignal(period=0.3, high=8.0, seed=4), size_out=2)
+    sources = [net.Ensemble(3, 1, neuron_type=mb.LIFRate()) for _ in range(3)]
+    for k in range(several + others):
+        ens = net.Ensemble(200 + k, 2)
+        net.Connection(stim, ens, synapse=mb.Lowpass(0.005))
+        for source in sources if k < several else ():
+            net.Connection(source.neurons, ens.neurons, transform=np.full((200 + k, 3), 1e-3), synapse=None)
+    with Simulator(net, seed=1, event_calibration_steps=0) as sim:
+        plan, = [p for p in sim._plans if getattr(p, "name", "") == "hipra_gemv.wave_ref_lif"
+                 and any(p.prog.geometry[b]["y_len"] >= 200 for b in p.members)]
+        counts = [len(plan.prog.geometry[b]["dots"]) for b in plan.members]
+        assert sum(c > 1 for c in counts) == several
+        assert (plan.laid_out is not None) == expected
