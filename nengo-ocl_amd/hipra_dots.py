@@ -36,6 +36,9 @@ GROUPS_FOR_FEW_ROWS = 2048  # of groups that are mostly empty
 #   200,000 x 8 14.4 / 17.3, x 32 17.2 / 19.8, x 64 19.2 / 18.2, x 100 28.7 / 25.9, 400,000 x 40 26.9 / 28.3, 130,000 x
 #   68 19.1 / 20.2, x 132 26.6 / 31.5; rows that are not on 16-byte boundaries 200,000 x 15 16.2 / 17.5, x 50 20.4 /
 #   18.0, x 66 41.8 / 26.1
+# - ... without filters, where rows as they lie are read faster: 40,000 x 128 20.1 / 16.6, 32 of 2000 x 128 22.1 / 24.4,
+#   80 of 2000 x 51 23.4 / 25.4, 64,000 x 200 25.9 / 29.3, 8 of 8000 x 256 26.1 / 28.0; not on 16-byte boundaries 40 of
+#   2000 x 66 28.0 / 25.6
 # Longer rows of up to 144 MB (250 to 1,700 columns, padded to twice that at most) are faster laid out throughout
 SMALL_ITEMS_BYTES, L2_BYTES = 20 << 20, 32 << 20
 
@@ -101,7 +104,7 @@ def _copy_units(plan, tiles, quads):
     return out
 
 
-def _reads_little(plan, tiles, quads, mats):
+def _reads_little(plan, filtered, tiles, quads, mats):
     """Is what the kernel reads of its copies and records little enough, against the matrices as they lie?"""
     if tiles > 2:
         return True
@@ -116,6 +119,8 @@ def _reads_little(plan, tiles, quads, mats):
         return read <= max(10 * useful, SMALL_ITEMS_BYTES)
     if read <= L2_BYTES or kind == (3, 0, 1):
         return True
+    if not filtered:
+        return False
     if kind == (3, STREAM_FLAT, 4):
         return cols > 16
     return cols > 32 and (2 * read <= 3 * useful or (read - useful <= L2_BYTES and 2 * read <= 5 * useful))
@@ -132,7 +137,8 @@ def matrix_spans(plan):
         return None
     mats = _copy_units(plan, *shape)
     size = sum(64 * key[2] * units for key, (units, _) in mats.items())
-    if size > (EVENT_MAX_BYTES if launch.events else MAX_BYTES) or not _reads_little(plan, *shape, mats):
+    if size > (EVENT_MAX_BYTES if launch.events else MAX_BYTES) or not _reads_little(
+            plan, launch.targets is not None, *shape, mats):
         return None
     return sorted({_span(plan.prog.A, a_j) for _, a_j in mats.values()} - {None})
 

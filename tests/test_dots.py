@@ -154,6 +154,17 @@ def test_launches_of_more_than_the_memory_side_cache_holds_read_matrices_as_they
     ([(180000, 40, 1)], True), ([(300000, 40, 1)], False), ([(120000, 68, 1)], False), ([(150000, 100, 1)], True),
     ([(60000, 132, 1)], False), ([(110000, 66, 1)], True), ([(9000, 520, 1)], True)])
 def test_copies_that_read_much_more_than_their_matrices_are_not_made(monkeypatch, shapes, expected):
+    check_layout(monkeypatch, shapes, expected, 0.005)
+
+
+@pytest.mark.parametrize("shapes,expected", [
+    ([(50000, 128, 1)], True), ([(64000, 128, 1)], False), ([(2000, 51, 40)], True), ([(2000, 51, 60)], False),
+    ([(27000, 200, 1)], True), ([(40000, 200, 1)], False), ([(2000, 66, 40)], True), ([(64, 4096, 40)], True)])
+def test_large_copies_are_not_made_for_launches_without_filters(monkeypatch, shapes, expected):
+    check_layout(monkeypatch, shapes, expected, None)
+
+
+def check_layout(monkeypatch, shapes, expected, synapse):
     from nengo_ocl_amd import minibuilder as mb
     from nengo_ocl_amd.simulator import Simulator
 
@@ -166,7 +177,8 @@ def test_copies_that_read_much_more_than_their_matrices_are_not_made(monkeypatch
             ens, out = net.Ensemble(n, 1, neuron_type=mb.LIFRate()), net.Node(None, size_in=m)
             net.Connection(stim, ens, synapse=None)
             weights = np.broadcast_to(np.float64(k + 1.0), (m, n))
-            net.Connection(ens.neurons, out, transform=weights, synapse=mb.Lowpass(0.005))
+            net.Connection(ens.neurons, out, transform=weights, synapse=synapse)
+            net.Probe(out[:1], synapse=0.01)
     with Simulator(net, seed=1) as sim:
         plan, = [p for p in sim._plans if hasattr(p, "prog") and any(
             d["a_shape1"] == shapes[0][1] and p.prog.geometry[b]["y_len"] == shapes[0][0]
