@@ -9,9 +9,9 @@
 // have read its activities steps the filters.
 //
 // 2000 x 2000: 13.9 -> 9.1 us (counters of arrivals: 9.8; nothing requested behind a wait or a condition: 9.1; in a
-// kernel trace of whole calls 10.0), whole steps 24.8 -> 19.0.  What is left, from the first group's start: record 0.5, vectors at 2.3, rows at 3.1 (5 TB/s
-// from there to the last), rule and stores 1.1, sums 1.1 (both as long as LDS takes for 40 KB a wave's
-// row), last group's filters 1.6.  A plain kernel that reads and writes 16.8 MB takes 4.4 us of a launch.
+// kernel trace of whole calls 10.0), whole steps 24.8 -> 19.0.  What is left, from the first group's start: record 0.5,
+// vectors at 2.3, rows at 3.1 (5 TB/s from there to the last), rule and stores 1.1, sums 1.1 (both as long as LDS
+// takes for 40 KB a wave's row), last group's filters 1.6.  A plain kernel that reads and writes 16.8 MB takes 4.4 us of a launch.
 //
 // A row in LDS lies in tiles of 128 columns, 132 words apart: the sum of a tile is four strided
 // partial sums (clra_gemv.py:1043-1058, :1148-1153), a lane each, sixteen tiles side by side, and
@@ -61,6 +61,7 @@ constexpr int LCOUNTERS = 32, LCOUNTER_WORDS = 32;  // counters of arrivals (and
 typedef float learn_f4 __attribute__((ext_vector_type(4)));
 typedef float learn_q4 __attribute__((ext_vector_type(4), aligned(4)));  // at any element of a row
 typedef int learn_i16 __attribute__((ext_vector_type(16)));
+typedef int learn_i8 __attribute__((ext_vector_type(8)));
 #define LEARN_INLINE __attribute__((always_inline))
 
 // LDS written by some lanes of a wave is read by others
@@ -430,64 +431,95 @@ __global__ __launch_bounds__(NHIP_WG) void gemv_learn_kernel(
     }
     const bool own = task.own_groups > 0;  // activities of its item's groups alone: their last one replaces those
     if (!own && n_filters == 0) return;
+    typedef const __attribute__((address_space(4))) learn_i8 const_i8;
+    learn_i8 f2 = learn_i8{}, f3 = learn_i8{};
+    if (n_filters > 2) {
+        const const_i8* more = reinterpret_cast<const const_i8*>(reinterpret_cast<uintptr_t>(filters));
+        f2 = more[2];
+        f3 = more[min(3, n_filters - 1)];
+    }
     __syncthreads();
     if (lds.last == 0) return;
     struct TwoFilters { LearnFilter a, b; };
     const TwoFilters here = __builtin_bit_cast(TwoFilters, fw);
-    auto step = [&](const LearnFilter& fa, const LearnFilter& fb) LEARN_INLINE {  // in quads
-        constexpr int U = 2;  // quads of a thread requested together, of each filter
+    // Q filters by T threads, of which this one is t: in quads, and what is left behind the last quad an element a
+    // thread; all of it requested together.
+    auto step = [&](const auto& f, int t, auto threads) LEARN_INLINE {
+        constexpr int T = decltype(threads)::value, U = 2;  // quads of a thread, of each filter
+        constexpr int Q = sizeof(f) / sizeof(f[0]);
         const auto stepped = [](const LearnFilter& f, float s, float old) LEARN_INLINE {
             const float bx = __fmul_rn(f.b, s);
             return f.has_a ? __fsub_rn(bx, __fmul_rn(f.a, old)) : bx;
         };
-        const auto element = [&](const LearnFilter& f) LEARN_INLINE {  // behind the last quad
-            const int i = (f.n & ~3) + tid;
-            if (i < f.n) {
-                float* F = filter.F + f.f_start + (size_t)i;
-                *F = stepped(f, X[f.s_start + (size_t)i], *F);
+        float st[Q], vt[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int i = (f[q].n & ~3) + t;
+            st[q] = vt[q] = 0.0f;
+            if (i < f[q].n) {
+                st[q] = X[f[q].s_start + (size_t)i];
+                vt[q] = filter.F[f[q].f_start + (size_t)i];
             }
-        };
-        for (int i0 = 4 * tid; i0 < max(fa.n, fb.n); i0 += 4 * U * NHIP_WG) {
-            learn_f4 sa[U], va[U], sb[U], vb[U];
-            const auto request = [&](const LearnFilter& f, learn_f4 (&s)[U], learn_f4 (&v)[U]) LEARN_INLINE {
+        }
+        int longest = 0;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) longest = max(longest, f[q].n);
+        for (int i0 = 4 * t; i0 < longest; i0 += 4 * U * T) {
+            learn_f4 s[Q][U], v[Q][U];
+#pragma unroll
+            for (int q = 0; q < Q; ++q)
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    const int i = i0 + 4 * u * NHIP_WG;
-                    s[u] = v[u] = learn_f4{};
-                    if (i + 4 <= f.n) {
-                        s[u] = *reinterpret_cast<const learn_q4*>(X + f.s_start + (size_t)i);
-                        v[u] = *reinterpret_cast<const learn_q4*>(filter.F + f.f_start + (size_t)i);
+                    const int i = i0 + 4 * u * T;
+                    s[q][u] = v[q][u] = learn_f4{};
+                    if (i + 4 <= f[q].n) {
+                        s[q][u] = *reinterpret_cast<const learn_q4*>(X + f[q].s_start + (size_t)i);
+                        v[q][u] = *reinterpret_cast<const learn_q4*>(filter.F + f[q].f_start + (size_t)i);
                     }
                 }
-            };
-            const auto replace = [&](const LearnFilter& f, const learn_f4 (&s)[U], const learn_f4 (&v)[U]) LEARN_INLINE {
+#pragma unroll
+            for (int q = 0; q < Q; ++q)
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    const int i = i0 + 4 * u * NHIP_WG;
-                    if (i + 4 <= f.n) {
+                    const int i = i0 + 4 * u * T;
+                    if (i + 4 <= f[q].n) {
                         learn_f4 y;
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) y[e] = stepped(f, s[u][e], v[u][e]);
-                        *reinterpret_cast<learn_q4*>(filter.F + f.f_start + (size_t)i) = y;
+                        for (int e = 0; e < 4; ++e) y[e] = stepped(f[q], s[q][u][e], v[q][u][e]);
+                        *reinterpret_cast<learn_q4*>(filter.F + f[q].f_start + (size_t)i) = y;
                     }
                 }
-            };
-            request(fa, sa, va);
-            request(fb, sb, vb);
-            replace(fa, sa, va);
-            replace(fb, sb, vb);
         }
-        element(fa);
-        element(fb);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int i = (f[q].n & ~3) + t;
+            if (i < f[q].n) filter.F[f[q].f_start + (size_t)i] = stepped(f[q], st[q], vt[q]);
+        }
     };
-    if (own) {
-        step(filters[task.own_filter], LearnFilter{});
+    // The first two or four (the activities of both sides, the BCM rule's third) by all threads, the others by a wave
+    // each.  (Two after the other by all threads, elements behind the last quad after those: 18 filters of up to 257
+    // elements beside 21 groups, the launch 17.0 us, now 8.6; whole steps of the BCM rule on 2000 x 2000 14.5 -> 12.7,
+    // on 92 x 92 9.5 -> 8.7, of Oja's 12.9 -> 12.3 and 8.7 -> 8.5.  With the records of more than two filters
+    // requested at the kernel's begin 12.9, 8.9, 12.5, 8.7.)
+    constexpr std::integral_constant<int, NHIP_WG> group_threads{};
+    if (own || n_filters <= 2) {
+        LearnFilter both[2] = {here.a, here.b};
+        if (own) both[0] = filters[task.own_filter];
+        if (own || n_filters < 2) both[1].n = 0;
+        step(both, tid, group_threads);
         return;
     }
-    for (int k = 0; k < n_filters; k += 2) {  // two at a time (the activities of both sides)
-        LearnFilter fb = k == 0 ? here.b : filters[min(k + 1, n_filters - 1)];
-        if (k + 1 >= n_filters) fb.n = 0;
-        step(k == 0 ? here.a : filters[k], fb);
+    LearnFilter first[4] = {here.a, here.b, __builtin_bit_cast(LearnFilter, f2), __builtin_bit_cast(LearnFilter, f3)};
+    if (n_filters < 4) first[3].n = 0;
+    step(first, tid, group_threads);
+    for (int k = 4 + wave; k < n_filters; k += 4 * LROWS) {
+        LearnFilter more[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            more[q] = filters[min(k + q * LROWS, n_filters - 1)];
+            if (k + q * LROWS >= n_filters) more[q].n = 0;
+        }
+        step(more, lane, std::integral_constant<int, NHIP_WAVE>{});
     }
 }
 

@@ -268,3 +268,40 @@ def test_populations_that_spike_densely_beside_learned_rows(queue, n):
             for p, p_o in zip(probes, probes_o):
                 assert np.array_equal(gpu.data[p], cpu.data[p_o])
             assert_same_signals(gpu, cpu)
+
+
+# two and three filters of the rules and others of any length: all threads, waves with one to four each, two rounds of them
+@pytest.mark.gpu
+@pytest.mark.parametrize("rule", ["Oja", "BCM"])
+@pytest.mark.parametrize("sizes", [[], [1], [3, 70], [5, 64, 257, 30], [1030] + [2, 33, 257, 7] * 2, [9, 260, 2100, 61] * 5])
+def test_filters_behind_the_last_reader(queue, rule, sizes):
+    from nengo_ocl_amd import minibuilder as mb
+    from nengo_ocl_amd.simulator import Simulator
+    from oracle.oracle_sim import OracleSimulator
+
+    def make():
+        rng = np.random.RandomState(3)
+        net = mb.Network(seed=5, solver="surrogate")
+        stim = net.Node(mb.WhiteSignal(period=0.5, high=6.0, seed=3), size_out=2)
+        pre, post = net.Ensemble(130, 2), net.Ensemble(101, 2)
+        net.Connection(stim, pre, synapse=None)
+        learning = mb.Oja(learning_rate=1e-6, beta=0.7) if rule == "Oja" else mb.BCM(learning_rate=1e-9)
+        net.Connection(pre.neurons, post.neurons, transform=rng.normal(scale=1e-3, size=(101, 130)),
+                       learning_rule=learning, synapse=mb.Lowpass(0.005))
+        probes = [net.Probe(post.neurons, sample_every=0.005)]
+        for k, n in enumerate(sizes):
+            ens = net.Ensemble(n, 2)
+            net.Connection(stim, ens, synapse=None)
+            probes.append(net.Probe(ens.neurons, synapse=mb.Lowpass(0.002 + 0.001 * k), sample_every=0.005))
+        return net, probes
+
+    (net, probes), (net_o, probes_o) = make(), make()
+    with Simulator(net, seed=1) as gpu, OracleSimulator(net_o, seed=1) as cpu:
+        plan, = [p for p in gpu._plans if getattr(p, "learned_matrices", 0)]
+        assert plan.args[9] == (2 if rule == "Oja" else 3) + len(sizes)
+        for steps in (1, 30):
+            gpu.run_steps(steps)
+            cpu.run_steps(steps)
+            for p, p_o in zip(probes, probes_o):
+                assert np.array_equal(gpu.data[p], cpu.data[p_o])
+            assert_same_signals(gpu, cpu)
