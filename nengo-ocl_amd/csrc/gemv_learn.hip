@@ -9,7 +9,7 @@
 // have read its activities steps the filters.
 //
 // 2000 x 2000: 13.9 -> 9.1 us (counters of arrivals: 9.8; nothing requested behind a wait or a condition: 9.1; in a
-// kernel trace of whole calls 10.0), whole steps 24.8 -> 19.0.  What is left, from the first group's start: record 0.5,
+// kernel trace of whole calls 9.5), whole steps 24.8 -> 19.0.  What is left, from the first group's start: record 0.5,
 // vectors at 2.3, rows at 3.1 (5 TB/s from there to the last), rule and stores 1.1, sums 1.1 (both as long as LDS
 // takes for 40 KB a wave's row), last group's filters 1.6.  A plain kernel that reads and writes 16.8 MB takes 4.4 us of a launch.
 //
